@@ -1,0 +1,250 @@
+"""The state plan: its host arrays executed in numpy against the oracle (CPU),
+and the kernels on it against the oracle at the edges of their tiles, rows and
+windows (GPU).
+
+Tolerances, of each output's largest |value|: sums of at most 1e5 terms with
+one rounding each (1.1e-16) and cancelling partial sums at most 1e3 times the
+result stay below 1e-8."""
+import numpy as np
+import pytest
+
+import cases
+import tskit_amd as ta
+from oracle.oracle import Oracle
+
+TOL = 1e-8
+
+
+def from_parents(parents, times, samples, L=100.0):
+    """Tables of the trees given by one parent array each."""
+    T = len(parents)
+    bp = np.linspace(0, L, T + 1)
+    rows = []
+    for u in range(len(times)):
+        t = 0
+        while t < T:
+            p, e = parents[t][u], t + 1
+            while e < T and parents[e][u] == p:
+                e += 1
+            if p >= 0:
+                rows.append((bp[t], bp[e], p, u))
+            t = e
+    tc = ta.TableCollection(L)
+    flags = np.zeros(len(times), np.uint32)
+    flags[list(samples)] = 1
+    tc.set_nodes(flags, times)
+    a = np.array(rows)
+    tc.set_edges(a[:, 0], a[:, 1], a[:, 2].astype(np.int32), a[:, 3].astype(np.int32))
+    tc.sort_edges()
+    pos = bp[:-1] + 0.25 * (bp[1] - bp[0])
+    tc.site_position = pos
+    tc.ancestral_state = np.full(T, ord("0"), np.int8)
+    tc.ancestral_state_offset = np.arange(T + 1, dtype=np.uint64)
+    tc.mutation_site = np.arange(T, dtype=np.int32)
+    tc.mutation_node = np.array([t % len(times) for t in range(T)], np.int32)
+    tc.mutation_parent = np.full(T, -1, np.int32)
+    tc.derived_state = np.full(T, ord("1"), np.int8)
+    tc.derived_state_offset = np.arange(T + 1, dtype=np.uint64)
+    return tc
+
+
+def bushy(n=70, trees=60, seed=3):
+    """Nodes of many children that come and go, an internal sample, unary
+    nodes, samples without a parent."""
+    rng = np.random.default_rng(seed)
+    A, B, U, R = n, n + 1, n + 2, n + 3
+    times = np.concatenate([np.zeros(n), [1.0, 1.5, 2.0, 3.0]])
+    cur = rng.choice([A, B, U, R], n)
+    parents = []
+    for _ in range(trees):
+        for s in rng.choice(n, 4, replace=False):
+            cur[s] = rng.choice([A, B, U, R, -1])
+        parents.append(np.concatenate([cur, [U, R, R, -1]]))
+    return from_parents(parents, times, list(range(n)) + [B])
+
+
+def caterpillar(n=700):
+    """One ladder of n samples, then its two youngest rungs swapped."""
+    times = np.concatenate([np.zeros(n), np.arange(1, n)])
+    par = np.full(2 * n - 1, -1)
+    par[0] = n
+    par[1:n] = np.arange(n, 2 * n - 1)
+    par[n:2 * n - 2] = np.arange(n + 1, 2 * n - 1)
+    other = par.copy()
+    other[[2, 3]] = other[[3, 2]]
+    return from_parents([par, other], times, range(n))
+
+
+INPUTS = {
+    "paper": cases.paper_ex,
+    "single_tree": cases.single_tree_ex,
+    "nonbinary": cases.nonbinary_ex,
+    "generated": lambda: cases.generated(300, 3e5, 11),
+    "gapped": lambda: cases.gapped(120, 2e5, 12),
+    "multiallelic": lambda: cases.multiallelic(150, 2e5, 13),
+    "bushy": bushy,
+}
+
+
+def sets_of(ts, k, seed):
+    perm = np.random.default_rng(seed).permutation(ts.samples())
+    return [np.sort(x).astype(np.int32) for x in np.array_split(perm, k)]
+
+
+def counts(plan, n, sets, sample_index):
+    x = np.zeros((plan["states"], len(sets)), np.int64)
+    for k, s in enumerate(sets):
+        x[1 + sample_index[s], k] = 1
+    lev = plan["level0"]
+    assert lev[0] == 0 and lev[1] == 1 + n and lev[-1] == plan["states"]
+    for l in range(1, len(lev) - 1):
+        ins = plan["inputs"][lev[l] - 1 - n:lev[l + 1] - 1 - n]
+        assert ins.min() >= 0 and ins.max() < lev[l]  # of earlier levels
+        x[lev[l]:lev[l + 1]] = x[ins].sum(axis=1)
+    return x
+
+
+def summary(stat, x, size, i, j):
+    if stat == "diversity":
+        return x[:, i] * (size[i] - x[:, i]) / (size[i] * (size[i] - 1))
+    if stat == "divergence":
+        return x[:, i] * (size[j] - x[:, j]) / (size[i] * size[j])
+    return x[:, i] * x[:, j] / (size[i] * size[j])  # non-centred relatedness
+
+
+@pytest.mark.parametrize("name", list(INPUTS))
+@pytest.mark.parametrize("polarised", [False, True])
+def test_state_plan_executes_to_oracle(name, polarised):
+    tc = INPUTS[name]()
+    ts = tc.tree_sequence()
+    plan = ts.ll_tree_sequence.get_state_plan()
+    assert plan["usable"]
+    n, L = ts.num_samples, ts.sequence_length
+    index = np.full(ts.num_nodes, -1)
+    index[ts.samples()] = np.arange(n)
+    sets = sets_of(ts, 2, 5)
+    size = np.array([len(s) for s in sets], dtype=float)
+    x = counts(plan, n, sets, index).astype(float)
+    assert np.all(np.diff(plan["ev_pos"]) >= 0) and np.all(np.diff(plan["row_pos"]) >= 0)
+    assert np.all((plan["ev_state"] >= 0) & (plan["ev_state"] < plan["states"]))
+    orc = Oracle(tc)
+    win = np.array([0, 0.21 * L, 0.5 * L, 0.77 * L, L])
+    for stat, ij in [("diversity", (0, 0)), ("divergence", (0, 1)), ("nc", (0, 1))]:
+        if size[ij[0]] < 2:
+            continue
+        one = stat == "diversity"
+        name_ = "genetic_relatedness" if stat == "nc" else stat
+        kw = dict(centre=False) if stat == "nc" else {}
+
+        def F(v):
+            return summary(stat, v, size, *ij)
+
+        for mode in ("branch", "site"):
+            exp = orc.stat(name_, sets, None if one else [ij], win, mode, polarised=polarised,
+                           span_normalise=False, **kw)[:, 0]
+            got = np.zeros(4)
+            if mode == "branch":
+                v = x[plan["ev_state"]]
+                f = plan["ev_b"] * (F(v) if polarised else F(v) + F(size - v))
+                w = np.clip(np.searchsorted(win, plan["ev_pos"], side="right") - 1, 0, 3)
+                got = np.bincount(w, f * (win[w + 1] - plan["ev_pos"]), 4)
+                jump = np.concatenate([[0], np.cumsum(np.bincount(w, f, 4))[:-1]])
+                got = got + jump * np.diff(win)
+            else:
+                for r, pos in zip(plan["row_ref"], plan["row_pos"]):
+                    w = np.searchsorted(win, pos, side="right") - 1
+                    if r >= 0:
+                        v = x[r:r + 1]
+                        got[w] += (F(v) if polarised else F(v) + F(size - v))[0]
+                        continue
+                    ent = plan["list_ent"][plan["list_off"][-1 - r]:plan["list_off"][-r]]
+                    anc = plan["list_kind"][-1 - r] == 2
+                    v = (size if anc else 0) + sum(
+                        (-1 if e & 1 else 1) * x[e >> 1] for e in ent)
+                    v = np.broadcast_to(v, (1, 2)).astype(float)
+                    if not (anc and polarised):
+                        got[w] += F(v)[0]
+            scale = max(np.max(np.abs(exp)), 1e-300)
+            assert np.max(np.abs(got - exp)) <= TOL * scale, (stat, mode)
+
+
+def test_state_plan_limits():
+    """Trees of more merged levels than launches are worth stay on the chunk
+    plans."""
+    ts = caterpillar().tree_sequence()
+    assert not ts.ll_tree_sequence.get_state_plan_sizes()["usable"]
+    assert caterpillar(200).tree_sequence().ll_tree_sequence.get_state_plan_sizes()["usable"]
+
+
+def stats_of(K):
+    out = [("diversity", None), ("segregating_sites", None)]
+    if K >= 2:
+        out.append(("divergence", [(i, (i + 1) % K) for i in range(K)]))
+        out.append(("genetic_relatedness", [(0, 1), (1, 0)]))
+    if K >= 4:
+        out.append(("f4", [(0, 1, 2, 3), (3, 1, 0, 2)]))
+    return out
+
+
+def close(got, exp):
+    scale = np.maximum(np.max(np.abs(exp), axis=0, keepdims=True), 1e-300)
+    return float(np.max(np.abs(np.asarray(got).reshape(exp.shape) - exp) / scale))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 8, 9, 17, 33, 64])
+def test_row_widths(require_gpu, K):
+    """Every row layout (1, 2 and 4-word loads, several parts a row), with
+    more windows than events and windows between two events."""
+    tc = cases.generated(300, 3e5, 11)
+    ts, orc = tc.tree_sequence(), Oracle(tc)
+    sets = [s[:max(2, len(s) - 1)] for s in cases.sample_sets(300, K, max(2, 300 // K - 1), K)]
+    L = tc.sequence_length
+    for W in (1, 7, 3000):
+        win = np.linspace(0, L, W + 1)
+        for mode in ("branch", "site"):
+            for name, idx in stats_of(K):
+                print("[case]", K, W, mode, name, flush=True)
+                pol = name == "genetic_relatedness"
+                exp = orc.stat(name, sets, idx, win, mode, polarised=pol)
+                kw = dict(windows=win, mode=mode)
+                if idx is not None:
+                    kw["indexes"] = idx
+                if pol:
+                    kw["proportion"] = False
+                err = close(getattr(ts, name)(sets, **kw), exp)
+                assert err <= TOL, (name, mode, W, err)
+    assert ts.ll_tree_sequence.get_last_store() == 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["paper", "single_tree", "nonbinary", "gapped", "multiallelic",
+                                  "bushy"])
+def test_shapes_of_trees(require_gpu, name):
+    tc = INPUTS[name]()
+    ts, orc = tc.tree_sequence(), Oracle(tc)
+    sets = sets_of(ts, 2, 5)
+    win = np.linspace(0, tc.sequence_length, 6)
+    for mode in ("branch", "site"):
+        for stat, idx in [("diversity", None), ("segregating_sites", None), ("divergence", [(0, 1)]),
+                          ("Y2", [(0, 1)]), ("f2", [(1, 0)])]:
+            if min(len(s) for s in sets) < 2:
+                continue
+            exp = orc.stat(stat, sets, idx, win, mode)
+            kw = dict(indexes=idx) if idx is not None else {}
+            print("[case]", name, mode, stat, flush=True)
+            got = getattr(ts, stat)(sets, windows=win, mode=mode, **kw)
+            assert close(got, exp) <= TOL, (stat, mode)
+
+
+@pytest.mark.gpu
+def test_more_than_16_bits(require_gpu):
+    """A set of more than 65535 samples takes 32-bit counts."""
+    tc = cases.generated(70000, 2e4, 5)
+    ts, orc = tc.tree_sequence(), Oracle(tc)
+    sets = [np.arange(66000, dtype=np.int32), np.arange(66000, 70000, dtype=np.int32)]
+    for mode in ("branch", "site"):
+        exp = orc.stat("divergence", sets, [(0, 1)], np.array([0, 1e4, 2e4]), mode)
+        got = ts.divergence(sets, indexes=[(0, 1)], windows=[0, 1e4, 2e4], mode=mode)
+        assert close(got, exp) <= TOL
+    assert ts.ll_tree_sequence.get_last_store() == 2

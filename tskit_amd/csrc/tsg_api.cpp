@@ -31,6 +31,7 @@
 #include "tsg_common.h"
 #include "tsg_launch.h"
 #include "tsg_relvec.h"
+#include "tsg_states.h"
 #include "tsg_treeseq.h"
 
 void tsg_build_index(const double *left, const double *right, const int32_t *parent,
@@ -49,6 +50,9 @@ struct DevBuf {
 struct Workspace {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipEvent_t ev2 = nullptr;       // runs on the state plan, when profiled
+    // the state plan's count rows and window sums
+    DevBuf state_x, state_wsum, state_tw;
     DevBuf seed_off, seed_ps;
     DevBuf seedbuf;                 // seeded slot counts shared with the next run
     DevBuf pair_s, pair_c, tot, outs, queries, windows, cq_wfirst, cq_nwin, cq_poff, partial, dR,
@@ -58,7 +62,7 @@ struct Workspace {
     // one launch over several batches' sweeps: their argument blocks and
     // chunk prefixes; their finish phases (run blocks, block prefixes) and
     // results, copied back in one transfer
-    DevBuf margs, mcpre, mfin, mpre, mout;
+    DevBuf margs, mcpre, mfin, mpre, mout, sargs, spre;
     void *mout_h = nullptr;
     size_t mout_h_bytes = 0;
     // a batch's host arrays, packed into one pinned buffer and sent with one
@@ -327,24 +331,17 @@ struct Pack {
         total = off + std::max<size_t>(bytes, 8);
         return (int) parts.size() - 1;
     }
-    int send(Workspace *ws, hipStream_t s) const {
-        int ret = ensure(ws, ws->arena, total);
+    // The arrays into the workspace's pinned staging buffer, the arena sized
+    // for them.
+    int fill(Workspace *ws) const {
+        const size_t padded = (total + 15) & ~(size_t) 15;
+        int ret = ensure(ws, ws->arena, padded);
         if (ret != 0) return ret;
-        if (ws->fixed != nullptr) {
-            // no pinned staging: one copy from host memory the workspace
-            // keeps until the run has synchronised
-            ws->fixed_stage.assign(total, 0);
-            for (const Part &pt : parts) {
-                if (pt.bytes) std::memcpy(ws->fixed_stage.data() + pt.off, pt.p, pt.bytes);
-            }
-            return hip_check(hipMemcpyAsync(ws->arena.p, ws->fixed_stage.data(), total,
-                                            hipMemcpyHostToDevice, s));
-        }
-        if (ws->stage_bytes < total) {
+        if (ws->stage_bytes < padded) {
             if (ws->stage_h != nullptr) (void) hipHostFree(ws->stage_h);
             ws->stage_h = nullptr;
             ws->stage_bytes = 0;
-            const size_t want = std::max(total + total / 2, (size_t) 1 << 16);
+            const size_t want = std::max(padded + padded / 2, (size_t) 1 << 16);
             if (hipHostMalloc(&ws->stage_h, want) != hipSuccess) {
                 (void) hipGetLastError();
                 ws->stage_h = nullptr;
@@ -355,6 +352,22 @@ struct Pack {
         for (const Part &pt : parts) {
             if (pt.bytes) std::memcpy((char *) ws->stage_h + pt.off, pt.p, pt.bytes);
         }
+        return 0;
+    }
+    int send(Workspace *ws, hipStream_t s) const {
+        int ret;
+        if (ws->fixed != nullptr) {
+            if ((ret = ensure(ws, ws->arena, total))) return ret;
+            // no pinned staging: one copy from host memory the workspace
+            // keeps until the run has synchronised
+            ws->fixed_stage.assign(total, 0);
+            for (const Part &pt : parts) {
+                if (pt.bytes) std::memcpy(ws->fixed_stage.data() + pt.off, pt.p, pt.bytes);
+            }
+            return hip_check(hipMemcpyAsync(ws->arena.p, ws->fixed_stage.data(), total,
+                                            hipMemcpyHostToDevice, s));
+        }
+        if ((ret = fill(ws))) return ret;
         return hip_check(
             hipMemcpyAsync(ws->arena.p, ws->stage_h, total, hipMemcpyHostToDevice, s));
     }
@@ -1324,6 +1337,334 @@ void batch_deliver(const BatchRun &r) {
     }
 }
 
+// ---- runs on the state plan ------------------------------------------------
+// The batch's queries of both modes in one run: one set of count rows, one
+// launch per phase (tsg_states.h).
+constexpr int TSG_NOT_ON_STATES = 1;  // not a run for the state plan
+
+// Device bytes of one run's count rows: beyond this the chunk sweeps, which
+// hold counts in LDS, take the run.
+constexpr size_t TSG_STATE_ROWS_MAX = (size_t) 4 << 30;
+// Host arrays up to this size are brought over by the run's first kernel
+// from pinned memory, larger ones by the copy engine (a copy and the wait of
+// the kernel behind it measured 28 us for 20 KB, the kernel 5 us); results
+// up to it are written to pinned memory by the last kernel.
+constexpr size_t TSG_STATE_DIRECT = (size_t) 256 << 10;
+// A query's segment sums beyond this are first added up per window by a
+// workgroup per window; below it the last kernel reads them directly (one
+// launch less).  Decided per query, so that its sums have the same order
+// whatever it is fused with.
+constexpr size_t TSG_STATE_SEGMENTS = (size_t) 256 << 10;
+
+struct StateRun {
+    tsg_treeseq *ts = nullptr;
+    std::vector<Query *> batch;
+    Workspace *ws = nullptr;
+    TsgStateLaunch l;
+    int Q = 0;
+    bool branch = false, site = false;
+    std::vector<int64_t> outbase;  // per query, in doubles
+    int64_t outcount = 0;
+    bool direct = false;           // results written to the pinned buffer
+    std::vector<char> on_dev;
+    const double *results_h = nullptr;
+};
+
+int pinned_out(Workspace *ws, size_t bytes) {
+    bytes = std::max<size_t>(bytes, 8);
+    if (ws->out_h_bytes >= bytes) return 0;
+    if (ws->out_h != nullptr) (void) hipHostFree(ws->out_h);
+    ws->out_h = nullptr;
+    ws->out_h_bytes = 0;
+    const size_t want = std::max(bytes + bytes / 2, (size_t) 1 << 16);
+    if (hipHostMalloc(&ws->out_h, want) != hipSuccess) {
+        (void) hipGetLastError();
+        ws->out_h = nullptr;
+        return TSG_ERR_NO_MEMORY;
+    }
+    ws->out_h_bytes = want;
+    return 0;
+}
+
+// Host work of a run on the state plan. TSG_NOT_ON_STATES where the plan
+// does not take it: no usable plan, a testing hook asks for another one, more
+// than 64 columns, tiles that do not fit in LDS, rows beyond
+// TSG_STATE_ROWS_MAX, or buffers that do not fit (the device's memory, or a
+// no-allocation run's region). many: one of several runs launched together;
+// the caller says where its results go (l.a.out).
+int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws,
+                  StateRun &r, bool many = false) {
+    const tsg_stateplan &sp = ts->states;
+    if (!sp.usable || ws->force_full || ws->force_c32) return TSG_NOT_ON_STATES;
+    r.ts = ts;
+    r.ws = ws;
+    r.batch.clear();
+    for (uint32_t mode : {TSG_STAT_BRANCH, TSG_STAT_SITE}) {
+        for (Query *q : queries) {
+            if (q->mode == mode) r.batch.push_back(q);
+        }
+    }
+    const int Q = r.Q = (int) r.batch.size();
+    int ret;
+    Fused fz;
+    fuse_queries(r.batch, fz);
+    const int K = fz.K;
+    const bool wgt = fz.weighted;
+    if (K < 1 || K > 64) return TSG_NOT_ON_STATES;
+    const int type = wgt ? TSG_ROW_F64
+                     : *std::max_element(fz.col_total.begin(), fz.col_total.end()) <= 65535
+                         ? TSG_ROW_U16
+                         : TSG_ROW_I32;
+    r.branch = r.batch.front()->mode == TSG_STAT_BRANCH;
+    r.site = r.batch.back()->mode == TSG_STAT_SITE;
+    const size_t lds = (size_t) ws->lds_limit - 1024;
+    if ((r.branch && tsg_state_shmem(K, type, true) > lds) ||
+        (r.site && tsg_state_shmem(K, type, false) > lds)) {
+        return TSG_NOT_ON_STATES;
+    }
+    const int RW = tsg_state_row_words(K, type);
+    const size_t rows = (size_t) sp.num_states * RW * 4;
+    if (rows > TSG_STATE_ROWS_MAX) return TSG_NOT_ON_STATES;
+
+    std::vector<TsgStateQuery> qs(Q);
+    std::vector<TsgFinalHost> fin;
+    std::vector<int32_t> ipar;
+    std::vector<double> dpar;
+    r.outbase.assign(Q, 0);
+    r.outcount = 0;
+    int64_t seg = 0, wsum = 0, raw = 0, fincount = 0;
+    int64_t wg = 0, fg = 0, tw = 0;
+    for (int qi = 0; qi < Q; qi++) {
+        const Query &q = *r.batch[qi];
+        const TsgQuery &f = fz.qs[qi];
+        TsgStateQuery &t = qs[qi];
+        t = TsgStateQuery{};
+        t.W = f.W;
+        t.M = f.M;
+        t.mbase = f.mbase;
+        t.flags = f.flags;
+        t.branch = q.mode == TSG_STAT_BRANCH ? 1 : 0;
+        t.win_off = f.win_off;
+        const int32_t tiles = t.branch ? sp.btiles : sp.stiles;
+        t.new_windows = !(qi > 0 && qs[qi - 1].branch == t.branch &&
+                          r.batch[qi - 1]->windows == q.windows);
+        t.tw = t.new_windows ? (int32_t) tw : qs[qi - 1].tw;
+        if (t.new_windows) tw += (int64_t) tiles + 1;
+        for (int m = f.mbase; m < f.mbase + f.M; m++) {
+            const TsgOut &o = fz.outs[m];
+            if (o.stat == TSG_STAT_RELATEDNESS) {
+                t.rel_c0 = o.cbase;
+                t.rel_cn = o.ccount;
+            }
+        }
+        const int per = t.branch ? 2 : 1;
+        t.pbase = seg;
+        t.cbase = wsum;
+        const int64_t own = ((int64_t) tiles + t.W) * t.M * per;
+        t.by_window = (size_t) own * 8 > TSG_STATE_SEGMENTS ? 1 : 0;
+        seg += own;
+        t.wbase = (int32_t) wg;
+        t.bbase = (int32_t) fg;
+        if (t.by_window) {
+            wsum += (int64_t) t.W * t.M * per;
+            wg += t.W;
+        }
+        fg += (t.M + TSG_FINISH_OUTPUTS - 1) / TSG_FINISH_OUTPUTS;
+        r.outbase[qi] = r.outcount;
+        r.outcount += (int64_t) t.W * q.P;
+        t.to_out = q.final_kind == TSG_FINAL_NONE ? 1 : 0;
+        t.obase = t.to_out ? r.outbase[qi] : raw;
+        if (t.to_out) continue;
+        TsgFinalHost h{};
+        h.kind = q.final_kind;
+        h.Kq = (int32_t) q.sets.size();
+        h.P = q.P;
+        h.W = t.W;
+        h.rawbase = raw;
+        h.outbase = r.outbase[qi];
+        h.Mraw = t.M;
+        if (q.final_kind == TSG_FINAL_TAJIMAS_D) {
+            h.pbase = (int64_t) dpar.size();
+            dpar.insert(dpar.end(), q.fin_dpar.begin(), q.fin_dpar.end());
+        } else {
+            h.pbase = (int64_t) ipar.size();
+            ipar.insert(ipar.end(), q.fin_ipar.begin(), q.fin_ipar.end());
+        }
+        fin.push_back(h);
+        raw += (int64_t) t.W * t.M;
+        fincount += (int64_t) t.W * q.P;
+    }
+    if (wg > INT32_MAX || fg > INT32_MAX || tw > INT32_MAX / 2 || fincount > (int64_t) INT32_MAX * 128) {
+        return TSG_NOT_ON_STATES;
+    }
+    Pack pk;
+    const int p_ps = pk.add(fz.pair_s), p_pc = pk.add(fz.pair_c), p_outs = pk.add(fz.outs);
+    const int p_qs = pk.add(qs), p_win = pk.add(fz.wins), p_tot = pk.add(fz.col_total);
+    const int p_fin = pk.add(fin), p_ip = pk.add(ipar), p_dp = pk.add(dpar);
+    int p_pw = -1, p_tw = -1, p_op = -1;
+    if (wgt) {
+        p_pw = pk.add(fz.pair_w);
+        p_tw = pk.add(fz.col_total_w);
+        p_op = pk.add(fz.opar);
+    }
+    r.on_dev.assign(Q, 0);
+    bool any_dev = false;
+    for (int qi = 0; qi < Q; qi++) {
+        r.on_dev[qi] = is_device_ptr(r.batch[qi]->result);
+        any_dev |= r.on_dev[qi] != 0;
+    }
+    r.direct = !many && !any_dev && ws->fixed == nullptr &&
+               (size_t) r.outcount * 8 <= TSG_STATE_DIRECT;
+    if (r.direct && (ret = pinned_out(ws, (size_t) r.outcount * 8))) return ret;
+    const bool by_kernel = ws->fixed == nullptr && pk.total <= TSG_STATE_DIRECT;
+    ret = ensure(ws, ws->state_x, rows);
+    if (ret == 0) ret = ensure(ws, ws->partial, (size_t) seg * 8);
+    if (ret == 0 && wsum > 0) ret = ensure(ws, ws->state_wsum, (size_t) wsum * 8);
+    if (ret == 0) ret = ensure(ws, ws->state_tw, (size_t) tw * 4);
+    if (ret == 0) ret = ensure(ws, ws->raw, (size_t) raw * 8);
+    if (ret == 0 && !many && !r.direct) ret = ensure(ws, ws->out, (size_t) r.outcount * 8);
+    if (ret == 0) ret = by_kernel ? pk.fill(ws) : pk.send(ws, ws->stream);
+    if (ret == TSG_ERR_DEVICE_MEMORY || ret == TSG_ERR_SCRATCH_TOO_SMALL) {
+        ws->fixed_used = 0;
+        return TSG_NOT_ON_STATES;
+    }
+    if (ret != 0) return ret;
+
+    const TsgStateDevice &d = sp.dev;
+    TsgStateArgs &a = r.l.a;
+    a = TsgStateArgs{};
+    a.in = d.in;
+    a.ev_state = d.ev_state;
+    a.ev_b = d.ev_b;
+    a.ev_pos = d.ev_pos;
+    a.btile_pos = d.btile_pos;
+    a.row_ref = d.row_ref;
+    a.row_pos = d.row_pos;
+    a.stile_pos = d.stile_pos;
+    a.list_off = d.list_off;
+    a.list_kind = d.list_kind;
+    a.list_ent = d.list_ent;
+    a.num_states = sp.num_states;
+    a.num_samples = ts->num_samples;
+    a.nev = (int32_t) sp.ev_state.size();
+    a.nrow = (int32_t) sp.row_ref.size();
+    a.btiles = sp.btiles;
+    a.stiles = sp.stiles;
+    a.K = K;
+    a.RW = RW;
+    a.x = (uint32_t *) ws->state_x.p;
+    a.npairs = (int32_t) fz.pair_s.size();
+    a.pair_sample = pk.dev<const int32_t>(ws, p_ps);
+    a.pair_col = pk.dev<const int32_t>(ws, p_pc);
+    a.col_total = pk.dev<const int32_t>(ws, p_tot);
+    if (wgt) {
+        a.pair_w = pk.dev<const double>(ws, p_pw);
+        a.col_total_w = pk.dev<const double>(ws, p_tw);
+        a.opar = pk.dev<const double>(ws, p_op);
+    }
+    a.QB = 0;
+    while (a.QB < Q && qs[a.QB].branch) a.QB++;
+    a.Q = Q;
+    a.outs = pk.dev<const TsgOut>(ws, p_outs);
+    a.queries = pk.dev<const TsgStateQuery>(ws, p_qs);
+    a.windows = pk.dev<const double>(ws, p_win);
+    a.tile_w = (int32_t *) ws->state_tw.p;
+    a.ntile_w = (int32_t) tw;
+    a.partial = (double *) ws->partial.p;
+    a.wsum = (double *) ws->state_wsum.p;
+    a.raw = (double *) ws->raw.p;
+    a.out = many ? nullptr : r.direct ? (double *) ws->out_h : (double *) ws->out.p;
+    if (by_kernel) {
+        a.stage_src = (const uint4 *) ws->stage_h;
+        a.stage_dst = (uint4 *) ws->arena.p;
+        a.stage_words = (int64_t) ((pk.total + 15) / 16);
+    }
+    a.fin = pk.dev<const void>(ws, p_fin);
+    a.nfin = (int32_t) fin.size();
+    a.ipar = pk.dev<const int32_t>(ws, p_ip);
+    a.dpar = pk.dev<const double>(ws, p_dp);
+    a.fincount = fincount;
+    r.l.type = type;
+    r.l.level0 = sp.level0.data();
+    r.l.levels = (int) sp.level0.size() - 1;
+    r.l.wgroups = (int) wg;
+    r.l.fgroups = (int) fg;
+    ws->last_store = type == TSG_ROW_U16 ? TSG_STORE_HOT16
+                     : type == TSG_ROW_I32 ? TSG_STORE_HOT
+                                           : TSG_STORE_HOTW;
+    return 0;
+}
+
+// Device copies of the results that go to device memory, and the others'
+// copy to the host (queued on stream s).
+int state_results(StateRun &r, const double *out, hipStream_t s) {
+    int ret;
+    Workspace *ws = r.ws;
+    bool host = false;
+    for (int qi = 0; qi < r.Q; qi++) {
+        const size_t n = (size_t) (r.batch[qi]->windows.size() - 1) * r.batch[qi]->P * 8;
+        const bool fixed = ws->fixed != nullptr;
+        if (!r.on_dev[qi] && !fixed) host = true;
+        if (n == 0 || (!r.on_dev[qi] && !fixed)) continue;
+        if ((ret = hip_check(hipMemcpyAsync(
+                 r.batch[qi]->result, out + r.outbase[qi], n,
+                 r.on_dev[qi] ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s)))) {
+            return ret;
+        }
+    }
+    if (!host || r.results_h != nullptr || r.outcount == 0) return 0;
+    if ((ret = pinned_out(ws, (size_t) r.outcount * 8))) return ret;
+    return hip_check(hipMemcpyAsync(ws->out_h, out, (size_t) r.outcount * 8,
+                                    hipMemcpyDeviceToHost, s));
+}
+
+// After the stream has finished: the results of host buffers.
+void state_deliver(const StateRun &r) {
+    if (r.ws->fixed != nullptr) return;
+    const double *src = r.results_h != nullptr ? r.results_h : (const double *) r.ws->out_h;
+    for (int qi = 0; qi < r.Q; qi++) {
+        if (r.on_dev[qi]) continue;
+        const Query &q = *r.batch[qi];
+        std::memcpy(q.result, src + r.outbase[qi], (q.windows.size() - 1) * (size_t) q.P * 8);
+    }
+}
+
+// Queries of one tree sequence (either mode or both) on the state plan, with
+// a leased workspace; TSG_NOT_ON_STATES where it does not take them.
+int run_states(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws) {
+    StateRun r;
+    int ret = state_prepare(ts, queries, ws, r);
+    if (ret != 0) return ret;
+    hipStream_t s = ws->stream;
+    const bool prof = ws->profile;
+    if (prof && ws->ev2 == nullptr && (ret = hip_check(hipEventCreate(&ws->ev2)))) return ret;
+    ret = hip_check(tsg_launch_states(r.l, prof ? ws->ev0 : nullptr, prof ? ws->ev1 : nullptr,
+                                      prof ? ws->ev2 : nullptr, s));
+    if (ret == 0 && !r.direct) ret = state_results(r, r.l.a.out, s);
+    const int sret = hip_check(hipStreamSynchronize(s));
+    if (ret == 0) ret = sret;
+    if (ret != 0) return ret;
+    state_deliver(r);
+    if (prof) {
+        // the counts are the branch queries' when there are any
+        float ms[2] = {0, 0};
+        (void) hipEventElapsedTime(&ms[0], ws->ev0, ws->ev1);
+        (void) hipEventElapsedTime(&ms[1], ws->ev1, ws->ev2);
+        if (!r.branch) {
+            ms[1] += ms[0];
+            ms[0] = 0;
+        }
+        for (int m = 0; m < 2; m++) {
+            if (!(m == 0 ? r.branch : r.site)) continue;
+            ws->sweep_ms += ms[m];
+            ws->sweep_launches += 1;
+            ws->mode_ms[m] += ms[m];
+            ws->mode_launches[m] += 1;
+        }
+    }
+    return 0;
+}
+
 // Runs a batch of queries (same tree sequence, same mode) in one sweep.
 int run_batch(tsg_treeseq *ts, std::vector<Query *> &batch) {
     int ret;
@@ -1334,6 +1675,7 @@ int run_batch(tsg_treeseq *ts, std::vector<Query *> &batch) {
     Lease lease(ts);
     Workspace *ws = lease.ws;
     if (ws == nullptr) return TSG_ERR_DEVICE;
+    if ((ret = run_states(ts, batch, ws)) != TSG_NOT_ON_STATES) return ret;
     BatchRun r;
     if ((ret = batch_prepare(ts, batch, ws, ws->stream, r))) return ret;
     if (ws->profile) (void) hipEventRecord(ws->ev0, r.s);
@@ -1465,6 +1807,22 @@ int device_upload(tsg_treeseq *ts) {
             (ret = upload_ptr(&h.mut_slot, hp.mut_slot, hb)) ||
             (ret = upload_ptr(&h.t0_parent, hp.t0_parent, hb)) ||
             (ret = upload_ptr(&h.t0_bl, hp.t0_bl, hb))) {
+            return ret;
+        }
+    }
+    if (ts->states.usable) {
+        const tsg_stateplan &sp = ts->states;
+        TsgStateDevice &h = ts->states.dev;
+        size_t &hb = h.bytes;
+        if ((ret = upload_ptr(&h.in, sp.in, hb)) || (ret = upload_ptr(&h.ev_state, sp.ev_state, hb)) ||
+            (ret = upload_ptr(&h.ev_b, sp.ev_b, hb)) || (ret = upload_ptr(&h.ev_pos, sp.ev_pos, hb)) ||
+            (ret = upload_ptr(&h.row_ref, sp.row_ref, hb)) ||
+            (ret = upload_ptr(&h.row_pos, sp.row_pos, hb)) ||
+            (ret = upload_ptr(&h.list_off, sp.list_off, hb)) ||
+            (ret = upload_ptr(&h.list_kind, sp.list_kind, hb)) ||
+            (ret = upload_ptr(&h.list_ent, sp.list_ent, hb)) ||
+            (ret = upload_ptr(&h.btile_pos, sp.btile_pos, hb)) ||
+            (ret = upload_ptr(&h.stile_pos, sp.stile_pos, hb))) {
             return ret;
         }
     }
@@ -1660,7 +2018,7 @@ void free_one_workspace(Workspace *ws) {
                       &ws->scale,
                       &ws->kout, &ws->wk0, &ws->wk1, &ws->sel, &ws->gslab, &ws->geno, &ws->x0,
                       &ws->r0part, &ws->bsum, &ws->margs, &ws->mcpre, &ws->mfin, &ws->mpre,
-                      &ws->mout, &ws->arena,
+                      &ws->mout, &ws->sargs, &ws->spre, &ws->arena, &ws->state_x, &ws->state_wsum, &ws->state_tw,
                       &ws->rv_E, &ws->rv_I, &ws->rv_z0, &ws->rv_d0, &ws->rv_esum, &ws->rv_y,
                       &ws->sitecol2, &ws->gt2, &ws->cmat2, &ws->wk0b, &ws->wk1b, &ws->row2};
     for (DevBuf *b : bufs) {
@@ -1675,6 +2033,7 @@ void free_one_workspace(Workspace *ws) {
     }
     if (ws->ev0) (void) hipEventDestroy(ws->ev0);
     if (ws->ev1) (void) hipEventDestroy(ws->ev1);
+    if (ws->ev2) (void) hipEventDestroy(ws->ev2);
     if (ws->stream) (void) hipStreamDestroy(ws->stream);
     delete ws;
 }
@@ -1713,6 +2072,15 @@ void tsg_hot_device_free(TsgHotDevice *h) {
         if (p != nullptr) (void) hipFree(p);
     }
     *h = TsgHotDevice();
+}
+
+void tsg_state_device_free(TsgStateDevice *h) {
+    void *ptrs[] = {h->in, h->ev_state, h->ev_b, h->ev_pos, h->row_ref, h->row_pos, h->list_off,
+                    h->list_kind, h->list_ent, h->btile_pos, h->stile_pos};
+    for (void *p : ptrs) {
+        if (p != nullptr) (void) hipFree(p);
+    }
+    *h = TsgStateDevice();
 }
 
 namespace {
@@ -1852,7 +2220,16 @@ int tsg_treeseq_init(tsg_treeseq **out, double sequence_length, uint64_t num_nod
                              derived_state_offset);
     if (ret != 0) return ret;
     ts->full_chunks = default_num_chunks(ts.get());
+    // the state plan on a thread of its own beside the (threaded) hot plan
+    std::thread states([&]() {
+        try {
+            (void) tsg_build_states(ts.get());
+        } catch (const std::bad_alloc &) {
+            ts->states = tsg_stateplan();
+        }
+    });
     ret = tsg_build_hot_plan(ts.get(), default_hot_chunks(ts.get()), true);
+    states.join();
     if (ret != 0) return ret;
     *out = ts.release();
     return 0;
@@ -1865,6 +2242,7 @@ int tsg_treeseq_free(tsg_treeseq *ts) {
         free_workspace(ts);
         tsg_device_free(&ts->dev);
         tsg_hot_device_free(&ts->hot.dev);
+        tsg_state_device_free(&ts->states.dev);
     }
     delete ts;
     return 0;
@@ -1878,6 +2256,7 @@ int tsg_treeseq_set_num_chunks(tsg_treeseq *ts, uint32_t num_chunks) {
     free_workspace(ts);
     tsg_device_free(&ts->dev);
     tsg_hot_device_free(&ts->hot.dev);
+    tsg_state_device_free(&ts->states.dev);
     ts->full_chunks = (int32_t) std::min<uint32_t>(num_chunks, INT32_MAX);
     ts->full_built = false;
     const int ret = tsg_build_hot_plan(ts, ts->full_chunks, false);
@@ -1925,7 +2304,7 @@ uint64_t tsg_treeseq_get_num_chunks(const tsg_treeseq *ts) {
 }
 double tsg_treeseq_get_sequence_length(const tsg_treeseq *ts) { return ts->L; }
 uint64_t tsg_treeseq_get_device_bytes(const tsg_treeseq *ts) {
-    return (uint64_t) (ts->dev.bytes + ts->hot.dev.bytes);
+    return (uint64_t) (ts->dev.bytes + ts->hot.dev.bytes + ts->states.dev.bytes);
 }
 uint64_t tsg_treeseq_get_max_chunk_nodes(const tsg_treeseq *ts) {
     return (uint64_t) full_plan(ts)->max_nloc;
@@ -2070,6 +2449,41 @@ int tsg_treeseq_copy_hot_afs_plan(const tsg_treeseq *ts, int32_t *slot_node, int
 
 // Profiling of the sweep kernel: HIP events on the library's stream around
 // every sweep launch.
+// Host copy of the state plan; sizes = {usable, states, levels, branch events,
+// site rows, lists, list entries}
+int tsg_treeseq_get_state_plan_sizes(const tsg_treeseq *ts, uint64_t *sizes) {
+    const tsg_stateplan &sp = ts->states;
+    sizes[0] = sp.usable ? 1 : 0;
+    sizes[1] = (uint64_t) sp.num_states;
+    sizes[2] = sp.level0.empty() ? 0 : sp.level0.size() - 1;
+    sizes[3] = sp.ev_state.size();
+    sizes[4] = sp.row_ref.size();
+    sizes[5] = sp.list_kind.size();
+    sizes[6] = sp.list_ent.size();
+    return 0;
+}
+
+int tsg_treeseq_copy_state_plan(const tsg_treeseq *ts, int32_t *level0, int32_t *in,
+                                int32_t *ev_state, double *ev_b, double *ev_pos, int32_t *row_ref,
+                                double *row_pos, int32_t *list_off, int32_t *list_kind,
+                                int32_t *list_ent) {
+    const tsg_stateplan &sp = ts->states;
+    auto put = [](auto *dst, const auto &src) {
+        if (dst != nullptr) std::copy(src.begin(), src.end(), dst);
+    };
+    put(level0, sp.level0);
+    put(in, sp.in);
+    put(ev_state, sp.ev_state);
+    put(ev_b, sp.ev_b);
+    put(ev_pos, sp.ev_pos);
+    put(row_ref, sp.row_ref);
+    put(row_pos, sp.row_pos);
+    put(list_off, sp.list_off);
+    put(list_kind, sp.list_kind);
+    put(list_ent, sp.list_ent);
+    return 0;
+}
+
 int tsg_treeseq_set_profiling(tsg_treeseq *ts, int enable) {
     Use use(ts);
     int ret = tsg_treeseq_upload(ts);
@@ -3297,6 +3711,32 @@ int run_fused_modes(tsg_batch *b) {
     }
     if (groups.empty()) return 0;
     if (groups.size() == 1) return run_batch(b->ts, groups[0]);
+    {
+        // both modes in one run on the state plan
+        std::vector<Query *> all(groups[0]);
+        all.insert(all.end(), groups[1].begin(), groups[1].end());
+        int ret;
+        {
+            std::lock_guard<std::mutex> lock(g_mutex);
+            if ((ret = device_upload(b->ts))) return ret;
+        }
+        Lease lease(b->ts);
+        if (lease.ws == nullptr) return TSG_ERR_DEVICE;
+        if ((ret = run_states(b->ts, all, lease.ws)) != TSG_NOT_ON_STATES) return ret;
+        // (more than 64 columns together, say) or the modes one by one
+        std::vector<bool> done(2, false);
+        for (int i = 0; i < 2; i++) {
+            ret = run_states(b->ts, groups[i], lease.ws);
+            if (ret == 0) {
+                done[i] = true;
+            } else if (ret != TSG_NOT_ON_STATES) {
+                return ret;
+            }
+        }
+        if (done[0] && done[1]) return 0;
+        if (done[0] || done[1]) groups.erase(groups.begin() + (done[0] ? 0 : 1));
+    }
+    if (groups.size() == 1) return run_batch(b->ts, groups[0]);
     std::vector<std::unique_ptr<Lease>> leases;
     std::vector<BatchRun> runs;
     int ret = run_two_modes(b->ts, groups, leases, runs);
@@ -3373,6 +3813,11 @@ __attribute__((visibility("hidden"))) int tsg_batch_run_fixed(tsg_batch *b, void
         }
         if (group.empty()) continue;
         w.fixed_used = 0;
+        if ((ret = run_states(ts, group, &w)) != TSG_NOT_ON_STATES) {
+            if (ret != 0) break;
+            continue;
+        }
+        w.fixed_used = 0;
         BatchRun r;
         ret = batch_prepare(ts, group, &w, w.stream, r);
         if (ret == 0) ret = batch_sweep(r);
@@ -3385,23 +3830,145 @@ __attribute__((visibility("hidden"))) int tsg_batch_run_fixed(tsg_batch *b, void
 }
 
 namespace {
-// The runs of tsg_batch_run_multi: prepared in parallel, each on its
+// The batches of a tsg_batch_run_multi that the state plan takes: prepared in
+// parallel, then one launch per phase over all of them (per row type), every
+// run's results into one device buffer and back in one copy.  taken[i]: batch
+// i's branch and site queries are done once the leases' streams have finished.
+int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lease>> &leases,
+                     std::deque<StateRun> &runs, std::vector<char> &taken) {
+    int ret;
+    taken.assign(n, 0);
+    struct Prep {
+        uint64_t i;
+        Workspace *ws;
+        std::vector<Query *> queries;
+        StateRun run;
+        int ret = 0;
+    };
+    std::deque<Prep> preps;
+    for (uint64_t i = 0; i < n; i++) {
+        tsg_batch *b = bs[i];
+        {
+            std::lock_guard<std::mutex> lock(g_mutex);
+            if ((ret = device_upload(b->ts))) return ret;
+        }
+        std::vector<Query *> qs;
+        for (auto &q : b->queries) {
+            if (q->mode != TSG_STAT_NODE) qs.push_back(q.get());
+        }
+        if (qs.empty()) {
+            taken[i] = 1;
+            continue;
+        }
+        if (!b->ts->states.usable) continue;
+        leases.push_back(std::make_unique<Lease>(b->ts));
+        if (leases.back()->ws == nullptr) return TSG_ERR_DEVICE;
+        preps.push_back(Prep{i, leases.back()->ws, std::move(qs), StateRun(), 0});
+    }
+    {
+        std::atomic<size_t> next{0};
+        auto work = [&]() {
+            for (size_t p; (p = next.fetch_add(1)) < preps.size();) {
+                Prep &t = preps[p];
+                t.ret = state_prepare(bs[t.i]->ts, t.queries, t.ws, t.run, true);
+                // (arrays too large for the first kernel go over on the
+                // run's own stream)
+                if (t.ret == 0) t.ret = hip_check(hipEventRecord(t.ws->ev0, t.ws->stream));
+            }
+        };
+        std::vector<std::thread> pool;
+        const size_t T = std::min<size_t>(preps.size(), 8);
+        for (size_t t = 1; t < T; t++) pool.emplace_back(work);
+        work();
+        for (std::thread &th : pool) th.join();
+    }
+    std::map<int, std::vector<Prep *>> byt;
+    int64_t outcount = 0;
+    Workspace *ws0 = nullptr;
+    for (Prep &t : preps) {
+        if (t.ret == TSG_NOT_ON_STATES) continue;
+        if (t.ret != 0) return t.ret;
+        if (ws0 == nullptr) ws0 = t.ws;
+        byt[t.run.l.type].push_back(&t);
+        outcount += t.run.outcount;
+    }
+    if (ws0 == nullptr) return 0;
+    if ((ret = ensure(ws0->mout, (size_t) std::max<int64_t>(outcount, 1) * 8))) return ret;
+    const size_t bytes = (size_t) std::max<int64_t>(outcount, 1) * 8;
+    if (ws0->mout_h_bytes < bytes) {
+        if (ws0->mout_h != nullptr) (void) hipHostFree(ws0->mout_h);
+        ws0->mout_h = nullptr;
+        ws0->mout_h_bytes = 0;
+        const size_t want = std::max(bytes + bytes / 2, (size_t) 1 << 16);
+        if (hipHostMalloc(&ws0->mout_h, want) != hipSuccess) {
+            (void) hipGetLastError();
+            return TSG_ERR_NO_MEMORY;
+        }
+        ws0->mout_h_bytes = want;
+    }
+    hipStream_t s0 = ws0->stream;
+    std::vector<TsgStateArgs> args;
+    std::vector<int32_t> pre;
+    std::vector<std::vector<int32_t>> pres;
+    std::vector<std::vector<TsgStateLaunch>> launches;
+    int64_t off = 0;
+    for (auto &kv : byt) {
+        launches.emplace_back();
+        for (Prep *t : kv.second) {
+            t->run.l.a.out = (double *) ws0->mout.p + off;
+            t->run.results_h = (const double *) ws0->mout_h + off;
+            off += t->run.outcount;
+            launches.back().push_back(t->run.l);
+            args.push_back(t->run.l.a);
+            if (t->ws != ws0 && (ret = hip_check(hipStreamWaitEvent(s0, t->ws->ev0, 0)))) return ret;
+        }
+        pres.emplace_back();
+        if (tsg_state_prefixes(launches.back().data(), (int) launches.back().size(),
+                               pres.back()) != 0) {
+            return TSG_ERR_BAD_PARAM_VALUE;
+        }
+        pre.insert(pre.end(), pres.back().begin(), pres.back().end());
+    }
+    if ((ret = upload(ws0->sargs, args, s0)) || (ret = upload(ws0->spre, pre, s0))) return ret;
+    size_t aoff = 0, poff = 0;
+    for (size_t g = 0; g < launches.size(); g++) {
+        if ((ret = hip_check(tsg_launch_states_multi(
+                 launches[g].data(), (const TsgStateArgs *) ws0->sargs.p + aoff,
+                 (int) launches[g].size(), pres[g], (const int32_t *) ws0->spre.p + poff, s0)))) {
+            return ret;
+        }
+        aoff += launches[g].size();
+        poff += pres[g].size();
+    }
+    if (outcount > 0 && (ret = hip_check(hipMemcpyAsync(ws0->mout_h, ws0->mout.p,
+                                                        (size_t) outcount * 8,
+                                                        hipMemcpyDeviceToHost, s0)))) {
+        return ret;
+    }
+    for (auto &kv : byt) {
+        for (Prep *t : kv.second) {
+            if ((ret = state_results(t->run, t->run.l.a.out, s0))) return ret;
+            taken[t->i] = 1;
+            runs.push_back(std::move(t->run));
+        }
+    }
+    return 0;
+}
+
+// The runs of tsg_batch_run_multi on the chunk plans: prepared in parallel, each on its
 // workspace's stream; runs on the hot plan whose outputs fit one slice share
 // one sweep launch per (mode, node store, outputs per lane) on the first
 // run's stream, the rest launch on their own there; then each run finishes
 // on its own stream.
-int run_multi(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lease>> &leases,
+int run_multi(tsg_batch **bs, uint64_t n, const std::vector<char> &taken,
+              std::vector<std::unique_ptr<Lease>> &leases,
               std::deque<std::vector<Query *>> &groups, std::deque<BatchRun> &runs) {
     int ret;
     std::vector<tsg_treeseq *> run_ts;
     std::vector<Workspace *> run_ws;
     for (uint64_t i = 0; i < n; i++) {
         tsg_batch *b = bs[i];
-        if (b == nullptr) return TSG_ERR_BAD_PARAM_VALUE;
-        {
-            std::lock_guard<std::mutex> lock(g_mutex);
-            if ((ret = device_upload(b->ts))) return ret;
-        }
+        if (taken[i]) continue;
         for (uint32_t mode : {TSG_STAT_BRANCH, TSG_STAT_SITE}) {
             std::vector<Query *> g;
             for (auto &q : b->queries) {
@@ -3579,7 +4146,10 @@ int tsg_batch_run_multi(tsg_batch **batches, uint64_t n) {
     std::vector<std::unique_ptr<Lease>> leases;
     std::deque<std::vector<Query *>> groups;
     std::deque<BatchRun> runs;
-    int ret = run_multi(batches, n, leases, groups, runs);
+    std::deque<StateRun> sruns;
+    std::vector<char> taken;
+    int ret = run_multi_states(batches, n, leases, sruns, taken);
+    if (ret == 0) ret = run_multi(batches, n, taken, leases, groups, runs);
     // the leases end (workspaces return to their pools) only once all work
     // queued on their streams has finished
     for (auto &l : leases) {
@@ -3588,6 +4158,7 @@ int tsg_batch_run_multi(tsg_batch **batches, uint64_t n) {
         if (ret == 0) ret = sret;
     }
     if (ret == 0) {
+        for (const StateRun &r : sruns) state_deliver(r);
         for (const BatchRun &r : runs) batch_deliver(r);
     }
     for (uint64_t i = 0; i < n && ret == 0; i++) ret = run_node_queries(batches[i]);

@@ -5,6 +5,7 @@
 #include <vector>
 
 #include "tsg_common.h"
+#include "tsg_states.h"
 
 // Query-independent data the sweep kernels read, resident in HBM.
 struct TsgDevice {
@@ -174,6 +175,7 @@ struct tsg_treeseq {
     bool full_built = false;              // the full plan above is built on first need
     int32_t full_chunks = 1;              // chunk count it is built with
     tsg_hotplan hot;
+    tsg_stateplan states;
 
     TsgDevice dev;
     void *workspace = nullptr;            // per-handle device scratch (tsg_api.cpp)

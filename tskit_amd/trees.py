@@ -262,6 +262,28 @@ class LowLevelTreeSequence:
         p["max_levels"] = max_levels
         return p
 
+    def get_state_plan_sizes(self):
+        sizes = (ctypes.c_uint64 * 7)()
+        self._lib.tsg_treeseq_get_state_plan_sizes(self._h, sizes)
+        keys = ["usable", "states", "levels", "events", "rows", "lists", "list_entries"]
+        return dict(zip(keys, [int(x) for x in sizes]))
+
+    def get_state_plan(self):
+        """The state plan's host arrays (include/tsgpu.h)."""
+        z = self.get_state_plan_sizes()
+        inner = max(0, z["states"] - 1 - self.get_num_samples())
+        out = dict(level0=np.zeros(z["levels"] + 1, np.int32),
+                   inputs=np.zeros((inner, 8), np.int32),
+                   ev_state=np.zeros(z["events"], np.int32), ev_b=np.zeros(z["events"]),
+                   ev_pos=np.zeros(z["events"]), row_ref=np.zeros(z["rows"], np.int32),
+                   row_pos=np.zeros(z["rows"]), list_off=np.zeros(z["lists"] + 1, np.int32),
+                   list_kind=np.zeros(z["lists"], np.int32),
+                   list_ent=np.zeros(z["list_entries"], np.int32))
+        check(self._lib.tsg_treeseq_copy_state_plan(
+            self._h, *[ptr(a, ctypes.c_double if a.dtype == np.float64 else ctypes.c_int32)
+                       for a in out.values()]))
+        return dict(z, **out)
+
     def set_sweep_plan(self, plan):
         """1: run statistics sweeps on the full plan; 2: on the hot plan with
         32-bit counts; 0: the library chooses."""
