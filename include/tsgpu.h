@@ -144,10 +144,12 @@ int tsg_treeseq_copy_hot_afs_plan(const tsg_treeseq_t *ts, int32_t *slot_node,
 /* host copy of the state plan (count states of the whole sequence, each the
  * sum of at most 8 earlier ones, and the events and site rows that read
  * them: the statistics' usual plan); sizes = {usable, states, levels, branch
- * events, site rows, lists, list entries}.  level0 has levels + 1 entries, in
- * 8 per state after the samples', list_off lists + 1. */
+ * events, site rows, lists, list entries}.  order: the states by level,
+ * level0 (levels + 1 entries) into it; in has 8 entries per state after the
+ * samples', list_off lists + 1. */
 int tsg_treeseq_get_state_plan_sizes(const tsg_treeseq_t *ts, uint64_t *sizes);
-int tsg_treeseq_copy_state_plan(const tsg_treeseq_t *ts, int32_t *level0, int32_t *in,
+int tsg_treeseq_copy_state_plan(const tsg_treeseq_t *ts, int32_t *level0, int32_t *order,
+    int32_t *in,
     int32_t *ev_state, double *ev_b, double *ev_pos, int32_t *row_ref, double *row_pos,
     int32_t *list_off, int32_t *list_kind, int32_t *list_ent);
 /* plan = 1: run statistics sweeps on the full plan; 2: on the hot plan with

@@ -97,10 +97,15 @@ def counts(plan, n, sets, sample_index):
         x[1 + sample_index[s], k] = 1
     lev = plan["level0"]
     assert lev[0] == 0 and lev[1] == 1 + n and lev[-1] == plan["states"]
+    assert np.array_equal(np.sort(plan["order"]), np.arange(plan["states"]))
+    assert np.array_equal(plan["order"][:1 + n], np.arange(1 + n))
+    level = np.zeros(plan["states"], np.int64)
     for l in range(1, len(lev) - 1):
-        ins = plan["inputs"][lev[l] - 1 - n:lev[l + 1] - 1 - n]
-        assert ins.min() >= 0 and ins.max() < lev[l]  # of earlier levels
-        x[lev[l]:lev[l + 1]] = x[ins].sum(axis=1)
+        here = plan["order"][lev[l]:lev[l + 1]]
+        ins = plan["inputs"][here - 1 - n]
+        level[here] = l
+        assert ins.min() >= 0 and np.all(level[ins] < l)
+        x[here] = x[ins].sum(axis=1)
     return x
 
 

@@ -18,13 +18,15 @@
 #include <condition_variable>
 #include <cstring>
 #include <deque>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <new>
 #include <numeric>
-#include <unordered_set>
+#include <system_error>
 #include <thread>
+#include <unordered_set>
 #include <tuple>
 #include <vector>
 
@@ -73,10 +75,9 @@ struct Workspace {
     // a batch's results, copied back in one transfer (pinned)
     void *out_h = nullptr;
     size_t out_h_bytes = 0;
-    // large results into pageable host memory: two pinned pieces in turn
-    // (copy_out)
-    void *cp_h[2] = {nullptr, nullptr};
-    hipEvent_t cp_ev[2] = {nullptr, nullptr};
+    // results into pageable host memory: a ring of pinned pieces (copy_out)
+    void *cp_h = nullptr;
+    hipEvent_t cp_ev[8] = {};
     // relatedness-vector route
     DevBuf rv_E, rv_I, rv_z0, rv_d0, rv_esum, rv_y;
     // relatedness-matrix route
@@ -221,6 +222,56 @@ int upload_ptr(T **dst, const std::vector<T> &v, size_t &bytes) {
     if (!v.empty()) return hip_check(hipMemcpy(*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
     return 0;
 }
+
+// Arrays that become resident together, in one device allocation (an
+// allocation and a transfer each cost tens of microseconds, more than the
+// arrays of a small tree sequence are worth): small ones go over in one
+// transfer, large ones each in their own.
+struct Arrays {
+    struct Part {
+        void **dst;
+        const void *src;
+        size_t bytes, off;
+    };
+    std::vector<Part> parts;
+    size_t total = 0;
+    template <typename T>
+    void add(T *&dst, const std::vector<T> &v) {
+        const size_t bytes = v.size() * sizeof(T);
+        parts.push_back({reinterpret_cast<void **>(&dst), v.data(), bytes, total});
+        total = (total + std::max<size_t>(bytes, 8) + 255) & ~(size_t) 255;
+    }
+    int upload(void *&block, size_t &held) {
+        if (hipMalloc(&block, std::max<size_t>(total, 256)) != hipSuccess) {
+            (void) hipGetLastError();
+            block = nullptr;
+            return TSG_ERR_DEVICE_MEMORY;
+        }
+        held += total;
+        char *const base = (char *) block;
+        int ret = 0;
+        if (total <= ((size_t) 4 << 20)) {
+            std::vector<char> all(total, 0);
+            for (const Part &p : parts) {
+                if (p.bytes) std::memcpy(all.data() + p.off, p.src, p.bytes);
+            }
+            ret = hip_check(hipMemcpy(base, all.data(), total, hipMemcpyHostToDevice));
+        } else {
+            for (const Part &p : parts) {
+                if (ret == 0 && p.bytes) {
+                    ret = hip_check(hipMemcpy(base + p.off, p.src, p.bytes, hipMemcpyHostToDevice));
+                }
+            }
+        }
+        if (ret != 0) {
+            (void) hipFree(block);
+            block = nullptr;
+            return ret;
+        }
+        for (const Part &p : parts) *p.dst = base + p.off;
+        return 0;
+    }
+};
 
 Resident *res_of(const tsg_treeseq *ts) { return reinterpret_cast<Resident *>(ts->workspace); }
 
@@ -590,11 +641,16 @@ bool is_device_ptr(const void *p) {
 
 // `bytes` of device memory src into the caller's dst, waiting for stream s
 // to finish: a device copy when dst is device memory, one transfer when it
-// is pinned host memory or small; otherwise through two pinned pieces in
-// turn, the transfer of one piece running while host threads copy the
-// previous one into dst (pageable memory takes its transfers slowly and its
-// first touch is paid in the copy; spread over threads, both go faster).
-constexpr size_t TSG_COPY_PIECE = (size_t) 64 << 20;
+// is pinned host memory or tiny; otherwise through a ring of pinned pieces,
+// each piece's transfer running while host threads copy earlier ones into
+// dst (pageable memory takes its transfers slowly and its first touch is paid
+// in the copy; spread over threads, both go faster).  Pieces of 2 MiB: the
+// last piece's host copy is all that the transfer does not hide.  (144 MB of
+// genotypes: 4.1 ms with two pieces of 64 MiB, threads started per piece; a
+// 50 MB matrix in pageable transfers 4.0 ms.)
+constexpr size_t TSG_COPY_PIECE = (size_t) 2 << 20;
+constexpr int TSG_COPY_RING = 8;
+constexpr size_t TSG_COPY_TINY = (size_t) 64 << 10;
 
 int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t bytes) {
     int ret;
@@ -606,58 +662,93 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
     } else {
         (void) hipGetLastError();
     }
-    if (type == hipMemoryTypeDevice || type == hipMemoryTypeHost || bytes <= TSG_COPY_PIECE ||
+    if (type == hipMemoryTypeDevice || type == hipMemoryTypeHost || bytes <= TSG_COPY_TINY ||
         ws->fixed != nullptr) {
         const hipMemcpyKind kind =
             type == hipMemoryTypeDevice ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
         if ((ret = hip_check(hipMemcpyAsync(dst, src, bytes, kind, s)))) return ret;
         return hip_check(hipStreamSynchronize(s));
     }
-    for (int b = 0; b < 2; b++) {
-        if (ws->cp_h[b] == nullptr && hipHostMalloc(&ws->cp_h[b], TSG_COPY_PIECE) != hipSuccess) {
-            (void) hipGetLastError();
-            ws->cp_h[b] = nullptr;
-            return TSG_ERR_NO_MEMORY;
-        }
+    const size_t np = (bytes + TSG_COPY_PIECE - 1) / TSG_COPY_PIECE;
+    if (ws->cp_h == nullptr &&
+        hipHostMalloc(&ws->cp_h, TSG_COPY_PIECE * TSG_COPY_RING) != hipSuccess) {
+        (void) hipGetLastError();
+        ws->cp_h = nullptr;
+        return TSG_ERR_NO_MEMORY;
+    }
+    for (int b = 0; b < TSG_COPY_RING; b++) {
         if (ws->cp_ev[b] == nullptr &&
             (ret = hip_check(hipEventCreateWithFlags(&ws->cp_ev[b], hipEventDisableTiming)))) {
             return ret;
         }
     }
+    // the copying threads (this one among them): one per 2 pieces, at most 8
     const unsigned hc = std::thread::hardware_concurrency();
-    const size_t T = std::max<size_t>(1, std::min<size_t>(8, hc == 0 ? 1 : hc));
-    auto host_copy = [&](char *to, const char *from, size_t n) {
-        const size_t per = (n + T - 1) / T;
-        std::vector<std::thread> pool;
-        for (size_t t = 1; t < T && t * per < n; t++) {
-            pool.emplace_back([=]() { std::memcpy(to + t * per, from + t * per, std::min(per, n - t * per)); });
-        }
-        std::memcpy(to, from, std::min(per, n));
-        for (auto &th : pool) th.join();
+    const size_t T = std::max<size_t>(
+        1, std::min<size_t>({8, hc == 0 ? 1 : hc, (np + 1) / 2}));
+    std::atomic<size_t> ready{0};  // pieces arrived in their pinned buffers
+    std::atomic<bool> failed{false};
+    std::vector<std::atomic<int>> done(np);  // threads through with each piece
+    for (auto &d : done) d.store(0, std::memory_order_relaxed);
+    auto size_of = [&](size_t i) { return std::min(TSG_COPY_PIECE, bytes - i * TSG_COPY_PIECE); };
+    auto share = [&](size_t i, size_t t) {  // thread t's part of piece i
+        const size_t n = size_of(i), per = ((n + T - 1) / T + 63) & ~(size_t) 63;
+        const size_t from = std::min(n, t * per), to = std::min(n, from + per);
+        std::memcpy((char *) dst + i * TSG_COPY_PIECE + from,
+                    (const char *) ws->cp_h + (i % TSG_COPY_RING) * TSG_COPY_PIECE + from,
+                    to - from);
+        done[i].fetch_add(1, std::memory_order_release);
     };
-    const size_t np = (bytes + TSG_COPY_PIECE - 1) / TSG_COPY_PIECE;
-    for (size_t i = 0; i <= np; i++) {
-        if (i < np) {
-            const size_t off = i * TSG_COPY_PIECE, n = std::min(TSG_COPY_PIECE, bytes - off);
-            const int b = (int) (i & 1);
-            if ((ret = hip_check(hipMemcpyAsync(ws->cp_h[b], (const char *) src + off, n,
-                                                hipMemcpyDeviceToHost, s))) ||
-                (ret = hip_check(hipEventRecord(ws->cp_ev[b], s)))) {
-                (void) hipStreamSynchronize(s);
-                return ret;
+    auto worker = [&](size_t t) {
+        for (size_t i = 0; i < np; i++) {
+            while (ready.load(std::memory_order_acquire) <= i) {
+                if (failed.load(std::memory_order_relaxed)) return;
+                std::this_thread::yield();
             }
+            share(i, t);
         }
-        if (i >= 1) {  // piece i - 1 has arrived in its pinned buffer
-            const size_t off = (i - 1) * TSG_COPY_PIECE, n = std::min(TSG_COPY_PIECE, bytes - off);
-            const int b = (int) ((i - 1) & 1);
-            if ((ret = hip_check(hipEventSynchronize(ws->cp_ev[b])))) {
-                (void) hipStreamSynchronize(s);
-                return ret;
-            }
-            host_copy((char *) dst + off, (const char *) ws->cp_h[b], n);
+    };
+    std::vector<std::thread> pool;
+    auto send = [&](size_t i) {
+        const int b = (int) (i % TSG_COPY_RING);
+        const int e = hip_check(hipMemcpyAsync((char *) ws->cp_h + b * TSG_COPY_PIECE,
+                                               (const char *) src + i * TSG_COPY_PIECE, size_of(i),
+                                               hipMemcpyDeviceToHost, s));
+        return e != 0 ? e : hip_check(hipEventRecord(ws->cp_ev[b], s));
+    };
+    size_t sent = 0;
+    ret = 0;
+    for (; ret == 0 && sent < std::min<size_t>(np, TSG_COPY_RING); sent++) ret = send(sent);
+    for (size_t t = 1; ret == 0 && t < T; t++) {
+        try {
+            pool.emplace_back(worker, t);
+        } catch (const std::system_error &) {  // no more threads: this one does their share
+            break;
         }
     }
-    return hip_check(hipStreamSynchronize(s));
+    const size_t mine = pool.size() + 1;
+    for (size_t i = 0; ret == 0 && i < np; i++) {
+        if ((ret = hip_check(hipEventSynchronize(ws->cp_ev[i % TSG_COPY_RING])))) break;
+        ready.store(i + 1, std::memory_order_release);
+        share(i, 0);
+        for (size_t t = mine; t < T; t++) share(i, t);
+        // refill the buffers every thread is through with
+        while (ret == 0 && sent < np &&
+               done[sent - TSG_COPY_RING].load(std::memory_order_acquire) == (int) T) {
+            ret = send(sent++);
+        }
+        // the next piece has to be on its way
+        while (ret == 0 && sent < np && sent <= i + 1) {
+            while (done[sent - TSG_COPY_RING].load(std::memory_order_acquire) != (int) T) {
+                std::this_thread::yield();
+            }
+            ret = send(sent++);
+        }
+    }
+    if (ret != 0) failed.store(true, std::memory_order_relaxed);
+    for (std::thread &t : pool) t.join();
+    const int sret = hip_check(hipStreamSynchronize(s));
+    return ret != 0 ? ret : sret;
 }
 
 // Device copies of the results of the queries whose buffers are device
@@ -1355,6 +1446,54 @@ constexpr size_t TSG_STATE_DIRECT = (size_t) 256 << 10;
 // launch less).  Decided per query, so that its sums have the same order
 // whatever it is fused with.
 constexpr size_t TSG_STATE_SEGMENTS = (size_t) 256 << 10;
+// ... and where a window has many tiles: the last kernel's threads add up a
+// window's segments one after the other.
+constexpr int32_t TSG_STATE_WINDOW_TILES = 16;
+
+// The evaluation kernels' record of an output.
+TsgStateOut state_out(const TsgOut &o, const Fused &fz) {
+    TsgStateOut t{};
+    t.stat = o.stat;
+    t.polarised = o.flags & 1;
+    const int32_t c[4] = {o.i, o.j, o.k, o.l};
+    for (int i = 0; i < 4; i++) {
+        t.c[i] = c[i];
+        t.n[i] = fz.weighted ? fz.col_total_w[c[i]] : (double) fz.col_total[c[i]];
+    }
+    t.par = o.par;
+    t.cbase = o.cbase;
+    t.ccount = o.ccount;
+    t.samples = o.ni;
+    t.scale = o.inv;
+    switch (o.stat) {
+    case TSG_STAT_DIVERSITY:
+        if (!t.polarised) t.scale *= 2;
+        break;
+    case TSG_STAT_RELATEDNESS:
+        if (!t.polarised) t.scale *= 2;
+        t.coef[0] = 1.0 / t.n[0];
+        t.coef[1] = 1.0 / t.n[1];
+        break;
+    case TSG_STAT_TRAIT_CORRELATION:  // slots: trait, frequency
+        t.c[1] = o.l;
+        t.n[1] = fz.col_total_w[o.l];
+        break;
+    case TSG_STAT_TRAIT_LINEAR_MODEL:
+    case TSG_STAT_RELATEDNESS_WEIGHTED_NONCENTRED:
+        t.scale = 1.0;
+        break;
+    case TSG_STAT_RELATEDNESS_WEIGHTED:  // slots: i, j, frequency
+        t.c[2] = o.l;
+        t.n[2] = fz.col_total_w[o.l];
+        t.coef[0] = fz.opar[o.par];
+        t.coef[1] = fz.opar[o.par + 1];
+        t.scale = 1.0;
+        break;
+    default:
+        break;
+    }
+    return t;
+}
 
 struct StateRun {
     tsg_treeseq *ts = nullptr;
@@ -1369,6 +1508,23 @@ struct StateRun {
     std::vector<char> on_dev;
     const double *results_h = nullptr;
 };
+
+// Whether the hot plan's chunk sweep would take the batch: weighted queries
+// and no-allocation runs are refused where it would not, on any plan.
+bool hot_takes(const tsg_treeseq *ts, const Workspace *ws, const Fused &fz, bool branch) {
+    const int K = fz.K, span = std::min(fz.M, 256);
+    const bool wgt = fz.weighted;
+    const bool hop = branch && tsg_sweep_needs_hop(fz.outs.data(), (int64_t) fz.outs.size(), K,
+                                                   wgt ? 1 : 0,
+                                                   wgt ? fz.col_total_w.data() : nullptr,
+                                                   wgt ? fz.opar.data() : nullptr) != 0;
+    const bool c16 = !wgt && *std::max_element(fz.col_total.begin(), fz.col_total.end()) <= 65535;
+    const size_t words = wgt ? TSG_SLOT_WORDS_W(K, branch) : TSG_SLOT_WORDS(K, c16, branch);
+    const size_t stage = (size_t) (wgt ? TSG_STAGE_INTS_W(K, span, hop)
+                                       : TSG_STAGE_INTS(K, span, hop)) * 4;
+    return ts->hot.usable &&
+           (size_t) ts->hot.max_slots * words * 4 + stage <= (size_t) ws->lds_limit;
+}
 
 int pinned_out(Workspace *ws, size_t bytes) {
     bytes = std::max<size_t>(bytes, 8);
@@ -1417,6 +1573,7 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
                          : TSG_ROW_I32;
     r.branch = r.batch.front()->mode == TSG_STAT_BRANCH;
     r.site = r.batch.back()->mode == TSG_STAT_SITE;
+    if ((wgt || ws->fixed != nullptr) && !hot_takes(ts, ws, fz, r.branch)) return TSG_NOT_ON_STATES;
     const size_t lds = (size_t) ws->lds_limit - 1024;
     if ((r.branch && tsg_state_shmem(K, type, true) > lds) ||
         (r.site && tsg_state_shmem(K, type, false) > lds)) {
@@ -1449,7 +1606,7 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
         t.new_windows = !(qi > 0 && qs[qi - 1].branch == t.branch &&
                           r.batch[qi - 1]->windows == q.windows);
         t.tw = t.new_windows ? (int32_t) tw : qs[qi - 1].tw;
-        if (t.new_windows) tw += (int64_t) tiles + 1;
+        if (t.new_windows) tw += (int64_t) tiles + 1 + t.W + 1;
         for (int m = f.mbase; m < f.mbase + f.M; m++) {
             const TsgOut &o = fz.outs[m];
             if (o.stat == TSG_STAT_RELATEDNESS) {
@@ -1461,7 +1618,8 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
         t.pbase = seg;
         t.cbase = wsum;
         const int64_t own = ((int64_t) tiles + t.W) * t.M * per;
-        t.by_window = (size_t) own * 8 > TSG_STATE_SEGMENTS ? 1 : 0;
+        t.by_window = (size_t) own * 8 > TSG_STATE_SEGMENTS ||
+                              tiles / t.W > TSG_STATE_WINDOW_TILES;
         seg += own;
         t.wbase = (int32_t) wg;
         t.bbase = (int32_t) fg;
@@ -1497,8 +1655,11 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
     if (wg > INT32_MAX || fg > INT32_MAX || tw > INT32_MAX / 2 || fincount > (int64_t) INT32_MAX * 128) {
         return TSG_NOT_ON_STATES;
     }
+    std::vector<TsgStateOut> outs;
+    outs.reserve(fz.outs.size());
+    for (const TsgOut &o : fz.outs) outs.push_back(state_out(o, fz));
     Pack pk;
-    const int p_ps = pk.add(fz.pair_s), p_pc = pk.add(fz.pair_c), p_outs = pk.add(fz.outs);
+    const int p_ps = pk.add(fz.pair_s), p_pc = pk.add(fz.pair_c), p_outs = pk.add(outs);
     const int p_qs = pk.add(qs), p_win = pk.add(fz.wins), p_tot = pk.add(fz.col_total);
     const int p_fin = pk.add(fin), p_ip = pk.add(ipar), p_dp = pk.add(dpar);
     int p_pw = -1, p_tw = -1, p_op = -1;
@@ -1533,6 +1694,7 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
     const TsgStateDevice &d = sp.dev;
     TsgStateArgs &a = r.l.a;
     a = TsgStateArgs{};
+    a.order = d.order;
     a.in = d.in;
     a.ev_state = d.ev_state;
     a.ev_b = d.ev_b;
@@ -1565,7 +1727,7 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
     a.QB = 0;
     while (a.QB < Q && qs[a.QB].branch) a.QB++;
     a.Q = Q;
-    a.outs = pk.dev<const TsgOut>(ws, p_outs);
+    a.outs = pk.dev<const TsgStateOut>(ws, p_outs);
     a.queries = pk.dev<const TsgStateQuery>(ws, p_qs);
     a.windows = pk.dev<const double>(ws, p_win);
     a.tile_w = (int32_t *) ws->state_tw.p;
@@ -1627,6 +1789,237 @@ void state_deliver(const StateRun &r) {
         const Query &q = *r.batch[qi];
         std::memcpy(q.result, src + r.outbase[qi], (q.windows.size() - 1) * (size_t) q.P * 8);
     }
+}
+
+// The plan, columns and counts of a run other than the sweeps' (node
+// statistics, the spectrum): type and rows of the columns, or
+// TSG_NOT_ON_STATES.
+int state_columns(const tsg_treeseq *ts, Workspace *ws, int K,
+                  const std::vector<int32_t> &col_total, TsgStateLaunch &l) {
+    const tsg_stateplan &sp = ts->states;
+    if (!sp.usable || ws->force_full || ws->force_c32 || K < 1 || K > 64) return TSG_NOT_ON_STATES;
+    l.type = *std::max_element(col_total.begin(), col_total.begin() + K) <= 65535 ? TSG_ROW_U16
+                                                                                  : TSG_ROW_I32;
+    const int RW = tsg_state_row_words(K, l.type);
+    const size_t rows = (size_t) sp.num_states * RW * 4;
+    if (rows > TSG_STATE_ROWS_MAX) return TSG_NOT_ON_STATES;
+    const int ret = ensure(ws, ws->state_x, rows);
+    if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? TSG_NOT_ON_STATES : ret;
+    const TsgStateDevice &d = sp.dev;
+    TsgStateArgs &a = l.a;
+    a = TsgStateArgs{};
+    a.order = d.order;
+    a.in = d.in;
+    a.row_ref = d.row_ref;
+    a.row_pos = d.row_pos;
+    a.list_off = d.list_off;
+    a.list_kind = d.list_kind;
+    a.list_ent = d.list_ent;
+    a.num_states = sp.num_states;
+    a.num_samples = ts->num_samples;
+    a.nrow = (int32_t) sp.row_ref.size();
+    a.K = K;
+    a.RW = RW;
+    a.x = (uint32_t *) ws->state_x.p;
+    l.level0 = sp.level0.data();
+    l.levels = (int) sp.level0.size() - 1;
+    return 0;
+}
+
+// The run's host arrays on their way: by its first kernel where they are
+// small.
+int state_send(Workspace *ws, const Pack &pk, TsgStateArgs &a) {
+    if (pk.total > TSG_STATE_DIRECT) return pk.send(ws, ws->stream);
+    const int ret = pk.fill(ws);
+    if (ret != 0) return ret;
+    a.stage_src = (const uint4 *) ws->stage_h;
+    a.stage_dst = (uint4 *) ws->arena.p;
+    a.stage_words = (int64_t) ((pk.total + 15) / 16);
+    return 0;
+}
+
+// The node statistics' and the spectrum's part of the plan, uploaded on
+// first need (called with g_mutex held).
+int ensure_state_nodes(tsg_treeseq *ts) {
+    TsgStateDevice &h = ts->states.dev;
+    if (h.nodes_block != nullptr) return 0;
+    TsgNodeRuns r;
+    tsg_node_runs(ts, r);
+    Arrays b;
+    b.add(h.run_node, r.node);
+    b.add(h.run_piece0, r.piece0);
+    b.add(h.run_state, r.state);
+    b.add(h.run_from, r.from);
+    h.runs = (int32_t) r.node.size();
+    return b.upload(h.nodes_block, h.bytes);
+}
+int ensure_state_spectrum(tsg_treeseq *ts) {
+    TsgStateDevice &h = ts->states.dev;
+    if (h.afs_block != nullptr) return 0;
+    Arrays b;
+    b.add(h.row_all, ts->states.row_all);
+    b.add(h.pieces, ts->states.pieces);
+    return b.upload(h.afs_block, h.bytes);
+}
+
+// A node-mode query on the state plan (trees.c:1788-1918), or
+// TSG_NOT_ON_STATES.
+int run_node_states(tsg_treeseq *ts, Query &q, const Fused &fz, Workspace *ws) {
+    StateRun r;
+    TsgStateLaunch &l = r.l;
+    int ret = state_columns(ts, ws, fz.K, fz.col_total, l);
+    if (ret != 0) return ret;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        if ((ret = ensure_state_nodes(ts))) return ret;
+    }
+    const int W = (int) q.windows.size() - 1;
+    const int64_t N = ts->num_nodes;
+    const bool composed = q.final_kind != TSG_FINAL_NONE;
+    const int64_t nres = (int64_t) W * N * fz.M, nout = (int64_t) W * N * q.P;
+    std::vector<TsgStateOut> outs;
+    for (const TsgOut &o : fz.outs) outs.push_back(state_out(o, fz));
+    std::vector<TsgStateQuery> qs(1);
+    qs[0].W = W;
+    qs[0].M = fz.M;
+    for (const TsgOut &o : fz.outs) {
+        if (o.stat == TSG_STAT_RELATEDNESS) {
+            qs[0].rel_c0 = o.cbase;
+            qs[0].rel_cn = o.ccount;
+        }
+    }
+    std::vector<TsgFinalHost> fin(1);
+    fin[0].kind = q.final_kind;
+    fin[0].Kq = (int32_t) q.sets.size();
+    fin[0].P = q.P;
+    fin[0].W = (int32_t) (W * N);
+    fin[0].Mraw = fz.M;
+    Pack pk;
+    const int p_ps = pk.add(fz.pair_s), p_pc = pk.add(fz.pair_c), p_tot = pk.add(fz.col_total);
+    const int p_outs = pk.add(outs), p_qs = pk.add(qs), p_win = pk.add(q.windows);
+    const int p_fin = pk.add(fin), p_ip = pk.add(q.fin_ipar), p_dp = pk.add(q.fin_dpar);
+    TsgStateArgs &a = l.a;
+    if ((ret = ensure(ws->raw, (size_t) nres * 8)) ||
+        (composed && (ret = ensure(ws->out, (size_t) nout * 8))) ||
+        (ret = state_send(ws, pk, a))) {
+        return ret;
+    }
+    a.npairs = (int32_t) fz.pair_s.size();
+    a.pair_sample = pk.dev<const int32_t>(ws, p_ps);
+    a.pair_col = pk.dev<const int32_t>(ws, p_pc);
+    a.col_total = pk.dev<const int32_t>(ws, p_tot);
+    a.outs = pk.dev<const TsgStateOut>(ws, p_outs);
+    a.queries = pk.dev<const TsgStateQuery>(ws, p_qs);
+    a.windows = pk.dev<const double>(ws, p_win);
+    const TsgStateDevice &d = ts->states.dev;
+    const TsgNodeArgs g{d.run_node, d.run_piece0, d.run_state, d.run_from, d.runs,
+                        N,          ts->L,        (double *) ws->raw.p};
+    hipStream_t s = ws->stream;
+    const uint32_t flags = q.span_normalise ? TSG_F_SPAN_NORMALISE : 0u;
+    if ((ret = hip_check(tsg_launch_fill_f64(g.res, nres, s)))) return ret;
+    if ((ret = hip_check(tsg_launch_state_counts(l, ws->profile ? ws->ev0 : nullptr, s))) ||
+        (ret = hip_check(tsg_launch_state_nodes(l, g, fz.M, s)))) {
+        return ret;
+    }
+    if (ws->profile) (void) hipEventRecord(ws->ev1, s);
+    if (flags != 0 && (ret = hip_check(tsg_launch_afs_branch_final(g.res, a.windows, W, N * fz.M,
+                                                                   flags, s)))) {
+        return ret;
+    }
+    if (composed && (ret = hip_check(tsg_launch_finals(
+                         pk.dev<const void>(ws, p_fin), 1, g.res, pk.dev<const int32_t>(ws, p_ip),
+                         pk.dev<const double>(ws, p_dp), (double *) ws->out.p, nout, s)))) {
+        return ret;
+    }
+    ws->last_store = TSG_STORE_HOT;
+    if ((ret = copy_out(ws, s, q.result, composed ? ws->out.p : ws->raw.p, (size_t) nout * 8))) {
+        return ret;
+    }
+    if (ws->profile) {
+        float ms = 0;
+        (void) hipEventElapsedTime(&ms, ws->ev0, ws->ev1);
+        ws->sweep_ms += ms;
+        ws->sweep_launches += 1;
+    }
+    return 0;
+}
+
+// The allele frequency spectrum on the state plan, or TSG_NOT_ON_STATES.
+int run_spectrum_states(tsg_treeseq *ts, const std::vector<std::vector<int32_t>> &sets,
+                        const std::vector<double> &win, const std::vector<double> &tw,
+                        const std::vector<int64_t> &dims, int64_t size, bool branch,
+                        uint32_t options, double *result, Workspace *ws) {
+    TsgStateLaunch l;
+    const int K = (int) sets.size();
+    std::vector<int32_t> pair_s, pair_c, col_total;
+    for (int k = 0; k < K; k++) {
+        for (int32_t s : sets[k]) {
+            pair_s.push_back(s);
+            pair_c.push_back(k);
+        }
+        col_total.push_back((int32_t) sets[k].size());
+    }
+    int ret = state_columns(ts, ws, K, col_total, l);
+    if (ret != 0) return ret;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        if ((ret = ensure_state_spectrum(ts))) return ret;
+    }
+    const int W = (int) win.size() - 1, TW = (int) tw.size() - 1;
+    const int64_t hist = (int64_t) W * TW * size;
+    Pack pk;
+    const int p_ps = pk.add(pair_s), p_pc = pk.add(pair_c), p_tot = pk.add(col_total);
+    const int p_win = pk.add(win), p_tw = pk.add(tw), p_dims = pk.add(dims);
+    TsgStateArgs &a = l.a;
+    if ((ret = ensure(ws->hist, (size_t) hist * 8)) ||
+        (!branch && (ret = ensure(ws->out, (size_t) hist * 8))) ||
+        (ret = state_send(ws, pk, a))) {
+        return ret;
+    }
+    a.npairs = (int32_t) pair_s.size();
+    a.pair_sample = pk.dev<const int32_t>(ws, p_ps);
+    a.pair_col = pk.dev<const int32_t>(ws, p_pc);
+    a.col_total = pk.dev<const int32_t>(ws, p_tot);
+    const tsg_stateplan &sp = ts->states;
+    TsgSpectrumArgs g{};
+    g.row_all = sp.dev.row_all;
+    g.pieces = sp.dev.pieces;
+    g.npieces = (int32_t) sp.pieces.size();
+    g.polarised = (options & TSG_STAT_POLARISED) ? 1 : 0;
+    g.W = W;
+    g.TW = TW;
+    g.windows = pk.dev<const double>(ws, p_win);
+    g.time_windows = pk.dev<const double>(ws, p_tw);
+    g.dims = pk.dev<const int64_t>(ws, p_dims);
+    g.size = size;
+    g.hist_u = (unsigned long long *) ws->hist.p;
+    g.hist_d = (double *) ws->hist.p;
+    hipStream_t s = ws->stream;
+    const uint32_t flags = (options & TSG_STAT_SPAN_NORMALISE) ? TSG_F_SPAN_NORMALISE : 0u;
+    if ((ret = hip_check(branch ? tsg_launch_fill_f64(g.hist_d, hist, s)
+                                : tsg_launch_fill_u64(g.hist_u, hist, s))) ||
+        (ret = hip_check(tsg_launch_state_counts(l, ws->profile ? ws->ev0 : nullptr, s))) ||
+        (ret = hip_check(tsg_launch_spectrum(l, g, branch, s)))) {
+        return ret;
+    }
+    if (ws->profile) (void) hipEventRecord(ws->ev1, s);
+    if (branch) {
+        ret = flags == 0 ? 0
+                         : hip_check(tsg_launch_afs_branch_final(g.hist_d, g.windows, W,
+                                                                 (int64_t) TW * size, flags, s));
+    } else {
+        ret = hip_check(tsg_launch_afs_site_final(g.hist_u, (double *) ws->out.p, g.windows, W,
+                                                  size, flags, s));
+    }
+    ws->last_store = TSG_STORE_HOT;
+    if (ret == 0) ret = copy_out(ws, s, result, branch ? ws->hist.p : ws->out.p, (size_t) hist * 8);
+    if (ret == 0 && ws->profile) {
+        float ms = 0;
+        (void) hipEventElapsedTime(&ms, ws->ev0, ws->ev1);
+        ws->sweep_ms += ms;
+        ws->sweep_launches += 1;
+    }
+    return ret;
 }
 
 // Queries of one tree sequence (either mode or both) on the state plan, with
@@ -1775,56 +2168,58 @@ int device_upload(tsg_treeseq *ts) {
     }
     int ret;
     TsgDevice &d = ts->dev;
-    size_t &by = d.bytes;
-    std::vector<int32_t> site_nalleles = ts->site_nalleles;
-    if ((ret = upload_ptr(&d.breakpoints, ts->breakpoints, by)) ||
-        (ret = upload_ptr(&d.tree_site0, ts->tree_site0, by)) ||
-        (ret = upload_ptr(&d.site_pos, ts->site_pos, by)) ||
-        (ret = upload_ptr(&d.site_mut0, ts->site_mut0, by)) ||
-        (ret = upload_ptr(&d.mut_allele, ts->mut_allele, by)) ||
-        (ret = upload_ptr(&d.mut_pallele, ts->mut_pallele, by)) ||
-        (ret = upload_ptr(&d.site_nalleles, site_nalleles, by))) {
-        return ret;
+    if (d.block == nullptr) {
+        Arrays b;
+        b.add(d.breakpoints, ts->breakpoints);
+        b.add(d.tree_site0, ts->tree_site0);
+        b.add(d.site_pos, ts->site_pos);
+        b.add(d.site_mut0, ts->site_mut0);
+        b.add(d.mut_allele, ts->mut_allele);
+        b.add(d.mut_pallele, ts->mut_pallele);
+        b.add(d.site_nalleles, ts->site_nalleles);
+        if ((ret = b.upload(d.block, d.bytes))) return ret;
     }
-    if (ts->hot.usable) {
+    if (ts->hot.usable && ts->hot.dev.block == nullptr) {
         const tsg_hotplan &hp = ts->hot;
         TsgHotDevice &h = ts->hot.dev;
-        size_t &hb = h.bytes;
-        if ((ret = upload_ptr(&h.chunk_tree0, hp.chunk_tree0, hb)) ||
-            (ret = upload_ptr(&h.chunk_slot0, hp.chunk_slot0, hb)) ||
-            (ret = upload_ptr(&h.slot_par, hp.slot_par, hb)) ||
-            (ret = upload_ptr(&h.slot_bl0, hp.slot_bl0, hb)) ||
-            (ret = upload_ptr(&h.chunk_lev0, hp.chunk_lev0, hb)) ||
-            (ret = upload_ptr(&h.lev_slot0, hp.lev_slot0, hb)) ||
-            (ret = upload_ptr(&h.sample_slot, block_sample_map(hp.sample_slot, hp.num_chunks,
-                                                              ts->num_samples), hb)) ||
-            (ret = upload_ptr(&h.tr_off, hp.tr_off, hb)) ||
-            (ret = upload_ptr(&h.tr_nrem, hp.tr_nrem, hb)) ||
-            (ret = upload_ptr(&h.ev_child, hp.ev_child, hb)) ||
-            (ret = upload_ptr(&h.ev_bl, hp.ev_bl, hb)) ||
-            (ret = upload_ptr(&h.ev_path0, hp.ev_path0, hb)) ||
-            (ret = upload_ptr(&h.path, hp.path, hb)) ||
-            (ret = upload_ptr(&h.mut_slot, hp.mut_slot, hb)) ||
-            (ret = upload_ptr(&h.t0_parent, hp.t0_parent, hb)) ||
-            (ret = upload_ptr(&h.t0_bl, hp.t0_bl, hb))) {
-            return ret;
-        }
+        const std::vector<uint16_t> map =
+            block_sample_map(hp.sample_slot, hp.num_chunks, ts->num_samples);
+        Arrays b;
+        b.add(h.chunk_tree0, hp.chunk_tree0);
+        b.add(h.chunk_slot0, hp.chunk_slot0);
+        b.add(h.slot_par, hp.slot_par);
+        b.add(h.slot_bl0, hp.slot_bl0);
+        b.add(h.chunk_lev0, hp.chunk_lev0);
+        b.add(h.lev_slot0, hp.lev_slot0);
+        b.add(h.sample_slot, map);
+        b.add(h.tr_off, hp.tr_off);
+        b.add(h.tr_nrem, hp.tr_nrem);
+        b.add(h.ev_child, hp.ev_child);
+        b.add(h.ev_bl, hp.ev_bl);
+        b.add(h.ev_path0, hp.ev_path0);
+        b.add(h.path, hp.path);
+        b.add(h.mut_slot, hp.mut_slot);
+        b.add(h.t0_parent, hp.t0_parent);
+        b.add(h.t0_bl, hp.t0_bl);
+        if ((ret = b.upload(h.block, h.bytes))) return ret;
     }
-    if (ts->states.usable) {
+    if (ts->states.usable && ts->states.dev.block == nullptr) {
         const tsg_stateplan &sp = ts->states;
         TsgStateDevice &h = ts->states.dev;
-        size_t &hb = h.bytes;
-        if ((ret = upload_ptr(&h.in, sp.in, hb)) || (ret = upload_ptr(&h.ev_state, sp.ev_state, hb)) ||
-            (ret = upload_ptr(&h.ev_b, sp.ev_b, hb)) || (ret = upload_ptr(&h.ev_pos, sp.ev_pos, hb)) ||
-            (ret = upload_ptr(&h.row_ref, sp.row_ref, hb)) ||
-            (ret = upload_ptr(&h.row_pos, sp.row_pos, hb)) ||
-            (ret = upload_ptr(&h.list_off, sp.list_off, hb)) ||
-            (ret = upload_ptr(&h.list_kind, sp.list_kind, hb)) ||
-            (ret = upload_ptr(&h.list_ent, sp.list_ent, hb)) ||
-            (ret = upload_ptr(&h.btile_pos, sp.btile_pos, hb)) ||
-            (ret = upload_ptr(&h.stile_pos, sp.stile_pos, hb))) {
-            return ret;
-        }
+        Arrays b;
+        if (!sp.order.empty()) b.add(h.order, sp.order);
+        b.add(h.in, sp.in);
+        b.add(h.ev_state, sp.ev_state);
+        b.add(h.ev_b, sp.ev_b);
+        b.add(h.ev_pos, sp.ev_pos);
+        b.add(h.row_ref, sp.row_ref);
+        b.add(h.row_pos, sp.row_pos);
+        b.add(h.list_off, sp.list_off);
+        b.add(h.list_kind, sp.list_kind);
+        b.add(h.list_ent, sp.list_ent);
+        b.add(h.btile_pos, sp.btile_pos);
+        b.add(h.stile_pos, sp.stile_pos);
+        if ((ret = b.upload(h.block, h.bytes))) return ret;
     }
     d.device = dev;
     return 0;
@@ -1923,6 +2318,7 @@ int run_node(tsg_treeseq *ts, Query &q) {
     Workspace *ws = lease.ws;
     if (ws == nullptr) return TSG_ERR_DEVICE;
     if (shmem > (size_t) ws->lds_limit) return TSG_ERR_UNSUPPORTED_INPUT;
+    if ((ret = run_node_states(ts, q, fz, ws)) != TSG_NOT_ON_STATES) return ret;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
         if ((ret = ensure_hot_node(ts))) return ret;
@@ -2027,9 +2423,9 @@ void free_one_workspace(Workspace *ws) {
     if (ws->stage_h != nullptr) (void) hipHostFree(ws->stage_h);
     if (ws->out_h != nullptr) (void) hipHostFree(ws->out_h);
     if (ws->mout_h != nullptr) (void) hipHostFree(ws->mout_h);
-    for (int b = 0; b < 2; b++) {
-        if (ws->cp_h[b] != nullptr) (void) hipHostFree(ws->cp_h[b]);
-        if (ws->cp_ev[b]) (void) hipEventDestroy(ws->cp_ev[b]);
+    if (ws->cp_h != nullptr) (void) hipHostFree(ws->cp_h);
+    for (hipEvent_t e : ws->cp_ev) {
+        if (e) (void) hipEventDestroy(e);
     }
     if (ws->ev0) (void) hipEventDestroy(ws->ev0);
     if (ws->ev1) (void) hipEventDestroy(ws->ev1);
@@ -2049,37 +2445,32 @@ void free_workspace(tsg_treeseq *ts) {
 
 }  // namespace
 
-void tsg_device_free(TsgDevice *d) {
-    void *ptrs[] = {d->chunk_tree0, d->chunk_node0, d->loc_parent0, d->loc_bl0, d->loc_time,
-                    d->loc_lastrem, d->tr_off, d->tr_nrem, d->ev_child, d->ev_parent, d->ev_bl,
-                    d->ev_path0, d->path,
-                    d->breakpoints, d->tree_site0, d->site_pos, d->site_mut0, d->mut_node,
-                    d->mut_allele, d->mut_pallele, d->site_nalleles};
+namespace {
+void free_all(std::initializer_list<void *> ptrs) {
     for (void *p : ptrs) {
         if (p != nullptr) (void) hipFree(p);
     }
+}
+}  // namespace
+
+// (the arrays of a block are freed with it; the others were uploaded on
+// first use, each on its own)
+void tsg_device_free(TsgDevice *d) {
+    free_all({d->block, d->chunk_tree0, d->chunk_node0, d->loc_parent0, d->loc_bl0, d->loc_time,
+              d->loc_lastrem, d->tr_off, d->tr_nrem, d->ev_child, d->ev_parent, d->ev_bl,
+              d->ev_path0, d->path, d->mut_node});
     *d = TsgDevice();
 }
 
 void tsg_hot_device_free(TsgHotDevice *h) {
-    void *ptrs[] = {h->chunk_tree0, h->chunk_slot0, h->slot_par, h->slot_bl0, h->chunk_lev0,
-                    h->lev_slot0, h->sample_slot, h->tr_off, h->tr_nrem, h->ev_child, h->ev_bl,
-                    h->ev_path0, h->path, h->mut_slot, h->t0_parent, h->t0_bl,
-                    h->slot_nsd, h->slot_tu, h->slot_last0, h->slot_ins0, h->slot_tp0,
-                    h->tl_parent, h->tl_time, h->tl_last, h->tl_ins, h->slot_node,
-                    h->node_last, h->node_lid};
-    for (void *p : ptrs) {
-        if (p != nullptr) (void) hipFree(p);
-    }
+    free_all({h->block, h->slot_nsd, h->slot_tu, h->slot_last0, h->slot_ins0, h->slot_tp0,
+              h->tl_parent, h->tl_time, h->tl_last, h->tl_ins, h->slot_node, h->node_last,
+              h->node_lid});
     *h = TsgHotDevice();
 }
 
 void tsg_state_device_free(TsgStateDevice *h) {
-    void *ptrs[] = {h->in, h->ev_state, h->ev_b, h->ev_pos, h->row_ref, h->row_pos, h->list_off,
-                    h->list_kind, h->list_ent, h->btile_pos, h->stile_pos};
-    for (void *p : ptrs) {
-        if (p != nullptr) (void) hipFree(p);
-    }
+    free_all({h->block, h->nodes_block, h->afs_block});
     *h = TsgStateDevice();
 }
 
@@ -2463,7 +2854,7 @@ int tsg_treeseq_get_state_plan_sizes(const tsg_treeseq *ts, uint64_t *sizes) {
     return 0;
 }
 
-int tsg_treeseq_copy_state_plan(const tsg_treeseq *ts, int32_t *level0, int32_t *in,
+int tsg_treeseq_copy_state_plan(const tsg_treeseq *ts, int32_t *level0, int32_t *order, int32_t *in,
                                 int32_t *ev_state, double *ev_b, double *ev_pos, int32_t *row_ref,
                                 double *row_pos, int32_t *list_off, int32_t *list_kind,
                                 int32_t *list_ent) {
@@ -2472,6 +2863,10 @@ int tsg_treeseq_copy_state_plan(const tsg_treeseq *ts, int32_t *level0, int32_t 
         if (dst != nullptr) std::copy(src.begin(), src.end(), dst);
     };
     put(level0, sp.level0);
+    if (order != nullptr) {
+        std::iota(order, order + sp.num_states, 0);
+        put(order, sp.order);
+    }
     put(in, sp.in);
     put(ev_state, sp.ev_state);
     put(ev_b, sp.ev_b);
@@ -3889,7 +4284,7 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
         if (t.ret == TSG_NOT_ON_STATES) continue;
         if (t.ret != 0) return t.ret;
         if (ws0 == nullptr) ws0 = t.ws;
-        byt[t.run.l.type].push_back(&t);
+        byt[2 * t.run.l.type + (t.run.l.a.K > TSG_STATE_F64_COLUMNS)].push_back(&t);
         outcount += t.run.outcount;
     }
     if (ws0 == nullptr) return 0;
@@ -4254,6 +4649,10 @@ int tsg_treeseq_allele_frequency_spectrum(tsg_treeseq *ts, uint64_t K, const uin
     Lease lease(ts);
     Workspace *ws = lease.ws;
     if (ws == nullptr) return TSG_ERR_DEVICE;
+    if ((ret = run_spectrum_states(ts, ss, win, tw, dims, afs_size, branch, options, result, ws)) !=
+        TSG_NOT_ON_STATES) {
+        return ret;
+    }
     hipStream_t s = ws->stream;
     const int KK = (int) K + 1;
     // The hot plan when its slots fit in LDS: per slot KK counts and, for

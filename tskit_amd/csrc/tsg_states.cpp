@@ -9,7 +9,7 @@
 // "The same samples" is decided by a 128-bit sum of pseudo-random sample
 // keys: two different sets agree with probability 2^-128.
 #include <algorithm>
-#include <cstring>
+#include <thread>
 #include <unordered_map>
 
 #include "tsg_states.h"
@@ -35,83 +35,120 @@ struct Wide {
     std::vector<std::vector<int32_t>> members, helper;  // per level
 };
 
+// What the pass keeps of a node: what a walk up a root path reads and writes
+// on one cache line, the rest on the next.
+struct alignas(128) Node {
+    Key key = 0;              // of the samples below
+    double time = 0;
+    double last = 0;          // last update (branch pieces)
+    int32_t par = TSG_NULL, stamp = -1, below = 0, state = 0;
+    int32_t in_state = 0;     // samples below it in the state it is in
+    int32_t last_piece = -1, lc = -1, rs = -1;
+
+    Key old_key = 0;
+    double ins = 0;           // its parent edge's insertion
+    double from = 0;          // where its state began
+    int32_t old_par = TSG_NULL, ls = -1, kids = 0, sample = TSG_NULL, slot = -1;
+};
+
+// Calls work(begin, end) over 0 .. count - 1, on a few threads where there is
+// enough of it.
+template <typename F>
+void over(int64_t count, F work) {
+    const int64_t P = std::max<int64_t>(
+        1, std::min<int64_t>({(int64_t) std::thread::hardware_concurrency(), 8, count / 65536}));
+    std::vector<std::thread> pool;
+    for (int64_t p = 1; p < P; p++) pool.emplace_back(work, count * p / P, count * (p + 1) / P);
+    work(0, count / P);
+    for (auto &th : pool) th.join();
+}
+
 struct Planner {
-    const tsg_treeseq *ts;
-    // states in creation order: their direct inputs, and the inputs after
-    // merging levels, with their level
-    std::vector<int64_t> dir0;
-    std::vector<int32_t> dir, level, in;
+    std::vector<Node> node;
+    // states in creation order: their level after merging, their direct inputs
+    // (two in place, more at `more`), and the inputs after merging levels
+    struct State {
+        int32_t level = 0, count = 0, d0 = 0, d1 = 0;
+    };
+    std::vector<State> state;
+    std::vector<int32_t> more;
+    std::vector<int32_t> *in = nullptr;
     std::unordered_map<int32_t, Wide> wide;
-    std::vector<int32_t> slot_of;
-    int64_t limit = 0;
-
-    int32_t n() const { return ts->num_samples; }
-    int32_t first() const { return 1 + ts->num_samples; }
-    int32_t count() const { return (int32_t) level.size(); }
-
-    const int32_t *inputs(int32_t s, int &m) const {
-        m = (int) (dir0[s + 1] - dir0[s]);
-        return dir.data() + dir0[s];
-    }
 
     // A new state summing list[0..m), m <= TSG_STATE_IN.  The deepest inputs
     // are replaced by their own inputs while the list has room: fewer levels
-    // (one launch each) for more gathers a state.  Measured on 2.8 M states
-    // of 20000 samples: 44 levels of 2 inputs, 16 of up to 4, 8 of up to 8.
+    // (one launch each) for more gathers a state.  On 2.8 M states of 20000
+    // samples: 44 levels of 2 inputs, 16 of up to 4, 8 of up to 8.
     int32_t add(const int32_t *list, int m) {
-        const int32_t id = count();
-        for (int i = 0; i < m; i++) dir.push_back(list[i]);
-        dir0.push_back((int64_t) dir.size());
-        int32_t l[TSG_STATE_IN];
-        std::copy(list, list + m, l);
-        for (;;) {
-            int deep = -1;
-            for (int i = 0; i < m; i++) {
-                if (level[l[i]] > 0 && (deep < 0 || level[l[i]] > level[l[deep]])) deep = i;
-            }
-            if (deep < 0) break;
-            int k;
-            const int32_t *src = inputs(l[deep], k);
-            if (m - 1 + k > TSG_STATE_IN) break;
-            l[deep] = src[0];
-            for (int i = 1; i < k; i++) l[m++] = src[i];
+        const int32_t id = (int32_t) state.size();
+        State made;
+        made.count = m;
+        if (m == 2) {
+            made.d0 = list[0];
+            made.d1 = list[1];
+        } else {
+            made.d0 = (int32_t) more.size();
+            more.insert(more.end(), list, list + m);
         }
-        int32_t lev = 0;
-        for (int i = 0; i < m; i++) lev = std::max(lev, level[l[i]]);
-        level.push_back(lev + 1);
-        for (int i = 0; i < TSG_STATE_IN; i++) in.push_back(i < m ? l[i] : 0);
+        const State *const st = state.data();
+        int32_t l[TSG_STATE_IN] = {}, lev[TSG_STATE_IN] = {};
+        for (int i = 0; i < m; i++) {
+            l[i] = list[i];
+            lev[i] = st[list[i]].level;
+        }
+        int32_t most;
+        for (;;) {
+            int32_t top = 0;  // level and place of the deepest input
+            for (int i = 0; i < TSG_STATE_IN; i++) top = std::max(top, lev[i] * TSG_STATE_IN + i);
+            most = top / TSG_STATE_IN;
+            if (most == 0) break;
+            const int deep = top % TSG_STATE_IN;
+            const State d = st[l[deep]];
+            if (m - 1 + d.count > TSG_STATE_IN) break;
+            if (d.count == 2) {
+                l[deep] = d.d0;
+                lev[deep] = st[d.d0].level;
+                l[m] = d.d1;
+                lev[m++] = st[d.d1].level;
+                continue;
+            }
+            const int32_t *src = more.data() + d.d0;
+            l[deep] = src[0];
+            lev[deep] = st[src[0]].level;
+            for (int i = 1; i < d.count; i++, m++) {
+                l[m] = src[i];
+                lev[m] = st[src[i]].level;
+            }
+        }
+        made.level = most + 1;
+        state.push_back(made);
+        in->insert(in->end(), l, l + TSG_STATE_IN);
         return id;
     }
 
-    // the state summing the inputs given: an existing one where there is at
-    // most one, helper states over groups where there are many
     int32_t sum(const int32_t *list, int m) {
-        if (m == 0) return 0;
-        if (m == 1) return list[0];
-        return add(list, m);
+        return m == 0 ? 0 : m == 1 ? list[0] : add(list, m);
     }
 
-    int32_t sum_wide(int32_t u, const std::vector<int32_t> &par, const std::vector<int32_t> &lc,
-                     const std::vector<int32_t> &rs, const std::vector<int32_t> &state) {
+    int32_t sum_wide(int32_t u) {
         Wide &w = wide[u];
         for (int32_t &c : w.slots) {
-            if (c >= 0 && par[c] != u) c = -1;
+            if (c >= 0 && node[c].par != u) c = -1;
         }
         size_t hole = 0;
-        for (int32_t c = lc[u]; c >= 0; c = rs[c]) {
-            if (slot_of[c] >= 0 && (size_t) slot_of[c] < w.slots.size() &&
-                w.slots[slot_of[c]] == c) {
-                continue;
-            }
+        for (int32_t c = node[u].lc; c >= 0; c = node[c].rs) {
+            const int32_t at = node[c].slot;
+            if (at >= 0 && (size_t) at < w.slots.size() && w.slots[at] == c) continue;
             while (hole < w.slots.size() && w.slots[hole] >= 0) hole++;
             if (hole == w.slots.size()) w.slots.push_back(-1);
             w.slots[hole] = c;
-            slot_of[c] = (int32_t) hole;
+            node[c].slot = (int32_t) hole;
         }
         std::vector<int32_t> cur(w.slots.size());
-        for (size_t i = 0; i < cur.size(); i++) cur[i] = w.slots[i] >= 0 ? state[w.slots[i]] : 0;
-        const int32_t own = ts->sample_index_map[u];
-        if (own != TSG_NULL) cur.insert(cur.begin(), 1 + own);
+        for (size_t i = 0; i < cur.size(); i++) {
+            cur[i] = w.slots[i] >= 0 ? node[w.slots[i]].state : 0;
+        }
+        if (node[u].sample != TSG_NULL) cur.insert(cur.begin(), 1 + node[u].sample);
         for (size_t lev = 0; cur.size() > 1; lev++) {
             if (w.members.size() <= lev) {
                 w.members.emplace_back();
@@ -141,6 +178,18 @@ struct Planner {
         }
         return cur.empty() ? 0 : cur[0];
     }
+
+    // the state of u's samples from its children's states
+    int32_t sum_of(int32_t u) {
+        if (node[u].kids + 1 > TSG_STATE_IN) return sum_wide(u);
+        int32_t l[TSG_STATE_IN];
+        int m = 0;
+        if (node[u].sample != TSG_NULL) l[m++] = 1 + node[u].sample;
+        for (int32_t c = node[u].lc; c >= 0; c = node[c].rs) {
+            if (node[c].state != 0) l[m++] = node[c].state;
+        }
+        return sum(l, m);
+    }
 };
 
 }  // namespace
@@ -156,154 +205,221 @@ int tsg_build_states(tsg_treeseq *ts) {
     const int32_t N = ts->num_nodes, E = ts->num_edges, T = ts->num_trees, n = ts->num_samples;
     const int32_t *I = ts->I.data(), *O = ts->O.data();
     constexpr int32_t MOST_LEVELS = 64;
+    // States from which they are numbered by level, so that a level's inputs
+    // and rows are contiguous; below, the plan is a few MB and stays as made,
+    // with a list of each level's states (half the memory written here).
+    constexpr int64_t RENUMBER = 1 << 18;
+    const int64_t most = 16 * ((int64_t) E + n) + 1024;
     Planner P;
-    P.ts = ts;
-    P.limit = 16 * ((int64_t) E + n) + 1024;
-    P.level.assign(1 + (size_t) n, 0);
-    P.dir0.assign(2 + (size_t) n, 0);
-    P.slot_of.assign(N, -1);
-    std::vector<int32_t> par(N, TSG_NULL), lc(N, -1), ls(N, -1), rs(N, -1), nch(N, 0);
-    std::vector<int32_t> state(N, 0), stamp(N, -1), old_par(N, TSG_NULL), touched;
-    std::vector<Key> key(N, 0), old_key(N, 0);
+    P.state.assign(1 + (size_t) n, Planner::State());
+    P.node.assign(N, Node());
+    Node *const node = P.node.data();
     for (int32_t u = 0; u < N; u++) {
-        const int32_t s = ts->sample_index_map[u];
+        node[u].time = ts->time[u];
+        const int32_t s = node[u].sample = ts->sample_index_map[u];
         if (s == TSG_NULL) continue;
-        state[u] = 1 + s;
-        key[u] = ((Key) mix64(2 * (uint64_t) s + 1) << 64) | mix64(2 * (uint64_t) s + 2);
+        node[u].state = 1 + s;
+        node[u].below = node[u].in_state = 1;
+        node[u].key = ((Key) mix64(2 * (uint64_t) s + 1) << 64) | mix64(2 * (uint64_t) s + 2);
     }
-    std::vector<int32_t> ev_state, row_ref, list_ent;
-    auto branch = [&](int32_t u, int32_t p) { return ts->time[p] - ts->time[u]; };
+    // (about 3 states and 6 events an edge on coalescent trees)
+    P.in = &sp.in;
+    P.state.reserve((size_t) n + 3 * (size_t) E);
+    sp.in.reserve((size_t) E * 3 * TSG_STATE_IN);
+    sp.ev_state.reserve((size_t) E * 6);
+    sp.ev_b.reserve((size_t) E * 6);
+    sp.ev_pos.reserve((size_t) E * 6);
+    sp.node_pieces.reserve((size_t) E * 4);
+    sp.pieces.reserve((size_t) E * 4);
+    auto event = [&](double b, double x, int32_t state) {
+        sp.ev_state.push_back(state);
+        sp.ev_b.push_back(b);
+        sp.ev_pos.push_back(x);
+    };
+    std::vector<int32_t> touched;
+    // the branch piece of u that ends here (see tsg_states.h)
+    auto update = [&](Node &v, double x) {
+        const double from = v.last;
+        if (!(from < x)) return;
+        v.last = x;
+        if (v.par == TSG_NULL || v.in_state <= 0 || v.in_state >= n) return;
+        const double tp = node[v.par].time;
+        if (v.last_piece >= 0) {
+            TsgBranchPiece &l = sp.pieces[v.last_piece];
+            if (l.to == from && l.state == v.state && l.tp == tp && l.ins == v.ins) {
+                l.to = x;
+                return;
+            }
+        }
+        v.last_piece = (int32_t) sp.pieces.size();
+        sp.pieces.push_back({v.time, tp, v.ins, from, x, v.state, 0});
+    };
     sp.list_off.assign(1, 0);
     int32_t j = 0, k = 0;
-    std::vector<int32_t> kids;
     for (int32_t t = 0; t < T; t++) {
         const double x = ts->breakpoints[t];
         touched.clear();
-        auto touch = [&](int32_t u) {
-            if (stamp[u] == t) return;
-            stamp[u] = t;
-            old_key[u] = key[u];
-            old_par[u] = par[u];
+        auto touch = [&](Node &v, int32_t u) {
+            if (v.stamp == t) return;
+            v.stamp = t;
+            v.old_key = v.key;
+            v.old_par = v.par;
             touched.push_back(u);
+        };
+        auto walk = [&](int32_t p, Key d, int32_t b) {  // up the root path
+            for (int32_t u = p; u != TSG_NULL; u = node[u].par) {
+                Node &v = node[u];
+                touch(v, u);
+                update(v, x);
+                v.key += d;
+                v.below += b;
+            }
         };
         while (k < E && ts->right[O[k]] == x) {
             const int32_t p = ts->parent[O[k]], c = ts->child[O[k]];
             k++;
-            touch(c);
-            for (int32_t u = p; u != TSG_NULL; u = par[u]) {
-                touch(u);
-                key[u] -= key[c];
-            }
-            if (ls[c] >= 0) rs[ls[c]] = rs[c];
-            else lc[p] = rs[c];
-            if (rs[c] >= 0) ls[rs[c]] = ls[c];
-            ls[c] = rs[c] = -1;
-            par[c] = TSG_NULL;
-            nch[p]--;
+            Node &v = node[c];
+            touch(v, c);
+            update(v, x);
+            walk(p, -v.key, -v.below);
+            if (v.ls >= 0) node[v.ls].rs = v.rs;
+            else node[p].lc = v.rs;
+            if (v.rs >= 0) node[v.rs].ls = v.ls;
+            v.ls = v.rs = -1;
+            v.par = TSG_NULL;
+            node[p].kids--;
         }
         while (j < E && ts->left[I[j]] == x) {
             const int32_t p = ts->parent[I[j]], c = ts->child[I[j]];
             j++;
-            touch(c);
-            for (int32_t u = p; u != TSG_NULL; u = par[u]) {
-                touch(u);
-                key[u] += key[c];
-            }
-            rs[c] = lc[p];
-            if (lc[p] >= 0) ls[lc[p]] = c;
-            lc[p] = c;
-            par[c] = p;
-            nch[p]++;
+            Node &v = node[c];
+            touch(v, c);
+            walk(p, v.key, v.below);
+            v.rs = node[p].lc;
+            if (v.rs >= 0) node[v.rs].ls = c;
+            node[p].lc = c;
+            v.par = p;
+            v.ins = x;
+            node[p].kids++;
         }
-        // children before parents: a child is younger than its parent
-        std::sort(touched.begin(), touched.end(), [&](int32_t a, int32_t b) {
-            return ts->time[a] != ts->time[b] ? ts->time[a] < ts->time[b] : a < b;
-        });
+        // children before parents: a child is younger than its parent (a few
+        // nodes, mostly in runs: by insertion; the first tree's by sorting)
+        auto younger = [&](int32_t a, int32_t b) {
+            return node[a].time != node[b].time ? node[a].time < node[b].time : a < b;
+        };
+        if (touched.size() > 64) {
+            std::sort(touched.begin(), touched.end(), younger);
+        } else {
+            for (size_t i = 1; i < touched.size(); i++) {
+                const int32_t u = touched[i];
+                size_t h = i;
+                for (; h > 0 && younger(u, touched[h - 1]); h--) touched[h] = touched[h - 1];
+                touched[h] = u;
+            }
+        }
         for (int32_t u : touched) {
-            const bool moved = key[u] != old_key[u];
-            const double was = old_par[u] != TSG_NULL ? branch(u, old_par[u]) : 0.0;
-            const double now = par[u] != TSG_NULL ? branch(u, par[u]) : 0.0;
-            if (!moved) {
-                if (now != was) {
-                    ev_state.push_back(state[u]);
-                    sp.ev_b.push_back(now - was);
-                    sp.ev_pos.push_back(x);
-                }
+            Node &v = node[u];
+            const double was = v.old_par != TSG_NULL ? node[v.old_par].time - v.time : 0.0;
+            const double now = v.par != TSG_NULL ? node[v.par].time - v.time : 0.0;
+            if (v.key == v.old_key) {
+                if (now != was) event(now - was, x, v.state);
                 continue;
             }
-            if (was != 0.0) {
-                ev_state.push_back(state[u]);
-                sp.ev_b.push_back(-was);
-                sp.ev_pos.push_back(x);
+            if (was != 0.0) event(-was, x, v.state);
+            const int32_t before = v.state;
+            v.state = P.sum_of(u);
+            v.in_state = v.below;
+            if (v.state != before) {
+                if (v.from < x) sp.node_pieces.push_back({u, before, v.from});
+                v.from = x;
             }
-            if (nch[u] + 1 > TSG_STATE_IN) {
-                state[u] = P.sum_wide(u, par, lc, rs, state);
-            } else {
-                int32_t l[TSG_STATE_IN];
-                int m = 0;
-                if (ts->sample_index_map[u] != TSG_NULL) l[m++] = 1 + ts->sample_index_map[u];
-                for (int32_t c = lc[u]; c >= 0; c = rs[c]) {
-                    if (state[c] != 0) l[m++] = state[c];
-                }
-                state[u] = P.sum(l, m);
-            }
-            if (now != 0.0) {
-                ev_state.push_back(state[u]);
-                sp.ev_b.push_back(now);
-                sp.ev_pos.push_back(x);
-            }
+            if (now != 0.0) event(now, x, v.state);
         }
-        if ((int64_t) P.level.size() > P.limit) return 0;
+        if ((int64_t) P.state.size() > most) {
+            sp = tsg_stateplan();
+            return 0;
+        }
         // the rows of this tree's sites, from the states of their mutations'
         // nodes
         for (int32_t s = ts->tree_site0[t]; s < ts->tree_site0[t + 1]; s++) {
             const int32_t m0 = ts->site_mut0[s], m1 = ts->site_mut0[s + 1];
             if (m1 == m0 + 1 && ts->mut_allele[m0] == 1 && ts->mut_pallele[m0] == 0) {
-                row_ref.push_back(state[ts->mut_node[m0]]);
+                const Node &v = node[ts->mut_node[m0]];
+                sp.row_ref.push_back(v.state);
                 sp.row_pos.push_back(ts->site_pos[s]);
+                sp.row_all.push_back(v.in_state);
                 continue;
             }
             for (int32_t al = 0; al < ts->site_nalleles[s]; al++) {
-                row_ref.push_back(-1 - sp.num_lists++);
+                sp.row_ref.push_back(-1 - sp.num_lists++);
                 sp.row_pos.push_back(ts->site_pos[s]);
                 sp.list_kind.push_back(al == 0 ? TSG_ROW_ANCESTRAL : TSG_ROW_DERIVED);
+                int32_t all = al == 0 ? n : 0;
                 for (int32_t m = m0; m < m1; m++) {
-                    const int32_t st = state[ts->mut_node[m]];
-                    if (ts->mut_allele[m] == al) list_ent.push_back(2 * st);
-                    if (ts->mut_pallele[m] == al) list_ent.push_back(2 * st + 1);
+                    const Node &v = node[ts->mut_node[m]];
+                    if (ts->mut_allele[m] == al) {
+                        sp.list_ent.push_back(2 * v.state);
+                        all += v.in_state;
+                    }
+                    if (ts->mut_pallele[m] == al) {
+                        sp.list_ent.push_back(2 * v.state + 1);
+                        all -= v.in_state;
+                    }
                 }
-                sp.list_off.push_back((int32_t) list_ent.size());
+                sp.row_all.push_back(all);
+                sp.list_off.push_back((int32_t) sp.list_ent.size());
             }
         }
     }
-    // number the states by level, within a level as created
-    const int32_t S = P.count();
-    if (S > INT32_MAX / 2 - 1 || ev_state.size() > (size_t) INT32_MAX ||
-        row_ref.size() > (size_t) INT32_MAX || list_ent.size() > (size_t) INT32_MAX) {
+    for (int32_t u = 0; u < N; u++) {
+        update(node[u], ts->L);
+        sp.node_pieces.push_back({u, node[u].state, node[u].from});
+    }
+    const int64_t S = (int64_t) P.state.size();
+    int32_t levels = 0;
+    for (const Planner::State &st : P.state) levels = std::max(levels, st.level + 1);
+    const size_t limit = (size_t) INT32_MAX / 2 - 1;
+    if ((size_t) S > limit || sp.ev_state.size() > limit || sp.row_ref.size() > limit ||
+        sp.list_ent.size() > limit || sp.node_pieces.size() > limit ||
+        sp.pieces.size() > limit || levels > MOST_LEVELS) {
+        sp = tsg_stateplan();
         return 0;
     }
-    int32_t levels = 0;
-    for (int32_t l : P.level) levels = std::max(levels, l + 1);
-    if (levels > MOST_LEVELS) return 0;
+    // the states by level, within a level as created
     sp.level0.assign(levels + 1, 0);
-    for (int32_t l : P.level) sp.level0[l + 1]++;
+    for (const Planner::State &st : P.state) sp.level0[st.level + 1]++;
     for (int32_t l = 0; l < levels; l++) sp.level0[l + 1] += sp.level0[l];
-    std::vector<int32_t> id(S), next(sp.level0.begin(), sp.level0.end() - 1);
-    for (int32_t s = 0; s < S; s++) id[s] = next[P.level[s]]++;
-    const int32_t f = P.first();
-    sp.in.resize((size_t) (S - f) * TSG_STATE_IN);
-    for (int32_t s = f; s < S; s++) {
-        const int32_t *src = P.in.data() + (size_t) (s - f) * TSG_STATE_IN;
-        int32_t *dst = sp.in.data() + (size_t) (id[s] - f) * TSG_STATE_IN;
-        for (int i = 0; i < TSG_STATE_IN; i++) dst[i] = id[src[i]];
+    std::vector<int32_t> next(sp.level0.begin(), sp.level0.end() - 1);
+    std::vector<int32_t> at(S);
+    for (int64_t s = 0; s < S; s++) at[s] = next[P.state[s].level]++;
+    if (S < RENUMBER) {
+        sp.order.resize(S);
+        for (int64_t s = 0; s < S; s++) sp.order[at[s]] = (int32_t) s;
+    } else {
+        const int32_t f = 1 + n;
+        std::vector<int32_t> in(sp.in.size());
+        over(S - f, [&](int64_t b, int64_t e) {
+            for (int64_t s = b; s < e; s++) {
+                const int32_t *src = sp.in.data() + s * TSG_STATE_IN;
+                int32_t *dst = in.data() + (int64_t) (at[s + f] - f) * TSG_STATE_IN;
+                for (int i = 0; i < TSG_STATE_IN; i++) dst[i] = at[src[i]];
+            }
+        });
+        sp.in.swap(in);
+        auto renumber = [&](auto &v, auto state) {
+            over((int64_t) v.size(), [&](int64_t b, int64_t e) {
+                for (int64_t i = b; i < e; i++) state(v[i]) = at[state(v[i])];
+            });
+        };
+        auto whole = [](int32_t &s) -> int32_t & { return s; };
+        auto member = [](auto &p) -> int32_t & { return p.state; };
+        renumber(sp.ev_state, whole);
+        renumber(sp.pieces, member);
+        renumber(sp.node_pieces, member);
+        for (int32_t &r : sp.row_ref) r = r >= 0 ? at[r] : r;
+        for (int32_t &e : sp.list_ent) e = 2 * at[e >> 1] + (e & 1);
     }
-    for (int32_t &s : ev_state) s = id[s];
-    for (int32_t &r : row_ref) r = r >= 0 ? id[r] : r;
-    for (int32_t &e : list_ent) e = 2 * id[e >> 1] + (e & 1);
-    sp.ev_state.swap(ev_state);
-    sp.row_ref.swap(row_ref);
-    sp.list_ent.swap(list_ent);
-    sp.num_states = S;
+    sp.num_states = (int32_t) S;
     auto tiles = [](const std::vector<double> &pos, int tile, int32_t &count,
                     std::vector<double> &first) {
         count = (int32_t) std::max<size_t>(1, (pos.size() + tile - 1) / tile);
@@ -316,4 +432,26 @@ int tsg_build_states(tsg_treeseq *ts) {
     tiles(sp.row_pos, TSG_SITE_TILE, sp.stiles, sp.stile_pos);
     sp.usable = true;
     return 0;
+}
+
+void tsg_node_runs(const tsg_treeseq *ts, TsgNodeRuns &r) {
+    const std::vector<TsgNodePiece> &pieces = ts->states.node_pieces;
+    const int32_t N = ts->num_nodes;
+    std::vector<int32_t> at(N + 1, 0);
+    for (const TsgNodePiece &q : pieces) at[q.node + 1]++;
+    for (int32_t u = 0; u < N; u++) at[u + 1] += at[u];
+    r.state.resize(pieces.size());
+    r.from.resize(pieces.size());
+    for (int32_t u = 0; u < N; u++) {
+        for (int32_t p = at[u]; p < at[u + 1]; p += TSG_NODE_RUN) {
+            r.node.push_back(u);
+            r.piece0.push_back(p);
+        }
+    }
+    r.piece0.push_back((int32_t) pieces.size());
+    for (const TsgNodePiece &q : pieces) {
+        const int32_t to = at[q.node]++;
+        r.state[to] = q.state;
+        r.from[to] = q.from;
+    }
 }

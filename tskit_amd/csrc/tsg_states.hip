@@ -82,6 +82,20 @@ __device__ __forceinline__ int window_of(const double *win, int W, double x) {
     return lo;
 }
 
+// first tile whose successor starts at x or later (or the last tile)
+__device__ __forceinline__ int first_tile(const double *tpos, int tiles, double x) {
+    int lo = 0, hi = tiles - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (tpos[mid + 1] >= x) {
+            hi = mid;
+        } else {
+            lo = mid + 1;
+        }
+    }
+    return lo;
+}
+
 template <int TYPE>
 __device__ __forceinline__ void seed(const TsgStateArgs &a, int64_t b) {
     const int64_t i = b * 256 + threadIdx.x;
@@ -108,9 +122,13 @@ __device__ __forceinline__ void seed(const TsgStateArgs &a, int64_t b) {
     const int t = (int) (j - Q.tw);
     const int tiles = Q.branch ? a.btiles : a.stiles;
     const double *tpos = Q.branch ? a.btile_pos : a.stile_pos;
-    a.tile_w[j] = t == 0 ? 0
-                  : t >= tiles ? Q.W - 1
-                               : window_of(a.windows + Q.win_off, Q.W, tpos[t]);
+    const double *win = a.windows + Q.win_off;
+    if (t <= tiles) {
+        a.tile_w[j] = t == 0 ? 0 : t >= tiles ? Q.W - 1 : window_of(win, Q.W, tpos[t]);
+    } else {
+        const int w = t - (tiles + 1);
+        a.tile_w[j] = w >= Q.W ? tiles - 1 : first_tile(tpos, tiles, win[w]);
+    }
 }
 int64_t seed_blocks(const TsgStateArgs &a) {
     return ((int64_t) a.npairs + a.ntile_w + 255) / 256;
@@ -145,15 +163,16 @@ __device__ __forceinline__ void store_words(uint32_t *p, const Words<V> &r) {
     }
 }
 
-// States s0 .. s1 - 1 of a level, V words a thread.  16-bit counts are added
+// States order[s0 .. s1 - 1] of a level, V words a thread.  16-bit counts are added
 // two to a word: no count exceeds its column's total, so none carries over.
 template <int V, bool F64>
 __device__ __forceinline__ void count(const TsgStateArgs &a, int s0, int s1, int64_t b) {
     const int parts = a.RW / V;
     const int64_t i = b * 256 + threadIdx.x;
-    const int64_t s = s0 + i / parts;
+    int64_t s = s0 + i / parts;
     const int p = (int) (i % parts) * V;
     if (s >= s1) return;
+    if (a.order != nullptr) s = a.order[s];
     const int4 *in =
         reinterpret_cast<const int4 *>(a.in + (s - 1 - a.num_samples) * TSG_STATE_IN);
     const int4 u = in[0], v = in[1];
@@ -196,25 +215,39 @@ __device__ __forceinline__ void count_rw(const TsgStateArgs &a, int s0, int s1, 
 
 // --- evaluation ---------------------------------------------------------------
 
-template <int TYPE>
-struct RowType {
+// What a tile holds a column as.  A site row's counts are sums of additions
+// and subtractions, so site tiles of counts hold 32 bits whatever the rows do.
+template <int TYPE, bool BRANCH, bool WIDE>
+struct TileType {
+    using T = double;
+};
+template <>
+struct TileType<TSG_ROW_U16, true, true> {
     using T = uint16_t;
 };
 template <>
-struct RowType<TSG_ROW_I32> {
+struct TileType<TSG_ROW_U16, false, true> {
     using T = int32_t;
 };
-template <>
-struct RowType<TSG_ROW_F64> {
-    using T = double;
+template <bool BRANCH>
+struct TileType<TSG_ROW_I32, BRANCH, true> {
+    using T = int32_t;
 };
-// A site row's counts are sums of additions and subtractions, so site tiles
-// hold 32-bit counts whatever the rows hold.
-template <int TYPE, bool BRANCH>
-struct TileType {
-    using T = typename std::conditional<!BRANCH && TYPE == TSG_ROW_U16, int32_t,
-                                        typename RowType<TYPE>::T>::type;
-};
+
+// A record of memory that no kernel of the run writes, at an address that is
+// the same for the whole wave: scalar loads.
+template <typename R>
+__device__ __forceinline__ R uniform(const R *p) {
+    typedef const __attribute__((address_space(4))) int32_t *Const;
+    static_assert(sizeof(R) % 4 == 0, "whole words");
+    Const q = (Const) (uintptr_t) p;
+    int32_t w[sizeof(R) / 4];
+#pragma unroll
+    for (size_t i = 0; i < sizeof(R) / 4; i++) w[i] = q[i];
+    R r;
+    __builtin_memcpy(&r, w, sizeof(R));
+    return r;
+}
 
 // first index of 0 .. n with pos[index] >= x (LDS)
 __device__ __forceinline__ int lower_bound(const double *pos, int n, double x) {
@@ -247,8 +280,11 @@ __device__ __forceinline__ double2 load2<double>(const double *col, int i) {
     return reinterpret_cast<const double2 *>(col)[i];
 }
 
-// Summary numerators at the counts x[0..3] (columns i, j, k, l) of sets of
-// n[0..3] samples: one(x) polarised, both(x) = one(x) + one(n - x).
+// Summary numerators at the counts x[0..3] (columns c[0..3]) of sets of
+// n[0..3] samples: one(x) polarised; both(x) = one(x) + one(n - x), an event
+// or a pair row of an unpolarised output; lone(x): a single allele of one.
+// Where one(x) = one(n - x), both(x) is one(x) and the output's scale has
+// the factor 2.
 struct Nums {
     double n[4];
 };
@@ -256,7 +292,8 @@ struct Diversity {
     static constexpr int S = 1;
     Nums p;
     __device__ double one(const double *x) const { return x[0] * (p.n[0] - x[0]); }
-    __device__ double both(const double *x) const { return 2.0 * one(x); }
+    __device__ double both(const double *x) const { return one(x); }
+    __device__ double lone(const double *x) const { return 0.5 * one(x); }
 };
 struct Segregating {
     static constexpr int S = 1;
@@ -266,6 +303,7 @@ struct Segregating {
     __device__ double both(const double *x) const {
         return (x[0] > 0 ? p.n[0] - x[0] : 0.0) + (x[0] < p.n[0] ? x[0] : 0.0);
     }
+    __device__ double lone(const double *x) const { return one(x); }
 };
 struct Y1 {
     static constexpr int S = 1;
@@ -277,6 +315,7 @@ struct Y1 {
     __device__ double both(const double *x) const {
         return x[0] * (p.n[0] - x[0]) * (p.n[0] - 2);
     }
+    __device__ double lone(const double *x) const { return one(x); }
 };
 struct Divergence {
     static constexpr int S = 2;
@@ -285,14 +324,16 @@ struct Divergence {
     __device__ double both(const double *x) const {
         return fma(x[0], p.n[1] - x[1], (p.n[0] - x[0]) * x[1]);
     }
+    __device__ double lone(const double *x) const { return one(x); }
 };
-struct Product {  // non-centred relatedness
+struct Product {  // non-centred relatedness, also of weights
     static constexpr int S = 2;
     Nums p;
     __device__ double one(const double *x) const { return x[0] * x[1]; }
     __device__ double both(const double *x) const {
         return fma(x[0], x[1], (p.n[0] - x[0]) * (p.n[1] - x[1]));
     }
+    __device__ double lone(const double *x) const { return one(x); }
 };
 template <typename D, int SLOTS>
 struct Complement {  // both() from one()
@@ -305,6 +346,7 @@ struct Complement {  // both() from one()
         for (int i = 0; i < SLOTS; i++) y[i] = p.n[i] - x[i];
         return static_cast<const D *>(this)->f(x) + static_cast<const D *>(this)->f(y);
     }
+    __device__ double lone(const double *x) const { return one(x); }
 };
 struct Y2 : Complement<Y2, 2> {
     __device__ double f(const double *x) const {
@@ -337,13 +379,17 @@ struct F4 {
     __device__ double both(const double *x) const {
         return fma(p.n[1], x[0], -(p.n[0] * x[1])) * b(x);
     }
+    __device__ double lone(const double *x) const { return one(x); }
 };
 // centred relatedness: slot 2 is the mean over the query's columns
 struct Relatedness {
-    Nums p;  // 1 / set size
+    static constexpr int S = 3;
+    double ri, rj;  // 1 / set size
     __device__ double one(const double *x) const {
-        return (x[0] * p.n[0] - x[2]) * (x[1] * p.n[1] - x[2]);
+        return (x[0] * ri - x[2]) * (x[1] * rj - x[2]);
     }
+    __device__ double both(const double *x) const { return one(x); }
+    __device__ double lone(const double *x) const { return 0.5 * one(x); }
 };
 // summaries of real-valued weights (p.n: the columns' totals)
 struct TraitCovariance {
@@ -354,29 +400,18 @@ struct TraitCovariance {
         const double y = p.n[0] - x[0];
         return fma(x[0], x[0], y * y);
     }
+    __device__ double lone(const double *x) const { return one(x); }
 };
-struct TraitCorrelation {  // slots: trait, frequency
-    static constexpr int S = 2;
-    Nums p;
-    __device__ double f(double x, double q) const {
-        return (q > 0.0 && q < 1.0) ? (x * x) / (q * (1 - q)) : 0.0;
-    }
-    __device__ double one(const double *x) const { return f(x[0], x[1]); }
-    __device__ double both(const double *x) const {
-        return f(x[0], x[1]) + f(p.n[0] - x[0], p.n[1] - x[1]);
+struct TraitCorrelation : Complement<TraitCorrelation, 2> {  // slots: trait, frequency
+    __device__ double f(const double *x) const {
+        const double q = x[1];
+        return (q > 0.0 && q < 1.0) ? (x[0] * x[0]) / (q * (1 - q)) : 0.0;
     }
 };
-struct RelatednessWeighted {  // slots: i, j, frequency
-    static constexpr int S = 3;
-    Nums p;
+struct RelatednessWeighted : Complement<RelatednessWeighted, 3> {  // slots: i, j, frequency
     double ca, cb;
     __device__ double f(const double *x) const {
         return (x[0] - ca * x[2]) * (x[1] - cb * x[2]);
-    }
-    __device__ double one(const double *x) const { return f(x); }
-    __device__ double both(const double *x) const {
-        const double y[3] = {p.n[0] - x[0], p.n[1] - x[1], p.n[2] - x[2]};
-        return f(x) + f(y);
     }
 };
 
@@ -387,26 +422,34 @@ struct LaneEvents {
     double wl[N], wb[N];
 };
 
+// The tile of one workgroup (LDS).
+template <typename T>
+struct Tile {
+    const double *mean;   // centred relatedness: the query's mean
+    const int32_t *kind;  // site rows
+    bool mixed;           // some row is not a pair
+    const T *cols;        // [K x TILE]
+};
+
 // how a row's value follows from the summary
 #define VALUE_ONE 0    // polarised, every row a pair or derived
 #define VALUE_BOTH 1   // unpolarised, every event or pair row
 #define VALUE_MIXED 2  // site tiles with other rows
 
-template <typename T, int TILE, bool BRANCH, int VALUE, typename F>
-__device__ __forceinline__ void add_up(const F &f, const T *const *col, const int32_t *kind,
-                                       bool polarised, int lane, const LaneEvents<TILE / WAVE> &ev,
-                                       double &L, double &J) {
+template <typename T, int TILE, bool BRANCH, int VALUE, typename F, typename C2>
+__device__ __forceinline__ void add_up(const F &f, const T *c0, const T *c1, const C2 *c2,
+                                       const T *c3, const int32_t *kind, bool polarised, int lane,
+                                       const LaneEvents<TILE / WAVE> &ev, double &L, double &J) {
     constexpr int N = TILE / WAVE;
 #pragma unroll
     for (int j = 0; j < N / 2; j++) {
-        double x0[F::S], x1[F::S];
+        double x0[4], x1[4];
         const int i = WAVE * j + lane;
-#pragma unroll
-        for (int s = 0; s < F::S; s++) {
-            const double2 v = load2<T>(col[s], i);
-            x0[s] = v.x;
-            x1[s] = v.y;
-        }
+        double2 v = load2<T>(c0, i);
+        x0[0] = v.x, x1[0] = v.y;
+        if constexpr (F::S > 1) v = load2<T>(c1, i), x0[1] = v.x, x1[1] = v.y;
+        if constexpr (F::S > 2) v = load2<C2>(c2, i), x0[2] = v.x, x1[2] = v.y;
+        if constexpr (F::S > 3) v = load2<T>(c3, i), x0[3] = v.x, x1[3] = v.y;
         double v0, v1;
         if constexpr (VALUE == VALUE_ONE) {
             v0 = f.one(x0);
@@ -416,11 +459,13 @@ __device__ __forceinline__ void add_up(const F &f, const T *const *col, const in
             v1 = f.both(x1);
         } else {
             const int2 k = reinterpret_cast<const int2 *>(kind)[i];
-            const bool both = !polarised;
-            v0 = (both && k.x == TSG_ROW_PAIR) ? f.both(x0) : f.one(x0);
-            v1 = (both && k.y == TSG_ROW_PAIR) ? f.both(x1) : f.one(x1);
-            if (polarised && k.x == TSG_ROW_ANCESTRAL) v0 = 0.0;
-            if (polarised && k.y == TSG_ROW_ANCESTRAL) v1 = 0.0;
+            if (polarised) {
+                v0 = k.x == TSG_ROW_ANCESTRAL ? 0.0 : f.one(x0);
+                v1 = k.y == TSG_ROW_ANCESTRAL ? 0.0 : f.one(x1);
+            } else {
+                v0 = k.x == TSG_ROW_PAIR ? f.both(x0) : f.lone(x0);
+                v1 = k.y == TSG_ROW_PAIR ? f.both(x1) : f.lone(x1);
+            }
         }
         L = fma(v0, ev.wl[2 * j], L);
         L = fma(v1, ev.wl[2 * j + 1], L);
@@ -431,23 +476,11 @@ __device__ __forceinline__ void add_up(const F &f, const T *const *col, const in
     }
 }
 
-template <typename T, int TILE, bool BRANCH, typename F>
-__device__ __forceinline__ void add_value(const F &f, const T *const *col, const int32_t *kind,
-                                          bool mixed, bool polarised, int lane,
-                                          const LaneEvents<TILE / WAVE> &ev, double &L, double &J) {
-    if (!BRANCH && mixed) {
-        add_up<T, TILE, BRANCH, VALUE_MIXED>(f, col, kind, polarised, lane, ev, L, J);
-    } else if (polarised) {
-        add_up<T, TILE, BRANCH, VALUE_ONE>(f, col, kind, true, lane, ev, L, J);
-    } else {
-        add_up<T, TILE, BRANCH, VALUE_BOTH>(f, col, kind, false, lane, ev, L, J);
-    }
-}
-
 // The trait regression's summary (trees.c:4108-4152) of event e, or of its
-// complement: covariates cbase .. with their row of V, the sample count x_l.
+// complement: covariates cbase .. with their row of V, the sample count in
+// column c[3].
 template <int TILE>
-__device__ __forceinline__ double regression(const TsgStateArgs &a, const TsgOut &o,
+__device__ __forceinline__ double regression(const TsgStateArgs &a, const TsgStateOut &o,
                                              const double *cols, int e, bool comp) {
     const double *v = a.opar + o.par;
     const double *tot = a.col_total_w;
@@ -455,9 +488,9 @@ __device__ __forceinline__ double regression(const TsgStateArgs &a, const TsgOut
         const double x = cols[c * TILE + e];
         return comp ? tot[c] - x : x;
     };
-    const double m = X(o.l), n = (double) o.ni;
-    if (!(m > 0.0 && m < n)) return 0.0;
-    double r = X(o.i), denom = m;
+    const double m = X(o.c[3]);
+    if (!(m > 0.0 && m < (double) o.samples)) return 0.0;
+    double r = X(o.c[0]), denom = m;
     for (int c = 0; c < o.ccount; c++) {
         const double z = X(o.cbase + c);
         r -= z * v[c];
@@ -466,222 +499,120 @@ __device__ __forceinline__ double regression(const TsgStateArgs &a, const TsgOut
     return denom < 1e-8 ? 0.0 : (r * r) / (2 * denom * denom);
 }
 
-template <int TILE, bool BRANCH>
-__device__ void add_regression(const TsgStateArgs &a, const TsgOut &o, const double *cols,
-                               const int32_t *kind, bool mixed, bool polarised, int lane,
-                               const LaneEvents<TILE / WAVE> &ev, double &L, double &J) {
-    constexpr int N = TILE / WAVE;
-    for (int j = 0; j < N; j++) {
-        const int e = 2 * WAVE * (j / 2) + 2 * lane + (j & 1);
-        const int k = (!BRANCH && mixed) ? kind[e] : TSG_ROW_PAIR;
-        double f = (polarised && k == TSG_ROW_ANCESTRAL) ? 0.0
-                                                         : regression<TILE>(a, o, cols, e, false);
-        if (!polarised && k == TSG_ROW_PAIR) f = f + regression<TILE>(a, o, cols, e, true);
-        double wl = 0, wb = 0;
-#pragma unroll
-        for (int r = 0; r < N; r++) {
-            if (r == j) {
-                wl = ev.wl[r];
-                wb = ev.wb[r];
-            }
-        }
-        L = fma(f, wl, L);
-        if constexpr (BRANCH) J = fma(f, wb, J);
+// Calls use(f, c2) with the summary f of output o and the column (or mean)
+// of its slot 2.
+template <int TYPE, int TILE, typename T, typename U>
+__device__ __forceinline__ void with_summary(const TsgStateOut &o, const Tile<T> &tile, U use) {
+    const T *c2 = tile.cols + o.c[2] * TILE;
+    const Nums n{{o.n[0], o.n[1], o.n[2], o.n[3]}};
+#define SUMMARY(ID, F) \
+    case ID: {         \
+        F f;           \
+        f.p = n;       \
+        use(f, c2);    \
+        break;         \
     }
-}
-
-// Output o's two sums over this lane's events, before the denominator.
-template <int TYPE, int TILE, bool BRANCH>
-__device__ __forceinline__ void add_output(const TsgStateArgs &a, const TsgOut &o,
-                                           const typename TileType<TYPE, BRANCH>::T *cols,
-                                           const double *mean, const int32_t *kind, bool mixed,
-                                           int lane, const LaneEvents<TILE / WAVE> &ev, double &L,
-                                           double &J) {
-    using T = typename TileType<TYPE, BRANCH>::T;
-    const bool pol = (o.flags & 1) != 0;
     if constexpr (TYPE == TSG_ROW_F64) {
-        const double *col[4] = {cols + o.i * TILE, cols + o.j * TILE, nullptr, nullptr};
-        const double *tot = a.col_total_w;
         switch (o.stat) {
-        case TSG_STAT_TRAIT_COVARIANCE:
-            add_value<T, TILE, BRANCH>(TraitCovariance{{{tot[o.i]}}}, col, kind, mixed, pol, lane,
-                                       ev, L, J);
+            SUMMARY(TSG_STAT_TRAIT_COVARIANCE, TraitCovariance)
+            SUMMARY(TSG_STAT_TRAIT_CORRELATION, TraitCorrelation)
+            SUMMARY(TSG_STAT_RELATEDNESS_WEIGHTED_NONCENTRED, Product)
+        case TSG_STAT_RELATEDNESS_WEIGHTED: {
+            RelatednessWeighted f;
+            f.p = n;
+            f.ca = o.coef[0];
+            f.cb = o.coef[1];
+            use(f, c2);
             break;
-        case TSG_STAT_TRAIT_CORRELATION:
-            col[1] = cols + o.l * TILE;
-            add_value<T, TILE, BRANCH>(TraitCorrelation{{{tot[o.i], tot[o.l]}}}, col, kind, mixed,
-                                       pol, lane, ev, L, J);
-            break;
-        case TSG_STAT_TRAIT_LINEAR_MODEL:
-            add_regression<TILE, BRANCH>(a, o, cols, kind, mixed, pol, lane, ev, L, J);
-            break;
-        case TSG_STAT_RELATEDNESS_WEIGHTED:
-            col[2] = cols + o.l * TILE;
-            add_value<T, TILE, BRANCH>(
-                RelatednessWeighted{
-                    {{tot[o.i], tot[o.j], tot[o.l]}}, a.opar[o.par], a.opar[o.par + 1]},
-                col, kind, mixed, pol, lane, ev, L, J);
-            break;
-        case TSG_STAT_RELATEDNESS_WEIGHTED_NONCENTRED:
-            add_value<T, TILE, BRANCH>(Product{{{tot[o.i], tot[o.j]}}}, col, kind, mixed, pol,
-                                       lane, ev, L, J);
-            break;
+        }
         default:
             break;
         }
     } else {
-        const T *col[4] = {cols + o.i * TILE, cols + o.j * TILE, cols + o.k * TILE,
-                           cols + o.l * TILE};
-        const Nums n = {{(double) o.ni, (double) o.nj, (double) o.nk, (double) o.nl}};
-#define SUMMARY(F)                                                                             \
-    {                                                                                          \
-        F f;                                                                                   \
-        f.p = n;                                                                               \
-        add_value<T, TILE, BRANCH>(f, col, kind, mixed, pol, lane, ev, L, J);                  \
-        break;                                                                                 \
-    }
         switch (o.stat) {
-        case TSG_STAT_DIVERSITY:
-            SUMMARY(Diversity)
-        case TSG_STAT_SEGREGATING_SITES:
-            SUMMARY(Segregating)
-        case TSG_STAT_Y1:
-            SUMMARY(Y1)
-        case TSG_STAT_DIVERGENCE:
-            SUMMARY(Divergence)
-        case TSG_STAT_RELATEDNESS_NONCENTRED:
-            SUMMARY(Product)
-        case TSG_STAT_Y2:
-            SUMMARY(Y2)
-        case TSG_STAT_F2:
-            SUMMARY(F2)
-        case TSG_STAT_Y3:
-            SUMMARY(Y3)
-        case TSG_STAT_F3:
-            SUMMARY(F3)
-        case TSG_STAT_F4:
-            SUMMARY(F4)
-#undef SUMMARY
-        case TSG_STAT_RELATEDNESS: {
-            constexpr int N = TILE / WAVE;
-            Relatedness f;
-            f.p = Nums{{1.0 / n.n[0], 1.0 / n.n[1], 0.0, 0.0}};
-#pragma unroll
-            for (int j = 0; j < N / 2; j++) {
-                const int i = WAVE * j + lane;
-                const double2 xi = load2<T>(col[0], i), xj = load2<T>(col[1], i);
-                const double2 mu = load2<double>(mean, i);
-                const double a0[3] = {xi.x, xj.x, mu.x}, a1[3] = {xi.y, xj.y, mu.y};
-                double v0 = f.one(a0), v1 = f.one(a1);
-                int2 k = make_int2(TSG_ROW_PAIR, TSG_ROW_PAIR);
-                if (!BRANCH && mixed) k = reinterpret_cast<const int2 *>(kind)[i];
-                if (pol) {
-                    v0 = k.x == TSG_ROW_ANCESTRAL ? 0.0 : v0;
-                    v1 = k.y == TSG_ROW_ANCESTRAL ? 0.0 : v1;
-                } else {
-                    v0 = k.x == TSG_ROW_PAIR ? 2.0 * v0 : v0;
-                    v1 = k.y == TSG_ROW_PAIR ? 2.0 * v1 : v1;
-                }
-                L = fma(v0, ev.wl[2 * j], L);
-                L = fma(v1, ev.wl[2 * j + 1], L);
-                if constexpr (BRANCH) {
-                    J = fma(v0, ev.wb[2 * j], J);
-                    J = fma(v1, ev.wb[2 * j + 1], J);
-                }
-            }
+            SUMMARY(TSG_STAT_DIVERSITY, Diversity)
+            SUMMARY(TSG_STAT_SEGREGATING_SITES, Segregating)
+            SUMMARY(TSG_STAT_Y1, Y1)
+            SUMMARY(TSG_STAT_DIVERGENCE, Divergence)
+            SUMMARY(TSG_STAT_RELATEDNESS_NONCENTRED, Product)
+            SUMMARY(TSG_STAT_Y2, Y2)
+            SUMMARY(TSG_STAT_F2, F2)
+            SUMMARY(TSG_STAT_Y3, Y3)
+            SUMMARY(TSG_STAT_F3, F3)
+            SUMMARY(TSG_STAT_F4, F4)
+        case TSG_STAT_RELATEDNESS:
+            use(Relatedness{o.coef[0], o.coef[1]}, tile.mean);
             break;
-        }
         default:
             break;
         }
     }
+#undef SUMMARY
 }
 
-// Output o's summary of event e alone, before the denominator.
-template <int TYPE, int TILE, bool BRANCH>
-__device__ __forceinline__ double value_of(const TsgStateArgs &a, const TsgOut &o,
-                                           const typename TileType<TYPE, BRANCH>::T *cols,
-                                           const double *mean, const int32_t *kind, int e) {
-    const bool pol = (o.flags & 1) != 0;
-    const int k = BRANCH ? TSG_ROW_PAIR : kind[e];
+// Output o's two sums over this lane's events, before the scale.
+template <int TYPE, int TILE, bool BRANCH, typename T>
+__device__ __forceinline__ void add_output(const TsgStateArgs &a, const TsgStateOut &o,
+                                           const Tile<T> &tile, int lane,
+                                           const LaneEvents<TILE / WAVE> &ev, double &L,
+                                           double &J) {
+    const bool pol = o.polarised != 0;
+    if constexpr (TYPE == TSG_ROW_F64) {
+        if (o.stat == TSG_STAT_TRAIT_LINEAR_MODEL) {
+            constexpr int N = TILE / WAVE;
+#pragma unroll
+            for (int r = 0; r < N; r++) {
+                const int e = 2 * WAVE * (r / 2) + 2 * lane + (r & 1);
+                const int k = (!BRANCH && tile.mixed) ? tile.kind[e] : TSG_ROW_PAIR;
+                double f = (pol && k == TSG_ROW_ANCESTRAL)
+                               ? 0.0
+                               : regression<TILE>(a, o, tile.cols, e, false);
+                if (!pol && k == TSG_ROW_PAIR) f = f + regression<TILE>(a, o, tile.cols, e, true);
+                L = fma(f, ev.wl[r], L);
+                if constexpr (BRANCH) J = fma(f, ev.wb[r], J);
+            }
+            return;
+        }
+    }
+    const T *c0 = tile.cols + o.c[0] * TILE, *c1 = tile.cols + o.c[1] * TILE;
+    const T *c3 = tile.cols + o.c[3] * TILE;
+    with_summary<TYPE, TILE>(o, tile, [&](const auto &f, const auto *c2) {
+        if (!BRANCH && tile.mixed) {
+            add_up<T, TILE, BRANCH, VALUE_MIXED>(f, c0, c1, c2, c3, tile.kind, pol, lane, ev, L,
+                                                 J);
+        } else if (pol) {
+            add_up<T, TILE, BRANCH, VALUE_ONE>(f, c0, c1, c2, c3, tile.kind, true, lane, ev, L, J);
+        } else {
+            add_up<T, TILE, BRANCH, VALUE_BOTH>(f, c0, c1, c2, c3, tile.kind, false, lane, ev, L,
+                                                J);
+        }
+    });
+}
+
+// Output o's summary of event e alone, before the scale.
+template <int TYPE, int TILE, bool BRANCH, typename T>
+__device__ __forceinline__ double value_of(const TsgStateArgs &a, const TsgStateOut &o,
+                                           const Tile<T> &tile, int e) {
+    const bool pol = o.polarised != 0;
+    const int k = BRANCH ? TSG_ROW_PAIR : tile.kind[e];
     if (pol && k == TSG_ROW_ANCESTRAL) return 0.0;
     const bool both = !pol && k == TSG_ROW_PAIR;
     if constexpr (TYPE == TSG_ROW_F64) {
-        const double *tot = a.col_total_w;
-        const double x[3] = {cols[o.i * TILE + e],
-                             cols[(o.stat == TSG_STAT_TRAIT_CORRELATION ? o.l : o.j) * TILE + e],
-                             cols[o.l * TILE + e]};
-        switch (o.stat) {
-        case TSG_STAT_TRAIT_COVARIANCE: {
-            const TraitCovariance f{{{tot[o.i]}}};
-            return both ? f.both(x) : f.one(x);
+        if (o.stat == TSG_STAT_TRAIT_LINEAR_MODEL) {
+            const double v = regression<TILE>(a, o, tile.cols, e, false);
+            return both ? v + regression<TILE>(a, o, tile.cols, e, true) : v;
         }
-        case TSG_STAT_TRAIT_CORRELATION: {
-            const TraitCorrelation f{{{tot[o.i], tot[o.l]}}};
-            return both ? f.both(x) : f.one(x);
-        }
-        case TSG_STAT_TRAIT_LINEAR_MODEL: {
-            const double v = regression<TILE>(a, o, cols, e, false);
-            return both ? v + regression<TILE>(a, o, cols, e, true) : v;
-        }
-        case TSG_STAT_RELATEDNESS_WEIGHTED: {
-            const RelatednessWeighted f{
-                {{tot[o.i], tot[o.j], tot[o.l]}}, a.opar[o.par], a.opar[o.par + 1]};
-            return both ? f.both(x) : f.one(x);
-        }
-        case TSG_STAT_RELATEDNESS_WEIGHTED_NONCENTRED: {
-            const Product f{{{tot[o.i], tot[o.j]}}};
-            return both ? f.both(x) : f.one(x);
-        }
-        default:
-            return 0.0;
-        }
-    } else {
-        const Nums n = {{(double) o.ni, (double) o.nj, (double) o.nk, (double) o.nl}};
-        double x[4] = {(double) cols[o.i * TILE + e], (double) cols[o.j * TILE + e], 0.0, 0.0};
-#define SUMMARY(F)                          \
-    {                                       \
-        F f;                                \
-        f.p = n;                            \
-        return both ? f.both(x) : f.one(x); \
     }
-        switch (o.stat) {
-        case TSG_STAT_DIVERSITY:
-            SUMMARY(Diversity)
-        case TSG_STAT_SEGREGATING_SITES:
-            SUMMARY(Segregating)
-        case TSG_STAT_Y1:
-            SUMMARY(Y1)
-        case TSG_STAT_DIVERGENCE:
-            SUMMARY(Divergence)
-        case TSG_STAT_RELATEDNESS_NONCENTRED:
-            SUMMARY(Product)
-        case TSG_STAT_Y2:
-            SUMMARY(Y2)
-        case TSG_STAT_F2:
-            SUMMARY(F2)
-        case TSG_STAT_RELATEDNESS: {
-            x[2] = mean[e];
-            const double v = Relatedness{{{1.0 / n.n[0], 1.0 / n.n[1], 0.0, 0.0}}}.one(x);
-            return both ? 2.0 * v : v;
-        }
-        default:
-            break;
-        }
-        x[2] = (double) cols[o.k * TILE + e];
-        x[3] = (double) cols[o.l * TILE + e];
-        switch (o.stat) {
-        case TSG_STAT_Y3:
-            SUMMARY(Y3)
-        case TSG_STAT_F3:
-            SUMMARY(F3)
-        case TSG_STAT_F4:
-            SUMMARY(F4)
-        default:
-            return 0.0;
-        }
-#undef SUMMARY
-    }
+    double x[4] = {(double) tile.cols[o.c[0] * TILE + e], 0.0, 0.0, 0.0};
+    double v = 0.0;
+    with_summary<TYPE, TILE>(o, tile, [&](const auto &f, const auto *c2) {
+        constexpr int S = std::decay<decltype(f)>::type::S;
+        if constexpr (S > 1) x[1] = (double) tile.cols[o.c[1] * TILE + e];
+        if constexpr (S > 2) x[2] = (double) c2[e];
+        if constexpr (S > 3) x[3] = (double) tile.cols[o.c[3] * TILE + e];
+        v = pol ? f.one(x) : both ? f.both(x) : f.lone(x);
+    });
+    return v;
 }
 
 // Four lane values a, b, c, d added up over the wave at once: lanes 0-15 get
@@ -724,12 +655,13 @@ __device__ __forceinline__ double wave_sums(double a, double b, double c, double
     return a;
 }
 
-// One tile: events (BRANCH) or site rows t TILE .. of the run.
-template <int TYPE, bool BRANCH>
+// One tile: events (BRANCH) or site rows t TILE .. of the run.  WIDE: more
+// columns than an FP64 tile takes.
+template <int TYPE, bool BRANCH, bool WIDE>
 __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
     constexpr int TILE = BRANCH ? TSG_BRANCH_TILE : TSG_SITE_TILE;
     constexpr int N = TILE / WAVE;
-    using T = typename TileType<TYPE, BRANCH>::T;
+    using T = typename TileType<TYPE, BRANCH, WIDE>::T;
     extern __shared__ double smem[];
     double *spos = smem;                                       // [TILE]
     double *sb = spos + TILE;                                  // [TILE] (branch)
@@ -768,7 +700,7 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                     if (2 * w < K) cols[(2 * w) * TILE + e] = (T) (v & 0xFFFFu);
                     if (2 * w + 1 < K) cols[(2 * w + 1) * TILE + e] = (T) (v >> 16);
                 } else if constexpr (TYPE == TSG_ROW_I32) {
-                    if (w < K) cols[w * TILE + e] = (T) v;
+                    if (w < K) cols[w * TILE + e] = (T) (int32_t) v;
                 } else {
                     if (w < 2 * K) {
                         reinterpret_cast<uint32_t *>(cols + (w / 2) * TILE + e)[w & 1] = v;
@@ -797,7 +729,7 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                     if constexpr (TYPE == TSG_ROW_F64) {
                         v = a.col_total_w[k];
                     } else {
-                        v = a.col_total[k];
+                        v = (T) a.col_total[k];
                     }
                 }
                 for (int i = a.list_off[l]; i < a.list_off[l + 1]; i++) {
@@ -805,9 +737,9 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                     const uint32_t *row = a.x + (int64_t) (ent >> 1) * RW;
                     T xv;
                     if constexpr (TYPE == TSG_ROW_U16) {
-                        xv = reinterpret_cast<const uint16_t *>(row)[k];
+                        xv = (T) reinterpret_cast<const uint16_t *>(row)[k];
                     } else if constexpr (TYPE == TSG_ROW_I32) {
-                        xv = (T) row[k];
+                        xv = (T) (int32_t) row[k];
                     } else {
                         xv = reinterpret_cast<const double *>(row)[k];
                     }
@@ -819,11 +751,12 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
     }
     const bool mixed = !BRANCH && __syncthreads_or(other) != 0;
     if constexpr (BRANCH) __syncthreads();
+    const Tile<T> tile{mean, kind, mixed, cols};
 
     const int q0 = BRANCH ? 0 : a.QB, q1 = BRANCH ? a.QB : a.Q;
     constexpr int PER = BRANCH ? 2 : 1;
     for (int q = q0; q < q1; q++) {
-        const TsgStateQuery &Q = a.queries[q];
+        const TsgStateQuery Q = uniform(a.queries + q);
         const double *win = a.windows + Q.win_off;
         const int M = Q.M;
         const int w0 = a.tile_w[Q.tw + t], w1 = a.tile_w[Q.tw + t + 1];
@@ -844,7 +777,7 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
         // A wave adds up an output's whole tile for each of its windows (about
         // 400 cycles); a thread a (window, output) pair's events one by one
         // (about 150 cycles each, 256 threads): whichever is less.  (Measured
-        // on 500 windows over 250 sites: 1634 -> 28 us.)
+        // on site tiles of up to 250 of 500 windows, 31 outputs: 1634 -> 71 us.)
         if ((int64_t) nw * nw * ((M + 3) / 4) * 8 >
             (int64_t) TILE * 3 * (((int64_t) nw * M + EVAL_THREADS - 1) / EVAL_THREADS)) {
             for (int64_t i = tid; i < (int64_t) nw * M; i += EVAL_THREADS) {
@@ -852,10 +785,10 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                 const int ea = w == w0 ? 0 : lower_bound(spos, ne, win[w]);
                 const int eb = w == w1 ? ne : lower_bound(spos, ne, win[w + 1]);
                 const double wr = win[w + 1];
-                const TsgOut o = a.outs[Q.mbase + m];
+                const TsgStateOut o = a.outs[Q.mbase + m];
                 double L = 0, J = 0;
                 for (int e = ea; e < eb; e++) {
-                    const double v = value_of<TYPE, TILE, BRANCH>(a, o, cols, mean, kind, e);
+                    const double v = value_of<TYPE, TILE, BRANCH>(a, o, tile, e);
                     if constexpr (BRANCH) {
                         const double b = sb[e];
                         L = fma(v, b * (wr - spos[e]), L);
@@ -864,12 +797,10 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                         L += v;
                     }
                 }
-                if (isfinite(o.inv)) {
-                    L *= o.inv;
-                    J *= o.inv;
-                } else {
-                    L = J = eb > ea ? NAN : 0.0;
-                }
+                // (a zero denominator: 0 x inf is the reference's NaN at every
+                // state, but a window without events has 0)
+                L = eb > ea ? L * o.scale : 0.0;
+                J = eb > ea ? J * o.scale : 0.0;
                 double *dst = a.partial + Q.pbase + ((int64_t) (t + w) * M + m) * PER;
                 dst[0] = L;
                 if constexpr (BRANCH) dst[1] = J;
@@ -895,31 +826,33 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                 }
             }
             // outputs wave, wave + 4, ...: two (branch: sums L and J) or four
-            // (site) of them a round
+            // (site) of them a round; lanes 0, 16, 32, 48 hold acc 0, 2, 1, 3
             constexpr int ROUND = BRANCH ? 2 : 4;
-            double *dst = a.partial + Q.pbase + (int64_t) (t + w) * M * PER;
+            const int row = lane / 16;
+            const int at = row == 1 ? 2 : (row == 2 ? 1 : row);
+            double *dst = a.partial + Q.pbase + (int64_t) (t + w) * M * PER +
+                          (BRANCH ? (at / 2) * WAVES * 2 + (at & 1) : at * WAVES);
             for (int m0 = wave; m0 < M; m0 += WAVES * ROUND) {
-                double acc[4] = {0, 0, 0, 0};
-                double unused = 0;
+                double acc[4] = {0, 0, 0, 0}, scale[ROUND], unused = 0;
 #pragma unroll
                 for (int i = 0; i < ROUND; i++) {
-                    const int m = m0 + i * WAVES;
-                    if (m >= M) break;
-                    add_output<TYPE, TILE, BRANCH>(a, a.outs[Q.mbase + m], cols, mean, kind, mixed,
-                                                   lane, ev, acc[BRANCH ? 2 * i : i],
-                                                   BRANCH ? acc[2 * i + 1] : unused);
+                    const int m = min(m0 + i * WAVES, M - 1);
+                    const TsgStateOut o = uniform(a.outs + Q.mbase + m);
+                    scale[i] = o.scale;
+                    if (m0 + i * WAVES < M) {
+                        add_output<TYPE, TILE, BRANCH>(a, o, tile, lane, ev,
+                                                       acc[BRANCH ? 2 * i : i],
+                                                       BRANCH ? acc[2 * i + 1] : unused);
+                    }
                 }
-                const double v = wave_sums(acc[0], acc[1], acc[2], acc[3]);
-                // lanes 0, 16, 32, 48 hold acc 0, 2, 1, 3
-                const int row = lane / 16;
-                const int at = row == 1 ? 2 : (row == 2 ? 1 : row);
-                const int m = m0 + (BRANCH ? at / 2 : at) * WAVES;
-                if (lane % 16 == 0 && m < M) {
-                    // a zero denominator: NaN at every state (trees.c:2097-2220
-                    // lets it through), none where there is no event
-                    const double inv = a.outs[Q.mbase + m].inv;
-                    const double r = isfinite(inv) ? v * inv : (eb > ea ? NAN : 0.0);
-                    dst[BRANCH ? 2 * m + (at & 1) : m] = r;
+                double v = wave_sums(acc[0], acc[1], acc[2], acc[3]);
+                if (lane % 16 == 0 && m0 + (BRANCH ? at / 2 : at) * WAVES < M) {
+                    double sc = scale[0];
+#pragma unroll
+                    for (int i = 1; i < ROUND; i++) {
+                        if ((BRANCH ? at / 2 : at) == i) sc = scale[i];
+                    }
+                    dst[m0 * PER] = eb > ea ? v * sc : 0.0;
                 }
             }
         }
@@ -927,20 +860,6 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
 }
 
 // --- window sums ----------------------------------------------------------------
-
-// first tile whose successor starts at x or later (or the last tile)
-__device__ __forceinline__ int first_tile(const double *tpos, int tiles, double x) {
-    int lo = 0, hi = tiles - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (tpos[mid + 1] >= x) {
-            hi = mid;
-        } else {
-            lo = mid + 1;
-        }
-    }
-    return lo;
-}
 
 __device__ __forceinline__ int pow2_at_least(int m, int most) {
     int p = 1;
@@ -955,19 +874,17 @@ __device__ __forceinline__ void window_sums(const TsgStateArgs &a, int b) {
     while (q + 1 < a.Q && a.queries[q + 1].wbase <= b) q++;
     const TsgStateQuery &Q = a.queries[q];
     const int w = b - Q.wbase;
-    const double *win = a.windows + Q.win_off;
-    const double *tpos = Q.branch ? a.btile_pos : a.stile_pos;
     const int tiles = Q.branch ? a.btiles : a.stiles;
     const int M = Q.M, per = Q.branch ? 2 : 1;
-    const int tlo = first_tile(tpos, tiles, win[w]);
-    const double wr = win[w + 1];
+    const int32_t *first = a.tile_w + Q.tw + tiles + 1;
+    const int tlo = first[w], thi = first[w + 1];
     const int mb = pow2_at_least(M, 64), tl = 256 / mb;
     const int mi = threadIdx.x & (mb - 1), ti = threadIdx.x / mb;
     for (int m0 = 0; m0 < M; m0 += mb) {
         const int m = m0 + mi;
         double L = 0, J = 0;
         if (m < M) {
-            for (int t = tlo + ti; t == tlo || (t < tiles && tpos[t] < wr); t += tl) {
+            for (int t = tlo + ti; t <= thi; t += tl) {
                 const double *src = a.partial + Q.pbase + ((int64_t) (t + w) * M + m) * per;
                 L += src[0];
                 if (per == 2) J += src[1];
@@ -1002,7 +919,6 @@ __device__ __forceinline__ void finish(const TsgStateArgs &a, int b) {
     while (q + 1 < a.Q && a.queries[q + 1].bbase <= b) q++;
     const TsgStateQuery &Q = a.queries[q];
     const double *win = a.windows + Q.win_off;
-    const double *tpos = Q.branch ? a.btile_pos : a.stile_pos;
     const int tiles = Q.branch ? a.btiles : a.stiles;
     const int M = Q.M, W = Q.W, per = Q.branch ? 2 : 1;
     const int mb = pow2_at_least(M, TSG_FINISH_OUTPUTS), S = FINISH_THREADS / mb;
@@ -1010,8 +926,8 @@ __device__ __forceinline__ void finish(const TsgStateArgs &a, int b) {
     const int m = (b - Q.bbase) * TSG_FINISH_OUTPUTS + mi;
     const bool on = m < M;
     const int wa = (int) ((int64_t) W * seg / S), wb = (int) ((int64_t) W * (seg + 1) / S);
-    int t = 0;
-    // window w's two sums; with the segments, tile t moves along
+    const int32_t *first = a.tile_w + Q.tw + tiles + 1;
+    // window w's two sums
     auto sums = [&](int w, double &L, double &J) {
         L = J = 0;
         if (Q.by_window) {
@@ -1020,23 +936,17 @@ __device__ __forceinline__ void finish(const TsgStateArgs &a, int b) {
             if (per == 2) J = src[1];
             return;
         }
-        const double wr = win[w + 1];
-        for (;;) {
+        const int thi = first[w + 1];
+        for (int t = first[w]; t <= thi; t++) {
             const double *src = a.partial + Q.pbase + ((int64_t) (t + w) * M + m) * per;
             L += src[0];
             if (per == 2) J += src[1];
-            if (t + 1 < tiles && tpos[t + 1] < wr) {
-                t++;
-            } else {
-                break;
-            }
         }
     };
     double R = 0;
     if (per == 2) {
         double acc = 0;
         if (on && wa < wb) {
-            t = Q.by_window ? 0 : first_tile(tpos, tiles, win[wa]);
             for (int w = wa; w < wb; w++) {
                 double L, J;
                 sums(w, L, J);
@@ -1055,7 +965,6 @@ __device__ __forceinline__ void finish(const TsgStateArgs &a, int b) {
         R = seg > 0 ? scan[threadIdx.x - mb] : 0.0;
     }
     if (!on || wa >= wb) return;
-    t = Q.by_window ? 0 : first_tile(tpos, tiles, win[wa]);
     double *dst = (Q.to_out ? a.out : a.raw) + Q.obase;
     for (int w = wa; w < wb; w++) {
         double L, J;
@@ -1069,6 +978,192 @@ __device__ __forceinline__ void finish(const TsgStateArgs &a, int b) {
 }
 
 }  // namespace
+
+// --- node statistics --------------------------------------------------------------
+
+// Column k of state s.
+template <int TYPE>
+__device__ __forceinline__ double row_value(const TsgStateArgs &a, int s, int k) {
+    const uint32_t *row = a.x + (int64_t) s * a.RW;
+    return TYPE == TSG_ROW_U16 ? (double) reinterpret_cast<const uint16_t *>(row)[k]
+                               : (double) (int32_t) row[k];
+}
+
+// Output o's summary at state s, before the scale.
+template <int TYPE>
+__device__ __forceinline__ double state_value(const TsgStateArgs &a, const TsgStateOut &o,
+                                              const TsgStateQuery &Q, int s) {
+    double mean = 0;
+    if (Q.rel_cn > 0) {
+        for (int c = Q.rel_c0; c < Q.rel_c0 + Q.rel_cn; c++) {
+            mean += row_value<TYPE>(a, s, c) / (double) a.col_total[c];
+        }
+        mean /= (double) Q.rel_cn;
+    }
+    double x[4] = {row_value<TYPE>(a, s, o.c[0]), row_value<TYPE>(a, s, o.c[1]), 0.0, 0.0};
+    double v = 0.0;
+    const Tile<double> none{&mean, nullptr, false, nullptr};
+    with_summary<TYPE, 1>(o, none, [&](const auto &f, const auto *) {
+        using F = typename std::decay<decltype(f)>::type;
+        if constexpr (std::is_same<F, Relatedness>::value) {
+            x[2] = mean;
+        } else {
+            if constexpr (F::S > 2) x[2] = row_value<TYPE>(a, s, o.c[2]);
+            if constexpr (F::S > 3) x[3] = row_value<TYPE>(a, s, o.c[3]);
+        }
+        v = o.polarised ? f.one(x) : f.both(x);
+    });
+    return v;
+}
+
+// Thread (run, output): a run of one node's states along the genome, each
+// the summary times its span in every window it crosses, added to
+// res[(window x N + node) x M + output] once per run and window (FP64 atomic
+// adds: a node's runs meet there in any order).  A chunk sweep added at
+// every event of a node's path: on 8000 samples, 8 sets, 347 us; this, 22 us.
+template <int TYPE>
+__global__ void __launch_bounds__(256) k_state_nodes(const TsgStateArgs a, const TsgNodeArgs g) {
+    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    const TsgStateQuery &Q = a.queries[0];
+    const int M = Q.M, W = Q.W;
+    const int64_t r = i / M;
+    const int m = (int) (i % M);
+    if (r >= g.runs) return;
+    const TsgStateOut o = a.outs[m];
+    const double *win = a.windows;
+    const int node = g.run_node[r];
+    const int p0 = g.run_piece0[r], p1 = g.run_piece0[r + 1];
+    const bool last = r + 1 == g.runs || g.run_node[r + 1] != node;
+    int w = W > 1 ? window_of(win, W, g.run_from[p0]) : 0;
+    double acc = 0;
+    auto add = [&]() {
+        double *dst = g.res + ((int64_t) w * g.num_nodes + node) * M + m;
+        atomicAdd(dst, acc * o.scale);
+        acc = 0;
+    };
+    for (int p = p0; p < p1; p++) {
+        double from = g.run_from[p];
+        const double to = (p + 1 < p1 || !last) ? g.run_from[p + 1] : g.length;
+        const double f = state_value<TYPE>(a, o, Q, g.run_state[p]);
+        while (w + 1 < W && win[w + 1] <= to) {
+            acc = fma(f, win[w + 1] - from, acc);
+            add();
+            from = win[++w];
+        }
+        acc = fma(f, to - from, acc);
+    }
+    add();
+}
+
+// --- allele frequency spectrum ------------------------------------------------------
+// Columns are the sample sets; which alleles and branches cover some samples
+// and not all is in the plan (row_all, the pieces left out).
+
+namespace {
+
+// Index of counts c[0 .. K) in the spectrum of the sets' sizes; folded
+// (unpolarised): complemented where the allele is the minor one, ties broken
+// on the trailing sets (trees.c:3469-3496).
+__device__ __forceinline__ int64_t spectrum_index(const TsgSpectrumArgs &g, int K, int32_t *c) {
+    if (!g.polarised) {
+        double half = 0;
+        int sum = 0;
+        for (int k = 0; k < K; k++) {
+            half += (double) g.dims[k] - 1;
+            sum += c[k];
+        }
+        half /= 2;
+        int k = K;
+        while (sum == half && k > 0) {
+            k--;
+            half -= ((double) (g.dims[k] - 1)) / 2;
+            sum -= c[k];
+        }
+        if (sum > half) {
+            for (k = 0; k < K; k++) c[k] = (int32_t) g.dims[k] - 1 - c[k];
+        }
+    }
+    int64_t at = 0;
+    for (int k = 0; k < K; k++) at = at * g.dims[k] + c[k];
+    return at;
+}
+
+template <int TYPE>
+__device__ __forceinline__ int32_t row_count(const TsgStateArgs &a, int s, int k) {
+    const uint32_t *row = a.x + (int64_t) s * a.RW;
+    return TYPE == TSG_ROW_U16 ? (int32_t) reinterpret_cast<const uint16_t *>(row)[k]
+                               : (int32_t) row[k];
+}
+
+}  // namespace
+
+// Thread per site row: one (polarised) or a half (folded) per allele that is
+// not fixed, in half-units (integers: exact, whatever the order).
+template <int TYPE>
+__global__ void __launch_bounds__(256) k_spectrum_site(const TsgStateArgs a,
+                                                       const TsgSpectrumArgs g) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= a.nrow) return;
+    const int all = g.row_all[i];
+    if (all <= 0 || all >= a.num_samples) return;
+    const int ref = a.row_ref[i];
+    const int K = a.K;
+    unsigned long long *hist = g.hist_u + window_of(g.windows, g.W, a.row_pos[i]) * g.size;
+    int32_t c[TSG_SPECTRUM_SETS];
+    if (ref >= 0) {
+        for (int k = 0; k < K; k++) c[k] = row_count<TYPE>(a, ref, k);
+        if (g.polarised) {
+            atomicAdd(&hist[spectrum_index(g, K, c)], 2ull);
+            return;
+        }
+        atomicAdd(&hist[spectrum_index(g, K, c)], 1ull);
+        for (int k = 0; k < K; k++) c[k] = a.col_total[k] - row_count<TYPE>(a, ref, k);
+        atomicAdd(&hist[spectrum_index(g, K, c)], 1ull);
+        return;
+    }
+    const int l = -1 - ref;
+    const bool ancestral = a.list_kind[l] == TSG_ROW_ANCESTRAL;
+    if (ancestral && g.polarised) return;
+    for (int k = 0; k < K; k++) {
+        int32_t v = ancestral ? a.col_total[k] : 0;
+        for (int e = a.list_off[l]; e < a.list_off[l + 1]; e++) {
+            const int32_t x = row_count<TYPE>(a, a.list_ent[e] >> 1, k);
+            v += (a.list_ent[e] & 1) ? -x : x;
+        }
+        c[k] = v;
+    }
+    atomicAdd(&hist[spectrum_index(g, K, c)], g.polarised ? 2ull : 1ull);
+}
+
+// Thread per branch piece: its span times the branch's length in each time
+// window, cut at the windows it crosses; a piece that ends at a window's end
+// counts where the edge was there before it (trees.c:3650-3690).
+template <int TYPE>
+__global__ void __launch_bounds__(256) k_spectrum_branch(const TsgStateArgs a,
+                                                         const TsgSpectrumArgs g) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= g.npieces) return;
+    const TsgBranchPiece p = g.pieces[i];
+    int32_t c[TSG_SPECTRUM_SETS];
+    for (int k = 0; k < a.K; k++) c[k] = row_count<TYPE>(a, p.state, k);
+    const int64_t at = spectrum_index(g, a.K, c);
+    auto add = [&](int w, double span) {
+        for (int tw = 0; tw < g.TW && g.time_windows[tw] < p.tp; tw++) {
+            const double length = fmax(0.0, fmin(g.time_windows[tw + 1], p.tp) -
+                                                fmax(g.time_windows[tw], p.tu));
+            atomicAdd(&g.hist_d[((int64_t) w * g.TW + tw) * g.size + at], span * length);
+        }
+    };
+    int w = window_of(g.windows, g.W, p.from);
+    double from = p.from;
+    while (w < g.W && g.windows[w + 1] <= p.to) {
+        const double end = g.windows[w + 1];
+        if (p.ins < end) add(w, end - from);
+        from = end;
+        w++;
+    }
+    if (w < g.W && p.to > from) add(w, p.to - from);
+}
 
 // --- one run ----------------------------------------------------------------------
 
@@ -1084,11 +1179,11 @@ __global__ void __launch_bounds__(256) k_state_count(const TsgStateArgs a, int s
     const int b = xcd_block(blockIdx.x, nb);
     if (b < nb) count_rw<F64>(a, s0, s1, b);
 }
-template <int TYPE, bool BRANCH>
+template <int TYPE, bool BRANCH, bool WIDE>
 __global__ void __launch_bounds__(EVAL_THREADS) k_state_eval(const TsgStateArgs a) {
     const int tiles = BRANCH ? a.btiles : a.stiles;
     const int t = xcd_block(blockIdx.x, tiles);
-    if (t < tiles) evaluate<TYPE, BRANCH>(a, t);
+    if (t < tiles) evaluate<TYPE, BRANCH, WIDE>(a, t);
 }
 __global__ void __launch_bounds__(256) k_state_windows(const TsgStateArgs a) {
     window_sums(a, blockIdx.x);
@@ -1134,14 +1229,14 @@ __global__ void __launch_bounds__(256) k_states_count(const TsgStateArgs *args, 
     const int r = run_at(pre, nrun, b);
     count_rw<F64>(args[r], lev[2 * r], lev[2 * r + 1], b - pre[r]);
 }
-template <int TYPE, bool BRANCH>
+template <int TYPE, bool BRANCH, bool WIDE>
 __global__ void __launch_bounds__(EVAL_THREADS) k_states_eval(const TsgStateArgs *args,
                                                               const int32_t *pre, int nrun,
                                                               int nb) {
     const int b = xcd_block(blockIdx.x, nb);
     if (b >= nb) return;
     const int r = run_at(pre, nrun, b);
-    evaluate<TYPE, BRANCH>(args[r], b - pre[r]);
+    evaluate<TYPE, BRANCH, WIDE>(args[r], b - pre[r]);
 }
 __global__ void __launch_bounds__(256) k_states_windows(const TsgStateArgs *args,
                                                         const int32_t *pre, int nrun) {
@@ -1166,7 +1261,9 @@ __global__ void __launch_bounds__(256) k_states_finals(const TsgStateArgs *args,
 
 size_t tsg_state_shmem(int K, int type, bool branch) {
     const size_t tile = branch ? TSG_BRANCH_TILE : TSG_SITE_TILE;
-    const size_t el = type == TSG_ROW_F64 ? 8 : (type == TSG_ROW_U16 && branch) ? 2 : 4;
+    const size_t el = (type == TSG_ROW_F64 || K <= TSG_STATE_F64_COLUMNS) ? 8
+                      : (type == TSG_ROW_U16 && branch)                   ? 2
+                                                                          : 4;
     return tile * (8 + 8 + (branch ? 8 : 4) + el * (size_t) K);
 }
 
@@ -1182,19 +1279,25 @@ hipError_t allow(F *fn, size_t shmem) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, most);
 }
 
+template <int TYPE, bool BRANCH, bool WIDE>
+hipError_t launch_eval_as(const TsgStateArgs &a, hipStream_t s) {
+    const size_t sh = tsg_state_shmem(a.K, TYPE, BRANCH);
+    hipError_t e = allow(&k_state_eval<TYPE, BRANCH, WIDE>, sh);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_state_eval<TYPE, BRANCH, WIDE>),
+                       dim3(xcd_grid(BRANCH ? a.btiles : a.stiles)), dim3(EVAL_THREADS), sh, s, a);
+    return hipGetLastError();
+}
 template <int TYPE, bool BRANCH>
 hipError_t launch_eval(const TsgStateArgs &a, hipStream_t s) {
-    const size_t sh = tsg_state_shmem(a.K, TYPE, BRANCH);
-    hipError_t e = allow(&k_state_eval<TYPE, BRANCH>, sh);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_state_eval<TYPE, BRANCH>), dim3(xcd_grid(BRANCH ? a.btiles : a.stiles)),
-                       dim3(EVAL_THREADS), sh, s, a);
-    return hipGetLastError();
+    if (TYPE == TSG_ROW_F64 || a.K <= TSG_STATE_F64_COLUMNS) {
+        return launch_eval_as<TYPE, BRANCH, false>(a, s);
+    }
+    return launch_eval_as<TYPE, BRANCH, TYPE != TSG_ROW_F64>(a, s);
 }
 
 template <int TYPE>
-hipError_t launch_run(const TsgStateLaunch &r, hipEvent_t begin, hipEvent_t mid, hipEvent_t end,
-                      hipStream_t s) {
+hipError_t launch_counts(const TsgStateLaunch &r, hipEvent_t begin, hipStream_t s) {
     const TsgStateArgs &a = r.a;
     constexpr bool F64 = TYPE == TSG_ROW_F64;
     hipLaunchKernelGGL(k_state_stage, dim3((unsigned) stage_blocks(a)), dim3(256), 0, s, a);
@@ -1209,6 +1312,15 @@ hipError_t launch_run(const TsgStateLaunch &r, hipEvent_t begin, hipEvent_t mid,
         hipLaunchKernelGGL((k_state_count<F64>), dim3(xcd_grid(nb)), dim3(256), 0, s, a, s0, s1,
                            (int) nb);
     }
+    return hipGetLastError();
+}
+
+template <int TYPE>
+hipError_t launch_run(const TsgStateLaunch &r, hipEvent_t begin, hipEvent_t mid, hipEvent_t end,
+                      hipStream_t s) {
+    const TsgStateArgs &a = r.a;
+    hipError_t e = launch_counts<TYPE>(r, begin, s);
+    if (e != hipSuccess) return e;
     if (a.QB > 0 && (e = launch_eval<TYPE, true>(a, s)) != hipSuccess) return e;
     if (mid != nullptr && (e = hipEventRecord(mid, s)) != hipSuccess) return e;
     if (a.Q > a.QB && (e = launch_eval<TYPE, false>(a, s)) != hipSuccess) return e;
@@ -1234,6 +1346,45 @@ int levels_of(const TsgStateLaunch *runs, int nrun) {
     return l;
 }
 }  // namespace
+
+hipError_t tsg_launch_state_counts(const TsgStateLaunch &r, hipEvent_t begin, hipStream_t s) {
+    switch (r.type) {
+    case TSG_ROW_U16:
+        return launch_counts<TSG_ROW_U16>(r, begin, s);
+    case TSG_ROW_I32:
+        return launch_counts<TSG_ROW_I32>(r, begin, s);
+    default:
+        return launch_counts<TSG_ROW_F64>(r, begin, s);
+    }
+}
+
+hipError_t tsg_launch_state_nodes(const TsgStateLaunch &r, const TsgNodeArgs &g, int M,
+                                  hipStream_t s) {
+    const unsigned nb = (unsigned) (((int64_t) g.runs * M + 255) / 256);
+    if (nb == 0) return hipSuccess;
+    if (r.type == TSG_ROW_U16) {
+        hipLaunchKernelGGL((k_state_nodes<TSG_ROW_U16>), dim3(nb), dim3(256), 0, s, r.a, g);
+    } else {
+        hipLaunchKernelGGL((k_state_nodes<TSG_ROW_I32>), dim3(nb), dim3(256), 0, s, r.a, g);
+    }
+    return hipGetLastError();
+}
+
+hipError_t tsg_launch_spectrum(const TsgStateLaunch &r, const TsgSpectrumArgs &g, bool branch,
+                               hipStream_t s) {
+    const unsigned nb = (unsigned) (((branch ? g.npieces : r.a.nrow) + 255) / 256);
+    if (nb == 0) return hipSuccess;
+    if (branch && r.type == TSG_ROW_U16) {
+        hipLaunchKernelGGL((k_spectrum_branch<TSG_ROW_U16>), dim3(nb), dim3(256), 0, s, r.a, g);
+    } else if (branch) {
+        hipLaunchKernelGGL((k_spectrum_branch<TSG_ROW_I32>), dim3(nb), dim3(256), 0, s, r.a, g);
+    } else if (r.type == TSG_ROW_U16) {
+        hipLaunchKernelGGL((k_spectrum_site<TSG_ROW_U16>), dim3(nb), dim3(256), 0, s, r.a, g);
+    } else {
+        hipLaunchKernelGGL((k_spectrum_site<TSG_ROW_I32>), dim3(nb), dim3(256), 0, s, r.a, g);
+    }
+    return hipGetLastError();
+}
 
 hipError_t tsg_launch_states(const TsgStateLaunch &r, hipEvent_t begin, hipEvent_t mid,
                              hipEvent_t end, hipStream_t s) {
@@ -1286,7 +1437,7 @@ int tsg_state_prefixes(const TsgStateLaunch *runs, int nrun, std::vector<int32_t
 }
 
 namespace {
-template <int TYPE>
+template <int TYPE, bool WIDE>
 hipError_t launch_multi(const TsgStateLaunch *runs, const TsgStateArgs *args, int nrun,
                         const std::vector<int32_t> &pre_h, const int32_t *pre, hipStream_t s) {
     constexpr bool F64 = TYPE == TSG_ROW_F64;
@@ -1314,14 +1465,14 @@ hipError_t launch_multi(const TsgStateLaunch *runs, const TsgStateArgs *args, in
     }
     hipError_t e;
     if (total(PH_BRANCH) > 0) {
-        if ((e = allow(&k_states_eval<TYPE, true>, sb)) != hipSuccess) return e;
-        hipLaunchKernelGGL((k_states_eval<TYPE, true>), dim3(xcd_grid(total(PH_BRANCH))),
+        if ((e = allow(&k_states_eval<TYPE, true, WIDE>, sb)) != hipSuccess) return e;
+        hipLaunchKernelGGL((k_states_eval<TYPE, true, WIDE>), dim3(xcd_grid(total(PH_BRANCH))),
                            dim3(EVAL_THREADS), sb, s, args, at(PH_BRANCH), nrun,
                            total(PH_BRANCH));
     }
     if (total(PH_SITE) > 0) {
-        if ((e = allow(&k_states_eval<TYPE, false>, ss)) != hipSuccess) return e;
-        hipLaunchKernelGGL((k_states_eval<TYPE, false>), dim3(xcd_grid(total(PH_SITE))),
+        if ((e = allow(&k_states_eval<TYPE, false, WIDE>, ss)) != hipSuccess) return e;
+        hipLaunchKernelGGL((k_states_eval<TYPE, false, WIDE>), dim3(xcd_grid(total(PH_SITE))),
                            dim3(EVAL_THREADS), ss, s, args, at(PH_SITE), nrun, total(PH_SITE));
     }
     if (total(PH_WINDOWS) > 0) {
@@ -1341,12 +1492,15 @@ hipError_t launch_multi(const TsgStateLaunch *runs, const TsgStateArgs *args, in
 hipError_t tsg_launch_states_multi(const TsgStateLaunch *runs, const TsgStateArgs *args, int nrun,
                                    const std::vector<int32_t> &pre_h, const int32_t *pre,
                                    hipStream_t s) {
+    const bool wide = runs[0].a.K > TSG_STATE_F64_COLUMNS;
     switch (runs[0].type) {
     case TSG_ROW_U16:
-        return launch_multi<TSG_ROW_U16>(runs, args, nrun, pre_h, pre, s);
+        return wide ? launch_multi<TSG_ROW_U16, true>(runs, args, nrun, pre_h, pre, s)
+                    : launch_multi<TSG_ROW_U16, false>(runs, args, nrun, pre_h, pre, s);
     case TSG_ROW_I32:
-        return launch_multi<TSG_ROW_I32>(runs, args, nrun, pre_h, pre, s);
+        return wide ? launch_multi<TSG_ROW_I32, true>(runs, args, nrun, pre_h, pre, s)
+                    : launch_multi<TSG_ROW_I32, false>(runs, args, nrun, pre_h, pre, s);
     default:
-        return launch_multi<TSG_ROW_F64>(runs, args, nrun, pre_h, pre, s);
+        return launch_multi<TSG_ROW_F64, false>(runs, args, nrun, pre_h, pre, s);
     }
 }

@@ -81,25 +81,35 @@ int check_tables(const tsg_treeseq *ts) {
 void tsg_build_index(const double *left, const double *right, const int32_t *parent,
                      const int32_t *child, const double *time, int32_t E, int32_t *I,
                      int32_t *O) {
-    std::vector<int32_t> idx(E);
-    std::iota(idx.begin(), idx.end(), 0);
-    std::sort(idx.begin(), idx.end(), [&](int32_t a, int32_t b) {
-        if (left[a] != left[b]) return left[a] < left[b];
-        const double ta = time[parent[a]], tb = time[parent[b]];
-        if (ta != tb) return ta < tb;
-        if (parent[a] != parent[b]) return parent[a] < parent[b];
-        return child[a] < child[b];
-    });
-    std::copy(idx.begin(), idx.end(), I);
-    std::iota(idx.begin(), idx.end(), 0);
-    std::sort(idx.begin(), idx.end(), [&](int32_t a, int32_t b) {
-        if (right[a] != right[b]) return right[a] < right[b];
-        const double ta = time[parent[a]], tb = time[parent[b]];
-        if (ta != tb) return ta > tb;
-        if (parent[a] != parent[b]) return parent[a] > parent[b];
-        return child[a] > child[b];
-    });
-    std::copy(idx.begin(), idx.end(), O);
+    auto insertion = [&]() {
+        std::iota(I, I + E, 0);
+        std::sort(I, I + E, [&](int32_t a, int32_t b) {
+            if (left[a] != left[b]) return left[a] < left[b];
+            const double ta = time[parent[a]], tb = time[parent[b]];
+            if (ta != tb) return ta < tb;
+            if (parent[a] != parent[b]) return parent[a] < parent[b];
+            return child[a] < child[b];
+        });
+    };
+    auto removal = [&]() {
+        std::iota(O, O + E, 0);
+        std::sort(O, O + E, [&](int32_t a, int32_t b) {
+            if (right[a] != right[b]) return right[a] < right[b];
+            const double ta = time[parent[a]], tb = time[parent[b]];
+            if (ta != tb) return ta > tb;
+            if (parent[a] != parent[b]) return parent[a] > parent[b];
+            return child[a] > child[b];
+        });
+    };
+    // the two orders side by side, where they are worth a thread
+    if (E < 2048) {
+        insertion();
+        removal();
+        return;
+    }
+    std::thread other(removal);
+    insertion();
+    other.join();
 }
 
 // Fills samples, breakpoints, per-tree site ranges and allele encoding, and

@@ -10,6 +10,7 @@
 // Query-independent data the sweep kernels read, resident in HBM.
 struct TsgDevice {
     int device = -1;
+    void *block = nullptr;            // holds breakpoints .. site_nalleles
     // per chunk [C+1]
     int32_t *chunk_tree0 = nullptr;   // first tree of each chunk (last entry = T)
     int64_t *chunk_node0 = nullptr;   // offset of each chunk's local-node block
@@ -41,6 +42,7 @@ struct TsgDevice {
 
 // Device copy of a hot plan (see tsg_hotplan).
 struct TsgHotDevice {
+    void *block = nullptr;            // holds chunk_tree0 .. t0_bl
     int32_t *chunk_tree0 = nullptr;
     int64_t *chunk_slot0 = nullptr;
     int32_t *slot_par = nullptr;

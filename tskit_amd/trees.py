@@ -273,6 +273,7 @@ class LowLevelTreeSequence:
         z = self.get_state_plan_sizes()
         inner = max(0, z["states"] - 1 - self.get_num_samples())
         out = dict(level0=np.zeros(z["levels"] + 1, np.int32),
+                   order=np.zeros(z["states"], np.int32),
                    inputs=np.zeros((inner, 8), np.int32),
                    ev_state=np.zeros(z["events"], np.int32), ev_b=np.zeros(z["events"]),
                    ev_pos=np.zeros(z["events"]), row_ref=np.zeros(z["rows"], np.int32),
