@@ -1658,6 +1658,11 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
     std::vector<TsgStateOut> outs;
     outs.reserve(fz.outs.size());
     for (const TsgOut &o : fz.outs) outs.push_back(state_out(o, fz));
+    for (size_t m = outs.size(); m-- > 0;) {  // (a kernel's runs end with the query)
+        const bool more = m + 1 < outs.size() && outs[m + 1].stat == outs[m].stat &&
+                          outs[m + 1].polarised == outs[m].polarised;
+        outs[m].run = more ? outs[m + 1].run + 1 : 1;
+    }
     Pack pk;
     const int p_ps = pk.add(fz.pair_s), p_pc = pk.add(fz.pair_c), p_outs = pk.add(outs);
     const int p_qs = pk.add(qs), p_win = pk.add(fz.wins), p_tot = pk.add(fz.col_total);

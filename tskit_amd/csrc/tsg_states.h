@@ -125,7 +125,8 @@ struct TsgStateOut {
     int32_t par;             // weighted summaries: offset of their parameters in opar
     int32_t cbase, ccount;   // trait regression: its covariates
     int32_t samples;         // ... and the number of samples
-    int32_t pad[2];
+    int32_t run;             // outputs from this one on of the same summary
+    int32_t pad;
     double n[4];
     double scale;            // 1 / denominator, twice that where one(x) = one(n - x)
     double coef[2];          // centred relatedness: 1 / n; weighted: its parameters

@@ -234,6 +234,15 @@ struct TileType<TSG_ROW_I32, BRANCH, true> {
     using T = int32_t;
 };
 
+// Elements from one column of a tile to the next: a few more than its
+// events, so that threads reading one event of different columns read
+// different banks (without: 20 conflict cycles per LDS instruction on 64
+// columns), and aligned for the paired loads.
+template <typename T>
+constexpr int stride_of(int tile) {
+    return tile + 2;
+}
+
 // A record of memory that no kernel of the run writes, at an address that is
 // the same for the whole wave: scalar loads.
 template <typename R>
@@ -485,7 +494,7 @@ __device__ __forceinline__ double regression(const TsgStateArgs &a, const TsgSta
     const double *v = a.opar + o.par;
     const double *tot = a.col_total_w;
     auto X = [&](int c) {
-        const double x = cols[c * TILE + e];
+        const double x = cols[c * stride_of<double>(TILE) + e];
         return comp ? tot[c] - x : x;
     };
     const double m = X(o.c[3]);
@@ -499,37 +508,37 @@ __device__ __forceinline__ double regression(const TsgStateArgs &a, const TsgSta
     return denom < 1e-8 ? 0.0 : (r * r) / (2 * denom * denom);
 }
 
-// Calls use(f, c2) with the summary f of output o and the column (or mean)
-// of its slot 2.
-template <int TYPE, int TILE, typename T, typename U>
-__device__ __forceinline__ void with_summary(const TsgStateOut &o, const Tile<T> &tile, U use) {
-    const T *c2 = tile.cols + o.c[2] * TILE;
-    const Nums n{{o.n[0], o.n[1], o.n[2], o.n[3]}};
-#define SUMMARY(ID, F) \
-    case ID: {         \
-        F f;           \
-        f.p = n;       \
-        use(f, c2);    \
-        break;         \
-    }
+// Calls use(make) for the summary `stat`, make(o) being the summary of output
+// o of that kind.
+template <int TYPE, typename U>
+__device__ __forceinline__ void with_summary(int stat, U use) {
+#define SUMMARY(ID, F)                                                  \
+    case ID:                                                            \
+        use([](const TsgStateOut &o) {                                  \
+            F f;                                                        \
+            f.p = Nums{{o.n[0], o.n[1], o.n[2], o.n[3]}};               \
+            return f;                                                   \
+        });                                                             \
+        break;
     if constexpr (TYPE == TSG_ROW_F64) {
-        switch (o.stat) {
+        switch (stat) {
             SUMMARY(TSG_STAT_TRAIT_COVARIANCE, TraitCovariance)
             SUMMARY(TSG_STAT_TRAIT_CORRELATION, TraitCorrelation)
             SUMMARY(TSG_STAT_RELATEDNESS_WEIGHTED_NONCENTRED, Product)
-        case TSG_STAT_RELATEDNESS_WEIGHTED: {
-            RelatednessWeighted f;
-            f.p = n;
-            f.ca = o.coef[0];
-            f.cb = o.coef[1];
-            use(f, c2);
+        case TSG_STAT_RELATEDNESS_WEIGHTED:
+            use([](const TsgStateOut &o) {
+                RelatednessWeighted f;
+                f.p = Nums{{o.n[0], o.n[1], o.n[2], o.n[3]}};
+                f.ca = o.coef[0];
+                f.cb = o.coef[1];
+                return f;
+            });
             break;
-        }
         default:
             break;
         }
     } else {
-        switch (o.stat) {
+        switch (stat) {
             SUMMARY(TSG_STAT_DIVERSITY, Diversity)
             SUMMARY(TSG_STAT_SEGREGATING_SITES, Segregating)
             SUMMARY(TSG_STAT_Y1, Y1)
@@ -541,7 +550,7 @@ __device__ __forceinline__ void with_summary(const TsgStateOut &o, const Tile<T>
             SUMMARY(TSG_STAT_F3, F3)
             SUMMARY(TSG_STAT_F4, F4)
         case TSG_STAT_RELATEDNESS:
-            use(Relatedness{o.coef[0], o.coef[1]}, tile.mean);
+            use([](const TsgStateOut &o) { return Relatedness{o.coef[0], o.coef[1]}; });
             break;
         default:
             break;
@@ -549,45 +558,9 @@ __device__ __forceinline__ void with_summary(const TsgStateOut &o, const Tile<T>
     }
 #undef SUMMARY
 }
-
-// Output o's two sums over this lane's events, before the scale.
-template <int TYPE, int TILE, bool BRANCH, typename T>
-__device__ __forceinline__ void add_output(const TsgStateArgs &a, const TsgStateOut &o,
-                                           const Tile<T> &tile, int lane,
-                                           const LaneEvents<TILE / WAVE> &ev, double &L,
-                                           double &J) {
-    const bool pol = o.polarised != 0;
-    if constexpr (TYPE == TSG_ROW_F64) {
-        if (o.stat == TSG_STAT_TRAIT_LINEAR_MODEL) {
-            constexpr int N = TILE / WAVE;
-#pragma unroll
-            for (int r = 0; r < N; r++) {
-                const int e = 2 * WAVE * (r / 2) + 2 * lane + (r & 1);
-                const int k = (!BRANCH && tile.mixed) ? tile.kind[e] : TSG_ROW_PAIR;
-                double f = (pol && k == TSG_ROW_ANCESTRAL)
-                               ? 0.0
-                               : regression<TILE>(a, o, tile.cols, e, false);
-                if (!pol && k == TSG_ROW_PAIR) f = f + regression<TILE>(a, o, tile.cols, e, true);
-                L = fma(f, ev.wl[r], L);
-                if constexpr (BRANCH) J = fma(f, ev.wb[r], J);
-            }
-            return;
-        }
-    }
-    const T *c0 = tile.cols + o.c[0] * TILE, *c1 = tile.cols + o.c[1] * TILE;
-    const T *c3 = tile.cols + o.c[3] * TILE;
-    with_summary<TYPE, TILE>(o, tile, [&](const auto &f, const auto *c2) {
-        if (!BRANCH && tile.mixed) {
-            add_up<T, TILE, BRANCH, VALUE_MIXED>(f, c0, c1, c2, c3, tile.kind, pol, lane, ev, L,
-                                                 J);
-        } else if (pol) {
-            add_up<T, TILE, BRANCH, VALUE_ONE>(f, c0, c1, c2, c3, tile.kind, true, lane, ev, L, J);
-        } else {
-            add_up<T, TILE, BRANCH, VALUE_BOTH>(f, c0, c1, c2, c3, tile.kind, false, lane, ev, L,
-                                                J);
-        }
-    });
-}
+// its slot 2 is the query's mean, not a column
+template <typename F>
+constexpr bool reads_mean = std::is_same<F, Relatedness>::value;
 
 // Output o's summary of event e alone, before the scale.
 template <int TYPE, int TILE, bool BRANCH, typename T>
@@ -603,13 +576,19 @@ __device__ __forceinline__ double value_of(const TsgStateArgs &a, const TsgState
             return both ? v + regression<TILE>(a, o, tile.cols, e, true) : v;
         }
     }
-    double x[4] = {(double) tile.cols[o.c[0] * TILE + e], 0.0, 0.0, 0.0};
+    constexpr int STRIDE = stride_of<T>(TILE);
+    double x[4] = {(double) tile.cols[o.c[0] * STRIDE + e], 0.0, 0.0, 0.0};
     double v = 0.0;
-    with_summary<TYPE, TILE>(o, tile, [&](const auto &f, const auto *c2) {
-        constexpr int S = std::decay<decltype(f)>::type::S;
-        if constexpr (S > 1) x[1] = (double) tile.cols[o.c[1] * TILE + e];
-        if constexpr (S > 2) x[2] = (double) c2[e];
-        if constexpr (S > 3) x[3] = (double) tile.cols[o.c[3] * TILE + e];
+    with_summary<TYPE>(o.stat, [&](auto make) {
+        const auto f = make(o);
+        using F = typename std::decay<decltype(f)>::type;
+        if constexpr (F::S > 1) x[1] = (double) tile.cols[o.c[1] * STRIDE + e];
+        if constexpr (reads_mean<F>) {
+            x[2] = tile.mean[e];
+        } else if constexpr (F::S > 2) {
+            x[2] = (double) tile.cols[o.c[2] * STRIDE + e];
+        }
+        if constexpr (F::S > 3) x[3] = (double) tile.cols[o.c[3] * STRIDE + e];
         v = pol ? f.one(x) : both ? f.both(x) : f.lone(x);
     });
     return v;
@@ -655,6 +634,86 @@ __device__ __forceinline__ double wave_sums(double a, double b, double c, double
     return a;
 }
 
+// A round's sums of a wave into the segment: two outputs (branch: sums L and
+// J) or four (site); lanes 0, 16, 32, 48 hold acc 0, 2, 1, 3.
+template <bool BRANCH, int WAVES>
+__device__ __forceinline__ void store_round(const double (&acc)[4], const double (&scale)[4],
+                                            int m0, int count, int lane, bool any, double *dst) {
+    constexpr int PER = BRANCH ? 2 : 1;
+    const double v = wave_sums(acc[0], acc[1], acc[2], acc[3]);
+    const int row = lane / 16;
+    const int at = row == 1 ? 2 : (row == 2 ? 1 : row);
+    const int i = BRANCH ? at / 2 : at;
+    if (lane % 16 == 0 && m0 + i * WAVES < count) {
+        const double sc = i == 0 ? scale[0] : i == 1 ? scale[1] : i == 2 ? scale[2] : scale[3];
+        // (a zero denominator: 0 x inf is the reference's NaN at every state,
+        // but a window without events has 0)
+        dst[(m0 + i * WAVES) * PER + (BRANCH ? (at & 1) : 0)] = any ? v * sc : 0.0;
+    }
+}
+
+// `count` outputs of one summary over the window's events: this wave's are
+// wave, wave + 4, ...; the next round's records are read while a round is
+// summed.
+template <typename T, int TILE, bool BRANCH, int VALUE, typename Make>
+__device__ __forceinline__ void add_run(Make make, const TsgStateOut *outs, int count,
+                                        const Tile<T> &tile, bool polarised, int wave, int lane,
+                                        const LaneEvents<TILE / WAVE> &ev, bool any, double *dst) {
+    constexpr int WAVES = EVAL_THREADS / WAVE, ROUND = BRANCH ? 2 : 4, STRIDE = stride_of<T>(TILE);
+    if (wave >= count) return;
+    TsgStateOut o[ROUND];
+#pragma unroll
+    for (int i = 0; i < ROUND; i++) o[i] = uniform(outs + min(wave + i * WAVES, count - 1));
+    for (int m0 = wave; m0 < count; m0 += WAVES * ROUND) {
+        double acc[4] = {0, 0, 0, 0}, scale[4] = {0, 0, 0, 0}, unused = 0;
+#pragma unroll
+        for (int i = 0; i < ROUND; i++) {
+            const auto f = make(o[i]);
+            using F = typename std::decay<decltype(f)>::type;
+            scale[i] = o[i].scale;
+            const T *c0 = tile.cols + o[i].c[0] * STRIDE, *c1 = tile.cols + o[i].c[1] * STRIDE;
+            const T *c2 = tile.cols + o[i].c[2] * STRIDE, *c3 = tile.cols + o[i].c[3] * STRIDE;
+            o[i] = uniform(outs + min(m0 + (i + ROUND) * WAVES, count - 1));
+            if (i > 0 && m0 + i * WAVES >= count) continue;
+            double &L = acc[BRANCH ? 2 * i : i], &J = BRANCH ? acc[(2 * i + 1) & 3] : unused;
+            if constexpr (reads_mean<F>) {
+                add_up<T, TILE, BRANCH, VALUE>(f, c0, c1, tile.mean, c3, tile.kind, polarised, lane,
+                                               ev, L, J);
+            } else {
+                add_up<T, TILE, BRANCH, VALUE>(f, c0, c1, c2, c3, tile.kind, polarised, lane, ev, L,
+                                               J);
+            }
+        }
+        store_round<BRANCH, WAVES>(acc, scale, m0, count, lane, any, dst);
+    }
+}
+
+template <int TILE, bool BRANCH>
+__device__ __forceinline__ void add_regressions(const TsgStateArgs &a, const TsgStateOut *outs,
+                                                int count, const Tile<double> &tile, int wave,
+                                                int lane, const LaneEvents<TILE / WAVE> &ev,
+                                                bool any, double *dst) {
+    constexpr int WAVES = EVAL_THREADS / WAVE, N = TILE / WAVE;
+    for (int m = wave; m < count; m += WAVES) {
+        const TsgStateOut o = uniform(outs + m);
+        const bool pol = o.polarised != 0;
+        double L = 0, J = 0;
+#pragma unroll
+        for (int r = 0; r < N; r++) {
+            const int e = 2 * WAVE * (r / 2) + 2 * lane + (r & 1);
+            const int k = (!BRANCH && tile.mixed) ? tile.kind[e] : TSG_ROW_PAIR;
+            double f = (pol && k == TSG_ROW_ANCESTRAL)
+                           ? 0.0
+                           : regression<TILE>(a, o, tile.cols, e, false);
+            if (!pol && k == TSG_ROW_PAIR) f = f + regression<TILE>(a, o, tile.cols, e, true);
+            L = fma(f, ev.wl[r], L);
+            if constexpr (BRANCH) J = fma(f, ev.wb[r], J);
+        }
+        const double acc[4] = {L, J, 0, 0}, scale[4] = {o.scale, 0, 0, 0};
+        store_round<BRANCH, WAVES>(acc, scale, m, m + 1, lane, any, dst);
+    }
+}
+
 // One tile: events (BRANCH) or site rows t TILE .. of the run.  WIDE: more
 // columns than an FP64 tile takes.
 template <int TYPE, bool BRANCH, bool WIDE>
@@ -662,6 +721,7 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
     constexpr int TILE = BRANCH ? TSG_BRANCH_TILE : TSG_SITE_TILE;
     constexpr int N = TILE / WAVE;
     using T = typename TileType<TYPE, BRANCH, WIDE>::T;
+    constexpr int STRIDE = stride_of<T>(TILE);
     extern __shared__ double smem[];
     double *spos = smem;                                       // [TILE]
     double *sb = spos + TILE;                                  // [TILE] (branch)
@@ -671,7 +731,6 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
     const int tid = threadIdx.x;
     const int lane = tid & (WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    constexpr int WAVES = EVAL_THREADS / WAVE;
     const int K = a.K, RW = a.RW;
     const int total = BRANCH ? a.nev : a.nrow;
     const int e0 = t * TILE;
@@ -697,13 +756,13 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
             const uint32_t *row = a.x + (int64_t) ref * RW;
             auto put = [&](int w, uint32_t v) {  // word w of the row
                 if constexpr (TYPE == TSG_ROW_U16) {
-                    if (2 * w < K) cols[(2 * w) * TILE + e] = (T) (v & 0xFFFFu);
-                    if (2 * w + 1 < K) cols[(2 * w + 1) * TILE + e] = (T) (v >> 16);
+                    if (2 * w < K) cols[(2 * w) * STRIDE + e] = (T) (v & 0xFFFFu);
+                    if (2 * w + 1 < K) cols[(2 * w + 1) * STRIDE + e] = (T) (v >> 16);
                 } else if constexpr (TYPE == TSG_ROW_I32) {
-                    if (w < K) cols[w * TILE + e] = (T) (int32_t) v;
+                    if (w < K) cols[w * STRIDE + e] = (T) (int32_t) v;
                 } else {
                     if (w < 2 * K) {
-                        reinterpret_cast<uint32_t *>(cols + (w / 2) * TILE + e)[w & 1] = v;
+                        reinterpret_cast<uint32_t *>(cols + (w / 2) * STRIDE + e)[w & 1] = v;
                     }
                 }
             };
@@ -745,7 +804,7 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                     }
                     v = (ent & 1) ? v - xv : v + xv;
                 }
-                cols[k * TILE + e] = v;
+                cols[k * STRIDE + e] = v;
             }
         }
     }
@@ -766,7 +825,7 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                 for (int e = tid; e < TILE; e += EVAL_THREADS) {
                     double s = 0;
                     for (int c = Q.rel_c0; c < Q.rel_c0 + Q.rel_cn; c++) {
-                        s += (double) cols[c * TILE + e] / (double) a.col_total[c];
+                        s += (double) cols[c * STRIDE + e] / (double) a.col_total[c];
                     }
                     mean[e] = s / (double) Q.rel_cn;
                 }
@@ -825,35 +884,32 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                     ev.wb[r] = 0.0;
                 }
             }
-            // outputs wave, wave + 4, ...: two (branch: sums L and J) or four
-            // (site) of them a round; lanes 0, 16, 32, 48 hold acc 0, 2, 1, 3
-            constexpr int ROUND = BRANCH ? 2 : 4;
-            const int row = lane / 16;
-            const int at = row == 1 ? 2 : (row == 2 ? 1 : row);
-            double *dst = a.partial + Q.pbase + (int64_t) (t + w) * M * PER +
-                          (BRANCH ? (at / 2) * WAVES * 2 + (at & 1) : at * WAVES);
-            for (int m0 = wave; m0 < M; m0 += WAVES * ROUND) {
-                double acc[4] = {0, 0, 0, 0}, scale[ROUND], unused = 0;
-#pragma unroll
-                for (int i = 0; i < ROUND; i++) {
-                    const int m = min(m0 + i * WAVES, M - 1);
-                    const TsgStateOut o = uniform(a.outs + Q.mbase + m);
-                    scale[i] = o.scale;
-                    if (m0 + i * WAVES < M) {
-                        add_output<TYPE, TILE, BRANCH>(a, o, tile, lane, ev,
-                                                       acc[BRANCH ? 2 * i : i],
-                                                       BRANCH ? acc[2 * i + 1] : unused);
+            double *dst = a.partial + Q.pbase + (int64_t) (t + w) * M * PER;
+            for (int m = 0; m < M;) {
+                // a run of outputs of one summary, polarised or not
+                const TsgStateOut first = uniform(a.outs + Q.mbase + m);
+                const TsgStateOut *outs = a.outs + Q.mbase + m;
+                const int count = min(first.run, M - m);
+                if constexpr (TYPE == TSG_ROW_F64) {
+                    if (first.stat == TSG_STAT_TRAIT_LINEAR_MODEL) {
+                        add_regressions<TILE, BRANCH>(a, outs, count, tile, wave, lane, ev, eb > ea,
+                                                      dst + m * PER);
                     }
                 }
-                double v = wave_sums(acc[0], acc[1], acc[2], acc[3]);
-                if (lane % 16 == 0 && m0 + (BRANCH ? at / 2 : at) * WAVES < M) {
-                    double sc = scale[0];
-#pragma unroll
-                    for (int i = 1; i < ROUND; i++) {
-                        if ((BRANCH ? at / 2 : at) == i) sc = scale[i];
+                with_summary<TYPE>(first.stat, [&](auto make) {
+                    if (!BRANCH && mixed) {
+                        add_run<T, TILE, BRANCH, VALUE_MIXED>(make, outs, count, tile,
+                                                              first.polarised != 0, wave, lane, ev,
+                                                              eb > ea, dst + m * PER);
+                    } else if (first.polarised) {
+                        add_run<T, TILE, BRANCH, VALUE_ONE>(make, outs, count, tile, true, wave,
+                                                            lane, ev, eb > ea, dst + m * PER);
+                    } else {
+                        add_run<T, TILE, BRANCH, VALUE_BOTH>(make, outs, count, tile, false, wave,
+                                                             lane, ev, eb > ea, dst + m * PER);
                     }
-                    dst[m0 * PER] = eb > ea ? v * sc : 0.0;
-                }
+                });
+                m += count;
             }
         }
     }
@@ -943,15 +999,24 @@ __device__ __forceinline__ void finish(const TsgStateArgs &a, int b) {
             if (per == 2) J += src[1];
         }
     };
+    // a run's first windows stay in registers between the two passes
+    constexpr int KEEP = 8;
+    double Lk[KEEP], Jk[KEEP];
+    const int n = on ? wb - wa : 0;
+#pragma unroll
+    for (int i = 0; i < KEEP; i++) {
+        Lk[i] = Jk[i] = 0;
+        if (i < n) sums(wa + i, Lk[i], Jk[i]);
+    }
     double R = 0;
     if (per == 2) {
         double acc = 0;
-        if (on && wa < wb) {
-            for (int w = wa; w < wb; w++) {
-                double L, J;
-                sums(w, L, J);
-                acc += J;
-            }
+#pragma unroll
+        for (int i = 0; i < KEEP; i++) acc += Jk[i];
+        for (int i = KEEP; i < n; i++) {
+            double L, J;
+            sums(wa + i, L, J);
+            acc += J;
         }
         scan[threadIdx.x] = acc;
         __syncthreads();
@@ -964,16 +1029,22 @@ __device__ __forceinline__ void finish(const TsgStateArgs &a, int b) {
         }
         R = seg > 0 ? scan[threadIdx.x - mb] : 0.0;
     }
-    if (!on || wa >= wb) return;
     double *dst = (Q.to_out ? a.out : a.raw) + Q.obase;
-    for (int w = wa; w < wb; w++) {
-        double L, J;
-        sums(w, L, J);
+    auto put = [&](int w, double L, double J) {
         const double span = win[w + 1] - win[w];
         double v = L + R * span;
         if (Q.flags & TSG_F_SPAN_NORMALISE) v /= span;
         dst[(int64_t) w * M + m] = v;
         R += J;
+    };
+#pragma unroll
+    for (int i = 0; i < KEEP; i++) {
+        if (i < n) put(wa + i, Lk[i], Jk[i]);
+    }
+    for (int i = KEEP; i < n; i++) {
+        double L, J;
+        sums(wa + i, L, J);
+        put(wa + i, L, J);
     }
 }
 
@@ -1002,10 +1073,10 @@ __device__ __forceinline__ double state_value(const TsgStateArgs &a, const TsgSt
     }
     double x[4] = {row_value<TYPE>(a, s, o.c[0]), row_value<TYPE>(a, s, o.c[1]), 0.0, 0.0};
     double v = 0.0;
-    const Tile<double> none{&mean, nullptr, false, nullptr};
-    with_summary<TYPE, 1>(o, none, [&](const auto &f, const auto *) {
+    with_summary<TYPE>(o.stat, [&](auto make) {
+        const auto f = make(o);
         using F = typename std::decay<decltype(f)>::type;
-        if constexpr (std::is_same<F, Relatedness>::value) {
+        if constexpr (reads_mean<F>) {
             x[2] = mean;
         } else {
             if constexpr (F::S > 2) x[2] = row_value<TYPE>(a, s, o.c[2]);
@@ -1264,7 +1335,7 @@ size_t tsg_state_shmem(int K, int type, bool branch) {
     const size_t el = (type == TSG_ROW_F64 || K <= TSG_STATE_F64_COLUMNS) ? 8
                       : (type == TSG_ROW_U16 && branch)                   ? 2
                                                                           : 4;
-    return tile * (8 + 8 + (branch ? 8 : 4) + el * (size_t) K);
+    return tile * (8 + 8 + (branch ? 8 : 4)) + el * (tile + 2) * (size_t) K + 16;
 }
 
 namespace {
