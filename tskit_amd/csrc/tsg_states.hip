@@ -42,6 +42,7 @@
 #define WAVE 64
 #define EVAL_THREADS 256
 #define FINISH_THREADS 1024
+#define SPECTRUM_SLOTS 1024
 
 namespace {
 
@@ -1209,31 +1210,59 @@ __global__ void __launch_bounds__(256) k_spectrum_site(const TsgStateArgs a,
 // Thread per branch piece: its span times the branch's length in each time
 // window, cut at the windows it crosses; a piece that ends at a window's end
 // counts where the edge was there before it (trees.c:3650-3690).
+//
+// Bound by adds to one address: most branches lie above one or two samples,
+// so a few cells of each window take most of them.  The pieces are in order
+// of their ends, so those of a workgroup fall into one or two windows; it
+// adds into SPECTRUM_SLOTS cells of LDS, a cell to the first index that
+// claims it, and sends each on once; other indexes go to memory directly.
 template <int TYPE>
 __global__ void __launch_bounds__(256) k_spectrum_branch(const TsgStateArgs a,
-                                                         const TsgSpectrumArgs g) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= g.npieces) return;
-    const TsgBranchPiece p = g.pieces[i];
-    int32_t c[TSG_SPECTRUM_SETS];
-    for (int k = 0; k < a.K; k++) c[k] = row_count<TYPE>(a, p.state, k);
-    const int64_t at = spectrum_index(g, a.K, c);
-    auto add = [&](int w, double span) {
-        for (int tw = 0; tw < g.TW && g.time_windows[tw] < p.tp; tw++) {
-            const double length = fmax(0.0, fmin(g.time_windows[tw + 1], p.tp) -
-                                                fmax(g.time_windows[tw], p.tu));
-            atomicAdd(&g.hist_d[((int64_t) w * g.TW + tw) * g.size + at], span * length);
-        }
-    };
-    int w = window_of(g.windows, g.W, p.from);
-    double from = p.from;
-    while (w < g.W && g.windows[w + 1] <= p.to) {
-        const double end = g.windows[w + 1];
-        if (p.ins < end) add(w, end - from);
-        from = end;
-        w++;
+                                                         const TsgSpectrumArgs g, int per) {
+    __shared__ unsigned long long cell[SPECTRUM_SLOTS];  // index + 1, 0: free
+    __shared__ double sum[SPECTRUM_SLOTS];
+    for (int i = threadIdx.x; i < SPECTRUM_SLOTS; i += 256) {
+        cell[i] = 0;
+        sum[i] = 0;
     }
-    if (w < g.W && p.to > from) add(w, p.to - from);
+    __syncthreads();
+    const int64_t first = (int64_t) blockIdx.x * per;
+    const int last = (int) min(first + per, (int64_t) g.npieces);
+    for (int i = (int) first + threadIdx.x; i < last; i += 256) {
+        const TsgBranchPiece p = g.pieces[i];
+        int32_t c[TSG_SPECTRUM_SETS];
+        for (int k = 0; k < a.K; k++) c[k] = row_count<TYPE>(a, p.state, k);
+        const int64_t at = spectrum_index(g, a.K, c);
+        auto add = [&](int w, double span) {
+            for (int tw = 0; tw < g.TW && g.time_windows[tw] < p.tp; tw++) {
+                const double length = fmax(0.0, fmin(g.time_windows[tw + 1], p.tp) -
+                                                    fmax(g.time_windows[tw], p.tu));
+                const int64_t to = ((int64_t) w * g.TW + tw) * g.size + at;
+                const int slot = (int) (((uint64_t) to * 0x9e3779b97f4a7c15ull) >> 54);
+                static_assert(SPECTRUM_SLOTS == 1 << (64 - 54), "slot bits");
+                const unsigned long long key = (unsigned long long) to + 1;
+                const unsigned long long was = atomicCAS(&cell[slot], 0ull, key);
+                if (was == 0 || was == key) {
+                    unsafeAtomicAdd(&sum[slot], span * length);
+                } else {
+                    unsafeAtomicAdd(&g.hist_d[to], span * length);
+                }
+            }
+        };
+        int w = window_of(g.windows, g.W, p.from);
+        double from = p.from;
+        while (w < g.W && g.windows[w + 1] <= p.to) {
+            const double end = g.windows[w + 1];
+            if (p.ins < end) add(w, end - from);
+            from = end;
+            w++;
+        }
+        if (w < g.W && p.to > from) add(w, p.to - from);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < SPECTRUM_SLOTS; i += 256) {
+        if (cell[i] != 0) unsafeAtomicAdd(&g.hist_d[cell[i] - 1], sum[i]);
+    }
 }
 
 // --- one run ----------------------------------------------------------------------
@@ -1443,12 +1472,15 @@ hipError_t tsg_launch_state_nodes(const TsgStateLaunch &r, const TsgNodeArgs &g,
 
 hipError_t tsg_launch_spectrum(const TsgStateLaunch &r, const TsgSpectrumArgs &g, bool branch,
                                hipStream_t s) {
-    const unsigned nb = (unsigned) (((branch ? g.npieces : r.a.nrow) + 255) / 256);
-    if (nb == 0) return hipSuccess;
+    const int64_t n = branch ? g.npieces : r.a.nrow;
+    if (n == 0) return hipSuccess;
+    // (branch: at most 1024 workgroups, so that each adds up more of them)
+    const int per = branch ? 256 * (int) ((n + 256 * 1024 - 1) / (256 * 1024)) : 256;
+    const unsigned nb = (unsigned) ((n + per - 1) / per);
     if (branch && r.type == TSG_ROW_U16) {
-        hipLaunchKernelGGL((k_spectrum_branch<TSG_ROW_U16>), dim3(nb), dim3(256), 0, s, r.a, g);
+        hipLaunchKernelGGL((k_spectrum_branch<TSG_ROW_U16>), dim3(nb), dim3(256), 0, s, r.a, g, per);
     } else if (branch) {
-        hipLaunchKernelGGL((k_spectrum_branch<TSG_ROW_I32>), dim3(nb), dim3(256), 0, s, r.a, g);
+        hipLaunchKernelGGL((k_spectrum_branch<TSG_ROW_I32>), dim3(nb), dim3(256), 0, s, r.a, g, per);
     } else if (r.type == TSG_ROW_U16) {
         hipLaunchKernelGGL((k_spectrum_site<TSG_ROW_U16>), dim3(nb), dim3(256), 0, s, r.a, g);
     } else {
