@@ -639,37 +639,53 @@ bool is_device_ptr(const void *p) {
     return attr.type == hipMemoryTypeDevice;
 }
 
-// `bytes` of device memory src into the caller's dst, waiting for stream s
-// to finish: a device copy when dst is device memory, one transfer when it
-// is pinned host memory or tiny; otherwise through a ring of pinned pieces,
-// each piece's transfer running while host threads copy earlier ones into
-// dst (pageable memory takes its transfers slowly and its first touch is paid
-// in the copy; spread over threads, both go faster).  Pieces of 2 MiB: the
-// last piece's host copy is all that the transfer does not hide.  (144 MB of
-// genotypes: 4.1 ms with two pieces of 64 MiB, threads started per piece; a
-// 50 MB matrix in pageable transfers 4.0 ms.)
-constexpr size_t TSG_COPY_PIECE = (size_t) 2 << 20;
-constexpr int TSG_COPY_RING = 8;
+// Whether a result at dst goes through the ring of copy_out.
 constexpr size_t TSG_COPY_TINY = (size_t) 64 << 10;
-
-int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t bytes) {
-    int ret;
-    if (bytes == 0) return hip_check(hipStreamSynchronize(s));
+bool through_ring(const Workspace *ws, const void *dst, size_t bytes, hipMemoryType *at) {
     hipPointerAttribute_t attr;
-    hipMemoryType type = hipMemoryTypeUnregistered;
+    *at = hipMemoryTypeUnregistered;
     if (hipPointerGetAttributes(&attr, dst) == hipSuccess) {
-        type = attr.type;
+        *at = attr.type;
     } else {
         (void) hipGetLastError();
     }
-    if (type == hipMemoryTypeDevice || type == hipMemoryTypeHost || bytes <= TSG_COPY_TINY ||
-        ws->fixed != nullptr) {
+    return *at != hipMemoryTypeDevice && *at != hipMemoryTypeHost && bytes > TSG_COPY_TINY &&
+           ws->fixed == nullptr;
+}
+
+// `bytes` of results into the caller's dst, waiting for stream s to finish: a
+// device copy when dst is device memory, one transfer when it is pinned host
+// memory or tiny; otherwise through a ring of pinned pieces, each piece's
+// transfer running while host threads copy earlier ones into dst.  `widen`:
+// src holds int8 values and dst takes them as int32 (only through the ring).
+//
+// Bound by the host: the first touch of the caller's pages costs more than
+// the bytes (50 MB into fresh pages of 4 KB: 5 ms with one thread), so the
+// threads touch their shares before the first piece is there, while the
+// kernels still run (MADV_POPULATE_WRITE was slower: pages one by one); the last piece's host copy is all that the transfer
+// does not hide, so there are at least 8 pieces where they are 2 MiB or more
+// (each costs about 12 us between two transfers).
+constexpr size_t TSG_COPY_PIECE = (size_t) 4 << 20;
+constexpr int TSG_COPY_RING = 8;
+constexpr size_t TSG_COPY_THREADS = 8;
+
+int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t bytes,
+             bool widen = false) {
+    int ret;
+    if (bytes == 0) return hip_check(hipStreamSynchronize(s));
+    hipMemoryType type;
+    if (!through_ring(ws, dst, bytes, &type)) {
         const hipMemcpyKind kind =
             type == hipMemoryTypeDevice ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
         if ((ret = hip_check(hipMemcpyAsync(dst, src, bytes, kind, s)))) return ret;
         return hip_check(hipStreamSynchronize(s));
     }
-    const size_t np = (bytes + TSG_COPY_PIECE - 1) / TSG_COPY_PIECE;
+    const size_t out_per = widen ? 4 : 1;  // bytes of dst a byte of src
+    const size_t total = bytes / out_per;
+    const size_t piece = std::min(
+        TSG_COPY_PIECE / (widen ? 2 : 1),
+        std::max<size_t>((total / 8 + 0xffff) & ~(size_t) 0xffff, (size_t) 2 << 20));
+    const size_t np = (total + piece - 1) / piece;
     if (ws->cp_h == nullptr &&
         hipHostMalloc(&ws->cp_h, TSG_COPY_PIECE * TSG_COPY_RING) != hipSuccess) {
         (void) hipGetLastError();
@@ -682,37 +698,61 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
             return ret;
         }
     }
-    // the copying threads (this one among them): one per 2 pieces, at most 8
+    // the copying threads (this one among them): one per 512 KiB, at most 8
     const unsigned hc = std::thread::hardware_concurrency();
     const size_t T = std::max<size_t>(
-        1, std::min<size_t>({8, hc == 0 ? 1 : hc, (np + 1) / 2}));
+        1, std::min<size_t>({TSG_COPY_THREADS, hc == 0 ? 1 : hc, bytes >> 19}));
     std::atomic<size_t> ready{0};  // pieces arrived in their pinned buffers
     std::atomic<bool> failed{false};
     std::vector<std::atomic<int>> done(np);  // threads through with each piece
     for (auto &d : done) d.store(0, std::memory_order_relaxed);
-    auto size_of = [&](size_t i) { return std::min(TSG_COPY_PIECE, bytes - i * TSG_COPY_PIECE); };
-    auto share = [&](size_t i, size_t t) {  // thread t's part of piece i
+    auto size_of = [&](size_t i) { return std::min(piece, total - i * piece); };
+    // thread t's part of piece i, in bytes of src
+    auto part = [&](size_t i, size_t t, size_t &from, size_t &to) {
         const size_t n = size_of(i), per = ((n + T - 1) / T + 63) & ~(size_t) 63;
-        const size_t from = std::min(n, t * per), to = std::min(n, from + per);
-        std::memcpy((char *) dst + i * TSG_COPY_PIECE + from,
-                    (const char *) ws->cp_h + (i % TSG_COPY_RING) * TSG_COPY_PIECE + from,
-                    to - from);
+        from = std::min(n, t * per);
+        to = std::min(n, from + per);
+    };
+    auto touch = [&](size_t i, size_t t) {  // a byte of every page
+        size_t from, to;
+        part(i, t, from, to);
+        volatile char *d = (volatile char *) dst + i * piece * out_per;
+        for (size_t k = from * out_per; k < to * out_per; k += 4096) d[k] = 0;
+    };
+    auto share = [&](size_t i, size_t t) {
+        size_t from, to;
+        part(i, t, from, to);
+        const char *p = (const char *) ws->cp_h + (i % TSG_COPY_RING) * TSG_COPY_PIECE;
+        char *d = (char *) dst + i * piece * out_per;
+        if (widen) {
+            int32_t *o = (int32_t *) d;
+            const int8_t *v = (const int8_t *) p;
+            for (size_t k = from; k < to; k++) o[k] = v[k];
+        } else {
+            std::memcpy(d + from, p + from, to - from);
+        }
         done[i].fetch_add(1, std::memory_order_release);
     };
     auto worker = [&](size_t t) {
+        size_t here = 0;  // pieces whose pages are there
         for (size_t i = 0; i < np; i++) {
             while (ready.load(std::memory_order_acquire) <= i) {
                 if (failed.load(std::memory_order_relaxed)) return;
-                std::this_thread::yield();
+                if (here < np) {
+                    touch(here++, t);
+                } else {
+                    std::this_thread::yield();
+                }
             }
             share(i, t);
+            here = std::max(here, i + 1);
         }
     };
     std::vector<std::thread> pool;
     auto send = [&](size_t i) {
         const int b = (int) (i % TSG_COPY_RING);
         const int e = hip_check(hipMemcpyAsync((char *) ws->cp_h + b * TSG_COPY_PIECE,
-                                               (const char *) src + i * TSG_COPY_PIECE, size_of(i),
+                                               (const char *) src + i * piece, size_of(i),
                                                hipMemcpyDeviceToHost, s));
         return e != 0 ? e : hip_check(hipEventRecord(ws->cp_ev[b], s));
     };
@@ -727,6 +767,14 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
         }
     }
     const size_t mine = pool.size() + 1;
+    if (ret == 0) {
+        size_t here = 0;
+        while (here < np && hipEventQuery(ws->cp_ev[0]) == hipErrorNotReady) {
+            touch(here, 0);
+            for (size_t t = mine; t < T; t++) touch(here, t);
+            here++;
+        }
+    }
     for (size_t i = 0; ret == 0 && i < np; i++) {
         if ((ret = hip_check(hipEventSynchronize(ws->cp_ev[i % TSG_COPY_RING])))) break;
         ready.store(i + 1, std::memory_order_release);
