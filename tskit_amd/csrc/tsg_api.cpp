@@ -3355,9 +3355,9 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
     const int ns = ts->num_samples;
     const int n_pad = ((ns + 127) / 128) * 128;
     const int NW = (ns + 31) / 32;
-    // per window: the bit rows of its sites, padded to a multiple of 64
-    // columns of Gt -- sites with at most two alleles in Gt, the rows of the
-    // others in Gt2
+    // per window: the bit rows of its sites, padded to a multiple of 128
+    // columns -- sites with at most two alleles in gt, the rows of the others
+    // in gt2
     std::vector<int64_t> wk0(W), wk1(W), wk0b(W), wk1b(W);
     std::vector<int32_t> sitecol, sitecol2;
     for (int w = 0; w < W; w++) {
@@ -3377,14 +3377,19 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
                 }
             }
         }
-        while (sitecol.size() % 64 != 0) sitecol.push_back(-1);
-        while (sitecol2.size() % 64 != 0) sitecol2.push_back(-1);
+        while (sitecol.size() % 128 != 0) sitecol.push_back(-1);
+        while (sitecol2.size() % 128 != 0) sitecol2.push_back(-1);
         wk1[w] = (int64_t) sitecol.size();
         wk1b[w] = (int64_t) sitecol2.size();
     }
-    if (sitecol.empty()) sitecol.assign(64, -1);
-    if (sitecol2.empty()) sitecol2.assign(64, -1);
+    if (sitecol.empty()) sitecol.assign(128, -1);
+    if (sitecol2.empty()) sitecol2.assign(128, -1);
     const int64_t Kp = (int64_t) sitecol.size(), Kp2 = (int64_t) sitecol2.size();
+    int64_t cols = 0, cols2 = 0;  // of the widest window
+    for (int w = 0; w < W; w++) {
+        cols = std::max(cols, wk1[w] - wk0[w]);
+        cols2 = std::max(cols2, wk1b[w] - wk0b[w]);
+    }
     std::vector<double> scale(W, 1.0);
     if (options & TSG_STAT_SPAN_NORMALISE) {
         for (int w = 0; w < W; w++) scale[w] = 1.0 / (win[w + 1] - win[w]);
@@ -3418,7 +3423,7 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
     const int64_t gstride = WB ? 1 : (int64_t) ts->max_nloc * (1 + NW);
     if (multi && ((ret = upload(ws->sitecol2, sitecol2, s)) || (ret = upload(ws->wk0b, wk0b, s)) ||
                   (ret = upload(ws->wk1b, wk1b, s)) || (ret = upload(ws->row2, site_row2, s)) ||
-                  (ret = ensure(ws->gt2, (size_t) n_pad * Kp2)) ||
+                  (ret = ensure(ws->gt2, (size_t) n_pad * Kp2 / 8)) ||
                   (ret = ensure(ws->cmat2, (size_t) W * n_pad * n_pad * 4)))) {
         return ret;
     }
@@ -3426,7 +3431,7 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
         (ret = ensure(ws->gslab, (size_t) (WB ? 1 : slots) * gstride * 4)) ||
         (ret = upload(ws->sitecol, sitecol, s)) || (ret = upload(ws->wk0, wk0, s)) ||
         (ret = upload(ws->wk1, wk1, s)) || (ret = upload(ws->scale, scale, s)) ||
-        (ret = upload(ws->sel, sel, s)) || (ret = ensure(ws->gt, (size_t) n_pad * Kp)) ||
+        (ret = upload(ws->sel, sel, s)) || (ret = ensure(ws->gt, (size_t) n_pad * Kp / 8)) ||
         (ret = ensure(ws->cmat, (size_t) W * n_pad * n_pad * 4)) ||
         (ret = ensure(ws->rowsum, (size_t) (W * (int64_t) n + W) * 8)) ||
         (ret = ensure(ws->kout, (size_t) W * n * (size_t) n * 8))) {
@@ -3483,24 +3488,24 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
     if (ws->profile) (void) hipEventRecord(ws->ev0, s);
     if ((ret = hip_check(WB ? tsg_launch_geno_hot(g, (size_t) ts->hot.max_slots * WB * 4, s)
                             : tsg_launch_geno_bits(g, s))) ||
-        (ret = hip_check(tsg_launch_bits_to_gt((const uint32_t *) ws->gbits.p, NW,
-                                               (const int32_t *) ws->sitecol.p, Kp, ns, n_pad,
-                                               (int8_t *) ws->gt.p, s))) ||
-        (ret = hip_check(tsg_launch_syrk_i8((const int8_t *) ws->gt.p, Kp, n_pad,
-                                            (const int64_t *) ws->wk0.p,
-                                            (const int64_t *) ws->wk1.p, W,
-                                            (int32_t *) ws->cmat.p, s)))) {
+        (ret = hip_check(tsg_launch_sample_bits((const uint32_t *) ws->gbits.p, NW,
+                                                (const int32_t *) ws->sitecol.p, Kp, n_pad,
+                                                (uint32_t *) ws->gt.p, s))) ||
+        (ret = hip_check(tsg_launch_syrk((const uint32_t *) ws->gt.p, Kp, n_pad,
+                                         (const int64_t *) ws->wk0.p,
+                                         (const int64_t *) ws->wk1.p, cols, W,
+                                         (int32_t *) ws->cmat.p, s)))) {
         return ret;
     }
     const int32_t *C2 = nullptr;
     if (multi) {
-        if ((ret = hip_check(tsg_launch_bits_to_gt((const uint32_t *) ws->gbits.p, NW,
-                                                   (const int32_t *) ws->sitecol2.p, Kp2, ns,
-                                                   n_pad, (int8_t *) ws->gt2.p, s))) ||
-            (ret = hip_check(tsg_launch_syrk_i8((const int8_t *) ws->gt2.p, Kp2, n_pad,
-                                                (const int64_t *) ws->wk0b.p,
-                                                (const int64_t *) ws->wk1b.p, W,
-                                                (int32_t *) ws->cmat2.p, s)))) {
+        if ((ret = hip_check(tsg_launch_sample_bits((const uint32_t *) ws->gbits.p, NW,
+                                                    (const int32_t *) ws->sitecol2.p, Kp2, n_pad,
+                                                    (uint32_t *) ws->gt2.p, s))) ||
+            (ret = hip_check(tsg_launch_syrk((const uint32_t *) ws->gt2.p, Kp2, n_pad,
+                                             (const int64_t *) ws->wk0b.p,
+                                             (const int64_t *) ws->wk1b.p, cols2, W,
+                                             (int32_t *) ws->cmat2.p, s)))) {
             return ret;
         }
         C2 = (const int32_t *) ws->cmat2.p;

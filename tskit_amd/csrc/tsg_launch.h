@@ -68,11 +68,12 @@ hipError_t tsg_launch_geno_hot(const TsgGenoArgs &a, size_t shmem, hipStream_t s
 // listed (site, sample) pairs
 hipError_t tsg_launch_genotypes(const TsgGenoArgs &a, size_t shmem, const int32_t *miss_site,
                                 const int32_t *miss_sample, int64_t nmiss, hipStream_t s);
-hipError_t tsg_launch_bits_to_gt(const uint32_t *gbits, int NW, const int32_t *site_of_col,
-                                 int64_t Kp, int n, int n_pad, int8_t *gt, hipStream_t s);
-hipError_t tsg_launch_syrk_i8(const int8_t *gt, int64_t Kp, int n_pad, const int64_t *win_k0,
-                              const int64_t *win_k1, int W, int32_t *C, hipStream_t s);
-// D = (C_ii + C_jj - 2 C_ij) * scale[w] over the selected samples
+hipError_t tsg_launch_sample_bits(const uint32_t *gbits, int NW, const int32_t *site_of_col,
+                                  int64_t Kp, int n_pad, uint32_t *bits, hipStream_t s);
+// most_cols: of a window
+hipError_t tsg_launch_syrk(const uint32_t *bits, int64_t Kp, int n_pad, const int64_t *win_k0,
+                           const int64_t *win_k1, int64_t most_cols, int W, int32_t *C,
+                           hipStream_t s);
 hipError_t tsg_launch_divergence(const int32_t *C, const int32_t *C2, const int32_t *sel, int n,
                                  int n_pad, int W, const double *scale, double *D,
                                  hipStream_t s);

@@ -12,18 +12,20 @@
 // so its rows d and B_a go into a second cross product C2 and, with
 // P = 2C + C2, D = (P_ii + P_jj)/2 - P_ij and K = J P J / 2.  C and C2 are
 // exact integer cross products (entries <= number of rows < 2^31), computed
-// here with int8 MFMA and int32 accumulation; the centring is FP64.
+// here on the matrix cores from the bits; the centring is FP64.
 //
 // Kernels:
 //   k_geno_bits  one wavefront per chunk: the chunk sweep with a per-node
 //                bitset of the samples below it (insert: OR, remove: AND-NOT);
 //                each site's row is the bitset of its mutation's node.
-//   k_bits_to_gt bit rows (site-major) -> int8 Gt (sample-major, each
-//                window's sites zero-padded to a multiple of 64).
-//   k_syrk_i8    C = Gt Gt^T on v_mfma_i32_32x32x32_i8, upper-triangular
-//                128x128 tiles, mirrored on store.
+//   k_sample_bits  bit rows by site -> by sample (each window's sites
+//                zero-padded to a multiple of 128).
+//   k_syrk       C = B B^T over the bits, upper-triangular 128x128 tiles,
+//                mirrored on store.
 //   k_centre     row sums, then K = (C - r_i/n - r_j/n + t/n^2) / span (FP64).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "tsg_common.h"
 #include "tsg_kernels.h"
@@ -237,58 +239,88 @@ __global__ void __launch_bounds__(WAVE) k_geno_hot(const TsgGenoArgs a) {
     }
 }
 
-// --- bits (site-major) -> int8 Gt (sample-major, K padded per window) -------
-// grid: (ceil(S_pad_total / 64), n_pad / 64); block 256.  Tile: 64 sites x
-// 64 samples.  site_of_col[k] maps a padded column to its site (-1 = pad).
-__global__ void __launch_bounds__(256) k_bits_to_gt(const uint32_t *gbits, int NW,
-                                                    const int32_t *site_of_col, int64_t Kp,
-                                                    int n, int8_t *gt) {
-    __shared__ uint32_t tile[64][2];  // 64 sites x 64 sample bits
-    const int64_t k0 = (int64_t) blockIdx.x * 64;
-    const int j0 = blockIdx.y * 64;  // first sample of the tile
-    const int tid = threadIdx.x;
-    if (tid < 128) {
-        const int r = tid >> 1, h = tid & 1;
-        const int64_t k = k0 + r;
-        uint32_t v = 0u;
-        const int w = (j0 >> 5) + h;
-        if (k < Kp) {
-            const int s = site_of_col[k];
-            if (s >= 0 && w < NW) v = gbits[(int64_t) s * NW + w];
+// --- bit rows by site -> by sample --------------------------------------------
+// bits: [n_pad x KW] words, bit k of sample j's row its genotype at column k;
+// site_of_col maps a padded column to its row of gbits (-1: zeros).  A wave
+// takes 256 columns of 128 samples: per 64 columns each lane reads one site's
+// 4 words and 128 ballots turn them; each lane then holds 32 bytes of two
+// samples' rows.  Bound by its ballots, about 2 instructions a sample and 64
+// sites (2500 samples x 56000 sites: the int8 expansion this replaced wrote
+// 143 MB, 66 us).
+__global__ void __launch_bounds__(256) k_sample_bits(const uint32_t *gbits, int NW,
+                                                     const int32_t *site_of_col, int64_t Kp,
+                                                     uint32_t *bits) {
+    const int lane = threadIdx.x % WAVE;
+    const int64_t k0 = ((int64_t) blockIdx.x * 4 + threadIdx.x / WAVE) * 256;
+    if (k0 >= Kp) return;
+    const int w0 = blockIdx.y * 4;
+    unsigned long long mine[2][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int64_t k = k0 + q * 64 + lane;
+        const int64_t site = k < Kp ? site_of_col[k] : -1;
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+            const uint32_t v = (site >= 0 && w0 + h < NW) ? gbits[site * NW + w0 + h] : 0u;
+            unsigned long long m = 0;
+#pragma unroll
+            for (int b = 0; b < 32; b++) {
+                const unsigned long long all = __ballot((v >> b) & 1u);
+                if (lane % 32 == b) m = all;
+            }
+            // word h's samples are 32 h + b: lanes 0-31 keep words 0 and 2,
+            // lanes 32-63 words 1 and 3
+            if (lane / 32 == h % 2) mine[h / 2][q] = m;
         }
-        tile[r][h] = v;
     }
-    __syncthreads();
-    // each thread writes 16 consecutive columns (sites) of one sample row
-    const int jj = tid >> 2;          // sample within tile, 0..63
-    const int kk = (tid & 3) * 16;    // 16-column group
-    const int j = j0 + jj;
-    if (k0 + kk >= Kp) return;
-    int8_t out[16];
-    for (int q = 0; q < 16; q++) {
-        const uint32_t wv = tile[kk + q][jj >> 5];
-        out[q] = (j < n) ? (int8_t) ((wv >> (jj & 31)) & 1u) : (int8_t) 0;
+    const int64_t KW = Kp / 32;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        uint32_t *row = bits + ((int64_t) blockIdx.y * 128 + r * 64 + lane) * KW + k0 / 32;
+#pragma unroll
+        for (int q = 0; q < 4; q += 2) {
+            if (k0 + q * 64 < Kp) {  // (Kp is a multiple of 128)
+                *reinterpret_cast<uint4 *>(row + 2 * q) =
+                    make_uint4((uint32_t) mine[r][q], (uint32_t) (mine[r][q] >> 32),
+                               (uint32_t) mine[r][q + 1], (uint32_t) (mine[r][q + 1] >> 32));
+            }
+        }
     }
-    int4 v;
-    __builtin_memcpy(&v, out, 16);
-    *reinterpret_cast<int4 *>(gt + (int64_t) j * Kp + k0 + kk) = v;
 }
 
-// --- SYRK on int8 MFMA --------------------------------------------------------
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
+// --- cross products of the bits ------------------------------------------------
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 
-#define BT 128        // output tile
-#define BK 64         // k per LDS stage
-#define LDSP 80       // padded LDS row (bytes): 64 + 16
+#define BT 128  // output tile
+// columns a wave may sum in FP32: whole numbers are exact below this
+#define SYRK_MOST ((int64_t) 1 << 24)
 
-// One workgroup (4 waves) per upper-triangular 128x128 tile of one window.
-// Wave (wy, wx) computes the 64x64 quadrant as 2x2 tiles of 32x32.
-__global__ void __launch_bounds__(256) k_syrk_i8(const int8_t *gt, int64_t Kp, int n_pad,
+// 32 bits as 32 FP4 values (E2M1: 1.0 is 0b0010).  The order of the values
+// along k does not matter, being the same for both operands.
+__device__ __forceinline__ v8i fp4(uint32_t b) {
+    v8i r = {};
+    r[0] = (int) ((b << 1) & 0x22222222u);
+    r[1] = (int) (b & 0x22222222u);
+    r[2] = (int) ((b >> 1) & 0x22222222u);
+    r[3] = (int) ((b >> 2) & 0x22222222u);
+    return r;
+}
+
+// One workgroup (4 waves) per upper-triangular 128x128 tile of one window and
+// part of its columns.  A genotype is one bit, so the bits are what is read
+// (a wave's 256 columns of 256 samples: 8 KB, straight into registers), and
+// FP4 matrix instructions multiply them: products of 0 and 1, summed in FP32,
+// are exact up to SYRK_MOST columns a wave.  Every wave computes the whole
+// tile over a quarter of the columns, 4 x 4 tiles of 32 x 32, so that 8
+// expansions (7 instructions each) feed 16 matrix instructions; the four
+// waves' sums are added in LDS, as integers.
+// (2500 samples x 56000 sites: 721 us with int8 operands staged in LDS, each
+// wave a quarter of the tile.)
+__global__ void __launch_bounds__(256, 1) k_syrk(const uint32_t *bits, int64_t KW, int n_pad,
                                                  const int64_t *win_k0, const int64_t *win_k1,
-                                                 int tiles_per_dim, int32_t *C) {
-    __shared__ __attribute__((aligned(16))) int8_t As[BT * LDSP];
-    __shared__ __attribute__((aligned(16))) int8_t Bs[BT * LDSP];
+                                                 int tiles_per_dim, bool add, int32_t *C) {
+    extern __shared__ float part[];  // [4 waves][4 tiles][16][64]
     const int w = blockIdx.y;  // window
     // invert the upper-triangular tile index
     int t = blockIdx.x, ti = 0;
@@ -300,50 +332,92 @@ __global__ void __launch_bounds__(256) k_syrk_i8(const int8_t *gt, int64_t Kp, i
     }
     const int tj = ti + t;
     const int i0 = ti * BT, j0 = tj * BT;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wy = wave >> 1, wx = wave & 1;
-    v16i acc[2][2];
-    for (int a = 0; a < 2; a++)
-        for (int b = 0; b < 2; b++)
-            for (int r = 0; r < 16; r++) acc[a][b][r] = 0;
-    const int64_t kbeg = win_k0[w], kend = win_k1[w];
-    for (int64_t k = kbeg; k < kend; k += BK) {
-        // stage 128 rows x 64 bytes of A (rows i0..) and B (rows j0..)
-        for (int q = tid; q < BT * 4; q += 256) {
-            const int r = q >> 2, seg = (q & 3) * 16;
-            *reinterpret_cast<int4 *>(As + r * LDSP + seg) =
-                *reinterpret_cast<const int4 *>(gt + (int64_t) (i0 + r) * Kp + k + seg);
-            *reinterpret_cast<int4 *>(Bs + r * LDSP + seg) =
-                *reinterpret_cast<const int4 *>(gt + (int64_t) (j0 + r) * Kp + k + seg);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    v16f acc[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
+    // this wave's chunks of 8 words (256 columns) of the window
+    const int64_t kbeg = win_k0[w] / 32, kend = win_k1[w] / 32;
+    const int64_t chunks = (kend - kbeg + 7) / 8;
+    const int64_t parts = (int64_t) gridDim.z * 4, p = (int64_t) blockIdx.z * 4 + wave;
+    const int64_t c0 = chunks * p / parts, c1 = chunks * (p + 1) / parts;
+    const uint32_t *ra = bits + (int64_t) (i0 + (lane & 31)) * KW;
+    const uint32_t *rb = bits + (int64_t) (j0 + (lane & 31)) * KW;
+    uint4 na[4], nb[4];
+    auto fetch = [&](int64_t c) {  // lanes 0-31 words 0-3 of the chunk, 32-63 words 4-7
+        const int64_t k = kbeg + c * 8 + 4 * (lane >> 5);
+        const bool in = c < c1 && k < kend;
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            na[a] = in ? *reinterpret_cast<const uint4 *>(ra + a * 32 * KW + k)
+                       : make_uint4(0, 0, 0, 0);
+            nb[a] = in ? *reinterpret_cast<const uint4 *>(rb + a * 32 * KW + k)
+                       : make_uint4(0, 0, 0, 0);
         }
-        __syncthreads();
-        for (int kk = 0; kk < BK; kk += 32) {
-            const int ko = kk + 16 * (lane >> 5);
-            v4i af[2], bf[2];
-            for (int a = 0; a < 2; a++) {
-                const int r = wy * 64 + a * 32 + (lane & 31);
-                af[a] = *reinterpret_cast<const v4i *>(As + r * LDSP + ko);
+    };
+    fetch(c0);
+    for (int64_t c = c0; c < c1; c++) {
+        uint4 ca[4], cb[4];
+#pragma unroll
+        for (int a = 0; a < 4; a++) ca[a] = na[a], cb[a] = nb[a];
+        fetch(c + 1);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            v8i af[4], bf[4];
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                af[a] = fp4(q == 0 ? ca[a].x : q == 1 ? ca[a].y : q == 2 ? ca[a].z : ca[a].w);
+                bf[a] = fp4(q == 0 ? cb[a].x : q == 1 ? cb[a].y : q == 2 ? cb[a].z : cb[a].w);
             }
-            for (int b = 0; b < 2; b++) {
-                const int r = wx * 64 + b * 32 + (lane & 31);
-                bf[b] = *reinterpret_cast<const v4i *>(Bs + r * LDSP + ko);
-            }
-            for (int a = 0; a < 2; a++)
-                for (int b = 0; b < 2; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[a], bf[b], acc[a][b], 0, 0, 0);
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+#pragma unroll
+                for (int b = 0; b < 4; b++)
+                    // (formats 4: FP4; scales 0: unscaled)
+                    acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                        af[a], bf[b], acc[a][b], 4, 4, 0, 0, 0, 0);
         }
-        __syncthreads();
     }
     int32_t *Cw = C + (int64_t) w * n_pad * n_pad;
-    for (int a = 0; a < 2; a++) {
-        for (int b = 0; b < 2; b++) {
-            const int col = j0 + wx * 64 + b * 32 + (lane & 31);
-            for (int r = 0; r < 16; r++) {
-                const int row = i0 + wy * 64 + a * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                const int32_t v = acc[a][b][r];
-                Cw[(int64_t) row * n_pad + col] = v;
-                Cw[(int64_t) col * n_pad + row] = v;
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+        // row of tiles a: every wave's sums into LDS, wave b adds up tile b
+        if (a > 0) __syncthreads();
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                part[((wave * 4 + b) * 16 + r) * WAVE + lane] = acc[a][b][r];
+        __syncthreads();
+        const int col = j0 + wave * 32 + (lane & 31);
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++) {
+            const int row = i0 + a * 32 + r4 * 8 + (lane >> 5) * 4;
+            int32_t v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                v[r] = 0;
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    v[r] += (int32_t) part[((u * 4 + wave) * 16 + r4 * 4 + r) * WAVE + lane];
+            }
+            int32_t *down = Cw + (int64_t) row * n_pad + col;
+            int32_t *across = Cw + (int64_t) col * n_pad + row;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (add) {
+                    atomicAdd(down + (int64_t) r * n_pad, v[r]);
+                    if (ti != tj) atomicAdd(across + r, v[r]);
+                } else {
+                    down[(int64_t) r * n_pad] = v[r];
+                }
+            }
+            if (!add && ti != tj) {
+                *reinterpret_cast<int4 *>(across) = make_int4(v[0], v[1], v[2], v[3]);
             }
         }
     }
@@ -514,18 +588,32 @@ hipError_t tsg_launch_genotypes(const TsgGenoArgs &a, size_t shmem, const int32_
     return hipGetLastError();
 }
 
-hipError_t tsg_launch_bits_to_gt(const uint32_t *gbits, int NW, const int32_t *site_of_col,
-                                 int64_t Kp, int n, int n_pad, int8_t *gt, hipStream_t s) {
-    dim3 grid((unsigned) ((Kp + 63) / 64), (unsigned) (n_pad / 64));
-    hipLaunchKernelGGL(k_bits_to_gt, grid, dim3(256), 0, s, gbits, NW, site_of_col, Kp, n, gt);
+hipError_t tsg_launch_sample_bits(const uint32_t *gbits, int NW, const int32_t *site_of_col,
+                                  int64_t Kp, int n_pad, uint32_t *bits, hipStream_t s) {
+    dim3 grid((unsigned) ((Kp + 1023) / 1024), (unsigned) (n_pad / 128));
+    hipLaunchKernelGGL(k_sample_bits, grid, dim3(256), 0, s, gbits, NW, site_of_col, Kp, bits);
     return hipGetLastError();
 }
 
-hipError_t tsg_launch_syrk_i8(const int8_t *gt, int64_t Kp, int n_pad, const int64_t *win_k0,
-                              const int64_t *win_k1, int W, int32_t *C, hipStream_t s) {
+// The columns of a window are split over workgroups, which then add into
+// zeroed products, where its tiles alone leave compute units idle (one
+// workgroup each: its registers), each wave keeping 8 chunks of 256 columns
+// or more; and where a wave's share would reach SYRK_MOST.
+hipError_t tsg_launch_syrk(const uint32_t *bits, int64_t Kp, int n_pad, const int64_t *win_k0,
+                           const int64_t *win_k1, int64_t most_cols, int W, int32_t *C,
+                           hipStream_t s) {
     const int tpd = n_pad / BT;
-    dim3 grid((unsigned) (tpd * (tpd + 1) / 2), (unsigned) W);
-    hipLaunchKernelGGL(k_syrk_i8, grid, dim3(256), 0, s, gt, Kp, n_pad, win_k0, win_k1, tpd, C);
+    const int64_t tiles = (int64_t) tpd * (tpd + 1) / 2 * W;
+    const int64_t split = std::max<int64_t>(std::min<int64_t>(256 / tiles, most_cols / (4 * 8 * 256)),
+                                            most_cols / (3 * SYRK_MOST) + 1);
+    const size_t shmem = 4 * 4 * 16 * WAVE * sizeof(float);
+    hipError_t e;
+    if (split > 1) {
+        const int64_t words = (int64_t) W * n_pad * n_pad / 2;
+        if ((e = tsg_launch_fill_u64((unsigned long long *) C, words, s)) != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(k_syrk, dim3((unsigned) (tpd * (tpd + 1) / 2), (unsigned) W, (unsigned) split),
+                       dim3(256), shmem, s, bits, Kp / 32, n_pad, win_k0, win_k1, tpd, split > 1, C);
     return hipGetLastError();
 }
 
