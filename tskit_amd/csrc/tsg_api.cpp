@@ -1915,6 +1915,50 @@ int ensure_state_spectrum(tsg_treeseq *ts) {
     return b.upload(h.afs_block, h.bytes);
 }
 
+// The genotype bits of every state of the state plan (tsg_relate.hip), queued:
+// g's part of them, or TSG_NOT_ON_STATES -- also where the rows would take
+// more than TSG_STATE_BITS_MAX, since the chunk walk needs none of that
+// memory (20000 samples: 400000 states).
+constexpr size_t TSG_STATE_BITS_MAX = (size_t) 1 << 30;
+int state_bits(tsg_treeseq *ts, Workspace *ws, TsgGenoArgs &g) {
+    const tsg_stateplan &sp = ts->states;
+    const int n = ts->num_samples, RW = ((n + 31) / 32 + 3) / 4 * 4;
+    const size_t rows = (size_t) sp.num_states * RW * 4;
+    if (!sp.usable || ws->force_full || rows > TSG_STATE_BITS_MAX) return TSG_NOT_ON_STATES;
+    int ret = ensure(ws->state_x, rows);
+    if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? TSG_NOT_ON_STATES : ret;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        TsgStateDevice &h = ts->states.dev;
+        if (h.bits_block == nullptr) {
+            Arrays b;
+            b.add(h.mut_state, sp.mut_state);
+            if ((ret = b.upload(h.bits_block, h.bytes))) return ret;
+        }
+    }
+    TsgStateLaunch l;
+    TsgStateArgs &a = l.a;
+    a = TsgStateArgs{};
+    a.order = sp.dev.order;
+    a.in = sp.dev.in;
+    a.num_states = sp.num_states;
+    a.num_samples = n;
+    a.RW = RW;
+    a.x = (uint32_t *) ws->state_x.p;
+    l.level0 = sp.level0.data();
+    l.levels = (int) sp.level0.size() - 1;
+    if ((ret = hip_check(tsg_launch_bits_seed(a.x, RW, n, ws->stream))) ||
+        (ret = hip_check(tsg_launch_state_levels(l, ws->stream)))) {
+        return ret;
+    }
+    g.x = a.x;
+    g.RW = RW;
+    g.num_sites = ts->num_sites;
+    g.mut_node = sp.dev.mut_state;
+    ws->last_store = TSG_STORE_HOT;
+    return 0;
+}
+
 // A node-mode query on the state plan (trees.c:1788-1918), or
 // TSG_NOT_ON_STATES.
 int run_node_states(tsg_treeseq *ts, Query &q, const Fused &fz, Workspace *ws) {
@@ -2523,7 +2567,7 @@ void tsg_hot_device_free(TsgHotDevice *h) {
 }
 
 void tsg_state_device_free(TsgStateDevice *h) {
-    free_all({h->block, h->nodes_block, h->afs_block});
+    free_all({h->block, h->nodes_block, h->afs_block, h->bits_block});
     *h = TsgStateDevice();
 }
 
@@ -3403,10 +3447,14 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
     Lease lease(ts);
     Workspace *ws = lease.ws;
     if (ws == nullptr) return TSG_ERR_DEVICE;
-    // genotype bitsets on the hot plan when a block of WB words per slot
+    TsgGenoArgs g{};
+    int ret_bits = state_bits(ts, ws, g);
+    if (ret_bits != 0 && ret_bits != TSG_NOT_ON_STATES) return ret_bits;
+    const bool on_states = ret_bits == 0;
+    // else genotype bitsets on the hot plan when a block of WB words per slot
     // fits in LDS (WB = 64, 32 or 16 words: a workgroup's share of samples)
     int WB = 0;
-    if (ts->hot.usable && !ws->force_full) {
+    if (!on_states && ts->hot.usable && !ws->force_full) {
         for (int wb : {64, 32, 16}) {
             if ((size_t) ts->hot.max_slots * wb * 4 <= (size_t) 48 * 1024) {
                 WB = wb;
@@ -3414,13 +3462,14 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
             }
         }
     }
-    if (WB == 0) {
+    if (!on_states && WB == 0) {
         std::lock_guard<std::mutex> lock(g_mutex);
         if ((ret = ensure_full(ts))) return ret;
     }
     hipStream_t s = ws->stream;
     const int slots = std::min(ts->num_chunks, 512);
-    const int64_t gstride = WB ? 1 : (int64_t) ts->max_nloc * (1 + NW);
+    const bool full = !on_states && WB == 0;
+    const int64_t gstride = full ? (int64_t) ts->max_nloc * (1 + NW) : 1;
     if (multi && ((ret = upload(ws->sitecol2, sitecol2, s)) || (ret = upload(ws->wk0b, wk0b, s)) ||
                   (ret = upload(ws->wk1b, wk1b, s)) || (ret = upload(ws->row2, site_row2, s)) ||
                   (ret = ensure(ws->gt2, (size_t) n_pad * Kp2 / 8)) ||
@@ -3428,7 +3477,7 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
         return ret;
     }
     if ((ret = ensure(ws->gbits, (size_t) std::max<int64_t>(nrows, 1) * NW * 4)) ||
-        (ret = ensure(ws->gslab, (size_t) (WB ? 1 : slots) * gstride * 4)) ||
+        (ret = ensure(ws->gslab, (size_t) (full ? slots : 1) * gstride * 4)) ||
         (ret = upload(ws->sitecol, sitecol, s)) || (ret = upload(ws->wk0, wk0, s)) ||
         (ret = upload(ws->wk1, wk1, s)) || (ret = upload(ws->scale, scale, s)) ||
         (ret = upload(ws->sel, sel, s)) || (ret = ensure(ws->gt, (size_t) n_pad * Kp / 8)) ||
@@ -3445,7 +3494,6 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
     }
     const TsgDevice &d = ts->dev;
     const TsgHotDevice &hd = ts->hot.dev;
-    TsgGenoArgs g{};
     g.tree_site0 = d.tree_site0;
     g.site_mut0 = d.site_mut0;
     g.num_samples = ns;
@@ -3454,7 +3502,7 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
     g.mut_allele = d.mut_allele;
     g.site_nalleles = d.site_nalleles;
     g.site_row2 = multi ? (const int32_t *) ws->row2.p : nullptr;
-    if (WB) {
+    if (WB != 0) {
         g.chunk_tree0 = hd.chunk_tree0;
         g.chunk_node0 = hd.chunk_slot0;
         g.tr_off = hd.tr_off;
@@ -3470,7 +3518,7 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
         g.num_chunks = ts->hot.num_chunks;
         g.WB = WB;
         ws->last_store = TSG_STORE_HOT;
-    } else {
+    } else if (full) {
         g.chunk_tree0 = d.chunk_tree0;
         g.chunk_node0 = d.chunk_node0;
         g.loc_parent0 = d.loc_parent0;
@@ -3486,8 +3534,9 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
         ws->last_store = TSG_STORE_GLOBAL;
     }
     if (ws->profile) (void) hipEventRecord(ws->ev0, s);
-    if ((ret = hip_check(WB ? tsg_launch_geno_hot(g, (size_t) ts->hot.max_slots * WB * 4, s)
-                            : tsg_launch_geno_bits(g, s))) ||
+    if ((ret = hip_check(on_states ? tsg_launch_site_bits(g, s)
+                         : full    ? tsg_launch_geno_bits(g, s)
+                                   : tsg_launch_geno_hot(g, (size_t) ts->hot.max_slots * WB * 4, s))) ||
         (ret = hip_check(tsg_launch_sample_bits((const uint32_t *) ws->gbits.p, NW,
                                                 (const int32_t *) ws->sitecol.p, Kp, n_pad,
                                                 (uint32_t *) ws->gt.p, s))) ||
@@ -3574,13 +3623,6 @@ int tsg_treeseq_divergence_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
 static void isolated_pairs(const tsg_treeseq *ts, std::vector<int32_t> &ms,
                            std::vector<int32_t> &mj) {
     const int32_t n = ts->num_samples;
-    std::vector<std::vector<std::pair<double, double>>> cover(n);
-    for (int32_t e = 0; e < ts->num_edges; e++) {
-        for (int32_t u : {ts->parent[e], ts->child[e]}) {
-            const int32_t j = ts->sample_index_map[u];
-            if (j != TSG_NULL) cover[j].emplace_back(ts->left[e], ts->right[e]);
-        }
-    }
     auto sites_in = [&](double a, double b, int32_t j) {
         const auto &pos = ts->site_pos;
         size_t s = std::lower_bound(pos.begin(), pos.end(), a) - pos.begin();
@@ -3596,15 +3638,18 @@ static void isolated_pairs(const tsg_treeseq *ts, std::vector<int32_t> &ms,
             }
         }
     };
-    for (int32_t j = 0; j < n; j++) {
-        auto &iv = cover[j];
-        std::sort(iv.begin(), iv.end());
-        double x = 0.0;  // covered up to x so far
-        for (const auto &[l, r] : iv) {
-            if (l > x) sites_in(x, l, j);
-            x = std::max(x, r);
+    // edges by their left ends: sample j is covered up to x[j] so far
+    std::vector<double> x(n, 0.0);
+    for (const int32_t e : ts->I) {
+        for (int32_t u : {ts->parent[e], ts->child[e]}) {
+            const int32_t j = ts->sample_index_map[u];
+            if (j == TSG_NULL) continue;
+            if (ts->left[e] > x[j]) sites_in(x[j], ts->left[e], j);
+            x[j] = std::max(x[j], ts->right[e]);
         }
-        if (x < ts->L) sites_in(x, ts->L, j);
+    }
+    for (int32_t j = 0; j < n; j++) {
+        if (x[j] < ts->L) sites_in(x[j], ts->L, j);
     }
 }
 
@@ -4015,43 +4060,53 @@ int tsg_treeseq_genotype_matrix(tsg_treeseq *ts, uint32_t options, int32_t *out)
     hipStream_t s = ws->stream;
     const int ns = ts->num_samples;
     const size_t cells = (size_t) ts->num_sites * ns;
-    if ((ret = ensure(ws->geno, cells * 4)) || (ret = upload(ws->wk0, ms, s)) ||
-        (ret = upload(ws->wk1, mj, s))) {
-        return ret;
-    }
+    if ((ret = upload(ws->wk0, ms, s)) || (ret = upload(ws->wk1, mj, s))) return ret;
     const TsgDevice &d = ts->dev;
     const TsgHotDevice &hd = ts->hot.dev;
     TsgGenoArgs g{};
-    g.tree_site0 = d.tree_site0;
     g.site_mut0 = d.site_mut0;
     g.num_samples = ns;
     g.NW = (ns + 31) / 32;
-    g.chunk_tree0 = hd.chunk_tree0;
-    g.chunk_node0 = hd.chunk_slot0;
-    g.tr_off = hd.tr_off;
-    g.tr_nrem = hd.tr_nrem;
-    g.ev_child = hd.ev_child;
-    g.ev_path0 = hd.ev_path0;
-    g.path = hd.path;
-    g.mut_node = hd.mut_slot;
-    g.slot_par = hd.slot_par;
-    g.chunk_lev0 = hd.chunk_lev0;
-    g.lev_slot0 = hd.lev_slot0;
-    g.sample_slot = hd.sample_slot;
-    g.num_chunks = ts->hot.num_chunks;
-    g.WB = WB;
     g.mut_allele = d.mut_allele;
-    g.geno = (int32_t *) ws->geno.p;
-    ws->last_store = TSG_STORE_HOT;
     if (ws->profile) (void) hipEventRecord(ws->ev0, s);
-    if ((ret = hip_check(tsg_launch_genotypes(g, (size_t) ts->hot.max_slots * WB * 4,
-                                              (const int32_t *) ws->wk0.p,
-                                              (const int32_t *) ws->wk1.p, (int64_t) ms.size(),
-                                              s)))) {
-        return ret;
+    // (a thread per 4 cells or more: one launch's limit)
+    ret = cells >> 33 != 0 ? TSG_NOT_ON_STATES : state_bits(ts, ws, g);
+    if (ret != 0 && ret != TSG_NOT_ON_STATES) return ret;
+    const bool on_states = ret == 0;
+    // where every allele index fits, a quarter of the bytes go to the host
+    hipMemoryType at;
+    const bool narrow = on_states && ts->max_alleles <= 128 && through_ring(ws, out, cells * 4, &at);
+    if ((ret = ensure(ws->geno, (cells * (narrow ? 1 : 4) + 15) / 16 * 16))) return ret;
+    g.geno = (int32_t *) ws->geno.p;
+    const int32_t *miss_site = (const int32_t *) ws->wk0.p, *miss_sample = (const int32_t *) ws->wk1.p;
+    if (on_states) {
+        ret = hip_check(tsg_launch_states_genotypes(g, narrow, miss_site, miss_sample,
+                                                    (int64_t) ms.size(), s));
+        if (ret != 0) return ret;
+    } else {
+        g.tree_site0 = d.tree_site0;
+        g.chunk_tree0 = hd.chunk_tree0;
+        g.chunk_node0 = hd.chunk_slot0;
+        g.tr_off = hd.tr_off;
+        g.tr_nrem = hd.tr_nrem;
+        g.ev_child = hd.ev_child;
+        g.ev_path0 = hd.ev_path0;
+        g.path = hd.path;
+        g.mut_node = hd.mut_slot;
+        g.slot_par = hd.slot_par;
+        g.chunk_lev0 = hd.chunk_lev0;
+        g.lev_slot0 = hd.lev_slot0;
+        g.sample_slot = hd.sample_slot;
+        g.num_chunks = ts->hot.num_chunks;
+        g.WB = WB;
+        ws->last_store = TSG_STORE_HOT;
+        if ((ret = hip_check(tsg_launch_genotypes(g, (size_t) ts->hot.max_slots * WB * 4, miss_site,
+                                                  miss_sample, (int64_t) ms.size(), s)))) {
+            return ret;
+        }
     }
     if (ws->profile) (void) hipEventRecord(ws->ev1, s);
-    if ((ret = copy_out(ws, s, out, ws->geno.p, cells * 4))) return ret;
+    if ((ret = copy_out(ws, s, out, ws->geno.p, cells * 4, narrow))) return ret;
     if (ws->profile) {
         float ms_ = 0;
         (void) hipEventElapsedTime(&ms_, ws->ev0, ws->ev1);

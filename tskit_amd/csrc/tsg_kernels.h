@@ -207,6 +207,9 @@ struct TsgGenoArgs {
     // (null: every site has at most two)
     const int32_t *site_row2;
     const int32_t *site_nalleles;
+    // on the state plan: bit rows of RW words a state, mut_node holding states
+    const uint32_t *x;
+    int32_t RW, num_sites;
 };
 
 struct TsgCombineArgs {

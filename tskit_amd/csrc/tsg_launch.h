@@ -68,6 +68,12 @@ hipError_t tsg_launch_geno_hot(const TsgGenoArgs &a, size_t shmem, hipStream_t s
 // listed (site, sample) pairs
 hipError_t tsg_launch_genotypes(const TsgGenoArgs &a, size_t shmem, const int32_t *miss_site,
                                 const int32_t *miss_sample, int64_t nmiss, hipStream_t s);
+// genotype bits on the state plan: rows 0 .. n of x; the rows of all sites from
+// all states'; genotypes into a.geno, int32 or (narrow) int8, whole 16 bytes
+hipError_t tsg_launch_bits_seed(uint32_t *x, int RW, int n, hipStream_t s);
+hipError_t tsg_launch_site_bits(const TsgGenoArgs &a, hipStream_t s);
+hipError_t tsg_launch_states_genotypes(const TsgGenoArgs &a, bool narrow, const int32_t *miss_site,
+                                       const int32_t *miss_sample, int64_t nmiss, hipStream_t s);
 hipError_t tsg_launch_sample_bits(const uint32_t *gbits, int NW, const int32_t *site_of_col,
                                   int64_t Kp, int n_pad, uint32_t *bits, hipStream_t s);
 // most_cols: of a window

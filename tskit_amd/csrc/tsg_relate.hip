@@ -18,6 +18,8 @@
 //   k_geno_bits  one wavefront per chunk: the chunk sweep with a per-node
 //                bitset of the samples below it (insert: OR, remove: AND-NOT);
 //                each site's row is the bitset of its mutation's node.
+//   k_site_bits  the same rows from the states of the state plan, whose bits
+//                the plan's count kernel adds up (where the plan is usable).
 //   k_sample_bits  bit rows by site -> by sample (each window's sites
 //                zero-padded to a multiple of 128).
 //   k_syrk       C = B B^T over the bits, upper-triangular 128x128 tiles,
@@ -237,6 +239,72 @@ __global__ void __launch_bounds__(WAVE) k_geno_hot(const TsgGenoArgs a) {
             }
         }
     }
+}
+
+// --- genotype bits on the state plan ----------------------------------------------
+// The samples below a state as RW words: the states' counts (tsg_states.hip)
+// with a word of 32 samples in place of a column, since the sets that a state
+// sums are disjoint and so add up without carries.  All states of a level at
+// once; the chunk walk (k_geno_hot) is a chain of dependent LDS updates per
+// chunk.  (2500 samples, 177000 states of 79 words, 56000 sites: 383 us by
+// chunks, TODO us here.)
+
+// Rows 0 (no samples) and 1 + s (sample s), 4 words a thread.
+__global__ void __launch_bounds__(256) k_bits_seed(uint32_t *x, int RW, int64_t n) {
+    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    const int64_t r = i / (RW / 4);
+    const int w = (int) (i % (RW / 4)) * 4;
+    if (r > n) return;
+    uint32_t v[4] = {0, 0, 0, 0};
+    if (r > 0 && (int) ((r - 1) >> 7) == w / 4) v[((r - 1) >> 5) & 3] = 1u << ((r - 1) & 31);
+    *reinterpret_cast<uint4 *>(x + r * RW + w) = make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+// Thread per (site, word): the site's bit rows from its mutations' states.
+__global__ void __launch_bounds__(256) k_site_bits(const TsgGenoArgs a) {
+    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    const int64_t site = i / a.NW;
+    if (site >= a.num_sites) return;
+    const int w = (int) (i % a.NW);
+    site_rows(a, (int) site, w, a.NW, [&](int st) { return a.x[(int64_t) st * a.RW + w]; });
+}
+
+// Genotypes as G, site after site, 16 bytes a thread: cells q .. of one site
+// or, at a site's end, of the next too.  A cell's value is the allele of the
+// last of its site's mutations with the sample below it.
+template <typename G>
+__global__ void __launch_bounds__(256) k_genotypes(const TsgGenoArgs a, G *geno, int64_t cells) {
+    constexpr int CELLS = 16 / (int) sizeof(G);
+    const int64_t q = ((int64_t) blockIdx.x * 256 + threadIdx.x) * CELLS;
+    if (q >= cells) return;
+    const int n = a.num_samples;
+    int64_t site = q / n;
+    int j = (int) (q % n);
+    uint32_t v[4] = {0, 0, 0, 0};
+    for (int done = 0; done < CELLS && site < a.num_sites; site++, j = 0) {
+        const int count = min(CELLS - done, n - j);
+        const uint32_t here = ((1u << count) - 1u) << done;
+        const int w = j >> 5;
+        for (int m = a.site_mut0[site]; m < a.site_mut0[site + 1]; m++) {
+            const uint32_t *row = a.x + (int64_t) a.mut_node[m] * a.RW;
+            const uint32_t hi = w + 1 < a.NW ? row[w + 1] : 0u;
+            // bits of samples j .. as cells done ..
+            const uint32_t b = ((uint32_t) ((((uint64_t) hi << 32) | row[w]) >> (j & 31)) << done) & here;
+            const uint32_t al = (uint32_t) a.mut_allele[m];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if constexpr (sizeof(G) == 1) {
+                    // 4 bits to 4 bytes of ones
+                    const uint32_t on = ((((b >> (4 * k)) & 15u) * 0x00204081u) & 0x01010101u) * 255u;
+                    v[k] = (v[k] & ~on) | (on & (al * 0x01010101u));
+                } else {
+                    if ((b >> k) & 1u) v[k] = al;
+                }
+            }
+        }
+        done += count;
+    }
+    *reinterpret_cast<uint4 *>(geno + q) = make_uint4(v[0], v[1], v[2], v[3]);
 }
 
 // --- bit rows by site -> by sample --------------------------------------------
@@ -573,19 +641,57 @@ hipError_t tsg_launch_geno_hot(const TsgGenoArgs &a, size_t shmem, hipStream_t s
 }
 
 // Missing data: geno[site * n + sample] = -1 for each listed pair.
-__global__ void k_mark_missing(int32_t *geno, int n, const int32_t *site, const int32_t *sample,
+template <typename G>
+__global__ void k_mark_missing(G *geno, int n, const int32_t *site, const int32_t *sample,
                                int64_t npairs) {
     const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < npairs) geno[(int64_t) site[i] * n + sample[i]] = -1;
+    if (i < npairs) geno[(int64_t) site[i] * n + sample[i]] = (G) -1;
+}
+template <typename G>
+hipError_t mark_missing(G *geno, int n, const int32_t *site, const int32_t *sample,
+                        int64_t npairs, hipStream_t s) {
+    if (npairs == 0) return hipGetLastError();
+    hipLaunchKernelGGL(k_mark_missing<G>, dim3((unsigned) ((npairs + 255) / 256)), dim3(256), 0, s,
+                       geno, n, site, sample, npairs);
+    return hipGetLastError();
 }
 
 hipError_t tsg_launch_genotypes(const TsgGenoArgs &a, size_t shmem, const int32_t *miss_site,
                                 const int32_t *miss_sample, int64_t nmiss, hipStream_t s) {
     hipError_t e = launch_geno_hot<true>(a, shmem, s);
-    if (e != hipSuccess || nmiss == 0) return e;
-    hipLaunchKernelGGL(k_mark_missing, dim3((unsigned) ((nmiss + 255) / 256)), dim3(256), 0, s,
-                       a.geno, a.num_samples, miss_site, miss_sample, nmiss);
+    if (e != hipSuccess) return e;
+    return mark_missing(a.geno, a.num_samples, miss_site, miss_sample, nmiss, s);
+}
+
+hipError_t tsg_launch_bits_seed(uint32_t *x, int RW, int n, hipStream_t s) {
+    const int64_t threads = (int64_t) (n + 1) * (RW / 4);
+    hipLaunchKernelGGL(k_bits_seed, dim3((unsigned) ((threads + 255) / 256)), dim3(256), 0, s, x, RW,
+                       (int64_t) n);
     return hipGetLastError();
+}
+
+hipError_t tsg_launch_site_bits(const TsgGenoArgs &a, hipStream_t s) {
+    const int64_t threads = (int64_t) a.num_sites * a.NW;
+    if (threads == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_site_bits, dim3((unsigned) ((threads + 255) / 256)), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+template <typename G>
+hipError_t launch_states_genotypes(const TsgGenoArgs &a, G *geno, const int32_t *miss_site,
+                                   const int32_t *miss_sample, int64_t nmiss, hipStream_t s) {
+    constexpr int CELLS = 16 / (int) sizeof(G);
+    const int64_t cells = (int64_t) a.num_sites * a.num_samples;
+    const int64_t threads = (cells + CELLS - 1) / CELLS;
+    hipLaunchKernelGGL(k_genotypes<G>, dim3((unsigned) ((threads + 255) / 256)), dim3(256), 0, s, a,
+                       geno, cells);
+    return mark_missing(geno, a.num_samples, miss_site, miss_sample, nmiss, s);
+}
+
+hipError_t tsg_launch_states_genotypes(const TsgGenoArgs &a, bool narrow, const int32_t *miss_site,
+                                       const int32_t *miss_sample, int64_t nmiss, hipStream_t s) {
+    return narrow ? launch_states_genotypes(a, (int8_t *) a.geno, miss_site, miss_sample, nmiss, s)
+                  : launch_states_genotypes(a, a.geno, miss_site, miss_sample, nmiss, s);
 }
 
 hipError_t tsg_launch_sample_bits(const uint32_t *gbits, int NW, const int32_t *site_of_col,

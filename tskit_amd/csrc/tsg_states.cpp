@@ -255,6 +255,7 @@ int tsg_build_states(tsg_treeseq *ts) {
         sp.pieces.push_back({v.time, tp, v.ins, from, x, v.state, 0});
     };
     sp.list_off.assign(1, 0);
+    sp.mut_state.resize(ts->mut_node.size());
     int32_t j = 0, k = 0;
     for (int32_t t = 0; t < T; t++) {
         const double x = ts->breakpoints[t];
@@ -343,6 +344,7 @@ int tsg_build_states(tsg_treeseq *ts) {
         // nodes
         for (int32_t s = ts->tree_site0[t]; s < ts->tree_site0[t + 1]; s++) {
             const int32_t m0 = ts->site_mut0[s], m1 = ts->site_mut0[s + 1];
+            for (int32_t m = m0; m < m1; m++) sp.mut_state[m] = node[ts->mut_node[m]].state;
             if (m1 == m0 + 1 && ts->mut_allele[m0] == 1 && ts->mut_pallele[m0] == 0) {
                 const Node &v = node[ts->mut_node[m0]];
                 sp.row_ref.push_back(v.state);
@@ -414,6 +416,7 @@ int tsg_build_states(tsg_treeseq *ts) {
         auto whole = [](int32_t &s) -> int32_t & { return s; };
         auto member = [](auto &p) -> int32_t & { return p.state; };
         renumber(sp.ev_state, whole);
+        renumber(sp.mut_state, whole);
         renumber(sp.pieces, member);
         renumber(sp.node_pieces, member);
         for (int32_t &r : sp.row_ref) r = r >= 0 ? at[r] : r;

@@ -65,9 +65,9 @@ struct TsgNodeRuns {
 };
 
 struct TsgStateDevice {
-    // allocations: the plan, and what node statistics and the allele
-    // frequency spectrum add on first use
-    void *block = nullptr, *nodes_block = nullptr, *afs_block = nullptr;
+    // allocations: the plan, and what node statistics, the allele frequency
+    // spectrum and genotypes add on first use
+    void *block = nullptr, *nodes_block = nullptr, *afs_block = nullptr, *bits_block = nullptr;
     int32_t *order = nullptr;      // [states] by level (null: the states are numbered so)
     int32_t *in = nullptr;         // [(states - 1 - n) x TSG_STATE_IN], of state 1 + n on
     int32_t *ev_state = nullptr;   // [events]
@@ -87,6 +87,8 @@ struct TsgStateDevice {
     // allele frequency spectrum (uploaded on first use)
     int32_t *row_all = nullptr;
     TsgBranchPiece *pieces = nullptr;
+    // genotypes
+    int32_t *mut_state = nullptr;
     size_t bytes = 0;
 };
 
@@ -112,6 +114,8 @@ struct tsg_stateplan {
     // all of them count nothing and are left out.
     std::vector<int32_t> row_all;
     std::vector<TsgBranchPiece> pieces;
+    // Genotypes: the state of each mutation's node at its site.
+    std::vector<int32_t> mut_state;
     TsgStateDevice dev;
 };
 
@@ -240,6 +244,8 @@ struct TsgSpectrumArgs {
 };
 // The counts alone (begin: recorded after the host arrays are over).
 hipError_t tsg_launch_state_counts(const TsgStateLaunch &r, hipEvent_t begin, hipStream_t s);
+// The levels from 1 on, of rows whose level 0 is there (16- or 32-bit words).
+hipError_t tsg_launch_state_levels(const TsgStateLaunch &r, hipStream_t s);
 hipError_t tsg_launch_state_nodes(const TsgStateLaunch &r, const TsgNodeArgs &g, int M,
                                   hipStream_t s);
 hipError_t tsg_launch_spectrum(const TsgStateLaunch &r, const TsgSpectrumArgs &g, bool branch,

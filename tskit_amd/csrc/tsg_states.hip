@@ -1396,14 +1396,9 @@ hipError_t launch_eval(const TsgStateArgs &a, hipStream_t s) {
     return launch_eval_as<TYPE, BRANCH, TYPE != TSG_ROW_F64>(a, s);
 }
 
-template <int TYPE>
-hipError_t launch_counts(const TsgStateLaunch &r, hipEvent_t begin, hipStream_t s) {
+template <bool F64>
+hipError_t launch_levels(const TsgStateLaunch &r, hipStream_t s) {
     const TsgStateArgs &a = r.a;
-    constexpr bool F64 = TYPE == TSG_ROW_F64;
-    hipLaunchKernelGGL(k_state_stage, dim3((unsigned) stage_blocks(a)), dim3(256), 0, s, a);
-    hipError_t e;
-    if (begin != nullptr && (e = hipEventRecord(begin, s)) != hipSuccess) return e;
-    hipLaunchKernelGGL((k_state_seed<TYPE>), dim3((unsigned) seed_blocks(a)), dim3(256), 0, s, a);
     for (int l = 1; l < r.levels; l++) {
         const int s0 = r.level0[l], s1 = r.level0[l + 1];
         const int64_t nb = count_blocks(a, s1 - s0);
@@ -1413,6 +1408,17 @@ hipError_t launch_counts(const TsgStateLaunch &r, hipEvent_t begin, hipStream_t 
                            (int) nb);
     }
     return hipGetLastError();
+}
+
+template <int TYPE>
+hipError_t launch_counts(const TsgStateLaunch &r, hipEvent_t begin, hipStream_t s) {
+    const TsgStateArgs &a = r.a;
+    constexpr bool F64 = TYPE == TSG_ROW_F64;
+    hipLaunchKernelGGL(k_state_stage, dim3((unsigned) stage_blocks(a)), dim3(256), 0, s, a);
+    hipError_t e;
+    if (begin != nullptr && (e = hipEventRecord(begin, s)) != hipSuccess) return e;
+    hipLaunchKernelGGL((k_state_seed<TYPE>), dim3((unsigned) seed_blocks(a)), dim3(256), 0, s, a);
+    return launch_levels<F64>(r, s);
 }
 
 template <int TYPE>
@@ -1456,6 +1462,10 @@ hipError_t tsg_launch_state_counts(const TsgStateLaunch &r, hipEvent_t begin, hi
     default:
         return launch_counts<TSG_ROW_F64>(r, begin, s);
     }
+}
+
+hipError_t tsg_launch_state_levels(const TsgStateLaunch &r, hipStream_t s) {
+    return launch_levels<false>(r, s);
 }
 
 hipError_t tsg_launch_state_nodes(const TsgStateLaunch &r, const TsgNodeArgs &g, int M,
