@@ -10,6 +10,9 @@
 // W x M doubles, C order); the callee zero-fills nothing the caller sees
 // until the result is complete.
 #include <hip/hip_runtime.h>
+#ifdef __SSE2__
+#include <emmintrin.h>
+#endif
 
 #include <algorithm>
 #include <atomic>
@@ -653,6 +656,52 @@ bool through_ring(const Workspace *ws, const void *dst, size_t bytes, hipMemoryT
            ws->fixed == nullptr;
 }
 
+// n bytes to d; large results past the caches, where reading a line only to
+// overwrite it costs as much as writing it.
+void copy_bytes(char *d, const char *p, size_t n, bool past) {
+#ifdef __SSE2__
+    if (past) {
+        const size_t head = std::min(n, (size_t) (-(uintptr_t) d & 15));
+        std::memcpy(d, p, head);
+        size_t k = head;
+        for (; k + 64 <= n; k += 64) {
+            const __m128i *v = (const __m128i *) (p + k);
+            const __m128i v0 = _mm_loadu_si128(v), v1 = _mm_loadu_si128(v + 1);
+            const __m128i v2 = _mm_loadu_si128(v + 2), v3 = _mm_loadu_si128(v + 3);
+            __m128i *o = (__m128i *) (d + k);
+            _mm_stream_si128(o, v0);
+            _mm_stream_si128(o + 1, v1);
+            _mm_stream_si128(o + 2, v2);
+            _mm_stream_si128(o + 3, v3);
+        }
+        std::memcpy(d + k, p + k, n - k);
+        _mm_sfence();
+        return;
+    }
+#endif
+    std::memcpy(d, p, n);
+}
+// n int8 values to int32
+void widen_bytes(int32_t *o, const int8_t *v, size_t n, bool past) {
+    size_t k = 0;
+#ifdef __SSE2__
+    if (past) {
+        for (; k < n && ((uintptr_t) (o + k) & 15) != 0; k++) o[k] = v[k];
+        for (; k + 16 <= n; k += 16) {
+            const __m128i x = _mm_loadu_si128((const __m128i *) (v + k));
+            const __m128i lo = _mm_unpacklo_epi8(x, x), hi = _mm_unpackhi_epi8(x, x);
+            __m128i *d = (__m128i *) (o + k);
+            _mm_stream_si128(d, _mm_srai_epi32(_mm_unpacklo_epi16(lo, lo), 24));
+            _mm_stream_si128(d + 1, _mm_srai_epi32(_mm_unpackhi_epi16(lo, lo), 24));
+            _mm_stream_si128(d + 2, _mm_srai_epi32(_mm_unpacklo_epi16(hi, hi), 24));
+            _mm_stream_si128(d + 3, _mm_srai_epi32(_mm_unpackhi_epi16(hi, hi), 24));
+        }
+        _mm_sfence();
+    }
+#endif
+    for (; k < n; k++) o[k] = v[k];
+}
+
 // `bytes` of results into the caller's dst, waiting for stream s to finish: a
 // device copy when dst is device memory, one transfer when it is pinned host
 // memory or tiny; otherwise through a ring of pinned pieces, each piece's
@@ -660,14 +709,16 @@ bool through_ring(const Workspace *ws, const void *dst, size_t bytes, hipMemoryT
 // src holds int8 values and dst takes them as int32 (only through the ring).
 //
 // Bound by the host: the first touch of the caller's pages costs more than
-// the bytes (50 MB into fresh pages of 4 KB: 5 ms with one thread), so the
-// threads touch their shares before the first piece is there, while the
-// kernels still run (MADV_POPULATE_WRITE was slower: pages one by one); the last piece's host copy is all that the transfer
-// does not hide, so there are at least 8 pieces where they are 2 MiB or more
-// (each costs about 12 us between two transfers).
+// the bytes.  So the threads (this one among them) claim blocks of dst in
+// turn and touch theirs before their piece is there, while the kernels still
+// run; a block is a whole huge page, since two threads that touch one at a
+// time clear it twice.  Pieces are 2 MiB at least (each costs about 12 us
+// between two transfers) and at least 8 where there is enough of them: the
+// last one's copy is all that the transfer does not hide.
 constexpr size_t TSG_COPY_PIECE = (size_t) 4 << 20;
 constexpr int TSG_COPY_RING = 8;
 constexpr size_t TSG_COPY_THREADS = 8;
+constexpr size_t TSG_COPY_HUGE = (size_t) 2 << 20;
 
 int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t bytes,
              bool widen = false) {
@@ -698,57 +749,63 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
             return ret;
         }
     }
-    // the copying threads (this one among them): one per 512 KiB, at most 8
+    // blocks of dst: to the first multiple of `block`, then whole ones; small
+    // results (on small pages) in a few a thread
     const unsigned hc = std::thread::hardware_concurrency();
     const size_t T = std::max<size_t>(
         1, std::min<size_t>({TSG_COPY_THREADS, hc == 0 ? 1 : hc, bytes >> 19}));
+    const bool large = bytes >= 2 * TSG_COPY_THREADS * TSG_COPY_HUGE;
+    const size_t block = large ? TSG_COPY_HUGE : (size_t) 128 << 10;
+    const size_t head = -(uintptr_t) dst & (block - 1);
+    const size_t nblocks = 1 + (bytes > head ? (bytes - head + block - 1) / block : 0);
+    auto from_of = [&](size_t b) { return b == 0 ? 0 : std::min(bytes, head + (b - 1) * block); };
+    std::atomic<size_t> next{0};   // blocks claimed
     std::atomic<size_t> ready{0};  // pieces arrived in their pinned buffers
     std::atomic<bool> failed{false};
-    std::vector<std::atomic<int>> done(np);  // threads through with each piece
+    std::vector<std::atomic<size_t>> done(np);  // bytes copied of each piece
     for (auto &d : done) d.store(0, std::memory_order_relaxed);
     auto size_of = [&](size_t i) { return std::min(piece, total - i * piece); };
-    // thread t's part of piece i, in bytes of src
-    auto part = [&](size_t i, size_t t, size_t &from, size_t &to) {
-        const size_t n = size_of(i), per = ((n + T - 1) / T + 63) & ~(size_t) 63;
-        from = std::min(n, t * per);
-        to = std::min(n, from + per);
-    };
-    auto touch = [&](size_t i, size_t t) {  // a byte of every page
-        size_t from, to;
-        part(i, t, from, to);
-        volatile char *d = (volatile char *) dst + i * piece * out_per;
-        for (size_t k = from * out_per; k < to * out_per; k += 4096) d[k] = 0;
-    };
-    auto share = [&](size_t i, size_t t) {
-        size_t from, to;
-        part(i, t, from, to);
-        const char *p = (const char *) ws->cp_h + (i % TSG_COPY_RING) * TSG_COPY_PIECE;
-        char *d = (char *) dst + i * piece * out_per;
-        if (widen) {
-            int32_t *o = (int32_t *) d;
-            const int8_t *v = (const int8_t *) p;
-            for (size_t k = from; k < to; k++) o[k] = v[k];
-        } else {
-            std::memcpy(d + from, p + from, to - from);
-        }
-        done[i].fetch_add(1, std::memory_order_release);
-    };
-    auto worker = [&](size_t t) {
-        size_t here = 0;  // pieces whose pages are there
-        for (size_t i = 0; i < np; i++) {
-            while (ready.load(std::memory_order_acquire) <= i) {
-                if (failed.load(std::memory_order_relaxed)) return;
-                if (here < np) {
-                    touch(here++, t);
-                } else {
-                    std::this_thread::yield();
+    // A thread's part: it claims blocks, touches them while it waits, and copies
+    // them in order; there(i): whether piece i has arrived.
+    auto work = [&](auto there) {
+        constexpr size_t HELD = 4;
+        size_t held[HELD], n = 0, first = 0;
+        auto claim = [&] {
+            const size_t b = next.fetch_add(1, std::memory_order_relaxed);
+            if (b >= nblocks) return false;
+            held[(first + n++) % HELD] = b;
+            return true;
+        };
+        bool more = true;
+        for (;;) {
+            if (n == 0 && !(more = more && claim())) return;
+            const size_t b = held[first];
+            for (size_t k = from_of(b) / out_per, to = from_of(b + 1) / out_per; k < to;) {
+                const size_t i = k / piece, end = std::min(to, (i + 1) * piece);
+                while (!there(i)) {
+                    if (failed.load(std::memory_order_relaxed)) return;
+                    if (n < HELD && more && (more = claim())) {
+                        const size_t c = held[(first + n - 1) % HELD];
+                        volatile char *d = (volatile char *) dst;
+                        for (size_t q = from_of(c); q < from_of(c + 1); q += 4096) d[q] = 0;
+                    } else {
+                        std::this_thread::yield();
+                    }
                 }
+                const char *p = (const char *) ws->cp_h + (i % TSG_COPY_RING) * TSG_COPY_PIECE +
+                                (k - i * piece);
+                if (widen) {
+                    widen_bytes((int32_t *) dst + k, (const int8_t *) p, end - k, large);
+                } else {
+                    copy_bytes((char *) dst + k, p, end - k, large);
+                }
+                done[i].fetch_add(end - k, std::memory_order_release);
+                k = end;
             }
-            share(i, t);
-            here = std::max(here, i + 1);
+            first = (first + 1) % HELD;
+            n--;
         }
     };
-    std::vector<std::thread> pool;
     auto send = [&](size_t i) {
         const int b = (int) (i % TSG_COPY_RING);
         const int e = hip_check(hipMemcpyAsync((char *) ws->cp_h + b * TSG_COPY_PIECE,
@@ -759,41 +816,43 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
     size_t sent = 0;
     ret = 0;
     for (; ret == 0 && sent < std::min<size_t>(np, TSG_COPY_RING); sent++) ret = send(sent);
+    // this thread passes on what has arrived and refills what is copied
+    auto pump = [&] {
+        size_t r = ready.load(std::memory_order_relaxed);
+        while (ret == 0 && r < sent) {
+            const hipError_t e = hipEventQuery(ws->cp_ev[r % TSG_COPY_RING]);
+            if (e == hipErrorNotReady) {
+                (void) hipGetLastError();
+                break;
+            }
+            if ((ret = hip_check(e)) == 0) ready.store(++r, std::memory_order_release);
+        }
+        while (ret == 0 && sent < np && sent - TSG_COPY_RING < r &&
+               done[sent - TSG_COPY_RING].load(std::memory_order_acquire) ==
+                   size_of(sent - TSG_COPY_RING)) {
+            ret = send(sent++);
+        }
+        if (ret != 0) failed.store(true, std::memory_order_relaxed);
+    };
+    std::vector<std::thread> pool;
     for (size_t t = 1; ret == 0 && t < T; t++) {
         try {
-            pool.emplace_back(worker, t);
-        } catch (const std::system_error &) {  // no more threads: this one does their share
+            pool.emplace_back(work, [&](size_t i) { return ready.load(std::memory_order_acquire) > i; });
+        } catch (const std::system_error &) {  // no more threads: fewer do the work
             break;
         }
     }
-    const size_t mine = pool.size() + 1;
     if (ret == 0) {
-        size_t here = 0;
-        while (here < np && hipEventQuery(ws->cp_ev[0]) == hipErrorNotReady) {
-            touch(here, 0);
-            for (size_t t = mine; t < T; t++) touch(here, t);
-            here++;
+        work([&](size_t i) {
+            pump();
+            return ready.load(std::memory_order_relaxed) > i;
+        });
+        // (the others may still wait for pieces)
+        while (ret == 0 && ready.load(std::memory_order_relaxed) < np) {
+            pump();
+            std::this_thread::yield();
         }
     }
-    for (size_t i = 0; ret == 0 && i < np; i++) {
-        if ((ret = hip_check(hipEventSynchronize(ws->cp_ev[i % TSG_COPY_RING])))) break;
-        ready.store(i + 1, std::memory_order_release);
-        share(i, 0);
-        for (size_t t = mine; t < T; t++) share(i, t);
-        // refill the buffers every thread is through with
-        while (ret == 0 && sent < np &&
-               done[sent - TSG_COPY_RING].load(std::memory_order_acquire) == (int) T) {
-            ret = send(sent++);
-        }
-        // the next piece has to be on its way
-        while (ret == 0 && sent < np && sent <= i + 1) {
-            while (done[sent - TSG_COPY_RING].load(std::memory_order_acquire) != (int) T) {
-                std::this_thread::yield();
-            }
-            ret = send(sent++);
-        }
-    }
-    if (ret != 0) failed.store(true, std::memory_order_relaxed);
     for (std::thread &t : pool) t.join();
     const int sret = hip_check(hipStreamSynchronize(s));
     return ret != 0 ? ret : sret;
