@@ -43,6 +43,8 @@
 #define EVAL_THREADS 256
 #define FINISH_THREADS 1024
 #define SPECTRUM_SLOTS 1024
+// windows whose first events a tile keeps at a time
+#define EDGES 256
 
 namespace {
 
@@ -563,38 +565,6 @@ __device__ __forceinline__ void with_summary(int stat, U use) {
 template <typename F>
 constexpr bool reads_mean = std::is_same<F, Relatedness>::value;
 
-// Output o's summary of event e alone, before the scale.
-template <int TYPE, int TILE, bool BRANCH, typename T>
-__device__ __forceinline__ double value_of(const TsgStateArgs &a, const TsgStateOut &o,
-                                           const Tile<T> &tile, int e) {
-    const bool pol = o.polarised != 0;
-    const int k = BRANCH ? TSG_ROW_PAIR : tile.kind[e];
-    if (pol && k == TSG_ROW_ANCESTRAL) return 0.0;
-    const bool both = !pol && k == TSG_ROW_PAIR;
-    if constexpr (TYPE == TSG_ROW_F64) {
-        if (o.stat == TSG_STAT_TRAIT_LINEAR_MODEL) {
-            const double v = regression<TILE>(a, o, tile.cols, e, false);
-            return both ? v + regression<TILE>(a, o, tile.cols, e, true) : v;
-        }
-    }
-    constexpr int STRIDE = stride_of<T>(TILE);
-    double x[4] = {(double) tile.cols[o.c[0] * STRIDE + e], 0.0, 0.0, 0.0};
-    double v = 0.0;
-    with_summary<TYPE>(o.stat, [&](auto make) {
-        const auto f = make(o);
-        using F = typename std::decay<decltype(f)>::type;
-        if constexpr (F::S > 1) x[1] = (double) tile.cols[o.c[1] * STRIDE + e];
-        if constexpr (reads_mean<F>) {
-            x[2] = tile.mean[e];
-        } else if constexpr (F::S > 2) {
-            x[2] = (double) tile.cols[o.c[2] * STRIDE + e];
-        }
-        if constexpr (F::S > 3) x[3] = (double) tile.cols[o.c[3] * STRIDE + e];
-        v = pol ? f.one(x) : both ? f.both(x) : f.lone(x);
-    });
-    return v;
-}
-
 // Four lane values a, b, c, d added up over the wave at once: lanes 0-15 get
 // a's sum, 16-31 c's, 32-47 b's, 48-63 d's (each swap halves the number of
 // values a lane holds: 3 swaps and 4 row rotations for 4 sums instead of 24
@@ -715,6 +685,85 @@ __device__ __forceinline__ void add_regressions(const TsgStateArgs &a, const Tsg
     }
 }
 
+// `count` outputs of one summary over cn windows of a tile: a thread adds up
+// the events of a (window, output) pair one by one.  Window i has the events
+// edge[i] .. edge[i + 1] and ends at wend[i]; its sums go to dst, windows M
+// outputs apart.
+template <int TYPE, int TILE, bool BRANCH, typename T>
+__device__ __forceinline__ void add_items(const TsgStateArgs &a, const TsgStateOut *outs,
+                                          const TsgStateOut &first, int count, const Tile<T> &tile,
+                                          const double *spos, const double *sb,
+                                          const int32_t *edge, const double *wend, int cn,
+                                          double *dst, int M) {
+    constexpr int STRIDE = stride_of<T>(TILE), PER = BRANCH ? 2 : 1;
+    const bool pol = first.polarised != 0;
+    auto items = [&](auto prepare) {
+        // a thread keeps its output while there is room for them all
+        for (int mc = 0; mc < count; mc += EVAL_THREADS) {
+            const int mn = min(EVAL_THREADS, count - mc), groups = EVAL_THREADS / mn;
+            const int m = mc + (int) threadIdx.x % mn;
+            if ((int) threadIdx.x >= groups * mn) continue;
+            const TsgStateOut o = outs[m];
+            const auto value = prepare(o);
+            for (int i = (int) threadIdx.x / mn; i < cn; i += groups) {
+                const int ea = edge[i], eb = edge[i + 1];
+                const double wr = wend[i];
+                double L = 0, J = 0;
+                for (int e = ea; e < eb; e++) {
+                    const double v = value(e);
+                    if constexpr (BRANCH) {
+                        const double b = sb[e];
+                        L = fma(v, b * (wr - spos[e]), L);
+                        J = fma(v, b, J);
+                    } else {
+                        L += v;
+                    }
+                }
+                // (a zero denominator: 0 x inf is the reference's NaN at every
+                // state, but a window without events has 0)
+                double *to = dst + ((int64_t) i * M + m) * PER;
+                to[0] = eb > ea ? L * o.scale : 0.0;
+                if constexpr (BRANCH) to[1] = eb > ea ? J * o.scale : 0.0;
+            }
+        }
+    };
+    if constexpr (TYPE == TSG_ROW_F64) {
+        if (first.stat == TSG_STAT_TRAIT_LINEAR_MODEL) {
+            items([&](const TsgStateOut &o) {
+                return [&](int e) {
+                    const int k = (!BRANCH && tile.mixed) ? tile.kind[e] : TSG_ROW_PAIR;
+                    if (pol && k == TSG_ROW_ANCESTRAL) return 0.0;
+                    double v = regression<TILE>(a, o, tile.cols, e, false);
+                    if (!pol && k == TSG_ROW_PAIR) v = v + regression<TILE>(a, o, tile.cols, e, true);
+                    return v;
+                };
+            });
+            return;
+        }
+    }
+    with_summary<TYPE>(first.stat, [&](auto make) {
+        items([&](const TsgStateOut &o) {
+            const auto f = make(o);
+            using F = typename std::decay<decltype(f)>::type;
+            const T *c0 = tile.cols + o.c[0] * STRIDE, *c1 = tile.cols + o.c[1] * STRIDE;
+            const T *c2 = tile.cols + o.c[2] * STRIDE, *c3 = tile.cols + o.c[3] * STRIDE;
+            return [=, &tile](int e) {
+                double x[4] = {(double) c0[e], 0.0, 0.0, 0.0};
+                if constexpr (F::S > 1) x[1] = (double) c1[e];
+                if constexpr (reads_mean<F>) {
+                    x[2] = tile.mean[e];
+                } else if constexpr (F::S > 2) {
+                    x[2] = (double) c2[e];
+                }
+                if constexpr (F::S > 3) x[3] = (double) c3[e];
+                const int k = (!BRANCH && tile.mixed) ? tile.kind[e] : TSG_ROW_PAIR;
+                if (pol) return k == TSG_ROW_ANCESTRAL ? 0.0 : f.one(x);
+                return k == TSG_ROW_PAIR ? f.both(x) : f.lone(x);
+            };
+        });
+    });
+}
+
 // One tile: events (BRANCH) or site rows t TILE .. of the run.  WIDE: more
 // columns than an FP64 tile takes.
 template <int TYPE, bool BRANCH, bool WIDE>
@@ -728,7 +777,9 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
     double *sb = spos + TILE;                                  // [TILE] (branch)
     double *mean = sb + (BRANCH ? TILE : 0);                   // [TILE]
     int32_t *kind = reinterpret_cast<int32_t *>(mean + TILE);  // [TILE] (site)
-    T *cols = reinterpret_cast<T *>(kind + (BRANCH ? 0 : TILE));  // [K x TILE]
+    double *wend = reinterpret_cast<double *>(kind + (BRANCH ? 0 : TILE));  // [EDGES]
+    int32_t *edge = reinterpret_cast<int32_t *>(wend + EDGES);              // [EDGES + 4]
+    T *cols = reinterpret_cast<T *>(edge + EDGES + 4);                      // [K x STRIDE]
     const int tid = threadIdx.x;
     const int lane = tid & (WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
@@ -836,34 +887,31 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
         const int nw = w1 - w0 + 1;
         // A wave adds up an output's whole tile for each of its windows (about
         // 400 cycles); a thread a (window, output) pair's events one by one
-        // (about 150 cycles each, 256 threads): whichever is less.  (Measured
-        // on site tiles of up to 250 of 500 windows, 31 outputs: 1634 -> 71 us.)
+        // (about 50 cycles an event, 150 a row, 256 threads): whichever is
+        // less.  (Branch tiles of 5 windows, 64 outputs: 107 us, 40 in pairs;
+        // of 20 windows, 31 outputs: 91 in pairs; site tiles of 2 or 3
+        // windows, 60 outputs: 40 us, 100 in pairs.)
         if ((int64_t) nw * nw * ((M + 3) / 4) * 8 >
-            (int64_t) TILE * 3 * (((int64_t) nw * M + EVAL_THREADS - 1) / EVAL_THREADS)) {
-            for (int64_t i = tid; i < (int64_t) nw * M; i += EVAL_THREADS) {
-                const int w = w0 + (int) (i / M), m = (int) (i % M);
-                const int ea = w == w0 ? 0 : lower_bound(spos, ne, win[w]);
-                const int eb = w == w1 ? ne : lower_bound(spos, ne, win[w + 1]);
-                const double wr = win[w + 1];
-                const TsgStateOut o = a.outs[Q.mbase + m];
-                double L = 0, J = 0;
-                for (int e = ea; e < eb; e++) {
-                    const double v = value_of<TYPE, TILE, BRANCH>(a, o, tile, e);
-                    if constexpr (BRANCH) {
-                        const double b = sb[e];
-                        L = fma(v, b * (wr - spos[e]), L);
-                        J = fma(v, b, J);
-                    } else {
-                        L += v;
-                    }
+            (int64_t) TILE * (BRANCH ? 1 : 3) *
+                (((int64_t) nw * M + EVAL_THREADS - 1) / EVAL_THREADS)) {
+            for (int c0 = w0; c0 <= w1; c0 += EDGES) {
+                const int cn = min(EDGES, w1 - c0 + 1);
+                // the windows' first events, found once for all outputs
+                __syncthreads();
+                for (int i = tid; i <= cn; i += EVAL_THREADS) {
+                    const int w = c0 + i;
+                    edge[i] = w == w0 ? 0 : w > w1 ? ne : lower_bound(spos, ne, win[w]);
+                    if (i < cn) wend[i] = win[w + 1];
                 }
-                // (a zero denominator: 0 x inf is the reference's NaN at every
-                // state, but a window without events has 0)
-                L = eb > ea ? L * o.scale : 0.0;
-                J = eb > ea ? J * o.scale : 0.0;
-                double *dst = a.partial + Q.pbase + ((int64_t) (t + w) * M + m) * PER;
-                dst[0] = L;
-                if constexpr (BRANCH) dst[1] = J;
+                __syncthreads();
+                for (int m = 0; m < M;) {
+                    const TsgStateOut first = uniform(a.outs + Q.mbase + m);
+                    const int count = min(first.run, M - m);
+                    double *dst = a.partial + Q.pbase + ((int64_t) (t + c0) * M + m) * PER;
+                    add_items<TYPE, TILE, BRANCH>(a, a.outs + Q.mbase + m, first, count, tile, spos,
+                                                  sb, edge, wend, cn, dst, M);
+                    m += count;
+                }
             }
             continue;
         }
@@ -1364,7 +1412,8 @@ size_t tsg_state_shmem(int K, int type, bool branch) {
     const size_t el = (type == TSG_ROW_F64 || K <= TSG_STATE_F64_COLUMNS) ? 8
                       : (type == TSG_ROW_U16 && branch)                   ? 2
                                                                           : 4;
-    return tile * (8 + 8 + (branch ? 8 : 4)) + el * (tile + 2) * (size_t) K + 16;
+    return tile * (8 + 8 + (branch ? 8 : 4)) + EDGES * 8 + (EDGES + 4) * 4 +
+           el * (tile + 2) * (size_t) K + 16;
 }
 
 namespace {
