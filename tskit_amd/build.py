@@ -4,10 +4,12 @@
 into ``tskit_amd/libtsgpu.so``.  The library exposes a C ABI (see
 ``include/tsgpu.h``) and is loaded with ctypes by ``tskit_amd._lib``.
 """
+import concurrent.futures
 import os
 import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -30,7 +32,6 @@ FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     f"--offload-arch={ARCH}",
     # summary values must round identically wherever they are evaluated
     "-ffp-contract=off",
@@ -51,10 +52,7 @@ def hipcc():
     return path
 
 
-def build(verbose=False):
-    srcs = [os.path.join(CSRC, s) for s in SOURCES]
-    tmp = LIB + ".tmp"
-    cmd = [hipcc(), *FLAGS, "-I", CSRC, "-o", tmp, *srcs]
+def run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -67,6 +65,20 @@ def build(verbose=False):
         raise RuntimeError(f"hipcc failed ({res.returncode}):\n{err}")
     if verbose and err.strip():
         print(err, file=sys.stderr)
+
+
+def build(verbose=False):
+    cc = hipcc()
+    tmp = LIB + ".tmp"
+    # one job a source (together 6 minutes, the longest alone 4)
+    with tempfile.TemporaryDirectory() as d:
+        objs = [os.path.join(d, s + ".o") for s in SOURCES]
+        with concurrent.futures.ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+            jobs = [pool.submit(run, [cc, *FLAGS, "-I", CSRC, "-c", os.path.join(CSRC, s), "-o", o],
+                                verbose) for s, o in zip(SOURCES, objs)]
+            for j in jobs:
+                j.result()
+        run([cc, "-fPIC", "-shared", f"--offload-arch={ARCH}", "-o", tmp, *objs], verbose)
     os.replace(tmp, LIB)
     return LIB
 
