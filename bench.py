@@ -501,9 +501,8 @@ def replicate_phase(om, with_cpu, inflight=4):
 
 
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "k_sweep_traffic.json")
-# the branch sweep of the scale workload: hot slots with 16-bit counts, one
-# output per lane, 8 hop groups per column (K = 8)
-SWEEP_KERNEL = "k_sweep<0, 3, 1, 8>"
+# the branch evaluation of the scale workload: 16-bit counts, tiles in FP64
+SWEEP_KERNEL = "k_state_eval<0, true, false>"
 
 
 def pmc_summary(fetch_csv, write_csv):
@@ -554,7 +553,9 @@ def measured_traffic(cfg_name):
             t = json.load(f)
     except (OSError, ValueError):
         return None
-    return t.get("traffic_bytes") if t.get("workload") == cfg_name else None
+    if t.get("workload") != cfg_name or t.get("kernel") != SWEEP_KERNEL:
+        return None
+    return t.get("traffic_bytes")
 
 
 def node_phase(ts, tc, sets, om, with_cpu, reps=3):
@@ -735,9 +736,9 @@ def main():
         f"branch {mode_ms['branch']:.3f} ms, site {mode_ms['site']:.3f} ms "
         f"({launches} launches)")
 
-    # roofline of the dominant kernel (the fused branch-mode sweep,
-    # k_sweep<0,...>): algorithmic bytes per launch / its average launch time
-    # from HIP events on the library's stream
+    # roofline of the dominant kernels (the counts of all states and the
+    # branch evaluation on them): algorithmic bytes per launch / their average
+    # time together from HIP events on the library's stream
     per_launch_queries = [(K, K + len(pairs)), (K, 2 * K), (K, len(quads))]
     alg_bytes = algorithmic_bytes(E, N, S, cfg["n"], per_launch_queries, cfg["W"])
     avg_launch_s = mode_ms["branch"] / 1e3
@@ -745,7 +746,7 @@ def main():
     roofline = {"bound": "hbm", "achieved": round(achieved, 3), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                 "traffic": None if args.small else measured_traffic(cfg["name"]),
-                "kernel": "k_sweep<0, 3, 1, 8> (branch, fused batch)", "bytes_per_launch": alg_bytes,
+                "kernel": "k_state_count + " + SWEEP_KERNEL + " (branch, fused batch)", "bytes_per_launch": alg_bytes,
                 "avg_launch_ms": round(avg_launch_s * 1e3, 4),
                 "site_sweep_ms": round(mode_ms["site"], 4)}
 

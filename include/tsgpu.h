@@ -104,7 +104,7 @@ int tsg_treeseq_copy_plan(const tsg_treeseq_t *ts, int32_t *chunk_tree0, int64_t
  * sets the number of (site, sample pair) with different alleles in the
  * window, over the pairs of the two sets, divided by the number of pairs
  * (trees.c:8876-8899) and, with TSG_STAT_SPAN_NORMALISE, by the window span;
- * from the same int8 cross products as the relatedness matrix: per window
+ * from the same cross products as the relatedness matrix: per window
  * P = 2 G1'G1 + G2'G2 (G1 the derived-allele rows of the sites with at most
  * two alleles, G2 the any-derived row and one row per derived allele of the
  * others), samples i and j differing at (P_ii + P_jj) / 2 - P_ij sites
@@ -153,13 +153,14 @@ int tsg_treeseq_copy_state_plan(const tsg_treeseq_t *ts, int32_t *level0, int32_
     int32_t *ev_state, double *ev_b, double *ev_pos, int32_t *row_ref, double *row_pos,
     int32_t *list_off, int32_t *list_kind, int32_t *list_ent);
 /* plan = 1: run statistics sweeps on the full plan; 2: on the hot plan with
- * 32-bit counts; 0: the library chooses (the hot plan whenever its slots fit
- * in LDS, 16-bit counts when every set has <= 65535 samples) -- a testing
- * hook */
+ * 32-bit counts; 0: the library chooses (the state plan where it is usable and
+ * takes the run, else the hot plan whenever its slots fit in LDS; 16-bit
+ * counts when every set has <= 65535 samples) -- a testing hook */
 int tsg_treeseq_set_sweep_plan(tsg_treeseq_t *ts, int plan);
 /* node store of the last statistics sweep: 0 HBM slabs, 1 LDS (full plan),
- * 2 LDS hot slots, 3 LDS hot slots with 16-bit counts, -1 before the first
- * sweep */
+ * 2 32-bit counts (LDS hot slots or rows of the state plan; also genotypes,
+ * node statistics and the spectrum), 3 16-bit counts, 4 FP64 weights, -1
+ * before the first sweep */
 int tsg_treeseq_get_last_store(const tsg_treeseq_t *ts);
 /* HIP-event timing of the sweep kernel on the library's stream */
 int tsg_treeseq_set_profiling(tsg_treeseq_t *ts, int enable);
@@ -322,7 +323,7 @@ int tsg_treeseq_allele_frequency_spectrum(tsg_treeseq_t *ts, uint64_t num_sample
  * genetic_relatedness_matrix(mode="site") of python/tskit/trees.py:8978-9102
  * (the divergence matrix of c/tskit/trees.c:8900-9001 double-centred) for
  * singleton sample sets (sample_sets NULL = every sample), computed as
- * K = J P J / 2 with P the int8 matrix-core cross product of the divergence
+ * K = J P J / 2 with P the matrix-core cross product of the divergence
  * matrix above (exact int32; K = J G^T G J when every site has at most two
  * alleles) and FP64 centring.  Windows need not span
  * the genome (as the reference's divergence matrix).  result: W x n x n. */

