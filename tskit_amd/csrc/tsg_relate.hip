@@ -313,8 +313,8 @@ __global__ void __launch_bounds__(256) k_genotypes(const TsgGenoArgs a, G *geno,
 // takes 256 columns of 128 samples: per 64 columns each lane reads one site's
 // 4 words and 128 ballots turn them; each lane then holds 32 bytes of two
 // samples' rows.  Bound by its ballots, about 2 instructions a sample and 64
-// sites (2500 samples x 56000 sites: the int8 expansion this replaced wrote
-// 143 MB, 66 us).
+// sites (2500 samples x 56000 sites: 48 us; the int8 expansion this replaced
+// wrote 143 MB, 66 us).
 __global__ void __launch_bounds__(256) k_sample_bits(const uint32_t *gbits, int NW,
                                                      const int32_t *site_of_col, int64_t Kp,
                                                      uint32_t *bits) {
@@ -383,8 +383,8 @@ __device__ __forceinline__ v8i fp4(uint32_t b) {
 // tile over a quarter of the columns, 4 x 4 tiles of 32 x 32, so that 8
 // expansions (7 instructions each) feed 16 matrix instructions; the four
 // waves' sums are added in LDS, as integers.
-// (2500 samples x 56000 sites: 721 us with int8 operands staged in LDS, each
-// wave a quarter of the tile.)
+// (2500 samples x 56000 sites: 114 us; 721 with int8 operands staged in LDS,
+// each wave a quarter of the tile.  5000 x 199000: 1322 us, 4693 before.)
 __global__ void __launch_bounds__(256, 1) k_syrk(const uint32_t *bits, int64_t KW, int n_pad,
                                                  const int64_t *win_k0, const int64_t *win_k1,
                                                  int tiles_per_dim, bool add, int32_t *C) {
