@@ -173,6 +173,121 @@ def test_state_plan_executes_to_oracle(name, polarised):
             assert np.max(np.abs(got - exp)) <= TOL * scale, (stat, mode)
 
 
+def forest(n, inner, trees, moves, seed):
+    """Samples that hop between a few inner nodes (the youngest a sample too,
+    the others under the last), so that nodes cross the number of children
+    one state takes in both directions, and subtrees move."""
+    rng = np.random.default_rng(seed)
+    hubs = list(range(n, n + inner))
+    root = n + inner
+    times = np.concatenate([np.zeros(n), 1.0 + np.arange(inner) / 8, [4.0]])
+    cur = rng.choice(hubs + [root], n)
+    up = np.array([rng.choice(hubs[i + 1:] + [root]) for i in range(inner)])
+    parents = []
+    for _ in range(trees):
+        for s in rng.choice(n, moves, replace=False):
+            cur[s] = rng.choice(hubs + [root, -1], p=[0.9 / inner] * inner + [0.05, 0.05])
+        i = rng.integers(inner)
+        if rng.random() < 0.3:
+            up[i] = rng.choice(hubs[i + 1:] + [root])
+        parents.append(np.concatenate([cur, up, [-1]]))
+    return parents, times, list(range(n)) + hubs[:1]
+
+
+def there_and_back():
+    """A child of one wide node that spends a tree below another, while the
+    first is narrow."""
+    par = np.concatenate([np.full(8, 20), np.full(12, 21), [22, 22, -1]])
+    moved = par.copy()
+    moved[7] = 21
+    return [par, moved, par], np.concatenate([np.zeros(20), [1.0, 1.0, 2.0]]), list(range(20))
+
+
+HOPS = {"there_and_back": there_and_back}
+HOPS.update({f"{n}_{inner}_{moves}_{seed}": (lambda a=(n, inner, 60, moves, seed): forest(*a))
+             for n, inner, moves in [(12, 2, 1), (20, 3, 2), (30, 3, 3), (40, 3, 3), (90, 2, 4)]
+             for seed in range(4)})
+
+
+def with_sites_everywhere(parents, times, samples):
+    """The trees' tables with a site per tree and node, one mutation each."""
+    tc = from_parents(parents, times, samples)
+    T, N = len(parents), len(times)
+    S, width = T * N, tc.sequence_length / T
+    tc.site_position = np.repeat(np.arange(T) * width, N) + np.tile(np.arange(N) * width / N, T)
+    tc.ancestral_state = np.full(S, ord("0"), np.int8)
+    tc.ancestral_state_offset = np.arange(S + 1, dtype=np.uint64)
+    tc.mutation_site = np.arange(S, dtype=np.int32)
+    tc.mutation_node = np.tile(np.arange(N), T).astype(np.int32)
+    tc.mutation_parent = np.full(S, -1, np.int32)
+    tc.derived_state = np.full(S, ord("1"), np.int8)
+    tc.derived_state_offset = np.arange(S + 1, dtype=np.uint64)
+    return tc
+
+
+def samples_below(par, times, samples):
+    """[nodes x samples] of one tree."""
+    below = np.zeros((len(times), len(samples)), np.int64)
+    below[samples, np.arange(len(samples))] = 1
+    for u in np.argsort(times, kind="stable"):
+        if par[u] >= 0:
+            below[par[u]] += below[u]
+    return below
+
+
+@pytest.mark.parametrize("name", list(HOPS))
+def test_states_are_the_samples_below(name):
+    """The plan's rows and branch events against the trees themselves, sample
+    by sample (a state's counts are whole numbers: equal; the branch lengths
+    of one set of samples: sums of a few dozen exactly representable terms)."""
+    parents, times, samples = HOPS[name]()
+    tc = with_sites_everywhere(parents, times, samples)
+    ts = tc.tree_sequence()
+    plan = ts.ll_tree_sequence.get_state_plan()
+    assert plan["usable"]
+    n, N, T = len(samples), len(times), len(parents)
+    index = np.full(N, -1)
+    index[samples] = np.arange(n)
+    x = counts(plan, n, [np.array([s]) for s in samples], index)
+    assert np.array_equal(plan["row_ref"] >= 0, np.ones(T * N, bool))
+    width = ts.sequence_length / T
+    have = {}
+    at = np.rint(plan["ev_pos"] / width).astype(int)
+    for t, par in enumerate(parents):
+        below = samples_below(par, times, samples)
+        assert np.array_equal(x[plan["row_ref"][t * N:(t + 1) * N]], below), t
+        for e in np.flatnonzero(at == t):
+            key = x[plan["ev_state"][e]].tobytes()
+            have[key] = have.get(key, 0.0) + plan["ev_b"][e]
+        want = {}
+        for u in range(N):
+            if par[u] >= 0:
+                key = below[u].tobytes()
+                want[key] = want.get(key, 0.0) + times[par[u]] - times[u]
+        for key in set(have) | set(want):
+            assert have.get(key, 0.0) == want.get(key, 0.0), t
+
+
+@pytest.mark.gpu
+def test_wide_nodes_on_the_device(require_gpu):
+    """Genotypes (bits that are added: equal) and the spectrum where children
+    hop between wide nodes."""
+    parents, times, samples = HOPS["40_3_3_1"]()
+    tc = with_sites_everywhere(parents, times, samples)
+    ts, orc = tc.tree_sequence(), Oracle(tc)
+    want = np.concatenate([samples_below(par, times, samples) for par in parents])
+    print("[case] genotypes", flush=True)
+    assert np.array_equal(ts.genotype_matrix(isolated_as_missing=False), want)
+    sets = sets_of(ts, 2, 5)
+    win = np.array([0, 33.0, 100.0])
+    for mode in ("site", "branch"):
+        print("[case] spectrum", mode, flush=True)
+        got = ts.allele_frequency_spectrum(sets, windows=win, mode=mode, polarised=True)
+        exp = orc.afs(sets, win, mode=mode, polarised=True)
+        err = float(np.max(np.abs(got - exp.reshape(got.shape))))
+        assert err <= TOL * float(np.max(exp)), err
+
+
 def test_state_plan_limits():
     """Trees of more merged levels than launches are worth stay on the chunk
     plans."""

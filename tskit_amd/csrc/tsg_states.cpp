@@ -132,8 +132,11 @@ struct Planner {
 
     int32_t sum_wide(int32_t u) {
         Wide &w = wide[u];
-        for (int32_t &c : w.slots) {
-            if (c >= 0 && node[c].par != u) c = -1;
+        // (a child that was under another wide node since may be in a slot it
+        // no longer names: it is in the one it names, or gets a new one)
+        for (size_t i = 0; i < w.slots.size(); i++) {
+            int32_t &c = w.slots[i];
+            if (c >= 0 && (node[c].par != u || node[c].slot != (int32_t) i)) c = -1;
         }
         size_t hole = 0;
         for (int32_t c = node[u].lc; c >= 0; c = node[c].rs) {
