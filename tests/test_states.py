@@ -5,6 +5,8 @@ windows (GPU).
 Tolerances, of each output's largest |value|: sums of at most 1e5 terms with
 one rounding each (1.1e-16) and cancelling partial sums at most 1e3 times the
 result stay below 1e-8."""
+import time
+
 import numpy as np
 import pytest
 
@@ -207,6 +209,7 @@ HOPS = {"there_and_back": there_and_back}
 HOPS.update({f"{n}_{inner}_{moves}_{seed}": (lambda a=(n, inner, 60, moves, seed): forest(*a))
              for n, inner, moves in [(12, 2, 1), (20, 3, 2), (30, 3, 3), (40, 3, 3), (90, 2, 4)]
              for seed in range(4)})
+HOPS["1200_2_40_0"] = lambda: forest(1200, 2, 12, 40, 0)  # four levels of groups
 
 
 def with_sites_everywhere(parents, times, samples):
@@ -266,6 +269,32 @@ def test_states_are_the_samples_below(name):
                 want[key] = want.get(key, 0.0) + times[par[u]] - times[u]
         for key in set(have) | set(want):
             assert have.get(key, 0.0) == want.get(key, 0.0), t
+
+
+def test_plan_of_wide_nodes_takes_no_pass_over_their_children():
+    """20000 samples below two nodes, one moving a tree: 0.1 s, where a visit
+    to every child at every move took 10 s."""
+    n, trees = 20000, 20000
+    rng = np.random.default_rng(1)
+    cur, since, rows = rng.integers(n, n + 2, n), np.zeros(n), []
+    for t in range(1, trees):
+        s = rng.integers(n)
+        rows.append((since[s], t, cur[s], s))
+        cur[s], since[s] = 2 * n + 1 - cur[s], t
+    rows += [(since[s], trees, cur[s], s) for s in range(n)]
+    rows += [(0, trees, n + 2, n), (0, trees, n + 2, n + 1)]
+    tc = ta.TableCollection(float(trees))
+    flags = np.zeros(n + 3, np.uint32)
+    flags[:n] = 1
+    tc.set_nodes(flags, np.concatenate([np.zeros(n), [1.0, 1.0, 2.0]]))
+    a = np.array([r for r in rows if r[0] < r[1]])
+    tc.set_edges(a[:, 0], a[:, 1], a[:, 2].astype(np.int32), a[:, 3].astype(np.int32))
+    tc.sort_edges()
+    t0 = time.perf_counter()
+    ts = tc.tree_sequence()
+    took = time.perf_counter() - t0
+    assert ts.ll_tree_sequence.get_state_plan_sizes()["usable"]
+    assert took < 3.0, took
 
 
 @pytest.mark.gpu
