@@ -12,6 +12,7 @@ import pytest
 
 import cases
 import tskit_amd as ta
+from tskit_amd import summaries
 from oracle.oracle import Oracle
 
 TOL = 1e-8
@@ -315,6 +316,59 @@ def test_wide_nodes_on_the_device(require_gpu):
         exp = orc.afs(sets, win, mode=mode, polarised=True)
         err = float(np.max(np.abs(got - exp.reshape(got.shape))))
         assert err <= TOL * float(np.max(exp)), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [np.nan, np.inf, 1e200])
+def test_one_window_keeps_its_infinities(require_gpu, value):
+    """A weight that is not finite, or whose square is not, reaches the windows
+    whose alleles (branches) are above its sample and no others: those are
+    what they are with a weight of zero there."""
+    tc = cases.generated(300, 3e5, 11)
+    ts = tc.tree_sequence()
+    ll, n, L = ts.ll_tree_sequence, ts.num_samples, ts.sequence_length
+    geno, pos = ts.genotype_matrix(isolated_as_missing=False), np.asarray(tc.site_position)
+    s = int(np.argmin(geno.sum(axis=0)))
+    with_s = pos[geno[:, s] > 0]
+    gaps = np.concatenate([[0.0], with_s, [L]])
+    g = int(np.argmax(np.diff(gaps)))
+    few = np.array([0.0, np.nextafter(gaps[g], L), gaps[g + 1], L])
+    rng = np.random.default_rng(4)
+    W = rng.normal(size=(n, 2))
+    Z = rng.normal(size=(n, 1)) / n
+    Z[s] = 0.0
+    W[s, 0] = 0.0
+    bad = W.copy()
+    bad[s, 0] = value
+    calls = [lambda w, v, m: ll.general_stat(v, summaries.trait_covariance(n), 2, w, m, 1, 0),
+             lambda w, v, m: ll.genetic_relatedness_weighted(v, [(0, 1)], w, m, 0, 1, 0)]
+    if np.isfinite(value):  # (the projection on the covariates is finite too)
+        calls.append(lambda w, v, m: ll.trait_linear_model(v, Z, w, m, 1, 0))
+    for i, call in enumerate(calls):
+        for win in (few, np.unique(np.concatenate([few, np.linspace(0, L, 400)]))):
+            print("[case]", value, i, len(win), flush=True)
+            free = np.histogram(with_s, win)[0] == 0
+            assert free.any() and not free.all()
+            got, want = call(win, bad, "site"), call(win, W, "site")
+            assert np.array_equal(got[free], want[free])
+            if i != 1:
+                assert not np.isfinite(got[~free][:, 0]).any()
+    # branches: a sample that joins the trees half way
+    par = np.array([4, 4, 5, 5, 6, 6, -1])
+    first = par.copy()
+    first[0] = -1
+    tc = from_parents([first] * 8 + [par] * 8, np.array([0, 0, 0, 0, 1.0, 1.5, 3.0]), range(4))
+    ll = tc.tree_sequence().ll_tree_sequence
+    W = rng.normal(size=(4, 2))
+    W[0, 0] = 0.0
+    bad = W.copy()
+    bad[0, 0] = value
+    for K in (4, 64):
+        win = np.linspace(0, 100.0, K + 1)
+        got, want = [ll.general_stat(v, summaries.trait_covariance(4), 2, win, "branch", 1, 0)
+                     for v in (bad, W)]
+        assert np.array_equal(got[:K // 2], want[:K // 2])
+        assert not np.isfinite(got[K // 2:, 0]).any()
 
 
 def test_state_plan_limits():

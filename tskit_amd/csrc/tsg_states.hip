@@ -428,10 +428,12 @@ struct RelatednessWeighted : Complement<RelatednessWeighted, 3> {  // slots: i, 
 };
 
 // A tile's events as one lane of a wave sees them: events 128 j + 2 lane and
-// the next, j < N / 2, with their weights in the window's two sums.
+// the next, j < N / 2, with their weights in the window's two sums (zero for
+// the others' events) and, bit by bit, which are the window's.
 template <int N>
 struct LaneEvents {
     double wl[N], wb[N];
+    uint32_t on;
 };
 
 // The tile of one workgroup (LDS).
@@ -448,7 +450,10 @@ struct Tile {
 #define VALUE_BOTH 1   // unpolarised, every event or pair row
 #define VALUE_MIXED 2  // site tiles with other rows
 
-template <typename T, int TILE, bool BRANCH, int VALUE, typename F, typename C2>
+// Summaries of counts are finite, so a weight of zero leaves an event out; of
+// weights (REAL) they may be infinite or NaN, and 0 x NaN would reach every
+// window of the tile.
+template <typename T, int TILE, bool BRANCH, bool REAL, int VALUE, typename F, typename C2>
 __device__ __forceinline__ void add_up(const F &f, const T *c0, const T *c1, const C2 *c2,
                                        const T *c3, const int32_t *kind, bool polarised, int lane,
                                        const LaneEvents<TILE / WAVE> &ev, double &L, double &J) {
@@ -478,6 +483,10 @@ __device__ __forceinline__ void add_up(const F &f, const T *c0, const T *c1, con
                 v0 = k.x == TSG_ROW_PAIR ? f.both(x0) : f.lone(x0);
                 v1 = k.y == TSG_ROW_PAIR ? f.both(x1) : f.lone(x1);
             }
+        }
+        if constexpr (REAL) {
+            v0 = (ev.on >> (2 * j)) & 1 ? v0 : 0.0;
+            v1 = (ev.on >> (2 * j + 1)) & 1 ? v1 : 0.0;
         }
         L = fma(v0, ev.wl[2 * j], L);
         L = fma(v1, ev.wl[2 * j + 1], L);
@@ -626,7 +635,7 @@ __device__ __forceinline__ void store_round(const double (&acc)[4], const double
 // `count` outputs of one summary over the window's events: this wave's are
 // wave, wave + 4, ...; the next round's records are read while a round is
 // summed.
-template <typename T, int TILE, bool BRANCH, int VALUE, typename Make>
+template <typename T, int TILE, bool BRANCH, bool REAL, int VALUE, typename Make>
 __device__ __forceinline__ void add_run(Make make, const TsgStateOut *outs, int count,
                                         const Tile<T> &tile, bool polarised, int wave, int lane,
                                         const LaneEvents<TILE / WAVE> &ev, bool any, double *dst) {
@@ -648,11 +657,11 @@ __device__ __forceinline__ void add_run(Make make, const TsgStateOut *outs, int 
             if (i > 0 && m0 + i * WAVES >= count) continue;
             double &L = acc[BRANCH ? 2 * i : i], &J = BRANCH ? acc[(2 * i + 1) & 3] : unused;
             if constexpr (reads_mean<F>) {
-                add_up<T, TILE, BRANCH, VALUE>(f, c0, c1, tile.mean, c3, tile.kind, polarised, lane,
-                                               ev, L, J);
+                add_up<T, TILE, BRANCH, REAL, VALUE>(f, c0, c1, tile.mean, c3, tile.kind, polarised,
+                                                     lane, ev, L, J);
             } else {
-                add_up<T, TILE, BRANCH, VALUE>(f, c0, c1, c2, c3, tile.kind, polarised, lane, ev, L,
-                                               J);
+                add_up<T, TILE, BRANCH, REAL, VALUE>(f, c0, c1, c2, c3, tile.kind, polarised, lane,
+                                                     ev, L, J);
             }
         }
         store_round<BRANCH, WAVES>(acc, scale, m0, count, lane, any, dst);
@@ -677,6 +686,7 @@ __device__ __forceinline__ void add_regressions(const TsgStateArgs &a, const Tsg
                            ? 0.0
                            : regression<TILE>(a, o, tile.cols, e, false);
             if (!pol && k == TSG_ROW_PAIR) f = f + regression<TILE>(a, o, tile.cols, e, true);
+            f = (ev.on >> r) & 1 ? f : 0.0;
             L = fma(f, ev.wl[r], L);
             if constexpr (BRANCH) J = fma(f, ev.wb[r], J);
         }
@@ -770,6 +780,7 @@ template <int TYPE, bool BRANCH, bool WIDE>
 __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
     constexpr int TILE = BRANCH ? TSG_BRANCH_TILE : TSG_SITE_TILE;
     constexpr int N = TILE / WAVE;
+    constexpr bool REAL = TYPE == TSG_ROW_F64;
     using T = typename TileType<TYPE, BRANCH, WIDE>::T;
     constexpr int STRIDE = stride_of<T>(TILE);
     extern __shared__ double smem[];
@@ -920,10 +931,12 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
             const int eb = w == w1 ? ne : lower_bound(spos, ne, win[w + 1]);
             const double wr = win[w + 1];
             LaneEvents<N> ev;
+            ev.on = 0;
 #pragma unroll
             for (int r = 0; r < N; r++) {
                 const int e = 2 * WAVE * (r / 2) + 2 * lane + (r & 1);
                 const bool on = e >= ea && e < eb;
+                if constexpr (REAL) ev.on |= (uint32_t) on << r;
                 if constexpr (BRANCH) {
                     const double b = on ? sb[e] : 0.0;
                     ev.wb[r] = b;
@@ -947,15 +960,17 @@ __device__ __forceinline__ void evaluate(const TsgStateArgs &a, int t) {
                 }
                 with_summary<TYPE>(first.stat, [&](auto make) {
                     if (!BRANCH && mixed) {
-                        add_run<T, TILE, BRANCH, VALUE_MIXED>(make, outs, count, tile,
-                                                              first.polarised != 0, wave, lane, ev,
-                                                              eb > ea, dst + m * PER);
+                        add_run<T, TILE, BRANCH, REAL, VALUE_MIXED>(
+                            make, outs, count, tile, first.polarised != 0, wave, lane, ev, eb > ea,
+                            dst + m * PER);
                     } else if (first.polarised) {
-                        add_run<T, TILE, BRANCH, VALUE_ONE>(make, outs, count, tile, true, wave,
-                                                            lane, ev, eb > ea, dst + m * PER);
+                        add_run<T, TILE, BRANCH, REAL, VALUE_ONE>(make, outs, count, tile, true,
+                                                                  wave, lane, ev, eb > ea,
+                                                                  dst + m * PER);
                     } else {
-                        add_run<T, TILE, BRANCH, VALUE_BOTH>(make, outs, count, tile, false, wave,
-                                                             lane, ev, eb > ea, dst + m * PER);
+                        add_run<T, TILE, BRANCH, REAL, VALUE_BOTH>(make, outs, count, tile, false,
+                                                                   wave, lane, ev, eb > ea,
+                                                                   dst + m * PER);
                     }
                 });
                 m += count;
