@@ -1,0 +1,152 @@
+"""The library's host code on a HIP runtime of host memory (host/
+host_runtime.cpp): which kernels a call launches, with what grids, and what it
+does where memory or threads are refused.  No kernel runs, so results are not
+looked at."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+PRELUDE = """
+import ctypes, json, sys
+sys.path[:0] = [%r, %r]
+import numpy as np
+import cases
+import tskit_amd as ta
+H = ctypes.CDLL(None)
+H.host_launches.restype = ctypes.c_char_p
+H.host_held.restype = H.host_most.restype = ctypes.c_size_t
+H.host_capacity.argtypes = [ctypes.c_size_t]
+
+def refuse(*sizes):
+    H.host_refuse((ctypes.c_size_t * len(sizes))(*sizes), len(sizes))
+
+def sizes():
+    out = (ctypes.c_size_t * 4096)()
+    return list(out[:H.host_sizes(out, 4096)])
+
+def launches():
+    rows = [r.split() for r in H.host_launches().decode().splitlines()]
+    return [(r[0], [int(v) for v in r[1:]]) for r in rows]
+
+def kernels():
+    return [k for k, _ in launches()]
+
+def on_states():
+    return any("k_state" in k or "k_genotypes" in k or "k_site_bits" in k for k in kernels())
+""" % (os.path.dirname(HERE), HERE)
+
+
+@pytest.fixture(scope="session")
+def host(tmp_path_factory):
+    """Runs a snippet in a process of its own on the host runtime; what it
+    assigns to ``out`` comes back."""
+    lib = str(tmp_path_factory.mktemp("host") / "host_runtime.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I",
+                    os.path.join(ROCM, "include"), "-o", lib,
+                    os.path.join(HERE, "host", "host_runtime.cpp"), "-ldl"], check=True)
+
+    def run(code):
+        env = dict(os.environ, LD_PRELOAD=lib, OPENBLAS_NUM_THREADS="1")
+        p = subprocess.run([sys.executable, "-c",
+                            PRELUDE + code + "\nprint('\\n' + json.dumps(out))"],
+                           env=env, capture_output=True, text=True, timeout=300)
+        assert p.returncode == 0, (p.returncode, p.stderr[-3000:])
+        return json.loads(p.stdout.splitlines()[-1])
+
+    return run
+
+
+CALLS = """
+sets = [np.arange(0, 100), np.arange(100, 300)]
+calls = {
+    "branch": lambda ts: ts.diversity(sets, mode="branch"),
+    "site": lambda ts: ts.diversity(sets, mode="site"),
+    "node": lambda ts: ts.diversity(sets, mode="node"),
+    "spectrum": lambda ts: ts.allele_frequency_spectrum([s[:5] for s in sets]),
+    "genotypes": lambda ts: ts.genotype_matrix(),
+    "matrix": lambda ts: ts.genetic_relatedness_matrix(),
+}
+tc = cases.generated(300, 3e5, 11)
+"""
+
+
+def test_plan_that_does_not_fit(host):
+    """Where the state plan, or the part of it that a call adds on its first
+    need, does not fit in device memory, the call runs on the chunk plans and
+    the resident bytes are those that are there."""
+    out = host(CALLS + """
+ts = tc.tree_sequence()
+ts.ll_tree_sequence.upload()
+plan = sizes()[-1]                       # uploaded last
+out = {"usual": {}, "refused": {}, "added": {}}
+for name, call in calls.items():
+    before = ts.ll_tree_sequence.get_device_bytes()
+    H.host_reset()
+    call(ts)
+    out["usual"][name] = on_states()
+    out["added"][name] = ts.ll_tree_sequence.get_device_bytes() - before
+ts = tc.tree_sequence()
+refuse(plan)
+ts.ll_tree_sequence.upload()
+out["held"] = [ts.ll_tree_sequence.get_device_bytes(), sum(sizes()[-2:])]
+for name, call in calls.items():
+    H.host_reset()
+    call(ts)
+    out["refused"][name] = on_states()
+for name in ("node", "spectrum", "genotypes", "matrix"):
+    refuse()
+    ts = tc.tree_sequence()
+    ts.ll_tree_sequence.upload()
+    refuse(out["added"][name] or out["added"]["genotypes"])
+    H.host_reset()
+    calls[name](ts)
+    out["refused"][name + " part"] = on_states()
+""")
+    assert all(out["usual"].values()), out
+    assert all(out["added"][k] > 0 for k in ("node", "spectrum", "genotypes")), out
+    assert not any(out["refused"].values()), out
+    assert out["held"][0] < out["held"][1] + 1024
+
+
+def test_rows_that_do_not_fit(host):
+    """Where the device holds the plans and what a call on the chunk plans
+    allocates, the call runs, whatever its rows on the state plan take."""
+    out = host(CALLS + """
+tc = cases.generated(3000, 1e6, 13)
+sets = [np.arange(100 * i, 100 * i + 100) for i in range(24)]
+calls["spectrum"] = lambda ts: ts.allele_frequency_spectrum([s[:2] for s in sets[:12]])
+out = {}
+for name, call in calls.items():
+    ts = tc.tree_sequence()
+    H.host_reset()
+    ts.ll_tree_sequence.upload()
+    plan = sizes()[-1]
+    call(ts)                             # (the parts a call adds are resident)
+    parts = ts.ll_tree_sequence.get_device_bytes()
+    del ts
+    ts = tc.tree_sequence()
+    refuse(plan)
+    H.host_reset()
+    ts.ll_tree_sequence.upload()
+    parts -= ts.ll_tree_sequence.get_device_bytes()
+    call(ts)
+    need = H.host_most()
+    del ts
+    refuse()
+    ts = tc.tree_sequence()
+    H.host_capacity(parts + need + 65536)
+    H.host_reset()
+    call(ts)
+    out[name] = kernels()
+    H.host_capacity(2 ** 64 - 1)
+    del ts
+""")
+    assert set(out) == {"branch", "site", "node", "spectrum", "genotypes", "matrix"}
+    for name, kernel in [("branch", "k_sweep"), ("site", "k_sweep"), ("matrix", "k_geno_hot")]:
+        assert any(kernel in k for k in out[name]), (name, out[name])

@@ -250,7 +250,6 @@ struct Arrays {
             block = nullptr;
             return TSG_ERR_DEVICE_MEMORY;
         }
-        held += total;
         char *const base = (char *) block;
         int ret = 0;
         if (total <= ((size_t) 4 << 20)) {
@@ -272,6 +271,7 @@ struct Arrays {
             return ret;
         }
         for (const Part &p : parts) *p.dst = base + p.off;
+        held += total;
         return 0;
     }
 };
@@ -1649,6 +1649,25 @@ int pinned_out(Workspace *ws, size_t bytes) {
     return 0;
 }
 
+// A run on the state plan whose buffers do not fit gives its own back and
+// goes to the chunk plans, which may do with less (a no-allocation run's are
+// pieces of its region).
+int state_gives_up(Workspace *ws) {
+    ws->fixed_used = 0;
+    if (ws->fixed != nullptr) return TSG_NOT_ON_STATES;
+    for (DevBuf *b : {&ws->state_x, &ws->state_wsum, &ws->state_tw, &ws->partial}) {
+        if (b->p != nullptr) (void) hipFree(b->p);
+        *b = DevBuf();
+    }
+    return TSG_NOT_ON_STATES;
+}
+
+// Whether the state plan is there to run on (not usable: see
+// tsg_build_states; not resident: it did not fit in device memory).
+bool states_resident(const tsg_treeseq *ts) {
+    return ts->states.usable && ts->states.dev.block != nullptr;
+}
+
 // Host work of a run on the state plan. TSG_NOT_ON_STATES where the plan
 // does not take it: no usable plan, a testing hook asks for another one, more
 // than 64 columns, tiles that do not fit in LDS, rows beyond
@@ -1658,7 +1677,7 @@ int pinned_out(Workspace *ws, size_t bytes) {
 int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws,
                   StateRun &r, bool many = false) {
     const tsg_stateplan &sp = ts->states;
-    if (!sp.usable || ws->force_full || ws->force_c32) return TSG_NOT_ON_STATES;
+    if (!states_resident(ts) || ws->force_full || ws->force_c32) return TSG_NOT_ON_STATES;
     r.ts = ts;
     r.ws = ws;
     r.batch.clear();
@@ -1797,10 +1816,7 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
     if (ret == 0) ret = ensure(ws, ws->raw, (size_t) raw * 8);
     if (ret == 0 && !many && !r.direct) ret = ensure(ws, ws->out, (size_t) r.outcount * 8);
     if (ret == 0) ret = by_kernel ? pk.fill(ws) : pk.send(ws, ws->stream);
-    if (ret == TSG_ERR_DEVICE_MEMORY || ret == TSG_ERR_SCRATCH_TOO_SMALL) {
-        ws->fixed_used = 0;
-        return TSG_NOT_ON_STATES;
-    }
+    if (ret == TSG_ERR_DEVICE_MEMORY || ret == TSG_ERR_SCRATCH_TOO_SMALL) return state_gives_up(ws);
     if (ret != 0) return ret;
 
     const TsgStateDevice &d = sp.dev;
@@ -1909,14 +1925,16 @@ void state_deliver(const StateRun &r) {
 int state_columns(const tsg_treeseq *ts, Workspace *ws, int K,
                   const std::vector<int32_t> &col_total, TsgStateLaunch &l) {
     const tsg_stateplan &sp = ts->states;
-    if (!sp.usable || ws->force_full || ws->force_c32 || K < 1 || K > 64) return TSG_NOT_ON_STATES;
+    if (!states_resident(ts) || ws->force_full || ws->force_c32 || K < 1 || K > 64) {
+        return TSG_NOT_ON_STATES;
+    }
     l.type = *std::max_element(col_total.begin(), col_total.begin() + K) <= 65535 ? TSG_ROW_U16
                                                                                   : TSG_ROW_I32;
     const int RW = tsg_state_row_words(K, l.type);
     const size_t rows = (size_t) sp.num_states * RW * 4;
     if (rows > TSG_STATE_ROWS_MAX) return TSG_NOT_ON_STATES;
     const int ret = ensure(ws, ws->state_x, rows);
-    if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? TSG_NOT_ON_STATES : ret;
+    if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? state_gives_up(ws) : ret;
     const TsgStateDevice &d = sp.dev;
     TsgStateArgs &a = l.a;
     a = TsgStateArgs{};
@@ -1983,16 +2001,19 @@ int state_bits(tsg_treeseq *ts, Workspace *ws, TsgGenoArgs &g) {
     const tsg_stateplan &sp = ts->states;
     const int n = ts->num_samples, RW = ((n + 31) / 32 + 3) / 4 * 4;
     const size_t rows = (size_t) sp.num_states * RW * 4;
-    if (!sp.usable || ws->force_full || rows > TSG_STATE_BITS_MAX) return TSG_NOT_ON_STATES;
+    if (!states_resident(ts) || ws->force_full || rows > TSG_STATE_BITS_MAX) {
+        return TSG_NOT_ON_STATES;
+    }
     int ret = ensure(ws->state_x, rows);
-    if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? TSG_NOT_ON_STATES : ret;
+    if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? state_gives_up(ws) : ret;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
         TsgStateDevice &h = ts->states.dev;
         if (h.bits_block == nullptr) {
             Arrays b;
             b.add(h.mut_state, sp.mut_state);
-            if ((ret = b.upload(h.bits_block, h.bytes))) return ret;
+            ret = b.upload(h.bits_block, h.bytes);
+            if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? state_gives_up(ws) : ret;
         }
     }
     TsgStateLaunch l;
@@ -2027,8 +2048,9 @@ int run_node_states(tsg_treeseq *ts, Query &q, const Fused &fz, Workspace *ws) {
     if (ret != 0) return ret;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        if ((ret = ensure_state_nodes(ts))) return ret;
+        ret = ensure_state_nodes(ts);
     }
+    if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? state_gives_up(ws) : ret;
     const int W = (int) q.windows.size() - 1;
     const int64_t N = ts->num_nodes;
     const bool composed = q.final_kind != TSG_FINAL_NONE;
@@ -2058,7 +2080,7 @@ int run_node_states(tsg_treeseq *ts, Query &q, const Fused &fz, Workspace *ws) {
     if ((ret = ensure(ws->raw, (size_t) nres * 8)) ||
         (composed && (ret = ensure(ws->out, (size_t) nout * 8))) ||
         (ret = state_send(ws, pk, a))) {
-        return ret;
+        return ret == TSG_ERR_DEVICE_MEMORY ? state_gives_up(ws) : ret;
     }
     a.npairs = (int32_t) fz.pair_s.size();
     a.pair_sample = pk.dev<const int32_t>(ws, p_ps);
@@ -2119,8 +2141,9 @@ int run_spectrum_states(tsg_treeseq *ts, const std::vector<std::vector<int32_t>>
     if (ret != 0) return ret;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        if ((ret = ensure_state_spectrum(ts))) return ret;
+        ret = ensure_state_spectrum(ts);
     }
+    if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? state_gives_up(ws) : ret;
     const int W = (int) win.size() - 1, TW = (int) tw.size() - 1;
     const int64_t hist = (int64_t) W * TW * size;
     Pack pk;
@@ -2130,7 +2153,7 @@ int run_spectrum_states(tsg_treeseq *ts, const std::vector<std::vector<int32_t>>
     if ((ret = ensure(ws->hist, (size_t) hist * 8)) ||
         (!branch && (ret = ensure(ws->out, (size_t) hist * 8))) ||
         (ret = state_send(ws, pk, a))) {
-        return ret;
+        return ret == TSG_ERR_DEVICE_MEMORY ? state_gives_up(ws) : ret;
     }
     a.npairs = (int32_t) pair_s.size();
     a.pair_sample = pk.dev<const int32_t>(ws, p_ps);
@@ -2375,7 +2398,8 @@ int device_upload(tsg_treeseq *ts) {
         b.add(h.list_ent, sp.list_ent);
         b.add(h.btile_pos, sp.btile_pos);
         b.add(h.stile_pos, sp.stile_pos);
-        if ((ret = b.upload(h.block, h.bytes))) return ret;
+        // (without it every call runs on the chunk plans)
+        if ((ret = b.upload(h.block, h.bytes)) && ret != TSG_ERR_DEVICE_MEMORY) return ret;
     }
     d.device = dev;
     return 0;
@@ -3509,48 +3533,57 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
     TsgGenoArgs g{};
     int ret_bits = state_bits(ts, ws, g);
     if (ret_bits != 0 && ret_bits != TSG_NOT_ON_STATES) return ret_bits;
-    const bool on_states = ret_bits == 0;
+    bool on_states = ret_bits == 0, full = false;
     // else genotype bitsets on the hot plan when a block of WB words per slot
     // fits in LDS (WB = 64, 32 or 16 words: a workgroup's share of samples)
-    int WB = 0;
-    if (!on_states && ts->hot.usable && !ws->force_full) {
-        for (int wb : {64, 32, 16}) {
-            if ((size_t) ts->hot.max_slots * wb * 4 <= (size_t) 48 * 1024) {
-                WB = wb;
-                break;
+    int WB = 0, slots = 0;
+    int64_t gstride = 1;
+    hipStream_t s = ws->stream;
+    auto buffers = [&]() -> int {
+        int ret;
+        if (!on_states && ts->hot.usable && !ws->force_full) {
+            for (int wb : {64, 32, 16}) {
+                if ((size_t) ts->hot.max_slots * wb * 4 <= (size_t) 48 * 1024) {
+                    WB = wb;
+                    break;
+                }
             }
         }
-    }
-    if (!on_states && WB == 0) {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        if ((ret = ensure_full(ts))) return ret;
-    }
-    hipStream_t s = ws->stream;
-    const int slots = std::min(ts->num_chunks, 512);
-    const bool full = !on_states && WB == 0;
-    const int64_t gstride = full ? (int64_t) ts->max_nloc * (1 + NW) : 1;
-    if (multi && ((ret = upload(ws->sitecol2, sitecol2, s)) || (ret = upload(ws->wk0b, wk0b, s)) ||
-                  (ret = upload(ws->wk1b, wk1b, s)) || (ret = upload(ws->row2, site_row2, s)) ||
-                  (ret = ensure(ws->gt2, (size_t) n_pad * Kp2 / 8)) ||
-                  (ret = ensure(ws->cmat2, (size_t) W * n_pad * n_pad * 4)))) {
-        return ret;
-    }
-    if ((ret = ensure(ws->gbits, (size_t) std::max<int64_t>(nrows, 1) * NW * 4)) ||
-        (ret = ensure(ws->gslab, (size_t) (full ? slots : 1) * gstride * 4)) ||
-        (ret = upload(ws->sitecol, sitecol, s)) || (ret = upload(ws->wk0, wk0, s)) ||
-        (ret = upload(ws->wk1, wk1, s)) || (ret = upload(ws->scale, scale, s)) ||
-        (ret = upload(ws->sel, sel, s)) || (ret = ensure(ws->gt, (size_t) n_pad * Kp / 8)) ||
-        (ret = ensure(ws->cmat, (size_t) W * n_pad * n_pad * 4)) ||
-        (ret = ensure(ws->rowsum, (size_t) (W * (int64_t) n + W) * 8)) ||
-        (ret = ensure(ws->kout, (size_t) W * n * (size_t) n * 8))) {
-        return ret;
-    }
-    if (!singletons) {
-        if ((ret = ensure(ws->out, (size_t) W * nsets * (size_t) nsets * 8)) ||
-            (ret = upload(ws->ipar, set_off, s))) {
+        full = !on_states && WB == 0;
+        if (full) {
+            std::lock_guard<std::mutex> lock(g_mutex);
+            if ((ret = ensure_full(ts))) return ret;
+        }
+        slots = std::min(ts->num_chunks, 512);
+        gstride = full ? (int64_t) ts->max_nloc * (1 + NW) : 1;
+        if (multi &&
+            ((ret = upload(ws->sitecol2, sitecol2, s)) || (ret = upload(ws->wk0b, wk0b, s)) ||
+             (ret = upload(ws->wk1b, wk1b, s)) || (ret = upload(ws->row2, site_row2, s)) ||
+             (ret = ensure(ws->gt2, (size_t) n_pad * Kp2 / 8)) ||
+             (ret = ensure(ws->cmat2, (size_t) W * n_pad * n_pad * 4)))) {
             return ret;
         }
+        if ((ret = ensure(ws->gbits, (size_t) std::max<int64_t>(nrows, 1) * NW * 4)) ||
+            (ret = ensure(ws->gslab, (size_t) (full ? slots : 1) * gstride * 4)) ||
+            (ret = upload(ws->sitecol, sitecol, s)) || (ret = upload(ws->wk0, wk0, s)) ||
+            (ret = upload(ws->wk1, wk1, s)) || (ret = upload(ws->scale, scale, s)) ||
+            (ret = upload(ws->sel, sel, s)) || (ret = ensure(ws->gt, (size_t) n_pad * Kp / 8)) ||
+            (ret = ensure(ws->cmat, (size_t) W * n_pad * n_pad * 4)) ||
+            (ret = ensure(ws->rowsum, (size_t) (W * (int64_t) n + W) * 8)) ||
+            (ret = ensure(ws->kout, (size_t) W * n * (size_t) n * 8))) {
+            return ret;
+        }
+        if (singletons) return 0;
+        if ((ret = ensure(ws->out, (size_t) W * nsets * (size_t) nsets * 8))) return ret;
+        return upload(ws->ipar, set_off, s);
+    };
+    ret = buffers();
+    if (ret == TSG_ERR_DEVICE_MEMORY && on_states) {  // without the states' rows
+        (void) state_gives_up(ws);
+        on_states = false;
+        ret = buffers();
     }
+    if (ret != 0) return ret;
     const TsgDevice &d = ts->dev;
     const TsgHotDevice &hd = ts->hot.dev;
     g.tree_site0 = d.tree_site0;
@@ -4131,11 +4164,17 @@ int tsg_treeseq_genotype_matrix(tsg_treeseq *ts, uint32_t options, int32_t *out)
     // (a thread per 4 cells or more: one launch's limit)
     ret = cells >> 33 != 0 ? TSG_NOT_ON_STATES : state_bits(ts, ws, g);
     if (ret != 0 && ret != TSG_NOT_ON_STATES) return ret;
-    const bool on_states = ret == 0;
+    bool on_states = ret == 0;
     // where every allele index fits, a quarter of the bytes go to the host
     hipMemoryType at;
-    const bool narrow = on_states && ts->max_alleles <= 128 && through_ring(ws, out, cells * 4, &at);
-    if ((ret = ensure(ws->geno, (cells * (narrow ? 1 : 4) + 15) / 16 * 16))) return ret;
+    bool narrow = on_states && ts->max_alleles <= 128 && through_ring(ws, out, cells * 4, &at);
+    ret = ensure(ws->geno, (cells * (narrow ? 1 : 4) + 15) / 16 * 16);
+    if (ret == TSG_ERR_DEVICE_MEMORY && on_states) {  // without the states' rows
+        (void) state_gives_up(ws);
+        on_states = narrow = false;
+        ret = ensure(ws->geno, (cells * 4 + 15) / 16 * 16);
+    }
+    if (ret != 0) return ret;
     g.geno = (int32_t *) ws->geno.p;
     const int32_t *miss_site = (const int32_t *) ws->wk0.p, *miss_sample = (const int32_t *) ws->wk1.p;
     if (on_states) {
@@ -4427,7 +4466,7 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
             taken[i] = 1;
             continue;
         }
-        if (!b->ts->states.usable) continue;
+        if (!states_resident(b->ts)) continue;
         leases.push_back(std::make_unique<Lease>(b->ts));
         if (leases.back()->ws == nullptr) return TSG_ERR_DEVICE;
         preps.push_back(Prep{i, leases.back()->ws, std::move(qs), StateRun(), 0});
