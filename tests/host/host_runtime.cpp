@@ -13,6 +13,7 @@
 #include <string.h>
 
 #include <map>
+#include <new>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -27,6 +28,7 @@ std::vector<size_t> refused;
 size_t held = 0, most = 0, capacity = SIZE_MAX;
 bool no_threads = false;
 int started = 0;
+size_t most_new = SIZE_MAX;
 }  // namespace
 
 extern "C" {
@@ -52,6 +54,7 @@ size_t host_held() { return held; }
 size_t host_most() { return most; }
 const char *host_launches() { return launches.c_str(); }  // "name x y z threads lds\n" each
 void host_no_threads(int on) { no_threads = on != 0; }
+void host_most_new(size_t n) { most_new = n; }  // larger host allocations throw
 int host_started() { return started; }
 
 // --- threads --------------------------------------------------------------------
@@ -62,6 +65,17 @@ int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), vo
     __atomic_fetch_add(&started, 1, __ATOMIC_RELAXED);
     return real(t, a, f, arg);
 }
+
+// --- memory ---------------------------------------------------------------------
+}
+void *operator new(size_t n) {
+    void *p = n <= most_new ? malloc(n ? n : 1) : nullptr;
+    if (p == nullptr) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+extern "C" {
 
 // --- the runtime ----------------------------------------------------------------
 void **__hipRegisterFatBinary(const void *) { return (void **) malloc(8); }

@@ -21,7 +21,7 @@ import tskit_amd as ta
 H = ctypes.CDLL(None)
 H.host_launches.restype = ctypes.c_char_p
 H.host_held.restype = H.host_most.restype = ctypes.c_size_t
-H.host_capacity.argtypes = [ctypes.c_size_t]
+H.host_capacity.argtypes = H.host_most_new.argtypes = [ctypes.c_size_t]
 
 def refuse(*sizes):
     H.host_refuse((ctypes.c_size_t * len(sizes))(*sizes), len(sizes))
@@ -150,3 +150,75 @@ for name, call in calls.items():
     assert set(out) == {"branch", "site", "node", "spectrum", "genotypes", "matrix"}
     for name, kernel in [("branch", "k_sweep"), ("site", "k_sweep"), ("matrix", "k_geno_hot")]:
         assert any(kernel in k for k in out[name]), (name, out[name])
+
+
+STARS = """
+def stars(n, trees):
+    rng = np.random.default_rng(2)
+    cur, since, rows = rng.integers(n, n + 2, n), np.zeros(n), []
+    for t in range(1, trees):
+        s = rng.integers(n)
+        rows.append((since[s], t, cur[s], s))
+        cur[s], since[s] = 2 * n + 1 - cur[s], t
+    rows += [(since[s], trees, cur[s], s) for s in range(n)]
+    rows += [(0, trees, n + 2, n), (0, trees, n + 2, n + 1)]
+    tc = ta.TableCollection(float(trees))
+    flags = np.zeros(n + 3, np.uint32)
+    flags[:n] = 1
+    tc.set_nodes(flags, np.concatenate([np.zeros(n), [1.0, 1.0, 2.0]]))
+    a = np.array([r for r in rows if r[0] < r[1]])
+    tc.set_edges(a[:, 0], a[:, 1], a[:, 2].astype(np.int32), a[:, 3].astype(np.int32))
+    tc.sort_edges()
+    return tc
+"""
+
+
+def test_no_more_threads(host):
+    """Where no thread can be started, the calling thread does their work: the
+    same plans, and the same launches."""
+    out = host("""
+tc = ta.simulate_tables(5000, 3e6, 1e4, 1e-8, 1e-8, 3)   # every pool is used
+plans, calls, count = [], [], []
+for none in (0, 1):
+    H.host_no_threads(none)
+    before = H.host_started()
+    H.host_reset()
+    ts = tc.tree_sequence()
+    ll = ts.ll_tree_sequence
+    plans.append([ll.get_state_plan(), ll.get_hot_plan()])
+    ts.diversity([np.arange(100)], mode="branch")
+    ts.genotype_matrix()
+    bs = []
+    for k in range(4):
+        bs.append(ts.batch())
+        bs[-1].diversity([np.arange(100 * k, 100 * k + 100)], mode="branch")
+        bs[-1].diversity([np.arange(70)] + [np.arange(k, 70 + j) for j in range(70)], mode="site")
+    ta.run_batches(bs)
+    calls.append(launches())
+    count.append(H.host_started() - before)
+same = all(np.array_equal(a[k], b[k]) for a, b in zip(*plans) for k in a)
+out = dict(same=bool(same), calls=calls[0] == calls[1], count=count)
+""")
+    assert out["same"] and out["calls"]
+    assert out["count"][0] > 8 and out["count"][1] == 0
+
+
+def test_no_more_memory(host):
+    """Where the host has no memory for the state plan the tree sequence does
+    without it; where it has none for the rest, that is an error."""
+    out = host(STARS + """
+tc = stars(200, 40000)
+E = tc.num_edges
+out = {}
+for name, most in [("plan", E * 90), ("rest", E * 8)]:
+    H.host_most_new(most)
+    try:
+        ts = tc.tree_sequence()
+        out[name] = ts.ll_tree_sequence.get_state_plan_sizes()["usable"]
+    except Exception as e:
+        out[name] = str(e)
+    H.host_most_new(2 ** 64 - 1)
+out["usual"] = tc.tree_sequence().ll_tree_sequence.get_state_plan_sizes()["usable"]
+""")
+    assert out["plan"] == 0 and out["usual"] == 1
+    assert "emory" in out["rest"]

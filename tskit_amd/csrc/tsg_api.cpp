@@ -27,7 +27,6 @@
 #include <mutex>
 #include <new>
 #include <numeric>
-#include <system_error>
 #include <thread>
 #include <unordered_set>
 #include <tuple>
@@ -37,6 +36,7 @@
 #include "tsg_launch.h"
 #include "tsg_relvec.h"
 #include "tsg_states.h"
+#include "tsg_threads.h"
 #include "tsg_treeseq.h"
 
 void tsg_build_index(const double *left, const double *right, const int32_t *parent,
@@ -764,6 +764,8 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
     std::atomic<bool> failed{false};
     std::vector<std::atomic<size_t>> done(np);  // bytes copied of each piece
     for (auto &d : done) d.store(0, std::memory_order_relaxed);
+    std::vector<std::thread> pool;
+    pool.reserve(T);
     auto size_of = [&](size_t i) { return std::min(piece, total - i * piece); };
     // A thread's part: it claims blocks, touches them while it waits, and copies
     // them in order; there(i): whether piece i has arrived.
@@ -834,11 +836,10 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
         }
         if (ret != 0) failed.store(true, std::memory_order_relaxed);
     };
-    std::vector<std::thread> pool;
     for (size_t t = 1; ret == 0 && t < T; t++) {
         try {
             pool.emplace_back(work, [&](size_t i) { return ready.load(std::memory_order_acquire) > i; });
-        } catch (const std::system_error &) {  // no more threads: fewer do the work
+        } catch (const std::exception &) {  // no more threads: fewer do the work
             break;
         }
     }
@@ -2315,10 +2316,7 @@ std::vector<uint16_t> block_sample_map(const std::vector<uint16_t> &map, int32_t
     };
     const int64_t P = std::max<int64_t>(
         1, std::min<int64_t>({(int64_t) std::thread::hardware_concurrency(), 16, nb}));
-    std::vector<std::thread> pool;
-    for (int64_t p = 1; p < P; p++) pool.emplace_back(work, nb * p / P, nb * (p + 1) / P);
-    work(0, nb / P);
-    for (auto &th : pool) th.join();
+    tsg_parallel((int) P, [&](int p) { work(nb * p / P, nb * (p + 1) / P); });
     return out;
 }
 
@@ -2743,7 +2741,7 @@ int tsg_treeseq_init(tsg_treeseq **out, double sequence_length, uint64_t num_nod
                      const int32_t *mutation_node, const int32_t *mutation_parent,
                      const char *derived_state, const uint64_t *derived_state_offset,
                      const int32_t *edge_insertion_order, const int32_t *edge_removal_order,
-                     uint32_t options) {
+                     uint32_t options) try {
     *out = nullptr;
     if (!(sequence_length > 0) || !std::isfinite(sequence_length)) return TSG_ERR_BAD_SEQUENCE_LENGTH;
     if (num_nodes > INT32_MAX || num_edges > INT32_MAX || num_sites > INT32_MAX ||
@@ -2792,18 +2790,23 @@ int tsg_treeseq_init(tsg_treeseq **out, double sequence_length, uint64_t num_nod
     if (ret != 0) return ret;
     ts->full_chunks = default_num_chunks(ts.get());
     // the state plan on a thread of its own beside the (threaded) hot plan
-    std::thread states([&]() {
+    const int chunks = default_hot_chunks(ts.get());
+    tsg_parallel(2, [&](int part) {
+        if (part == 0) {
+            ret = tsg_build_hot_plan(ts.get(), chunks, true);
+            return;
+        }
         try {
             (void) tsg_build_states(ts.get());
-        } catch (const std::bad_alloc &) {
+        } catch (const std::exception &) {  // (no memory for it: calls do without)
             ts->states = tsg_stateplan();
         }
     });
-    ret = tsg_build_hot_plan(ts.get(), default_hot_chunks(ts.get()), true);
-    states.join();
     if (ret != 0) return ret;
     *out = ts.release();
     return 0;
+} catch (const std::bad_alloc &) {
+    return TSG_ERR_NO_MEMORY;
 }
 
 int tsg_treeseq_free(tsg_treeseq *ts) {
@@ -4476,17 +4479,17 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
         auto work = [&]() {
             for (size_t p; (p = next.fetch_add(1)) < preps.size();) {
                 Prep &t = preps[p];
-                t.ret = state_prepare(bs[t.i]->ts, t.queries, t.ws, t.run, true);
+                try {
+                    t.ret = state_prepare(bs[t.i]->ts, t.queries, t.ws, t.run, true);
+                } catch (const std::bad_alloc &) {
+                    t.ret = TSG_ERR_NO_MEMORY;
+                }
                 // (arrays too large for the first kernel go over on the
                 // run's own stream)
                 if (t.ret == 0) t.ret = hip_check(hipEventRecord(t.ws->ev0, t.ws->stream));
             }
         };
-        std::vector<std::thread> pool;
-        const size_t T = std::min<size_t>(preps.size(), 8);
-        for (size_t t = 1; t < T; t++) pool.emplace_back(work);
-        work();
-        for (std::thread &th : pool) th.join();
+        tsg_parallel((int) std::min<size_t>(preps.size(), 8), [&](int) { work(); });
     }
     std::map<int, std::vector<Prep *>> byt;
     int64_t outcount = 0;
@@ -4600,15 +4603,15 @@ int run_multi(tsg_batch **bs, uint64_t n, const std::vector<char> &taken,
         auto work = [&]() {
             for (size_t i; (i = next.fetch_add(1)) < R;) {
                 Workspace *ws = run_ws[i];
-                rets[i] = batch_prepare(run_ts[i], groups[i], ws, ws->stream, runs[i]);
+                try {
+                    rets[i] = batch_prepare(run_ts[i], groups[i], ws, ws->stream, runs[i]);
+                } catch (const std::bad_alloc &) {
+                    rets[i] = TSG_ERR_NO_MEMORY;
+                }
                 if (rets[i] == 0) rets[i] = hip_check(hipEventRecord(ws->ev0, ws->stream));
             }
         };
-        std::vector<std::thread> pool;
-        const size_t T = std::min<size_t>(R, 8);
-        for (size_t t = 1; t < T; t++) pool.emplace_back(work);
-        work();
-        for (std::thread &th : pool) th.join();
+        tsg_parallel((int) std::min<size_t>(R, 8), [&](int) { work(); });
     }
     for (size_t i = 0; i < R; i++) {
         if (rets[i] != 0) return rets[i];

@@ -12,6 +12,7 @@
 #include <thread>
 
 #include "tsg_states.h"
+#include "tsg_threads.h"
 #include "tsg_treeseq.h"
 
 namespace {
@@ -81,10 +82,7 @@ template <typename F>
 void over(int64_t count, F work) {
     const int64_t P = std::max<int64_t>(
         1, std::min<int64_t>({(int64_t) std::thread::hardware_concurrency(), 8, count / 65536}));
-    std::vector<std::thread> pool;
-    for (int64_t p = 1; p < P; p++) pool.emplace_back(work, count * p / P, count * (p + 1) / P);
-    work(0, count / P);
-    for (auto &th : pool) th.join();
+    tsg_parallel((int) P, [&](int p) { work(count * p / P, count * (p + 1) / P); });
 }
 
 struct Planner {

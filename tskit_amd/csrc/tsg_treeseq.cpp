@@ -9,6 +9,7 @@
 //   samples              c/tskit/trees.c:404-453
 //   breakpoints / sites  c/tskit/trees.c:243-359
 //   allele table         c/tskit/trees.c:1525-1612 (allele order = first seen)
+#include "tsg_threads.h"
 #include "tsg_treeseq.h"
 
 #include <algorithm>
@@ -107,9 +108,7 @@ void tsg_build_index(const double *left, const double *right, const int32_t *par
         removal();
         return;
     }
-    std::thread other(removal);
-    insertion();
-    other.join();
+    tsg_parallel(2, [&](int p) { p == 0 ? insertion() : removal(); });
 }
 
 // Fills samples, breakpoints, per-tree site ranges and allele encoding, and
@@ -704,14 +703,7 @@ int build_hot_plan_bounds(tsg_treeseq *ts, std::vector<int32_t> bounds) {
     std::vector<int32_t> cb(P + 1);
     for (int32_t p = 0; p <= P; p++) cb[p] = (int32_t) ((int64_t) C * p / P);
     std::vector<HotPart> parts(P);
-    {
-        std::vector<std::thread> pool;
-        for (int32_t p = 1; p < P; p++) {
-            pool.emplace_back(plan_hot_range, ts, std::ref(hp), cb[p], cb[p + 1], std::ref(parts[p]));
-        }
-        plan_hot_range(ts, hp, cb[0], cb[1], parts[0]);
-        for (auto &th : pool) th.join();
-    }
+    tsg_parallel(P, [&](int p) { plan_hot_range(ts, hp, cb[p], cb[p + 1], parts[p]); });
     for (const HotPart &part : parts) {
         if (part.too_big) return 0;  // not representable: hp.usable stays false
     }
