@@ -222,3 +222,48 @@ out["usual"] = tc.tree_sequence().ll_tree_sequence.get_state_plan_sizes()["usabl
 """)
     assert out["plan"] == 0 and out["usual"] == 1
     assert "emory" in out["rest"]
+
+
+def test_launches_stay_below_their_limit(host):
+    """Grids of 2^32 threads or more are refused by the runtime: bit rows of
+    many sites go in several launches, a request of 17 million windows to the
+    chunk plans (which take no workgroup a window), and batches that are too
+    large together in several launches of some of them."""
+    out = host("""
+n, S, T = 60000, 2300000, 1
+tc = ta.TableCollection(1.0)
+flags = np.ones(n + 1, np.uint32)
+flags[n] = 0
+tc.set_nodes(flags, np.concatenate([np.zeros(n), [1.0]]))
+tc.set_edges(np.zeros(n), np.ones(n), np.full(n, n, np.int32), np.arange(n, dtype=np.int32))
+tc.site_position = np.arange(S) / S
+tc.ancestral_state = np.full(S, ord("0"), np.int8)
+tc.ancestral_state_offset = np.arange(S + 1, dtype=np.uint64)
+tc.mutation_site = np.arange(S, dtype=np.int32)
+tc.mutation_node = (np.arange(S) % n).astype(np.int32)
+tc.mutation_parent = np.full(S, -1, np.int32)
+tc.derived_state = np.full(S, ord("1"), np.int8)
+tc.derived_state_offset = np.arange(S + 1, dtype=np.uint64)
+ts = tc.tree_sequence()
+ts.genetic_relatedness_matrix(sample_sets=[[0], [1]])
+grids = [g for k, g in launches() if "k_site_bits" in k]
+out = dict(bits=[len(grids), sum(g[0] for g in grids) * 256 >= S * 1875])
+del ts, tc
+tc = cases.generated(300, 3e5, 11)
+ts = tc.tree_sequence()
+H.host_reset()
+W = 17000000
+ts.diversity([np.arange(100)], windows=np.linspace(0, 3e5, W + 1), mode="branch")
+out["windows"] = on_states()
+ts = [tc.tree_sequence() for _ in range(3)]
+bs = [t.batch() for t in ts]
+for b in bs:
+    b.diversity([np.arange(100)], windows=np.linspace(0, 3e5, 8000001), mode="branch")
+H.host_reset()
+ta.run_batches(bs)
+grids = [g for k, g in launches() if "k_states_windows" in k]
+out["batches"] = [len(grids), sum(g[0] for g in grids)]
+""")
+    assert out["bits"] == [3, True]
+    assert out["windows"] is False
+    assert out["batches"][0] > 1 and out["batches"][1] == 24000000

@@ -1779,7 +1779,9 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
         raw += (int64_t) t.W * t.M;
         fincount += (int64_t) t.W * q.P;
     }
-    if (wg > INT32_MAX || fg > INT32_MAX || tw > INT32_MAX / 2 || fincount > (int64_t) INT32_MAX * 128) {
+    // (one launch each; the other phases are bounded by the rows' bytes)
+    if (wg > TSG_LAUNCH_THREADS / 256 || fg > TSG_LAUNCH_THREADS / TSG_FINISH_THREADS ||
+        tw > INT32_MAX / 2 || fincount > TSG_LAUNCH_THREADS - 256) {
         return TSG_NOT_ON_STATES;
     }
     std::vector<TsgStateOut> outs;
@@ -4531,12 +4533,19 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
             args.push_back(t->run.l.a);
             if (t->ws != ws0 && (ret = hip_check(hipStreamWaitEvent(s0, t->ws->ev0, 0)))) return ret;
         }
-        pres.emplace_back();
-        if (tsg_state_prefixes(launches.back().data(), (int) launches.back().size(),
-                               pres.back()) != 0) {
-            return TSG_ERR_BAD_PARAM_VALUE;
+    }
+    // (runs too large together for one launch a phase: halves of them)
+    for (size_t g = 0; g < launches.size(); g++) {
+        std::vector<int32_t> p;
+        while (tsg_state_prefixes(launches[g].data(), (int) launches[g].size(), p) != 0) {
+            const size_t half = launches[g].size() / 2;
+            if (half == 0) return TSG_ERR_BAD_PARAM_VALUE;  // (state_prepare takes no such run)
+            launches.emplace(launches.begin() + g + 1, launches[g].begin() + half,
+                             launches[g].end());
+            launches[g].resize(half);
         }
-        pre.insert(pre.end(), pres.back().begin(), pres.back().end());
+        pre.insert(pre.end(), p.begin(), p.end());
+        pres.push_back(std::move(p));
     }
     if ((ret = upload(ws0->sargs, args, s0)) || (ret = upload(ws0->spre, pre, s0))) return ret;
     size_t aoff = 0, poff = 0;

@@ -4,6 +4,19 @@
 
 #include "tsg_kernels.h"
 
+// A launch takes fewer than 2^32 threads.
+#define TSG_LAUNCH_THREADS ((int64_t) UINT32_MAX)
+// `blocks` workgroups of 256 threads in as many launches as they need:
+// launch(first, count) each.
+template <typename F>
+hipError_t tsg_in_launches(int64_t blocks, F launch) {
+    constexpr int64_t most = (int64_t) 1 << 23;
+    for (int64_t b = 0; b < blocks; b += most) {
+        launch(b, (unsigned) (blocks - b < most ? blocks - b : most));
+    }
+    return hipGetLastError();
+}
+
 // the device's dynamic LDS limit per workgroup (set once, before launches)
 void tsg_set_lds_max(int bytes);
 int tsg_lds_max();

@@ -261,8 +261,8 @@ __global__ void __launch_bounds__(256) k_bits_seed(uint32_t *x, int RW, int64_t 
 }
 
 // Thread per (site, word): the site's bit rows from its mutations' states.
-__global__ void __launch_bounds__(256) k_site_bits(const TsgGenoArgs a) {
-    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+__global__ void __launch_bounds__(256) k_site_bits(const TsgGenoArgs a, int64_t b0) {
+    const int64_t i = (b0 + blockIdx.x) * 256 + threadIdx.x;
     const int64_t site = i / a.NW;
     if (site >= a.num_sites) return;
     const int w = (int) (i % a.NW);
@@ -672,9 +672,9 @@ hipError_t tsg_launch_bits_seed(uint32_t *x, int RW, int n, hipStream_t s) {
 
 hipError_t tsg_launch_site_bits(const TsgGenoArgs &a, hipStream_t s) {
     const int64_t threads = (int64_t) a.num_sites * a.NW;
-    if (threads == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_site_bits, dim3((unsigned) ((threads + 255) / 256)), dim3(256), 0, s, a);
-    return hipGetLastError();
+    return tsg_in_launches((threads + 255) / 256, [&](int64_t b, unsigned count) {
+        hipLaunchKernelGGL(k_site_bits, dim3(count), dim3(256), 0, s, a, b);
+    });
 }
 
 template <typename G>

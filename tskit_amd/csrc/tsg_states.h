@@ -33,8 +33,9 @@ struct tsg_treeseq;
 // conversion is paid once an event instead of once an output.
 #define TSG_STATE_F64_COLUMNS 16
 
-// outputs per workgroup of k_state_finish
+// outputs and threads per workgroup of k_state_finish
 #define TSG_FINISH_OUTPUTS 8
+#define TSG_FINISH_THREADS 1024
 
 // pieces of a node one thread adds up
 #define TSG_NODE_RUN 16
@@ -258,7 +259,8 @@ hipError_t tsg_launch_states(const TsgStateLaunch &r, hipEvent_t begin, hipEvent
 // Many runs of one row type, all of up to TSG_STATE_F64_COLUMNS columns or all
 // of more, one launch per phase: their arguments in device
 // memory, in the order of `runs`, and the block prefixes of the phases
-// (tsg_state_prefixes) on the host and in device memory.
+// (tsg_state_prefixes; -1: too many for one launch) on the host and in device
+// memory.
 int tsg_state_prefixes(const TsgStateLaunch *runs, int nrun, std::vector<int32_t> &pre);
 hipError_t tsg_launch_states_multi(const TsgStateLaunch *runs, const TsgStateArgs *args, int nrun,
                                    const std::vector<int32_t> &pre_h, const int32_t *pre,

@@ -41,7 +41,6 @@
 
 #define WAVE 64
 #define EVAL_THREADS 256
-#define FINISH_THREADS 1024
 #define SPECTRUM_SLOTS 1024
 // windows whose first events a tile keeps at a time
 #define EDGES 256
@@ -1034,14 +1033,14 @@ __device__ __forceinline__ void window_sums(const TsgStateArgs &a, int b) {
 // outputs, 128 runs: blocks of 64 outputs left one workgroup a query, 104 us
 // for 2000 windows of 64 outputs.)
 __device__ __forceinline__ void finish(const TsgStateArgs &a, int b) {
-    __shared__ double scan[FINISH_THREADS];
+    __shared__ double scan[TSG_FINISH_THREADS];
     int q = 0;
     while (q + 1 < a.Q && a.queries[q + 1].bbase <= b) q++;
     const TsgStateQuery &Q = a.queries[q];
     const double *win = a.windows + Q.win_off;
     const int tiles = Q.branch ? a.btiles : a.stiles;
     const int M = Q.M, W = Q.W, per = Q.branch ? 2 : 1;
-    const int mb = pow2_at_least(M, TSG_FINISH_OUTPUTS), S = FINISH_THREADS / mb;
+    const int mb = pow2_at_least(M, TSG_FINISH_OUTPUTS), S = TSG_FINISH_THREADS / mb;
     const int mi = threadIdx.x & (mb - 1), seg = threadIdx.x / mb;
     const int m = (b - Q.bbase) * TSG_FINISH_OUTPUTS + mi;
     const bool on = m < M;
@@ -1157,8 +1156,9 @@ __device__ __forceinline__ double state_value(const TsgStateArgs &a, const TsgSt
 // adds: a node's runs meet there in any order).  A chunk sweep added at
 // every event of a node's path: on 8000 samples, 8 sets, 347 us; this, 22 us.
 template <int TYPE>
-__global__ void __launch_bounds__(256) k_state_nodes(const TsgStateArgs a, const TsgNodeArgs g) {
-    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+__global__ void __launch_bounds__(256) k_state_nodes(const TsgStateArgs a, const TsgNodeArgs g,
+                                                     int64_t b0) {
+    const int64_t i = (b0 + blockIdx.x) * 256 + threadIdx.x;
     const TsgStateQuery &Q = a.queries[0];
     const int M = Q.M, W = Q.W;
     const int64_t r = i / M;
@@ -1351,7 +1351,7 @@ __global__ void __launch_bounds__(EVAL_THREADS) k_state_eval(const TsgStateArgs 
 __global__ void __launch_bounds__(256) k_state_windows(const TsgStateArgs a) {
     window_sums(a, blockIdx.x);
 }
-__global__ void __launch_bounds__(FINISH_THREADS) k_state_finish(const TsgStateArgs a) {
+__global__ void __launch_bounds__(TSG_FINISH_THREADS) k_state_finish(const TsgStateArgs a) {
     finish(a, blockIdx.x);
 }
 
@@ -1406,7 +1406,7 @@ __global__ void __launch_bounds__(256) k_states_windows(const TsgStateArgs *args
     const int r = run_at(pre, nrun, blockIdx.x);
     window_sums(args[r], blockIdx.x - pre[r]);
 }
-__global__ void __launch_bounds__(FINISH_THREADS) k_states_finish(const TsgStateArgs *args,
+__global__ void __launch_bounds__(TSG_FINISH_THREADS) k_states_finish(const TsgStateArgs *args,
                                                                   const int32_t *pre, int nrun) {
     const int r = run_at(pre, nrun, blockIdx.x);
     finish(args[r], blockIdx.x - pre[r]);
@@ -1498,7 +1498,7 @@ hipError_t launch_run(const TsgStateLaunch &r, hipEvent_t begin, hipEvent_t mid,
     if (r.wgroups > 0) {
         hipLaunchKernelGGL(k_state_windows, dim3((unsigned) r.wgroups), dim3(256), 0, s, a);
     }
-    hipLaunchKernelGGL(k_state_finish, dim3((unsigned) r.fgroups), dim3(FINISH_THREADS), 0, s, a);
+    hipLaunchKernelGGL(k_state_finish, dim3((unsigned) r.fgroups), dim3(TSG_FINISH_THREADS), 0, s, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (a.nfin > 0) {
         return tsg_launch_finals(a.fin, a.nfin, a.raw, a.ipar, a.dpar, a.out, a.fincount, s);
@@ -1534,14 +1534,13 @@ hipError_t tsg_launch_state_levels(const TsgStateLaunch &r, hipStream_t s) {
 
 hipError_t tsg_launch_state_nodes(const TsgStateLaunch &r, const TsgNodeArgs &g, int M,
                                   hipStream_t s) {
-    const unsigned nb = (unsigned) (((int64_t) g.runs * M + 255) / 256);
-    if (nb == 0) return hipSuccess;
-    if (r.type == TSG_ROW_U16) {
-        hipLaunchKernelGGL((k_state_nodes<TSG_ROW_U16>), dim3(nb), dim3(256), 0, s, r.a, g);
-    } else {
-        hipLaunchKernelGGL((k_state_nodes<TSG_ROW_I32>), dim3(nb), dim3(256), 0, s, r.a, g);
-    }
-    return hipGetLastError();
+    return tsg_in_launches(((int64_t) g.runs * M + 255) / 256, [&](int64_t b, unsigned count) {
+        if (r.type == TSG_ROW_U16) {
+            hipLaunchKernelGGL((k_state_nodes<TSG_ROW_U16>), dim3(count), dim3(256), 0, s, r.a, g, b);
+        } else {
+            hipLaunchKernelGGL((k_state_nodes<TSG_ROW_I32>), dim3(count), dim3(256), 0, s, r.a, g, b);
+        }
+    });
 }
 
 hipError_t tsg_launch_spectrum(const TsgStateLaunch &r, const TsgSpectrumArgs &g, bool branch,
@@ -1578,12 +1577,13 @@ hipError_t tsg_launch_states(const TsgStateLaunch &r, hipEvent_t begin, hipEvent
 int tsg_state_prefixes(const TsgStateLaunch *runs, int nrun, std::vector<int32_t> &pre) {
     const int levels = levels_of(runs, nrun);
     pre.clear();
-    auto phase = [&](auto blocks) {
+    auto phase = [&](auto blocks, int threads = 256) {
         int64_t at = 0;
         pre.push_back(0);
         for (int r = 0; r < nrun; r++) {
             at += blocks(runs[r]);
-            if (at > INT32_MAX / 2) return false;
+            // (with what rounding up to the 8 XCDs adds)
+            if ((at + 8) * threads > TSG_LAUNCH_THREADS) return false;
             pre.push_back((int32_t) at);
         }
         return true;
@@ -1595,7 +1595,7 @@ int tsg_state_prefixes(const TsgStateLaunch *runs, int nrun, std::vector<int32_t
                   return (int64_t) (r.a.Q > r.a.QB ? r.a.stiles : 0);
               }) &&
               phase([](const TsgStateLaunch &r) { return (int64_t) r.wgroups; }) &&
-              phase([](const TsgStateLaunch &r) { return (int64_t) r.fgroups; }) &&
+              phase([](const TsgStateLaunch &r) { return (int64_t) r.fgroups; }, TSG_FINISH_THREADS) &&
               phase([](const TsgStateLaunch &r) { return (r.a.fincount + 255) / 256; });
     for (int l = 1; ok && l < levels; l++) {
         ok = phase([l](const TsgStateLaunch &r) {
@@ -1656,7 +1656,7 @@ hipError_t launch_multi(const TsgStateLaunch *runs, const TsgStateArgs *args, in
         hipLaunchKernelGGL(k_states_windows, dim3(total(PH_WINDOWS)), dim3(256), 0, s, args,
                            at(PH_WINDOWS), nrun);
     }
-    hipLaunchKernelGGL(k_states_finish, dim3(total(PH_FINISH)), dim3(FINISH_THREADS), 0, s, args,
+    hipLaunchKernelGGL(k_states_finish, dim3(total(PH_FINISH)), dim3(TSG_FINISH_THREADS), 0, s, args,
                        at(PH_FINISH), nrun);
     if (total(PH_FINALS) > 0) {
         hipLaunchKernelGGL(k_states_finals, dim3(total(PH_FINALS)), dim3(256), 0, s, args,
