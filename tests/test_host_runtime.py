@@ -267,3 +267,34 @@ out["batches"] = [len(grids), sum(g[0] for g in grids)]
     assert out["bits"] == [3, True]
     assert out["windows"] is False
     assert out["batches"][0] > 1 and out["batches"][1] == 24000000
+
+
+def test_batches_of_more_columns_than_a_run(host):
+    """A batch that does not fit one run on the state plan goes there in
+    parts; the chunk sweeps take the queries that do not fit alone."""
+    out = host("""
+tc = cases.generated(300, 3e5, 11)
+def fill(widths):
+    b = tc.tree_sequence().batch()
+    for i, K in enumerate(widths):
+        sets = [np.arange(j, j + 5 + i) for j in range(K)]
+        for mode in ("branch", "site"):
+            b.diversity(sets, mode=mode)
+    return b
+out = {}
+for name, widths in [("fit", (40, 20, 30, 30)), ("one", (40, 70, 30))]:
+    H.host_reset()
+    fill(widths).run()
+    out[name] = kernels()
+    bs = [fill(widths) for _ in range(2)]
+    H.host_reset()
+    ta.run_batches(bs)
+    out[name + " together"] = kernels()
+""")
+    for name, ks in out.items():
+        many = "together" in name
+        evals = [k for k in ks if ("k_states_eval" if many else "k_state_eval") in k]
+        sweeps = [k for k in ks if "k_sweep" in k]
+        assert len(sweeps) == (2 if "one" in name else 0), (name, sweeps)
+        # two runs; together one launch a mode over all of them
+        assert len(evals) == (2 if many else 4), (name, evals)

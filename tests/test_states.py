@@ -441,6 +441,36 @@ def test_shapes_of_trees(require_gpu, name):
 
 
 @pytest.mark.gpu
+def test_company_of_more_columns_than_a_run(require_gpu):
+    """Queries of 1 to 70 columns, 250 together: the same bits alone, in a
+    batch and in several batches at once."""
+    tc = cases.generated(300, 3e5, 11)
+    ts = tc.tree_sequence()
+    win = np.linspace(0, tc.sequence_length, 8)
+    rng = np.random.default_rng(3)
+    asks = []
+    for K in (40, 1, 70, 30, 64, 5, 40):
+        sets = [np.sort(rng.choice(300, 9, replace=False)).astype(np.int32) for _ in range(K)]
+        asks += [("diversity", (sets,), dict(windows=win, mode=m)) for m in ("branch", "site")]
+    alone = [getattr(ts, name)(*a, **kw) for name, a, kw in asks]
+
+    def fill():
+        b = ts.batch()
+        return b, [getattr(b, name)(*a, **kw) for name, a, kw in asks]
+
+    for run in ("batch", "batches"):
+        print("[case]", run, flush=True)
+        made = [fill() for _ in range(1 if run == "batch" else 2)]
+        if run == "batch":
+            made[0][0].run()
+        else:
+            ta.run_batches([b for b, _ in made])
+        for _, pending in made:
+            for one, p, ask in zip(alone, pending, asks):
+                assert np.array_equal(p.result(), one), (len(ask[1][0]), ask[2]["mode"])
+
+
+@pytest.mark.gpu
 def test_more_than_16_bits(require_gpu):
     """A set of more than 65535 samples takes 32-bit counts."""
     tc = cases.generated(70000, 2e4, 5)

@@ -27,6 +27,7 @@
 #include <mutex>
 #include <new>
 #include <numeric>
+#include <set>
 #include <thread>
 #include <unordered_set>
 #include <tuple>
@@ -1540,6 +1541,7 @@ void batch_deliver(const BatchRun &r) {
 // The batch's queries of both modes in one run: one set of count rows, one
 // launch per phase (tsg_states.h).
 constexpr int TSG_NOT_ON_STATES = 1;  // not a run for the state plan
+constexpr int TSG_STATE_COLUMNS = 64;  // of one run
 
 // Device bytes of one run's count rows: beyond this the chunk sweeps, which
 // hold counts in LDS, take the run.
@@ -1668,6 +1670,10 @@ int state_gives_up(Workspace *ws) {
 bool states_resident(const tsg_treeseq *ts) {
     return ts->states.usable && ts->states.dev.block != nullptr;
 }
+// ... and no testing hook asks for another one.
+bool on_state_plan(const tsg_treeseq *ts, const Workspace *ws) {
+    return states_resident(ts) && !ws->force_full && !ws->force_c32;
+}
 
 // Host work of a run on the state plan. TSG_NOT_ON_STATES where the plan
 // does not take it: no usable plan, a testing hook asks for another one, more
@@ -1678,7 +1684,7 @@ bool states_resident(const tsg_treeseq *ts) {
 int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws,
                   StateRun &r, bool many = false) {
     const tsg_stateplan &sp = ts->states;
-    if (!states_resident(ts) || ws->force_full || ws->force_c32) return TSG_NOT_ON_STATES;
+    if (!on_state_plan(ts, ws)) return TSG_NOT_ON_STATES;
     r.ts = ts;
     r.ws = ws;
     r.batch.clear();
@@ -1693,7 +1699,7 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
     fuse_queries(r.batch, fz);
     const int K = fz.K;
     const bool wgt = fz.weighted;
-    if (K < 1 || K > 64) return TSG_NOT_ON_STATES;
+    if (K < 1 || K > TSG_STATE_COLUMNS) return TSG_NOT_ON_STATES;
     const int type = wgt ? TSG_ROW_F64
                      : *std::max_element(fz.col_total.begin(), fz.col_total.end()) <= 65535
                          ? TSG_ROW_U16
@@ -1928,9 +1934,7 @@ void state_deliver(const StateRun &r) {
 int state_columns(const tsg_treeseq *ts, Workspace *ws, int K,
                   const std::vector<int32_t> &col_total, TsgStateLaunch &l) {
     const tsg_stateplan &sp = ts->states;
-    if (!states_resident(ts) || ws->force_full || ws->force_c32 || K < 1 || K > 64) {
-        return TSG_NOT_ON_STATES;
-    }
+    if (!on_state_plan(ts, ws) || K < 1 || K > TSG_STATE_COLUMNS) return TSG_NOT_ON_STATES;
     l.type = *std::max_element(col_total.begin(), col_total.begin() + K) <= 65535 ? TSG_ROW_U16
                                                                                   : TSG_ROW_I32;
     const int RW = tsg_state_row_words(K, l.type);
@@ -2240,17 +2244,58 @@ int run_states(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *
     return 0;
 }
 
-// Runs a batch of queries (same tree sequence, same mode) in one sweep.
-int run_batch(tsg_treeseq *ts, std::vector<Query *> &batch) {
-    int ret;
-    {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        if ((ret = device_upload(ts))) return ret;
+// Queries that do not fit one run on the state plan, in parts: runs of them
+// of at most TSG_STATE_COLUMNS distinct sets, or halves where it is not the
+// columns (rows beyond TSG_STATE_ROWS_MAX).  So a query is on the state plan
+// in company wherever it is alone, and its results are the same bits.
+std::vector<std::vector<Query *>> state_parts(const std::vector<Query *> &queries) {
+    std::vector<std::vector<Query *>> parts(1);
+    std::set<std::vector<int32_t>> cols;
+    size_t own = 0;  // columns that are not shared (fuse_queries)
+    for (Query *q : queries) {
+        bool centred = false;
+        for (const Block &b : q->blocks) centred |= b.stat == TSG_STAT_RELATEDNESS;
+        std::vector<std::vector<int32_t>> add;
+        for (const std::vector<int32_t> &set : q->sets) {
+            if (centred) break;
+            add.push_back(set);
+            std::sort(add.back().begin(), add.back().end());
+        }
+        std::set<std::vector<int32_t>> both(cols);
+        both.insert(add.begin(), add.end());
+        if (centred) own += q->sets.size();
+        if (!parts.back().empty() && both.size() + own > (size_t) TSG_STATE_COLUMNS) {
+            parts.emplace_back();
+            both = std::set<std::vector<int32_t>>(add.begin(), add.end());
+            own = centred ? q->sets.size() : 0;
+        }
+        parts.back().push_back(q);
+        cols.swap(both);
     }
-    Lease lease(ts);
-    Workspace *ws = lease.ws;
-    if (ws == nullptr) return TSG_ERR_DEVICE;
-    if ((ret = run_states(ts, batch, ws)) != TSG_NOT_ON_STATES) return ret;
+    if (parts.size() > 1) return parts;
+    const auto half = queries.begin() + queries.size() / 2;
+    return {std::vector<Query *>(queries.begin(), half), std::vector<Query *>(half, queries.end())};
+}
+
+// Queries on the state plan, in parts where they need them; rest: those that
+// do not fit alone.
+int run_states_in_parts(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws,
+                        std::vector<Query *> &rest) {
+    int ret = run_states(ts, queries, ws);
+    if (ret != TSG_NOT_ON_STATES) return ret;
+    if (queries.size() < 2 || !on_state_plan(ts, ws)) {
+        rest.insert(rest.end(), queries.begin(), queries.end());
+        return 0;
+    }
+    for (const std::vector<Query *> &part : state_parts(queries)) {
+        if ((ret = run_states_in_parts(ts, part, ws, rest))) return ret;
+    }
+    return 0;
+}
+
+// A batch of queries (same tree sequence, same mode) in one chunk sweep.
+int run_sweep(tsg_treeseq *ts, std::vector<Query *> &batch, Workspace *ws) {
+    int ret;
     BatchRun r;
     if ((ret = batch_prepare(ts, batch, ws, ws->stream, r))) return ret;
     if (ws->profile) (void) hipEventRecord(ws->ev0, r.s);
@@ -2267,6 +2312,21 @@ int run_batch(tsg_treeseq *ts, std::vector<Query *> &batch) {
         ws->mode_launches[r.mode_id] += 1;
     }
     return 0;
+}
+
+// Runs a batch of queries (same tree sequence, same mode).
+int run_batch(tsg_treeseq *ts, std::vector<Query *> &batch) {
+    int ret;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        if ((ret = device_upload(ts))) return ret;
+    }
+    Lease lease(ts);
+    Workspace *ws = lease.ws;
+    if (ws == nullptr) return TSG_ERR_DEVICE;
+    std::vector<Query *> rest;
+    if ((ret = run_states_in_parts(ts, batch, ws, rest)) || rest.empty()) return ret;
+    return run_sweep(ts, rest, ws);
 }
 
 // While a batch is being filled, the validated query is handed to it
@@ -4309,23 +4369,17 @@ int run_node_queries(tsg_batch *b) {
     return 0;
 }
 
-// The branch and site queries of a batch: one fused sweep per mode.
+// The branch and site queries of a batch: both modes together on the state
+// plan, the rest in one fused sweep per mode.
 int run_fused_modes(tsg_batch *b) {
     Use use(b->ts);
-    std::vector<std::vector<Query *>> groups;
-    for (uint32_t mode : {TSG_STAT_BRANCH, TSG_STAT_SITE}) {
-        std::vector<Query *> group;
-        for (auto &q : b->queries) {
-            if (q->mode == mode) group.push_back(q.get());
-        }
-        if (!group.empty()) groups.push_back(std::move(group));
+    std::vector<Query *> all, rest;
+    for (auto &q : b->queries) {
+        if (q->mode != TSG_STAT_NODE) all.push_back(q.get());
     }
-    if (groups.empty()) return 0;
-    if (groups.size() == 1) return run_batch(b->ts, groups[0]);
+    if (all.empty()) return 0;
+    std::vector<std::vector<Query *>> groups;
     {
-        // both modes in one run on the state plan
-        std::vector<Query *> all(groups[0]);
-        all.insert(all.end(), groups[1].begin(), groups[1].end());
         int ret;
         {
             std::lock_guard<std::mutex> lock(g_mutex);
@@ -4333,21 +4387,16 @@ int run_fused_modes(tsg_batch *b) {
         }
         Lease lease(b->ts);
         if (lease.ws == nullptr) return TSG_ERR_DEVICE;
-        if ((ret = run_states(b->ts, all, lease.ws)) != TSG_NOT_ON_STATES) return ret;
-        // (more than 64 columns together, say) or the modes one by one
-        std::vector<bool> done(2, false);
-        for (int i = 0; i < 2; i++) {
-            ret = run_states(b->ts, groups[i], lease.ws);
-            if (ret == 0) {
-                done[i] = true;
-            } else if (ret != TSG_NOT_ON_STATES) {
-                return ret;
+        if ((ret = run_states_in_parts(b->ts, all, lease.ws, rest)) || rest.empty()) return ret;
+        for (uint32_t mode : {TSG_STAT_BRANCH, TSG_STAT_SITE}) {
+            std::vector<Query *> group;
+            for (Query *q : rest) {
+                if (q->mode == mode) group.push_back(q);
             }
+            if (!group.empty()) groups.push_back(std::move(group));
         }
-        if (done[0] && done[1]) return 0;
-        if (done[0] || done[1]) groups.erase(groups.begin() + (done[0] ? 0 : 1));
+        if (groups.size() == 1) return run_sweep(b->ts, groups[0], lease.ws);
     }
-    if (groups.size() == 1) return run_batch(b->ts, groups[0]);
     std::vector<std::unique_ptr<Lease>> leases;
     std::vector<BatchRun> runs;
     int ret = run_two_modes(b->ts, groups, leases, runs);
@@ -4441,14 +4490,15 @@ __attribute__((visibility("hidden"))) int tsg_batch_run_fixed(tsg_batch *b, void
 }
 
 namespace {
-// The batches of a tsg_batch_run_multi that the state plan takes: prepared in
-// parallel, then one launch per phase over all of them (per row type), every
-// run's results into one device buffer and back in one copy.  taken[i]: batch
-// i's branch and site queries are done once the leases' streams have finished.
+// The branch and site queries of a tsg_batch_run_multi that the state plan
+// takes: prepared in parallel, a batch that does not fit in parts, then one
+// launch per phase over all runs (per row type), every run's results into one
+// device buffer and back in one copy; done once the leases' streams have
+// finished.  rest[i]: batch i's others.
 int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lease>> &leases,
-                     std::deque<StateRun> &runs, std::vector<char> &taken) {
+                     std::deque<StateRun> &runs, std::vector<std::vector<Query *>> &rest) {
     int ret;
-    taken.assign(n, 0);
+    rest.assign(n, std::vector<Query *>());
     struct Prep {
         uint64_t i;
         Workspace *ws;
@@ -4467,19 +4517,20 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
         for (auto &q : b->queries) {
             if (q->mode != TSG_STAT_NODE) qs.push_back(q.get());
         }
-        if (qs.empty()) {
-            taken[i] = 1;
+        if (qs.empty()) continue;
+        if (!states_resident(b->ts)) {
+            rest[i] = std::move(qs);
             continue;
         }
-        if (!states_resident(b->ts)) continue;
         leases.push_back(std::make_unique<Lease>(b->ts));
         if (leases.back()->ws == nullptr) return TSG_ERR_DEVICE;
         preps.push_back(Prep{i, leases.back()->ws, std::move(qs), StateRun(), 0});
     }
-    {
-        std::atomic<size_t> next{0};
+    for (size_t from = 0; from < preps.size();) {
+        const size_t to = preps.size();
+        std::atomic<size_t> next{from};
         auto work = [&]() {
-            for (size_t p; (p = next.fetch_add(1)) < preps.size();) {
+            for (size_t p; (p = next.fetch_add(1)) < to;) {
                 Prep &t = preps[p];
                 try {
                     t.ret = state_prepare(bs[t.i]->ts, t.queries, t.ws, t.run, true);
@@ -4491,7 +4542,26 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
                 if (t.ret == 0) t.ret = hip_check(hipEventRecord(t.ws->ev0, t.ws->stream));
             }
         };
-        tsg_parallel((int) std::min<size_t>(preps.size(), 8), [&](int) { work(); });
+        tsg_parallel((int) std::min<size_t>(to - from, 8), [&](int) { work(); });
+        for (size_t p = from; p < to; p++) {
+            Prep &t = preps[p];
+            if (t.ret != TSG_NOT_ON_STATES) continue;
+            tsg_treeseq *ts = bs[t.i]->ts;
+            if (t.queries.size() < 2 || !on_state_plan(ts, t.ws)) {
+                rest[t.i].insert(rest[t.i].end(), t.queries.begin(), t.queries.end());
+                continue;
+            }
+            Workspace *ws = t.ws;  // the first part's; another one for each of the others
+            for (std::vector<Query *> &part : state_parts(t.queries)) {
+                if (ws == nullptr) {
+                    leases.push_back(std::make_unique<Lease>(ts));
+                    if ((ws = leases.back()->ws) == nullptr) return TSG_ERR_DEVICE;
+                }
+                preps.push_back(Prep{t.i, ws, std::move(part), StateRun(), 0});
+                ws = nullptr;
+            }
+        }
+        from = to;
     }
     std::map<int, std::vector<Prep *>> byt;
     int64_t outcount = 0;
@@ -4566,7 +4636,6 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
     for (auto &kv : byt) {
         for (Prep *t : kv.second) {
             if ((ret = state_results(t->run, t->run.l.a.out, s0))) return ret;
-            taken[t->i] = 1;
             runs.push_back(std::move(t->run));
         }
     }
@@ -4578,7 +4647,7 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
 // one sweep launch per (mode, node store, outputs per lane) on the first
 // run's stream, the rest launch on their own there; then each run finishes
 // on its own stream.
-int run_multi(tsg_batch **bs, uint64_t n, const std::vector<char> &taken,
+int run_multi(tsg_batch **bs, uint64_t n, const std::vector<std::vector<Query *>> &rest,
               std::vector<std::unique_ptr<Lease>> &leases,
               std::deque<std::vector<Query *>> &groups, std::deque<BatchRun> &runs) {
     int ret;
@@ -4586,11 +4655,10 @@ int run_multi(tsg_batch **bs, uint64_t n, const std::vector<char> &taken,
     std::vector<Workspace *> run_ws;
     for (uint64_t i = 0; i < n; i++) {
         tsg_batch *b = bs[i];
-        if (taken[i]) continue;
         for (uint32_t mode : {TSG_STAT_BRANCH, TSG_STAT_SITE}) {
             std::vector<Query *> g;
-            for (auto &q : b->queries) {
-                if (q->mode == mode) g.push_back(q.get());
+            for (Query *q : rest[i]) {
+                if (q->mode == mode) g.push_back(q);
             }
             if (g.empty()) continue;
             leases.push_back(std::make_unique<Lease>(b->ts));
@@ -4765,9 +4833,9 @@ int tsg_batch_run_multi(tsg_batch **batches, uint64_t n) {
     std::deque<std::vector<Query *>> groups;
     std::deque<BatchRun> runs;
     std::deque<StateRun> sruns;
-    std::vector<char> taken;
-    int ret = run_multi_states(batches, n, leases, sruns, taken);
-    if (ret == 0) ret = run_multi(batches, n, taken, leases, groups, runs);
+    std::vector<std::vector<Query *>> rest;
+    int ret = run_multi_states(batches, n, leases, sruns, rest);
+    if (ret == 0) ret = run_multi(batches, n, rest, leases, groups, runs);
     // the leases end (workspaces return to their pools) only once all work
     // queued on their streams has finished
     for (auto &l : leases) {

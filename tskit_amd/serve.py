@@ -20,9 +20,10 @@ launch per mode (``run_batches``).  ``one_per_launch=True, max_inflight=1``
 serves every request alone, one launch at a time: the plain path the served
 loop is measured against.
 
-Results do not depend on the company a request keeps: a fused sweep computes
-every output from its own columns in the same order as a sweep of that
-request alone.
+Results do not depend on the company a request keeps: a fused run computes
+every output from its own columns in the same order as a run of that request
+alone, and a request is on the same plan in company and alone (unless the
+device has no memory left for the run's counts).
 """
 import collections
 import concurrent.futures
