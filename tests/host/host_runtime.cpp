@@ -29,6 +29,25 @@ size_t held = 0, most = 0, capacity = SIZE_MAX;
 bool no_threads = false;
 int started = 0;
 size_t most_new = SIZE_MAX;
+int live = 0, most_live = 0;
+long waits = 0;
+bool then_fail = false;
+struct Start {
+    void *(*f)(void *);
+    void *arg;
+};
+void *run_thread(void *p) {
+    const Start s = *(Start *) p;
+    free(p);
+    {
+        std::lock_guard<std::mutex> lock(m);
+        if (++live > most_live) most_live = live;
+    }
+    void *r = s.f(s.arg);
+    std::lock_guard<std::mutex> lock(m);
+    live--;
+    return r;
+}
 }  // namespace
 
 extern "C" {
@@ -55,6 +74,9 @@ size_t host_most() { return most; }
 const char *host_launches() { return launches.c_str(); }  // "name x y z threads lds\n" each
 void host_no_threads(int on) { no_threads = on != 0; }
 void host_most_new(size_t n) { most_new = n; }  // larger host allocations throw
+int host_most_live() { return most_live; }  // threads at one time
+// the next n event queries are not ready, the others done or (fail) an error
+void host_events(long n, int fail) { waits = n, then_fail = fail != 0; }
 int host_started() { return started; }
 
 // --- threads --------------------------------------------------------------------
@@ -63,7 +85,9 @@ int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), vo
         dlsym(RTLD_NEXT, "pthread_create");
     if (no_threads) return EAGAIN;
     __atomic_fetch_add(&started, 1, __ATOMIC_RELAXED);
-    return real(t, a, f, arg);
+    Start *s = (Start *) malloc(sizeof(Start));
+    s->f = f, s->arg = arg;
+    return real(t, a, run_thread, s);
 }
 
 // --- memory ---------------------------------------------------------------------
@@ -142,7 +166,11 @@ hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuc
 hipError_t hipEventCreate(hipEvent_t *e) { return *e = (hipEvent_t) malloc(8), hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { return free(e), hipSuccess; }
-hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) {
+    std::lock_guard<std::mutex> lock(m);
+    if (waits > 0) return waits--, hipErrorNotReady;
+    return then_fail ? hipErrorUnknown : hipSuccess;
+}
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 0, hipSuccess; }
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }

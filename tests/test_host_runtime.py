@@ -298,3 +298,29 @@ for name, widths in [("fit", (40, 20, 30, 30)), ("one", (40, 70, 30))]:
         assert len(sweeps) == (2 if "one" in name else 0), (name, sweeps)
         # two runs; together one launch a mode over all of them
         assert len(evals) == (2 if many else 4), (name, evals)
+
+
+def test_large_results(host):
+    """A result that does not arrive leaves the caller's buffer as it was, and
+    calls at one time share the threads that copy their results."""
+    out = host("""
+import threading
+from tskit_amd import _lib
+tc = ta.simulate_tables(2000, 1e6, 1e4, 1e-8, 2e-8, 3)
+ts = tc.tree_sequence()
+ll, lib = ts.ll_tree_sequence, _lib.lib()
+shape = (ts.num_sites, 2000)
+got = np.full(shape, 7, np.int32)
+H.host_events(100000, 1)
+rc = lib.tsg_treeseq_genotype_matrix(ll._h, 1, got.ctypes.data)
+out = dict(bytes=got.nbytes, rc=rc, kept=bool((got == 7).all()))
+H.host_events(20000, 0)
+def call():
+    ts.genotype_matrix()
+python = [threading.Thread(target=call) for _ in range(6)]
+for t in python: t.start()
+for t in python: t.join()
+out["threads"] = H.host_most_live()
+""")
+    assert out["bytes"] > 2 ** 25 and out["rc"] != 0 and out["kept"]
+    assert out["threads"] <= 6 + 7

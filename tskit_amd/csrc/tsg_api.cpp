@@ -712,14 +712,41 @@ void widen_bytes(int32_t *o, const int8_t *v, size_t n, bool past) {
 // Bound by the host: the first touch of the caller's pages costs more than
 // the bytes.  So the threads (this one among them) claim blocks of dst in
 // turn and touch theirs before their piece is there, while the kernels still
-// run; a block is a whole huge page, since two threads that touch one at a
-// time clear it twice.  Pieces are 2 MiB at least (each costs about 12 us
+// run (dst keeps its contents until results arrive); a block is a whole huge
+// page, since two threads that touch one at a time clear it twice.  All calls
+// of the process share TSG_COPY_THREADS - 1 threads beside their own, which
+// wait for pieces by yielding.  Pieces are 2 MiB at least (each costs about 12 us
 // between two transfers) and at least 8 where there is enough of them: the
 // last one's copy is all that the transfer does not hide.
 constexpr size_t TSG_COPY_PIECE = (size_t) 4 << 20;
 constexpr int TSG_COPY_RING = 8;
 constexpr size_t TSG_COPY_THREADS = 8;
 constexpr size_t TSG_COPY_HUGE = (size_t) 2 << 20;
+
+std::atomic<int> g_copy_helpers{0};
+struct CopyHelpers {
+    int count = 0;  // of them this call's
+    explicit CopyHelpers(size_t want) {
+        int used = g_copy_helpers.load();
+        do {
+            count = (int) std::min<size_t>(want, TSG_COPY_THREADS - 1 - (size_t) used);
+        } while (!g_copy_helpers.compare_exchange_weak(used, used + count));
+    }
+    ~CopyHelpers() { g_copy_helpers -= count; }
+    CopyHelpers(const CopyHelpers &) = delete;
+    CopyHelpers &operator=(const CopyHelpers &) = delete;
+};
+
+// Faults the page of p in for writing and leaves its contents (a read first
+// would map the zero page and fault again at the write).
+void touch_page(char *p) {
+#ifdef __x86_64__
+    asm volatile("lock; orb $0, %0" : "+m"(*p));
+#else
+    volatile char *v = p;
+    *v = *v;
+#endif
+}
 
 int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t bytes,
              bool widen = false) {
@@ -753,8 +780,9 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
     // blocks of dst: to the first multiple of `block`, then whole ones; small
     // results (on small pages) in a few a thread
     const unsigned hc = std::thread::hardware_concurrency();
-    const size_t T = std::max<size_t>(
+    const size_t most = std::max<size_t>(
         1, std::min<size_t>({TSG_COPY_THREADS, hc == 0 ? 1 : hc, bytes >> 19}));
+    const CopyHelpers helpers(most - 1);
     const bool large = bytes >= 2 * TSG_COPY_THREADS * TSG_COPY_HUGE;
     const size_t block = large ? TSG_COPY_HUGE : (size_t) 128 << 10;
     const size_t head = -(uintptr_t) dst & (block - 1);
@@ -766,7 +794,7 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
     std::vector<std::atomic<size_t>> done(np);  // bytes copied of each piece
     for (auto &d : done) d.store(0, std::memory_order_relaxed);
     std::vector<std::thread> pool;
-    pool.reserve(T);
+    pool.reserve(helpers.count);
     auto size_of = [&](size_t i) { return std::min(piece, total - i * piece); };
     // A thread's part: it claims blocks, touches them while it waits, and copies
     // them in order; there(i): whether piece i has arrived.
@@ -789,8 +817,9 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
                     if (failed.load(std::memory_order_relaxed)) return;
                     if (n < HELD && more && (more = claim())) {
                         const size_t c = held[(first + n - 1) % HELD];
-                        volatile char *d = (volatile char *) dst;
-                        for (size_t q = from_of(c); q < from_of(c + 1); q += 4096) d[q] = 0;
+                        for (size_t q = from_of(c); q < from_of(c + 1); q += 4096) {
+                            touch_page((char *) dst + q);
+                        }
                     } else {
                         std::this_thread::yield();
                     }
@@ -837,7 +866,7 @@ int copy_out(Workspace *ws, hipStream_t s, void *dst, const void *src, size_t by
         }
         if (ret != 0) failed.store(true, std::memory_order_relaxed);
     };
-    for (size_t t = 1; ret == 0 && t < T; t++) {
+    for (int t = 0; ret == 0 && t < helpers.count; t++) {
         try {
             pool.emplace_back(work, [&](size_t i) { return ready.load(std::memory_order_acquire) > i; });
         } catch (const std::exception &) {  // no more threads: fewer do the work
