@@ -152,16 +152,19 @@ int tsg_treeseq_copy_state_plan(const tsg_treeseq_t *ts, int32_t *level0, int32_
     int32_t *in,
     int32_t *ev_state, double *ev_b, double *ev_pos, int32_t *row_ref, double *row_pos,
     int32_t *list_off, int32_t *list_kind, int32_t *list_ent);
-/* plan = 1: run statistics sweeps on the full plan; 2: on the hot plan with
- * 32-bit counts; 0: the library chooses (the state plan where it is usable and
- * takes the run, else the hot plan whenever its slots fit in LDS; 16-bit
- * counts when every set has <= 65535 samples) -- a testing hook */
+/* plan = 1: run statistics on the full plan; 2: on the hot plan with 32-bit
+ * counts; 3: on the hot plan with the width the library chooses; 0: the
+ * library chooses (the state plan where it is usable and takes the run, else
+ * the hot plan whenever its slots fit in LDS; 16-bit counts when every set
+ * has <= 65535 samples) -- a testing hook */
 int tsg_treeseq_set_sweep_plan(tsg_treeseq_t *ts, int plan);
-/* node store of the last statistics sweep: 0 HBM slabs, 1 LDS (full plan),
+/* node store of the last statistics run: 0 HBM slabs, 1 LDS (full plan),
  * 2 32-bit counts (LDS hot slots or rows of the state plan; also genotypes,
  * node statistics and the spectrum), 3 16-bit counts, 4 FP64 weights, -1
- * before the first sweep */
+ * before the first run */
 int tsg_treeseq_get_last_store(const tsg_treeseq_t *ts);
+/* its plan: 0 full, 1 hot, 2 state plan, -1 before the first run */
+int tsg_treeseq_get_last_plan(const tsg_treeseq_t *ts);
 /* HIP-event timing of the sweep kernel on the library's stream */
 int tsg_treeseq_set_profiling(tsg_treeseq_t *ts, int enable);
 int tsg_treeseq_get_profile(const tsg_treeseq_t *ts, double *sweep_ms, uint64_t *launches);

@@ -12,6 +12,8 @@ Tolerances (stated per statistic, the bar of the hot path):
     <= 1e-6 of the largest |value| of that output over the windows;
   * site-mode AFS: bit-exact.
 """
+import functools
+
 import numpy as np
 import pytest
 
@@ -40,10 +42,29 @@ def _check(name, got, exp):
     return err
 
 
-@pytest.fixture(scope="module")
-def small(require_gpu):
+# plans by name: the library's choice (the state plan, wherever a test does
+# not say otherwise), the chunk plans it falls back to
+PLANS = {"states": 0, "full": 1, "hot32": 2, "hot": 3}
+RAN = {"full": 0, "hot32": 1, "hot": 1, "states": 2}
+
+
+def _small(plan):
     tc = cases.generated(200, 2e5, 7)
-    return tc, tc.tree_sequence(), Oracle(tc)
+    ts = tc.tree_sequence()
+    ts.ll_tree_sequence.set_sweep_plan(PLANS[plan])
+    return tc, ts, Oracle(tc)
+
+
+@pytest.fixture(scope="module", params=["states", "hot"])
+def small(require_gpu, request):
+    """On the state plan and on the chunk sweeps it falls back to."""
+    return _small(request.param)
+
+
+@pytest.fixture(scope="module")
+def any_plan(require_gpu):
+    """For tests that choose the plan themselves."""
+    return _small("states")
 
 
 @pytest.fixture(scope="module")
@@ -171,12 +192,14 @@ def test_config1_headline(cfg1):
         _check("Fst", ts.Fst(sets, windows=w, mode=mode), fst(div, dvg, [(0, 1)])[:, 0])
 
 
+@pytest.mark.parametrize("plan", ["states", "hot"])
 @pytest.mark.parametrize("num_chunks", [1, 2, 37, 100000])
-def test_chunk_counts(require_gpu, num_chunks):
+def test_chunk_counts(require_gpu, num_chunks, plan):
     """Results do not depend on how the genome is cut into chunks."""
     tc = cases.generated(120, 1e5, 11)
     ts = tc.tree_sequence()
     ts.ll_tree_sequence.set_num_chunks(num_chunks)
+    ts.ll_tree_sequence.set_sweep_plan(PLANS[plan])
     orc = Oracle(tc)
     sets = cases.sample_sets(120, 3, 30, 5)
     w = np.linspace(0, tc.sequence_length, 7)
@@ -188,15 +211,15 @@ def test_chunk_counts(require_gpu, num_chunks):
                orc.stat("f4", sets + [sets[0]], [(0, 1, 2, 3)], w, mode)[:, 0])
 
 
-@pytest.mark.parametrize("plan", ["hot16", "hot32", "full"])
+@pytest.mark.parametrize("plan", ["states", "hot", "hot32", "full"])
 def test_node_stores(require_gpu, plan):
-    """The same statistics from the hot plan (slots in LDS, 16- or 32-bit
-    counts) and from the full plan, whose chunks are too large for LDS here
+    """The same statistics from the state plan, from the hot plan (slots in
+    LDS, 16- or 32-bit counts) and from the full plan, whose chunks are too large for LDS here
     and run from per-chunk HBM slabs."""
     tc = cases.generated(3000, 1e6, 13)
     ts = tc.tree_sequence()
     ll = ts.ll_tree_sequence
-    ll.set_sweep_plan({"hot16": 0, "full": 1, "hot32": 2}[plan])
+    ll.set_sweep_plan(PLANS[plan])
     orc = Oracle(tc)
     sets = cases.sample_sets(3000, 8, 100, 6)
     w = np.linspace(0, tc.sequence_length, 5)
@@ -205,17 +228,20 @@ def test_node_stores(require_gpu, plan):
         _say("store", plan, mode)
         _check("divergence", ts.divergence(sets, indexes=idx, windows=w, mode=mode),
                orc.stat("divergence", sets, idx, w, mode))
-        assert ll.get_last_store() == {"hot16": 3, "full": 0, "hot32": 2}[plan]
+        assert ll.get_last_store() == {"states": 3, "hot": 3, "full": 0, "hot32": 2}[plan]
+        assert ll.get_last_plan() == RAN[plan]
         _check("f4", ts.f4(sets[:4], windows=w, mode=mode),
                orc.stat("f4", sets[:4], [(0, 1, 2, 3)], w, mode)[:, 0])
 
 
+@pytest.mark.parametrize("plan", ["states", "hot"])
 @pytest.mark.parametrize("mode", ["branch", "site"])
-def test_gapped_stats(require_gpu, mode):
+def test_gapped_stats(require_gpu, mode, plan):
     """Statistics on trees with several roots and samples missing over gaps
     (nodes that lose their parent edge and regain it later)."""
     tc = cases.gapped(200, 2e5, 3)
     ts = tc.tree_sequence()
+    ts.ll_tree_sequence.set_sweep_plan(PLANS[plan])
     orc = Oracle(tc)
     sets = cases.sample_sets(200, 4, 40, 3)
     w = np.linspace(0, tc.sequence_length, 9)
@@ -326,22 +352,21 @@ def test_paper_ex_known_answers(require_gpu):
 
 
 def _afs_plan(ll, plan):
-    """1: the full plan (every node of each chunk); 0: the library's choice,
-    the hot plan here."""
-    ll.set_sweep_plan(1 if plan == "full" else 0)
+    ll.set_sweep_plan(PLANS[plan])
 
 
 def _afs_store_ok(ll, plan):
     store = ll.get_last_store()
-    assert (store == 2) if plan == "hot" else store in (0, 1)
+    assert store in (0, 1) if plan == "full" else store == 2
+    assert ll.get_last_plan() == RAN[plan]
 
 
-@pytest.mark.parametrize("plan", ["hot", "full"])
+@pytest.mark.parametrize("plan", ["states", "hot", "full"])
 @pytest.mark.parametrize("mode", ["site", "branch"])
 @pytest.mark.parametrize("nsets", [1, 2, 3])
 @pytest.mark.parametrize("polarised", [False, True])
-def test_afs(small, plan, mode, nsets, polarised):
-    tc, ts, orc = small
+def test_afs(any_plan, plan, mode, nsets, polarised):
+    tc, ts, orc = any_plan
     ll = ts.ll_tree_sequence
     sets = cases.sample_sets(200, nsets, 13, 8)
     w = np.linspace(0, tc.sequence_length, 5)
@@ -360,9 +385,9 @@ def test_afs(small, plan, mode, nsets, polarised):
         assert rel_err(got, exp, np.maximum(scale, 1e-300)) <= TOL
 
 
-@pytest.mark.parametrize("plan", ["hot", "full"])
-def test_afs_time_windows(small, plan):
-    tc, ts, orc = small
+@pytest.mark.parametrize("plan", ["states", "hot", "full"])
+def test_afs_time_windows(any_plan, plan):
+    tc, ts, orc = any_plan
     ll = ts.ll_tree_sequence
     sets = cases.sample_sets(200, 2, 20, 9)
     w = np.linspace(0, tc.sequence_length, 3)
@@ -379,7 +404,7 @@ def test_afs_time_windows(small, plan):
     assert rel_err(got, exp, scale) <= TOL
 
 
-@pytest.mark.parametrize("plan", ["hot", "full"])
+@pytest.mark.parametrize("plan", ["states", "hot", "full"])
 @pytest.mark.parametrize("polarised", [False, True])
 def test_afs_gapped(require_gpu, plan, polarised):
     """Trees with several roots and samples missing over gaps: nodes lose
@@ -426,7 +451,7 @@ def test_relatedness_matrix(require_gpu, windows):
     assert np.allclose(got, exp, rtol=1e-10, atol=1e-12 * np.max(np.abs(exp)))
 
 
-@pytest.mark.parametrize("plan", ["hot", "full"])
+@pytest.mark.parametrize("plan", ["states", "hot", "full"])
 def test_relatedness_matrix_wide(require_gpu, plan):
     """3000 samples: several workgroups per chunk split the sample bitsets
     (hot plan, 2048 samples each); the hot and full genotype sweeps give the
@@ -437,10 +462,11 @@ def test_relatedness_matrix_wide(require_gpu, plan):
     orc = Oracle(tc)
     w = np.array([0, 1.2e5, 3e5])
     _say("relatedness matrix wide", plan)
-    ll.set_sweep_plan(1 if plan == "full" else 0)
+    ll.set_sweep_plan(PLANS[plan])
     try:
         got = ts.genetic_relatedness_matrix(windows=w)
-        assert ll.get_last_store() == (2 if plan == "hot" else 0)
+        assert ll.get_last_store() == (0 if plan == "full" else 2)
+        assert ll.get_last_plan() == RAN[plan]
     finally:
         ll.set_sweep_plan(0)
     exp = orc.relatedness_matrix(w, True)
@@ -450,7 +476,8 @@ def test_relatedness_matrix_wide(require_gpu, plan):
 @pytest.mark.parametrize("case", ["paper_ex", "single_tree_ex", "nonbinary_ex", "generated",
                                   "gapped", "wide"])
 @pytest.mark.parametrize("missing", [True, False])
-def test_genotype_matrix(require_gpu, case, missing):
+@pytest.mark.parametrize("plan", ["states", "hot"])
+def test_genotype_matrix(require_gpu, case, missing, plan):
     """Device genotype decode equals the oracle's (pinned to the reference's
     tsk_variant_decode): multi-allelic sites with back and recurrent
     mutations (single_tree_ex), isolated samples as missing or ancestral
@@ -464,7 +491,8 @@ def test_genotype_matrix(require_gpu, case, missing):
     else:
         tc = getattr(cases, case)()
     ts = tc.tree_sequence()
-    _say("genotype matrix", case, missing)
+    _say("genotype matrix", case, missing, plan)
+    ts.ll_tree_sequence.set_sweep_plan(PLANS[plan])
     got = ts.genotype_matrix(isolated_as_missing=missing)
     exp = Oracle(tc).genotype_matrix(missing)
     assert got.dtype == np.int32 and np.array_equal(got, exp)
@@ -644,13 +672,15 @@ def _node_case(name):
 
 @pytest.mark.parametrize("name", ["generated", "gapped", "paper_ex", "nonbinary_ex",
                                   "single_tree_ex"])
-def test_node_mode(require_gpu, name):
+@pytest.mark.parametrize("plan", ["states", "hot"])
+def test_node_mode(require_gpu, name, plan):
     """Node statistics (trees.c:1788-1918) against the oracle, which is pinned
     to the reference's node outputs: one- and k-way summaries, polarised and
     not, span-normalised and not, several windows and none, and the composed
     Fst and Tajima's D; shapes as the reference's (windows, nodes, outputs)."""
     tc = _node_case(name)
     ts = tc.tree_sequence()
+    ts.ll_tree_sequence.set_sweep_plan(PLANS[plan])
     orc = Oracle(tc)
     n = int(np.sum(tc.node_flags & 1))
     N = tc.num_nodes
@@ -900,49 +930,57 @@ def test_relatedness_vector(require_gpu, case):
     check(got, W20, np.linspace(0, L, 4), True, True)
 
 
-@pytest.mark.parametrize("case", ["multiallelic", "single_tree_ex", "wide"])
-@pytest.mark.parametrize("plan", ["hot", "full"])
-def test_multiallelic_matrices(require_gpu, case, plan):
-    """Site divergence and relatedness matrices with back, recurrent and
-    stacked mutations (2 to 4 alleles per site): the extra allele rows go
-    into a second int8 cross product.  Against the genotype closed form on
-    the oracle's genotypes (pinned to tsk_variant_decode) and the reference's
-    tsk_treeseq_divergence_matrix when oracle/_ref is present; the
-    relatedness matrix against the reference's composition of the divergence
-    matrix (trees.py:9080-9102).  Integer cross products: rtol 1e-12."""
+@functools.lru_cache(maxsize=4)
+def _multiallelic_case(case):
+    """Tables, windows and the expected divergence of every two samples and of
+    three sets."""
     import test_oracle as to
-    from oracle import oracle as om
 
     tc = {"multiallelic": lambda: cases.multiallelic(150, 3e5, 5),
           "single_tree_ex": cases.single_tree_ex,
           "wide": lambda: cases.multiallelic(3000, 2e5, 9, every=2)}[case]()
-    ts = tc.tree_sequence()
-    ll = ts.ll_tree_sequence
     G = Oracle(tc).genotype_matrix(False)
-    n = G.shape[1]
-    L = tc.sequence_length
+    n, L = G.shape[1], tc.sequence_length
     w = np.array([0, 0.4 * L, L])
+    sets = [np.arange(0, n // 2, dtype=np.int32), np.arange(n // 2, n - 1, dtype=np.int32),
+            np.array([n - 1], np.int32)] if n >= 4 else None
+    span = np.diff(w)[:, None, None]
+    D = to._allele_divergence(G, tc.site_position, w) / span
+    of_sets = None
+    if sets is not None:
+        of_sets = to._allele_divergence(G, tc.site_position, w, [list(s) for s in sets]) / span
+    return tc, w, D, sets, of_sets
+
+
+@pytest.mark.parametrize("case", ["multiallelic", "single_tree_ex", "wide"])
+@pytest.mark.parametrize("plan", ["states", "hot", "full"])
+def test_multiallelic_matrices(require_gpu, case, plan):
+    """Site divergence and relatedness matrices with back, recurrent and
+    stacked mutations (2 to 4 alleles per site): the extra allele rows go
+    into a second cross product.  Against the genotype closed form on
+    the oracle's genotypes (pinned to tsk_variant_decode) and the reference's
+    tsk_treeseq_divergence_matrix when oracle/_ref is present; the
+    relatedness matrix against the reference's composition of the divergence
+    matrix (trees.py:9080-9102).  Integer cross products: rtol 1e-12."""
+    from oracle import oracle as om
+
+    tc, w, D, sets, of_sets = _multiallelic_case(case)
+    ts = tc.tree_sequence()
+    ll, n = ts.ll_tree_sequence, ts.num_samples
     _say("multiallelic matrices", case, plan)
-    ll.set_sweep_plan(1 if plan == "full" else 0)
-    try:
-        got = ts.divergence_matrix(windows=w)
-        exp = to._allele_divergence(G, tc.site_position, w) / np.diff(w)[:, None, None]
-        assert np.allclose(got, exp, rtol=1e-12, atol=0)
-        if om.reference_available() and n <= 300:
-            ref = om.Reference(tc).divergence_matrix(np.arange(n, dtype=np.int32), w, "site")
-            assert np.allclose(got, ref, rtol=1e-12, atol=0)
-        if n >= 4:
-            sets = [np.arange(0, n // 2, dtype=np.int32),
-                    np.arange(n // 2, n - 1, dtype=np.int32), np.array([n - 1], np.int32)]
-            got = ts.divergence_matrix(sample_sets=sets, windows=w)
-            exp = to._allele_divergence(G, tc.site_position, w, [list(s) for s in sets])
-            assert np.allclose(got, exp / np.diff(w)[:, None, None], rtol=1e-12, atol=0)
-        K = ts.genetic_relatedness_matrix(windows=w)
-        D = to._allele_divergence(G, tc.site_position, w) / np.diff(w)[:, None, None]
-        expK = np.array([_relatedness_from_divergence(D[j], np.ones(n)) for j in range(2)])
-        assert np.allclose(K, expK, rtol=1e-9, atol=1e-12 * np.max(np.abs(expK)))
-    finally:
-        ll.set_sweep_plan(0)
+    ll.set_sweep_plan(PLANS[plan])
+    got = ts.divergence_matrix(windows=w)
+    assert np.allclose(got, D, rtol=1e-12, atol=0)
+    assert ll.get_last_plan() == RAN[plan]
+    if om.reference_available() and n <= 300:
+        ref = om.Reference(tc).divergence_matrix(np.arange(n, dtype=np.int32), w, "site")
+        assert np.allclose(got, ref, rtol=1e-12, atol=0)
+    if sets is not None:
+        got = ts.divergence_matrix(sample_sets=sets, windows=w)
+        assert np.allclose(got, of_sets, rtol=1e-12, atol=0)
+    K = ts.genetic_relatedness_matrix(windows=w)
+    expK = np.array([_relatedness_from_divergence(D[j], np.ones(n)) for j in range(2)])
+    assert np.allclose(K, expK, rtol=1e-9, atol=1e-12 * np.max(np.abs(expK)))
 
 
 def test_branch_divergence_matrix_wide(require_gpu):
@@ -1021,9 +1059,10 @@ def test_autotune(require_gpu, tmp_path):
 
 
 @pytest.mark.parametrize("case", ["generated", "gapped", "multiallelic", "paper_ex"])
-def test_weighted_stats(require_gpu, case):
-    """general_stat of real-valued weights (FP64 state columns on the hot
-    plan): trait covariance, correlation and linear model, weighted genetic
+@pytest.mark.parametrize("plan", ["states", "hot"])
+def test_weighted_stats(require_gpu, case, plan):
+    """general_stat of real-valued weights (FP64 columns on the state plan
+    and on the hot plan): trait covariance, correlation and linear model, weighted genetic
     relatedness centred and not, both modes and polarisations, windows
     spanning the sequence and in pieces, one and several chunks, against the
     oracle (pinned to the compiled reference and to closed forms) and the
@@ -1057,6 +1096,7 @@ def test_weighted_stats(require_gpu, case):
     for chunks in (None, 1):
         if chunks:
             ll.set_num_chunks(chunks)
+        ll.set_sweep_plan(PLANS[plan])
         for w in [np.array([0.0, L]), np.array([0, 0.3 * L, 0.35 * L, L])]:
             for mode in ("branch", "site"):
                 for pol in (False, True):

@@ -471,6 +471,26 @@ def test_company_of_more_columns_than_a_run(require_gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("case", ["caterpillar", "columns"])
+def test_runs_the_plan_does_not_take(require_gpu, case):
+    """Trees of too many levels and queries of too many columns run on the
+    chunk sweeps."""
+    if case == "caterpillar":
+        tc, K = caterpillar(), 3
+    else:
+        tc, K = cases.generated(300, 3e5, 11), 65
+    ts, orc = tc.tree_sequence(), Oracle(tc)
+    rng = np.random.default_rng(5)
+    sets = [np.sort(rng.choice(300, 40, replace=False)).astype(np.int32) for _ in range(K)]
+    win = np.linspace(0, tc.sequence_length, 4)
+    for mode in ("branch", "site"):
+        print("[case]", case, mode, flush=True)
+        got = ts.diversity(sets, windows=win, mode=mode)
+        assert close(got, orc.stat("diversity", sets, None, win, mode)) <= TOL
+        assert ts.ll_tree_sequence.get_last_plan() == 1
+
+
+@pytest.mark.gpu
 def test_more_than_16_bits(require_gpu):
     """A set of more than 65535 samples takes 32-bit counts."""
     tc = cases.generated(70000, 2e4, 5)

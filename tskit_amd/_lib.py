@@ -69,6 +69,7 @@ SIGNATURES = {
     "tsg_treeseq_copy_state_plan": (ctypes.c_int, [c_void] + [c_void] * 11),
     "tsg_treeseq_set_sweep_plan": (ctypes.c_int, [c_void, ctypes.c_int]),
     "tsg_treeseq_get_last_store": (ctypes.c_int, [c_void]),
+    "tsg_treeseq_get_last_plan": (ctypes.c_int, [c_void]),
     "tsg_treeseq_set_profiling": (ctypes.c_int, [c_void, ctypes.c_int]),
     "tsg_treeseq_get_profile": (ctypes.c_int, [c_void, c_f64p, c_u64p]),
     "tsg_treeseq_get_profile_modes": (ctypes.c_int, [c_void, c_f64p, c_u64p]),

@@ -48,6 +48,9 @@ int tsg_init_trees(tsg_treeseq *ts, const char *ancestral_state,
 
 namespace {
 
+// plans of the last run
+constexpr int TSG_PLAN_FULL = 0, TSG_PLAN_HOT = 1, TSG_PLAN_STATES = 2;
+
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
@@ -97,7 +100,13 @@ struct Workspace {
     int lds_limit = 65536;          // dynamic LDS a sweep workgroup may use
     bool force_full = false;        // run sweeps on the full plan (testing hook)
     bool force_c32 = false;         // hot plan with 32-bit counts (testing hook)
-    int last_store = -1;            // node store of the last sweep (TSG_STORE_*)
+    bool force_hot = false;         // hot plan, not the state plan (testing hook)
+    int last_store = -1;            // node store of the last run (TSG_STORE_*)
+    int last_plan = -1;             // and its plan (TSG_PLAN_*)
+    void ran(int store, int plan) {
+        last_store = store;
+        last_plan = plan;
+    }
     // profiling of the dominant (sweep) kernel
     bool profile = false;
     double sweep_ms = 0;
@@ -113,8 +122,8 @@ struct Workspace {
 struct Resident {
     std::vector<Workspace *> all, idle;
     int lds_limit = 65536;
-    bool force_full = false, force_c32 = false, profile = false;
-    int last_store = -1;
+    bool force_full = false, force_c32 = false, force_hot = false, profile = false;
+    int last_store = -1, last_plan = -1;
 };
 
 // Guards device residency (uploads, plan builds), the workspace pools and
@@ -308,7 +317,8 @@ struct Lease {
         res->idle.pop_back();
         ws->force_full = res->force_full;
         ws->force_c32 = res->force_c32;
-        ws->last_store = -1;
+        ws->force_hot = res->force_hot;
+        ws->ran(-1, -1);
     }
     ~Lease() {
         if (ws == nullptr) return;
@@ -316,7 +326,10 @@ struct Lease {
         // next lease must find the stream (and its staging buffers) idle
         (void) hipStreamSynchronize(ws->stream);
         std::lock_guard<std::mutex> lock(g_mutex);
-        if (ws->last_store >= 0) res->last_store = ws->last_store;
+        if (ws->last_store >= 0) {
+            res->last_store = ws->last_store;
+            res->last_plan = ws->last_plan;
+        }
         res->idle.push_back(ws);
     }
     Lease(const Lease &) = delete;
@@ -1329,7 +1342,8 @@ int batch_prepare(tsg_treeseq *ts, std::vector<Query *> &batch, Workspace *ws, h
         a.ev_bl = d.ev_bl;
         a.mut_node = d.mut_node;
     }
-    ws->last_store = store;
+    ws->ran(store, store == TSG_STORE_GLOBAL || store == TSG_STORE_LDS ? TSG_PLAN_FULL
+                                                                       : TSG_PLAN_HOT);
     a.bp = d.breakpoints;
     a.tree_site0 = d.tree_site0;
     a.site_pos = d.site_pos;
@@ -1701,7 +1715,7 @@ bool states_resident(const tsg_treeseq *ts) {
 }
 // ... and no testing hook asks for another one.
 bool on_state_plan(const tsg_treeseq *ts, const Workspace *ws) {
-    return states_resident(ts) && !ws->force_full && !ws->force_c32;
+    return states_resident(ts) && !ws->force_full && !ws->force_c32 && !ws->force_hot;
 }
 
 // Host work of a run on the state plan. TSG_NOT_ON_STATES where the plan
@@ -1917,9 +1931,10 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
     r.l.levels = (int) sp.level0.size() - 1;
     r.l.wgroups = (int) wg;
     r.l.fgroups = (int) fg;
-    ws->last_store = type == TSG_ROW_U16 ? TSG_STORE_HOT16
-                     : type == TSG_ROW_I32 ? TSG_STORE_HOT
-                                           : TSG_STORE_HOTW;
+    ws->ran(type == TSG_ROW_U16   ? TSG_STORE_HOT16
+            : type == TSG_ROW_I32 ? TSG_STORE_HOT
+                                  : TSG_STORE_HOTW,
+            TSG_PLAN_STATES);
     return 0;
 }
 
@@ -2037,9 +2052,7 @@ int state_bits(tsg_treeseq *ts, Workspace *ws, TsgGenoArgs &g) {
     const tsg_stateplan &sp = ts->states;
     const int n = ts->num_samples, RW = ((n + 31) / 32 + 3) / 4 * 4;
     const size_t rows = (size_t) sp.num_states * RW * 4;
-    if (!states_resident(ts) || ws->force_full || rows > TSG_STATE_BITS_MAX) {
-        return TSG_NOT_ON_STATES;
-    }
+    if (!on_state_plan(ts, ws) || rows > TSG_STATE_BITS_MAX) return TSG_NOT_ON_STATES;
     int ret = ensure(ws->state_x, rows);
     if (ret != 0) return ret == TSG_ERR_DEVICE_MEMORY ? state_gives_up(ws) : ret;
     {
@@ -2071,7 +2084,7 @@ int state_bits(tsg_treeseq *ts, Workspace *ws, TsgGenoArgs &g) {
     g.RW = RW;
     g.num_sites = ts->num_sites;
     g.mut_node = sp.dev.mut_state;
-    ws->last_store = TSG_STORE_HOT;
+    ws->ran(TSG_STORE_HOT, TSG_PLAN_STATES);
     return 0;
 }
 
@@ -2145,7 +2158,7 @@ int run_node_states(tsg_treeseq *ts, Query &q, const Fused &fz, Workspace *ws) {
                          pk.dev<const double>(ws, p_dp), (double *) ws->out.p, nout, s)))) {
         return ret;
     }
-    ws->last_store = TSG_STORE_HOT;
+    ws->ran(TSG_STORE_HOT, TSG_PLAN_STATES);
     if ((ret = copy_out(ws, s, q.result, composed ? ws->out.p : ws->raw.p, (size_t) nout * 8))) {
         return ret;
     }
@@ -2226,7 +2239,7 @@ int run_spectrum_states(tsg_treeseq *ts, const std::vector<std::vector<int32_t>>
         ret = hip_check(tsg_launch_afs_site_final(g.hist_u, (double *) ws->out.p, g.windows, W,
                                                   size, flags, s));
     }
-    ws->last_store = TSG_STORE_HOT;
+    ws->ran(TSG_STORE_HOT, TSG_PLAN_STATES);
     if (ret == 0) ret = copy_out(ws, s, result, branch ? ws->hist.p : ws->out.p, (size_t) hist * 8);
     if (ret == 0 && ws->profile) {
         float ms = 0;
@@ -2641,7 +2654,7 @@ int run_node(tsg_treeseq *ts, Query &q) {
         return ret;
     }
     if (ws->profile) (void) hipEventRecord(ws->ev1, s);
-    ws->last_store = TSG_STORE_HOT;
+    ws->ran(TSG_STORE_HOT, TSG_PLAN_HOT);
     const uint32_t fflags = q.span_normalise ? TSG_F_SPAN_NORMALISE : 0u;
     if ((ret = hip_check(tsg_launch_afs_branch_final(raw, a.windows, W, N * M, fflags, s)))) {
         return ret;
@@ -2929,10 +2942,11 @@ int tsg_treeseq_set_num_chunks(tsg_treeseq *ts, uint32_t num_chunks) {
     return ret;
 }
 
-// Testing hook: plan = 1 runs every sweep on the full plan, 2 on the hot
-// plan with 32-bit counts, 0 lets the library choose (the hot plan whenever
-// its slots fit in LDS, with 16-bit counts when every set has <= 65535
-// samples).
+// Testing hook: plan = 1 runs on the full plan, 2 on the hot plan with 32-bit
+// counts, 3 on the hot plan with the counts' width by the library (16 bits
+// when every set has <= 65535 samples), 0 lets the library choose (the state
+// plan where it takes the run, else the hot plan whenever its slots fit in
+// LDS).
 int tsg_treeseq_set_sweep_plan(tsg_treeseq *ts, int plan) {
     Use use(ts);
     std::lock_guard<std::mutex> lock(g_mutex);
@@ -2940,16 +2954,23 @@ int tsg_treeseq_set_sweep_plan(tsg_treeseq *ts, int plan) {
     if (ret != 0) return ret;
     res_of(ts)->force_full = plan == 1;
     res_of(ts)->force_c32 = plan == 2;
+    res_of(ts)->force_hot = plan == 3;
     return 0;
 }
 
-// Node store of the last statistics sweep: 0 HBM slabs (full plan), 1 LDS
-// (full plan), 2 LDS hot slots, 3 LDS hot slots with 16-bit counts; -1
-// before the first sweep.
+// Node store of the last run: 0 HBM slabs, 1 LDS (full plan), 2 32-bit
+// counts, 3 16-bit counts, 4 FP64 weights; -1 before the first.
 int tsg_treeseq_get_last_store(const tsg_treeseq *ts) {
     std::lock_guard<std::mutex> lock(g_mutex);
     const Resident *res = res_of(ts);
     return res == nullptr ? -1 : res->last_store;
+}
+
+// Its plan: 0 full, 1 hot, 2 state plan.
+int tsg_treeseq_get_last_plan(const tsg_treeseq *ts) {
+    std::lock_guard<std::mutex> lock(g_mutex);
+    const Resident *res = res_of(ts);
+    return res == nullptr ? -1 : res->last_plan;
 }
 
 int tsg_treeseq_upload(tsg_treeseq *ts) {
@@ -3703,7 +3724,7 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
         g.sample_slot = hd.sample_slot;
         g.num_chunks = ts->hot.num_chunks;
         g.WB = WB;
-        ws->last_store = TSG_STORE_HOT;
+        ws->ran(TSG_STORE_HOT, TSG_PLAN_HOT);
     } else if (full) {
         g.chunk_tree0 = d.chunk_tree0;
         g.chunk_node0 = d.chunk_node0;
@@ -3717,7 +3738,7 @@ static int site_gram_matrix(tsg_treeseq *ts, uint64_t num_sample_sets,
         g.slots = slots;
         g.g_rec = (uint32_t *) ws->gslab.p;
         g.g_stride = gstride;
-        ws->last_store = TSG_STORE_GLOBAL;
+        ws->ran(TSG_STORE_GLOBAL, TSG_PLAN_FULL);
     }
     if (ws->profile) (void) hipEventRecord(ws->ev0, s);
     if ((ret = hip_check(on_states ? tsg_launch_site_bits(g, s)
@@ -4291,7 +4312,7 @@ int tsg_treeseq_genotype_matrix(tsg_treeseq *ts, uint32_t options, int32_t *out)
         g.sample_slot = hd.sample_slot;
         g.num_chunks = ts->hot.num_chunks;
         g.WB = WB;
-        ws->last_store = TSG_STORE_HOT;
+        ws->ran(TSG_STORE_HOT, TSG_PLAN_HOT);
         if ((ret = hip_check(tsg_launch_genotypes(g, (size_t) ts->hot.max_slots * WB * 4, miss_site,
                                                   miss_sample, (int64_t) ms.size(), s)))) {
             return ret;
@@ -4486,6 +4507,7 @@ __attribute__((visibility("hidden"))) int tsg_batch_run_fixed(tsg_batch *b, void
         w.lds_limit = res->lds_limit;
         w.force_c32 = res->force_c32;
         w.force_full = res->force_full;
+        w.force_hot = res->force_hot;
     }
     w.fixed = (char *) scratch;
     w.fixed_cap = cap;
@@ -5035,7 +5057,7 @@ int tsg_treeseq_allele_frequency_spectrum(tsg_treeseq *ts, uint64_t K, const uin
         a.slot_tp0 = h.slot_tp0;
         a.slot_last0 = h.slot_last0;
         a.slot_ins0 = h.slot_ins0;
-        ws->last_store = TSG_STORE_HOT;
+        ws->ran(TSG_STORE_HOT, TSG_PLAN_HOT);
     } else {
         std::vector<int32_t> cq_wfirst(C), cq_nwin(C);
         std::vector<int64_t> cq_poff(C, 0);
@@ -5076,7 +5098,7 @@ int tsg_treeseq_allele_frequency_spectrum(tsg_treeseq *ts, uint64_t K, const uin
         a.g_stride = (int64_t) ts->max_nloc * R;
         a.g_last = (double *) ws->last.p;
         a.g_last_stride = ts->max_nloc;
-        ws->last_store = lds ? TSG_STORE_LDS : TSG_STORE_GLOBAL;
+        ws->ran(lds ? TSG_STORE_LDS : TSG_STORE_GLOBAL, TSG_PLAN_FULL);
     }
     a.bp = d.breakpoints;
     a.tree_site0 = d.tree_site0;

@@ -286,14 +286,18 @@ class LowLevelTreeSequence:
         return dict(z, **out)
 
     def set_sweep_plan(self, plan):
-        """1: run statistics sweeps on the full plan; 2: on the hot plan with
-        32-bit counts; 0: the library chooses."""
+        """1: run statistics on the full plan; 2: on the hot plan with 32-bit
+        counts; 3: on the hot plan; 0: the library chooses."""
         check(self._lib.tsg_treeseq_set_sweep_plan(self._h, int(plan)))
 
     def get_last_store(self):
-        """Node store of the last sweep: 0 HBM slabs, 1 LDS full plan, 2 LDS hot
-        slots, 3 LDS hot slots with 16-bit counts."""
+        """Node store of the last run: 0 HBM slabs, 1 LDS full plan, 2 32-bit
+        counts, 3 16-bit counts, 4 FP64 weights."""
         return int(self._lib.tsg_treeseq_get_last_store(self._h))
+
+    def get_last_plan(self):
+        """Plan of the last run: 0 full, 1 hot, 2 state plan."""
+        return int(self._lib.tsg_treeseq_get_last_plan(self._h))
 
     def set_num_chunks(self, num_chunks):
         check(self._lib.tsg_treeseq_set_num_chunks(self._h, int(num_chunks)))
