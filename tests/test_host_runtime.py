@@ -324,3 +324,37 @@ out["threads"] = H.host_most_live()
 """)
     assert out["bytes"] > 2 ** 25 and out["rc"] != 0 and out["kept"]
     assert out["threads"] <= 6 + 7
+
+
+def test_tuning_the_chunks(host):
+    """The tuner times the chunk sweeps, and a change of the chunk count
+    leaves the state plan where it is."""
+    out = host(CALLS + """
+from tskit_amd import autotune
+ts = tc.tree_sequence()
+ll = ts.ll_tree_sequence
+ll.upload()
+plan = sizes()[-1]
+H.host_reset()
+got = autotune.tune(ts, candidates=(64, 256), reps=1, table={})
+out = dict(states=on_states(), sweeps=sum("k_sweep" in k for k in kernels()))
+b = [t.batch() for t in (ts, ts)]
+def run():
+    b = [ts.batch() for _ in range(2)]
+    for x in b:
+        x.diversity(sets, mode="branch")
+    ta.run_batches(b)
+import types
+sys.modules["torch"] = types.SimpleNamespace(cuda=types.SimpleNamespace(synchronize=lambda: None))
+H.host_reset()
+autotune.tune_batch([ts], run, candidates=(64, 256), reps=1)
+ks = kernels()
+out["joint"] = [sum("k_sweep" in k for k in ks), sum("k_states_eval" in k for k in ks)]
+out["sent"] = plan in sizes()
+H.host_reset()
+ts.diversity(sets, mode="branch")
+out["after"] = on_states()
+""")
+    assert out["sweeps"] == 4 and not out["states"]
+    assert out["joint"] == [4, 1]  # (the last run warms the usual plan)
+    assert out["after"] and not out["sent"]

@@ -1,5 +1,10 @@
 """Chunk-count autotuner for the sweep kernels.
 
+Statistics run on the state plan, which has no chunks; the chunk sweeps take
+what it does not (queries of more than 64 sample sets, very deep trees, runs
+whose counts do not fit in device memory), and the relatedness vector.  The
+tuner times the chunk sweeps themselves, whatever the state plan would take.
+
 The sweep cuts a tree sequence's trees into chunks, one wavefront each; a
 chunk is a serial chain of edge events, so more, shorter chunks run faster
 as long as their hot slots stay small enough for several chunks per CU.
@@ -19,6 +24,7 @@ import os
 import numpy as np
 
 CANDIDATES = (32, 64, 128, 256, 512)  # edge events per chunk
+HOT = 3  # the sweep plan of the chunk sweeps (set_num_chunks goes back to the usual one)
 
 
 def cache_path():
@@ -94,6 +100,7 @@ def tune(ts, candidates=CANDIDATES, reps=3, path=None, table=None):
     times = {}
     for epc in candidates:
         ts.ll_tree_sequence.set_num_chunks(chunks_for(ts, epc))
+        ts.ll_tree_sequence.set_sweep_plan(HOT)
         times[epc] = _probe(ts, reps)
     best = min(times, key=times.get)
     ts.ll_tree_sequence.set_num_chunks(chunks_for(ts, best))
@@ -121,7 +128,7 @@ def tune_batch(tss, run, candidates=CANDIDATES, reps=2):
     for epc in candidates:
         for ts in tss:
             ts.ll_tree_sequence.set_num_chunks(chunks_for(ts, epc))
-            ts.ll_tree_sequence.upload()
+            ts.ll_tree_sequence.set_sweep_plan(HOT)
         run()  # warm the workspaces at this plan
         torch.cuda.synchronize()
         best = float("inf")

@@ -2484,9 +2484,14 @@ int device_upload(tsg_treeseq *ts) {
         b.add(h.t0_bl, hp.t0_bl);
         if ((ret = b.upload(h.block, h.bytes))) return ret;
     }
+    // (on another device after tsg_treeseq_set_num_chunks: there)
+    if (ts->states.dev.block != nullptr && ts->states.dev.device != dev) {
+        tsg_state_device_free(&ts->states.dev);
+    }
     if (ts->states.usable && ts->states.dev.block == nullptr) {
         const tsg_stateplan &sp = ts->states;
         TsgStateDevice &h = ts->states.dev;
+        h.device = dev;
         Arrays b;
         if (!sp.order.empty()) b.add(h.order, sp.order);
         b.add(h.in, sp.in);
@@ -2927,14 +2932,14 @@ int tsg_treeseq_free(tsg_treeseq *ts) {
 }
 
 // Rebuilds the chunk plans with a given chunk count (autotuner hook); the
-// full plan is rebuilt on its next use.
+// full plan is rebuilt on its next use.  The state plan, which has no chunks,
+// stays where it is.
 int tsg_treeseq_set_num_chunks(tsg_treeseq *ts, uint32_t num_chunks) {
     if (ts == nullptr || num_chunks == 0) return TSG_ERR_BAD_PARAM_VALUE;
     std::unique_lock<std::mutex> lock = exclusive(ts);
     free_workspace(ts);
     tsg_device_free(&ts->dev);
     tsg_hot_device_free(&ts->hot.dev);
-    tsg_state_device_free(&ts->states.dev);
     ts->full_chunks = (int32_t) std::min<uint32_t>(num_chunks, INT32_MAX);
     ts->full_built = false;
     const int ret = tsg_build_hot_plan(ts, ts->full_chunks, false);

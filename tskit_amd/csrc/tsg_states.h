@@ -66,6 +66,7 @@ struct TsgNodeRuns {
 };
 
 struct TsgStateDevice {
+    int device = -1;
     // allocations: the plan, and what node statistics, the allele frequency
     // spectrum and genotypes add on first use
     void *block = nullptr, *nodes_block = nullptr, *afs_block = nullptr, *bits_block = nullptr;
