@@ -358,3 +358,50 @@ out["after"] = on_states()
     assert out["sweeps"] == 4 and not out["states"]
     assert out["joint"] == [4, 1]  # (the last run warms the usual plan)
     assert out["after"] and not out["sent"]
+
+
+def test_serving_estimates_cover_what_a_launch_allocates(host):
+    """The admission's estimate of a launch, on the state plan and on the
+    chunk plans, is at least what the launch allocates and within a few times
+    of it where that is large."""
+    out = host("""
+from tskit_amd import serve
+tc = cases.generated(3000, 1e6, 13)
+rng = np.random.default_rng(1)
+def sets(k, size=60):
+    return [rng.choice(3000, size, replace=False) for _ in range(k)]
+pairs = [(i, i + 1) for i in range(9)]
+w = np.linspace(0, 1e6, 41)
+launches_ = {
+    "one": [("diversity", dict(sample_sets=sets(1), mode="site"))],
+    "wide": [("diversity", dict(sample_sets=sets(64), mode="branch", windows=np.linspace(0, 1e6, 2001)))],
+    "mixed": [("Fst", dict(sample_sets=sets(10), indexes=pairs, windows=w, mode="branch")),
+              ("Tajimas_D", dict(sample_sets=sets(12), windows=w, mode="branch")),
+              ("f4", dict(sample_sets=sets(4), indexes=[(0, 1, 2, 3)], windows=w, mode="branch")),
+              ("genetic_relatedness", dict(sample_sets=sets(7), indexes=[(0, 1)], windows=w,
+                                           mode="branch"))],
+    "site": [("divergence", dict(sample_sets=sets(10), indexes=pairs, windows=w, mode="site"))
+             for _ in range(5)],
+    "columns": [("diversity", dict(sample_sets=sets(70), windows=w, mode="site")),
+                ("diversity", dict(sample_sets=sets(30), windows=w, mode="site")),
+                ("diversity", dict(sample_sets=sets(50), windows=w, mode="site"))],
+    "node": [("diversity", dict(sample_sets=sets(3), mode="node"))],
+    "spectrum": [("allele_frequency_spectrum", dict(sample_sets=sets(2, 40), windows=w))],
+}
+out = {}
+for name, asks in launches_.items():
+    ts = tc.tree_sequence()
+    srv = serve.StatServer([ts], max_inflight=1, memory_budget=1 << 40)
+    reqs = [serve.Request(i, 0, stat, kw) for i, (stat, kw) in enumerate(asks)]
+    for r in reqs:
+        r.normalise(ts)
+    resident, before = ts.ll_tree_sequence.get_device_bytes(), H.host_held()
+    H.host_reset()
+    srv._run([reqs])
+    assert all(r.error is None for r in reqs), reqs[0].error
+    parts = ts.ll_tree_sequence.get_device_bytes() - resident
+    out[name] = [H.host_most() - before - parts, srv.job_bytes([reqs])]
+""")
+    for name, (held, estimate) in out.items():
+        assert held <= estimate, (name, held, estimate)
+        assert estimate <= 3 * held + (1 << 20), (name, held, estimate)

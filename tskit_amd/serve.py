@@ -40,7 +40,7 @@ class Request:
     sequence ``ts_id``."""
 
     __slots__ = ("rid", "ts_id", "stat", "kwargs", "t_arrival", "t_start", "t_done", "result",
-                 "error", "launch", "sets")
+                 "error", "launch", "sets", "keys")
 
     def __init__(self, rid, ts_id, stat, kwargs, t_arrival=0.0):
         self.rid = rid
@@ -54,6 +54,7 @@ class Request:
         self.error = None  # the exception the request's launch raised, if any
         self.launch = None
         self.sets = None   # the sample sets as a list of arrays (set on submit)
+        self.keys = None   # and their identities: the sorted samples, as bytes (hashed in C)
 
     @property
     def mode(self):
@@ -68,6 +69,7 @@ class Request:
         elif len(sets) > 0 and np.ndim(sets[0]) == 0:
             sets = [sets]
         self.sets = [np.asarray(x, dtype=np.int64) for x in sets]
+        self.keys = {np.sort(s).tobytes() for s in self.sets}
 
     def shape(self):
         """(sample sets, outputs, windows) of the request."""
@@ -86,11 +88,85 @@ class Request:
 
 
 def launch_bytes(k, m, nw, chunks, samples=0):
-    """Device bytes one fused launch needs for a query of m outputs over nw
-    windows on a plan of `chunks` chunks: window partials (chunks + windows)
-    x m, the combined result and finals, the per-chunk branch sums, and the
-    (sample, column) seeds and per-(chunk, query) window tables."""
+    """Device bytes a fused launch needs on the chunk plans for a query of m
+    outputs over nw windows, on a plan of `chunks` chunks: window partials
+    (chunks + windows) x m, the combined result and finals, the per-chunk
+    branch sums, and the (sample, column) seeds and per-(chunk, query) window
+    tables."""
     return 8 * m * (3 * chunks + 3 * nw) + 64 * k + 16 * samples + 16 * chunks
+
+
+RUN_COLUMNS = 64  # sample sets of one run on the state plan
+
+
+def rows_bytes(plan, columns, wide):
+    """Device bytes of a launch's count rows on the state plan: a row a state,
+    16 bits a column (32 where a set has more than 65535 samples) in whole 4,
+    8 or 16 byte words; in parts of at most RUN_COLUMNS columns."""
+    def words(k):
+        w = k if wide else (k + 1) // 2
+        return w if w <= 2 else (w + 3) // 4 * 4
+
+    parts, left = divmod(columns, RUN_COLUMNS)
+    return 4 * plan["states"] * (parts * words(RUN_COLUMNS) + (words(left) if left else 0))
+
+
+def request_bytes(req, plan):
+    """Device bytes of one request of a launch on the state plan beside the
+    rows: its segment and window sums, tile tables, outputs and arguments."""
+    k, m, nw = req.shape()
+    samples = sum(len(x) for x in req.sets)
+    raw = 2 * m + 1 if req.stat == "Tajimas_D" else m + 1  # (before composites)
+    args = 8192 + 8 * samples + 128 * (raw + k) + 40 * (nw + 1)
+    if req.stat == "allele_frequency_spectrum":
+        tw = req.kwargs.get("time_windows")
+        cells = nw * (1 if tw is None else len(tw) - 1)
+        for x in req.sets:
+            cells *= len(x) + 1
+        return args + 16 * cells
+    if req.mode == "node":
+        return args + 8 * nw * plan["nodes"] * (raw + m)
+    branch = req.mode == "branch"
+    tiles = plan["events"] // 512 + 1 if branch else plan["rows"] // 256 + 1
+    sums = (2 if branch else 1) * (tiles + 2 * nw) * raw
+    return args + 8 * (sums + nw * (raw + m)) + 4 * (tiles + nw + 2)
+
+
+class _LaunchSize:
+    """Estimated device bytes of a launch, request by request; plan None:
+    chunk plans."""
+
+    def __init__(self, plan, chunks):
+        self.plan, self.chunks = plan, chunks
+        self.shared, self.own, self.wide, self.fixed = set(), 0, False, 0
+
+    def _add(self, r):
+        fixed = 0
+        # (a request that no run on the state plan takes goes to the chunks)
+        if self.plan is None or len(r.sets) > RUN_COLUMNS:
+            k, m, nw = r.shape()
+            fixed += launch_bytes(k, m, nw, self.chunks, sum(len(x) for x in r.sets))
+        if self.plan is not None:
+            fixed += request_bytes(r, self.plan)
+        # centred relatedness keeps its own columns
+        centred = r.stat == "genetic_relatedness" and r.kwargs.get("centre", True)
+        return (self.shared if centred else self.shared | r.keys,
+                self.own + (len(r.sets) if centred else 0),
+                self.wide or any(len(x) > 65535 for x in r.sets), self.fixed + fixed)
+
+    def _bytes(self, shared, own, wide, fixed):
+        if self.plan is None:
+            return fixed
+        return fixed + rows_bytes(self.plan, len(shared) + own, wide)
+
+    def add(self, r):
+        self.shared, self.own, self.wide, self.fixed = self._add(r)
+
+    def with_request(self, r):
+        return self._bytes(*self._add(r))
+
+    def bytes(self):
+        return self._bytes(self.shared, self.own, self.wide, self.fixed)
 
 
 def device_free_bytes():
@@ -128,6 +204,7 @@ class StatServer:
         self.inflight_bytes = 0
         self.deferred = 0  # launches that waited for device memory
         self.chunks = [ts.ll_tree_sequence.get_hot_plan_sizes()["chunks"] for ts in self.ts]
+        self.plans = [self._plan_sizes(ts) for ts in self.ts]
         self.launch_budget = launch_budget
         self.max_columns = max_columns
         self.max_outputs = max_outputs
@@ -139,6 +216,13 @@ class StatServer:
         self.queue = collections.deque()
         self.launches = 0
 
+    plans = None  # per tree sequence its state plan's sizes, None: chunk plans
+
+    @staticmethod
+    def _plan_sizes(ts):
+        sizes = ts.ll_tree_sequence.get_state_plan_sizes()
+        return dict(sizes, nodes=ts.num_nodes) if sizes["usable"] else None
+
     def close(self):
         if self.pool is not None:
             self.pool.shutdown(wait=True)
@@ -148,24 +232,21 @@ class StatServer:
         req.normalise(self.ts[req.ts_id])
         self.queue.append(req)
 
-    def _pack(self, reqs, chunks):
+    def _pack(self, reqs, chunks, plan=None):
         """Greedy packing of one group into launches under the column,
         output and memory limits; requests keep their arrival order."""
-        launches, cur, cols, outs, mem = [], [], set(), 0, 0
+        launches, cur, cols, outs, size = [], [], set(), 0, _LaunchSize(plan, chunks)
         for r in reqs:
-            k, m, nw = r.shape()
-            # a set's identity: its sorted samples, as bytes (hashed in C)
-            keys = {np.sort(s).tobytes() for s in r.sets}
-            b = launch_bytes(k, m, nw, chunks, sum(len(x) for x in r.sets))
-            full = cur and (len(cols | keys) > self.max_columns or outs + m > self.max_outputs
-                            or mem + b > self.launch_budget)
+            _, m, _ = r.shape()
+            full = cur and (len(cols | r.keys) > self.max_columns or outs + m > self.max_outputs
+                            or size.with_request(r) > self.launch_budget)
             if full or self.one_per_launch and cur:
                 launches.append(cur)
-                cur, cols, outs, mem = [], set(), 0, 0
+                cur, cols, outs, size = [], set(), 0, _LaunchSize(plan, chunks)
             cur.append(r)
-            cols |= keys
+            cols |= r.keys
             outs += m
-            mem += b
+            size.add(r)
         if cur:
             launches.append(cur)
         return launches
@@ -184,7 +265,7 @@ class StatServer:
                 alone.append([r])
         fused = []
         for (tid, _), reqs in groups.items():
-            fused.extend(self._pack(reqs, self.chunks[tid]))
+            fused.extend(self._pack(reqs, self.chunks[tid], self.plans and self.plans[tid]))
         if not self.multi:
             return [[launch] for launch in fused] + [[a] for a in alone]
         nj = max(1, min(njobs or self.max_inflight, len(fused)))
@@ -230,10 +311,11 @@ class StatServer:
         """Estimated device bytes of a job's launches."""
         total = 0
         for launch in job:
-            chunks = self.chunks[launch[0].ts_id]
+            tid = launch[0].ts_id
+            size = _LaunchSize(self.plans and self.plans[tid], self.chunks[tid])
             for r in launch:
-                k, m, nw = r.shape()
-                total += launch_bytes(k, m, nw, chunks, sum(len(x) for x in r.sets))
+                size.add(r)
+            total += size.bytes()
         return total
 
     def admits(self, job, inflight):
