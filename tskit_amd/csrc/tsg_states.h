@@ -28,7 +28,7 @@ struct tsg_treeseq;
 #define TSG_BRANCH_TILE 512
 #define TSG_SITE_TILE 256
 
-// Columns up to which a tile holds counts as FP64 (44 KB of LDS at 8 columns:
+// Columns up to which a tile holds counts as FP64 (48 KB of LDS at 8 columns:
 // three workgroups a CU, which is what their registers allow too): the
 // conversion is paid once an event instead of once an output.
 #define TSG_STATE_F64_COLUMNS 16
@@ -123,7 +123,7 @@ struct tsg_stateplan {
 
 // --- device side ------------------------------------------------------------
 // One output: a summary of the columns c[0..3] (set sizes or, for weights,
-// column totals n[]).  Read by scalar loads (one 96-byte record a wave).
+// column totals n[]).  Read by scalar loads (one 104-byte record a wave).
 struct TsgStateOut {
     int32_t stat;            // tsg_stat_id
     int32_t polarised;

@@ -245,8 +245,9 @@ constexpr int stride_of(int tile) {
     return tile + 2;
 }
 
-// A record of memory that no kernel of the run writes, at an address that is
-// the same for the whole wave: scalar loads.
+// A record at an address that is the same for the whole wave, written by no
+// kernel at the same time (k_state_stage, before this kernel, wrote it: the
+// scalar caches are clean at a kernel's start): scalar loads.
 template <typename R>
 __device__ __forceinline__ R uniform(const R *p) {
     typedef const __attribute__((address_space(4))) int32_t *Const;
