@@ -1141,12 +1141,13 @@ struct SeedShare {
 // share_out: this run writes its seeded counts for a later run (share_in).
 int batch_prepare(tsg_treeseq *ts, std::vector<Query *> &batch, Workspace *ws, hipStream_t s,
                   BatchRun &r, SeedShare *share_out = nullptr,
-                  const SeedShare *share_in = nullptr) {
+                  const SeedShare *share_in = nullptr, Fused *fused = nullptr) {
     int ret;
     const int Q = (int) batch.size();
     const uint32_t mode = batch[0]->mode;
-    Fused fz;
-    fuse_queries(batch, fz);
+    Fused own;
+    if (fused == nullptr) fuse_queries(batch, own);
+    Fused &fz = fused != nullptr ? *fused : own;
     std::vector<int32_t> &pair_s = fz.pair_s, &pair_c = fz.pair_c, &col_total = fz.col_total;
     std::vector<TsgOut> &outs = fz.outs;
     std::vector<TsgQuery> &qs = fz.qs;
@@ -1722,10 +1723,11 @@ bool on_state_plan(const tsg_treeseq *ts, const Workspace *ws) {
 // does not take it: no usable plan, a testing hook asks for another one, more
 // than 64 columns, tiles that do not fit in LDS, rows beyond
 // TSG_STATE_ROWS_MAX, or buffers that do not fit (the device's memory, or a
-// no-allocation run's region). many: one of several runs launched together;
-// the caller says where its results go (l.a.out).
+// no-allocation run's region). fz: the queries fused, also where the plan
+// does not take them for what they are. many: one of several runs launched
+// together; the caller says where its results go (l.a.out).
 int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws,
-                  StateRun &r, bool many = false) {
+                  StateRun &r, Fused &fz, bool many = false) {
     const tsg_stateplan &sp = ts->states;
     if (!on_state_plan(ts, ws)) return TSG_NOT_ON_STATES;
     r.ts = ts;
@@ -1738,7 +1740,7 @@ int state_prepare(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspac
     }
     const int Q = r.Q = (int) r.batch.size();
     int ret;
-    Fused fz;
+    fz = Fused();
     fuse_queries(r.batch, fz);
     const int K = fz.K;
     const bool wgt = fz.weighted;
@@ -2252,9 +2254,9 @@ int run_spectrum_states(tsg_treeseq *ts, const std::vector<std::vector<int32_t>>
 
 // Queries of one tree sequence (either mode or both) on the state plan, with
 // a leased workspace; TSG_NOT_ON_STATES where it does not take them.
-int run_states(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws) {
+int run_states(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws, Fused &fz) {
     StateRun r;
-    int ret = state_prepare(ts, queries, ws, r);
+    int ret = state_prepare(ts, queries, ws, r, fz);
     if (ret != 0) return ret;
     hipStream_t s = ws->stream;
     const bool prof = ws->profile;
@@ -2320,26 +2322,30 @@ std::vector<std::vector<Query *>> state_parts(const std::vector<Query *> &querie
 }
 
 // Queries on the state plan, in parts where they need them; rest: those that
-// do not fit alone.
+// do not fit alone; fz: the last of them fused (if it was).
 int run_states_in_parts(tsg_treeseq *ts, const std::vector<Query *> &queries, Workspace *ws,
-                        std::vector<Query *> &rest) {
-    int ret = run_states(ts, queries, ws);
+                        std::vector<Query *> &rest, Fused &fz) {
+    Fused here;
+    int ret = run_states(ts, queries, ws, here);
     if (ret != TSG_NOT_ON_STATES) return ret;
     if (queries.size() < 2 || !on_state_plan(ts, ws)) {
+        fz = queries.size() == 1 ? std::move(here) : Fused();
         rest.insert(rest.end(), queries.begin(), queries.end());
         return 0;
     }
     for (const std::vector<Query *> &part : state_parts(queries)) {
-        if ((ret = run_states_in_parts(ts, part, ws, rest))) return ret;
+        if ((ret = run_states_in_parts(ts, part, ws, rest, fz))) return ret;
     }
     return 0;
 }
 
-// A batch of queries (same tree sequence, same mode) in one chunk sweep.
-int run_sweep(tsg_treeseq *ts, std::vector<Query *> &batch, Workspace *ws) {
+// A batch of queries (same tree sequence, same mode) in one chunk sweep; fz: a
+// single one of them fused (K 0: not yet).
+int run_sweep(tsg_treeseq *ts, std::vector<Query *> &batch, Workspace *ws, Fused &fz) {
     int ret;
     BatchRun r;
-    if ((ret = batch_prepare(ts, batch, ws, ws->stream, r))) return ret;
+    Fused *const fused = batch.size() == 1 && fz.K > 0 ? &fz : nullptr;
+    if ((ret = batch_prepare(ts, batch, ws, ws->stream, r, nullptr, nullptr, fused))) return ret;
     if (ws->profile) (void) hipEventRecord(ws->ev0, r.s);
     if ((ret = batch_sweep(r))) return ret;
     if (ws->profile) (void) hipEventRecord(ws->ev1, r.s);
@@ -2367,8 +2373,9 @@ int run_batch(tsg_treeseq *ts, std::vector<Query *> &batch) {
     Workspace *ws = lease.ws;
     if (ws == nullptr) return TSG_ERR_DEVICE;
     std::vector<Query *> rest;
-    if ((ret = run_states_in_parts(ts, batch, ws, rest)) || rest.empty()) return ret;
-    return run_sweep(ts, rest, ws);
+    Fused fz;
+    if ((ret = run_states_in_parts(ts, batch, ws, rest, fz)) || rest.empty()) return ret;
+    return run_sweep(ts, rest, ws, fz);
 }
 
 // While a batch is being filled, the validated query is handed to it
@@ -4442,7 +4449,9 @@ int run_fused_modes(tsg_batch *b) {
         }
         Lease lease(b->ts);
         if (lease.ws == nullptr) return TSG_ERR_DEVICE;
-        if ((ret = run_states_in_parts(b->ts, all, lease.ws, rest)) || rest.empty()) return ret;
+        Fused fz;
+        ret = run_states_in_parts(b->ts, all, lease.ws, rest, fz);
+        if (ret != 0 || rest.empty()) return ret;
         for (uint32_t mode : {TSG_STAT_BRANCH, TSG_STAT_SITE}) {
             std::vector<Query *> group;
             for (Query *q : rest) {
@@ -4450,7 +4459,7 @@ int run_fused_modes(tsg_batch *b) {
             }
             if (!group.empty()) groups.push_back(std::move(group));
         }
-        if (groups.size() == 1) return run_sweep(b->ts, groups[0], lease.ws);
+        if (groups.size() == 1) return run_sweep(b->ts, groups[0], lease.ws, fz);
     }
     std::vector<std::unique_ptr<Lease>> leases;
     std::vector<BatchRun> runs;
@@ -4529,7 +4538,8 @@ __attribute__((visibility("hidden"))) int tsg_batch_run_fixed(tsg_batch *b, void
         }
         if (group.empty()) continue;
         w.fixed_used = 0;
-        if ((ret = run_states(ts, group, &w)) != TSG_NOT_ON_STATES) {
+        Fused fz;
+        if ((ret = run_states(ts, group, &w, fz)) != TSG_NOT_ON_STATES) {
             if (ret != 0) break;
             continue;
         }
@@ -4589,7 +4599,8 @@ int run_multi_states(tsg_batch **bs, uint64_t n, std::vector<std::unique_ptr<Lea
             for (size_t p; (p = next.fetch_add(1)) < to;) {
                 Prep &t = preps[p];
                 try {
-                    t.ret = state_prepare(bs[t.i]->ts, t.queries, t.ws, t.run, true);
+                    Fused fz;
+                    t.ret = state_prepare(bs[t.i]->ts, t.queries, t.ws, t.run, fz, true);
                 } catch (const std::bad_alloc &) {
                     t.ret = TSG_ERR_NO_MEMORY;
                 }
