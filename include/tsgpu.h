@@ -366,8 +366,10 @@ int tsg_batch_run_multi(tsg_batch_t **batches, uint64_t n);
  * (node mode: TSG_ERR_UNSUPPORTED_STAT_MODE); a batch needing more than the
  * 64 MiB returns TSG_ERR_SCRATCH_TOO_SMALL (-30006) with no result written.
  * Modes run one after the other on the null stream; results equal
- * tsg_batch_run's.  Calls on one GPU share its array: calls that overlap
- * on one GPU race, and the caller serialises them. */
+ * tsg_batch_run's (bit for bit where a mode's queries have at most 64
+ * distinct sets and the array holds their counts, else to rounding).  Calls
+ * on one GPU share its array: calls that overlap on one GPU race, and the
+ * caller serialises them. */
 int tsg_batch_run_noalloc(tsg_batch_t *batch);
 int tsg_batch_diversity(tsg_batch_t *batch, uint64_t num_sample_sets,
     const uint64_t *sample_set_sizes, const int32_t *sample_sets, uint64_t num_windows,
